@@ -6,21 +6,25 @@
 //   * PEC DOFs are eliminated implicitly: the operator is
 //     y = mask.(K (mask.x)) + (1 - mask).x, so x_PEC = 0 exactly and no
 //     reduced matrix is ever formed (solver.py:430-435 builds one per call);
-//   * SpMV is HBM-bound: 16-lane sub-waves per CSR row, coalesced loads of
-//     columns and values, complex128 or complex64 values;
+//   * the solver's own vectors hold the two modes of an entity side by side and
+//     its matrix 2x2 blocks in a real and an imaginary plane, the latter read
+//     only where there are losses ("packed solver layout" below);
 //   * Gram-Schmidt is classical, as a tiled multi-dot and a fused multi-AXPY
 //     + norm, so each Arnoldi step streams the basis twice instead of j
-//     times; a second pass runs only when the first cancelled 99% of the
-//     vector's squared norm (loss-of-orthogonality test on the norms);
+//     times; the multi-dot also brings the basis' Gram matrix up, which takes
+//     the place of a second pass (k_gram_correct);
 //   * the preconditioner is the inverse of the 2x2 blocks coupling the two
-//     modes of each edge / face;
+//     modes of each edge / face, with the gradient correction and the GMRES
+//     polynomial when set;
 //   * precision 32 runs GMRES in complex64 inside FP64 iterative refinement:
-//     the residual b - K x is always formed in complex128.
+//     the residual b - K x is always formed in complex128, and the cycles of
+//     one solve share their Krylov spaces (gmres_cycle).
 
 #include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <limits>
 #include <string>
 #include <vector>
 
@@ -28,23 +32,6 @@
 #include "emg_common.h"
 
 using emg::cplx;
-
-struct cplxf {
-    float re, im;
-    __host__ __device__ cplxf() : re(0), im(0) {}
-    __host__ __device__ cplxf(float r, float i = 0) : re(r), im(i) {}
-};
-
-template <typename T>
-struct Cx;
-template <>
-struct Cx<double> {
-    using C = cplx;
-};
-template <>
-struct Cx<float> {
-    using C = cplxf;
-};
 
 template <typename R>
 struct cx {
@@ -76,44 +63,55 @@ __device__ __forceinline__ void st(R *p, int64_t i, cx<R> v) {
     }
 }
 
+// Sum over groups of L = 4 .. 64 consecutive lanes, left in every lane: the steps within 16 lanes are
+// data-parallel-primitive adds (quad permutes, half-row and row mirrors), a few cycles each where a
+// shuffle through LDS takes over a hundred; the pairs added are those of the xor butterfly.
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+static constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140, DPP_ROR8 = 0x128;
+template <int L, typename T>
+__device__ __forceinline__ T lane_sum(T v) {
+    static_assert(L == 4 || L == 8 || L == 16 || L == 32 || L == 64, "lane_sum: group size");
+    v += dpp_mov<DPP_XOR1>(v);
+    v += dpp_mov<DPP_XOR2>(v);
+    if constexpr (L >= 8) v += dpp_mov<DPP_HALF_MIRROR>(v);
+    if constexpr (L >= 16) v += dpp_mov<DPP_MIRROR>(v);
+    if constexpr (L >= 32) v += __shfl_xor(v, 16, 64);
+    if constexpr (L >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
 static constexpr int SUB = 16;  // lanes per CSR row
 // (SpMV rows stay in dispatch order: giving each XCD a contiguous share of the
 // rows fetched a third fewer bytes but ran 30 % slower.)
 
-// y = mask.(A (mask.x)) + (1-mask).x   (mask == nullptr: plain y = A x)
-// If `b` is given, y = b - (that).  L lanes share one CSR row.  MC: apply the
-// column mask per entry (false when the masked columns are already zero in
-// vals, as in the solver's complex64 copy).
-template <typename R, int L, bool MC>
+// y = mask.(A (mask.x)) + (1-mask).x   (mask == nullptr: plain y = A x).  L lanes share one CSR row.
+template <int L>
 __global__ void __launch_bounds__(256) k_spmv(int64_t n, const int32_t *__restrict__ rowptr, const int32_t *__restrict__ cols,
-                                              const R *__restrict__ vals, const uint8_t *__restrict__ mask,
-                                              const R *__restrict__ x, const R *__restrict__ b, R *__restrict__ y) {
+                                              const double *__restrict__ vals, const uint8_t *__restrict__ mask,
+                                              const double *__restrict__ x, double *__restrict__ y) {
     const int64_t row = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / L;
     const int lane = threadIdx.x % L;
     if (row >= n) return;
     const bool keep = mask == nullptr || mask[row];
-    cx<R> acc;
+    cx<double> acc;
     if (keep) {
         const int32_t p0 = rowptr[row], p1 = rowptr[row + 1];
         for (int32_t p = p0 + lane; p < p1; p += L) {
             const int32_t c = cols[p];
-            if (MC && mask != nullptr && !mask[c]) continue;
+            if (mask != nullptr && !mask[c]) continue;
             acc = cadd(acc, cmul(ld(vals, p), ld(x, c)));
         }
     }
-#pragma unroll
-    for (int off = L / 2; off > 0; off >>= 1) {
-        acc.re += __shfl_xor(acc.re, off, L);
-        acc.im += __shfl_xor(acc.im, off, L);
-    }
-    if (lane == 0) {
-        cx<R> v = keep ? acc : ld(x, row);
-        if (b != nullptr) {
-            const cx<R> bb = ld(b, row);
-            v = cx<R>(bb.re - v.re, bb.im - v.im);
-        }
-        st(y, row, v);
-    }
+    acc = cx<double>(lane_sum<L>(acc.re), lane_sum<L>(acc.im));
+    if (lane == 0) st(y, row, keep ? acc : ld(x, row));
 }
 
 // Lanes per CSR row for the SpMV: EMG_SPMV_LANES (4, 8, 16 or 32) if set, else 16.
@@ -127,27 +125,16 @@ static int spmv_lanes() {
     return lanes;
 }
 
-template <typename R, bool MC>
-static void launch_spmv_l(hipStream_t st, int64_t n, const int32_t *rowptr, const int32_t *cols, const R *vals,
-                          const uint8_t *mask, const R *x, const R *b, R *y) {
+static void launch_spmv(hipStream_t st, int64_t n, const int32_t *rowptr, const int32_t *cols, const double *vals,
+                        const uint8_t *mask, const double *x, double *y) {
     const int L = spmv_lanes();
     const unsigned grid = (unsigned)((n * L + 255) / 256);
     switch (L) {
-        case 4: k_spmv<R, 4, MC><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, b, y); break;
-        case 8: k_spmv<R, 8, MC><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, b, y); break;
-        case 32: k_spmv<R, 32, MC><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, b, y); break;
-        default: k_spmv<R, 16, MC><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, b, y); break;
+        case 4: k_spmv<4><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, y); break;
+        case 8: k_spmv<8><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, y); break;
+        case 32: k_spmv<32><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, y); break;
+        default: k_spmv<16><<<grid, 256, 0, st>>>(n, rowptr, cols, vals, mask, x, y); break;
     }
-}
-
-// mask_cols false: vals already holds zeros in the masked columns.
-template <typename R>
-static void launch_spmv(hipStream_t st, int64_t n, const int32_t *rowptr, const int32_t *cols, const R *vals,
-                        const uint8_t *mask, const R *x, const R *b, R *y, bool mask_cols = true) {
-    if (mask_cols)
-        launch_spmv_l<R, true>(st, n, rowptr, cols, vals, mask, x, b, y);
-    else
-        launch_spmv_l<R, false>(st, n, rowptr, cols, vals, mask, x, b, y);
 }
 
 // SpMV of a matrix on an entity pattern (emg_pattern_csr): DOF = mode * ne +
@@ -156,16 +143,16 @@ static void launch_spmv(hipStream_t st, int64_t n, const int32_t *rowptr, const 
 // r_m + deg + j, r_0 = rowptr[e], r_1 = r_0 + half (half = nnz / 2).  One
 // group of L lanes computes both rows of entity e: each column index and each
 // pair of x gathers serves four matrix entries.  Same masking as k_spmv.
-template <typename R, int L, bool MC>
+template <int L>
 __global__ void __launch_bounds__(256) k_spmv_blk(int64_t ne, int64_t half, const int32_t *__restrict__ rowptr,
-                                                  const int32_t *__restrict__ cols, const R *__restrict__ vals,
-                                                  const uint8_t *__restrict__ mask, const R *__restrict__ x,
-                                                  const R *__restrict__ b, R *__restrict__ y) {
+                                                  const int32_t *__restrict__ cols, const double *__restrict__ vals,
+                                                  const uint8_t *__restrict__ mask, const double *__restrict__ x,
+                                                  const double *__restrict__ b, double *__restrict__ y) {
     const int64_t e = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / L;
     const int lane = threadIdx.x % L;
     if (e >= ne) return;
     const bool k0 = mask == nullptr || mask[e], k1 = mask == nullptr || mask[ne + e];
-    cx<R> a0, a1;
+    cx<double> a0, a1;
     if (k0 || k1) {
         const int32_t r0 = rowptr[e];
         // a row beyond the first half is not an entity pattern: read nothing past nnz
@@ -173,29 +160,24 @@ __global__ void __launch_bounds__(256) k_spmv_blk(int64_t ne, int64_t half, cons
         for (int32_t j = lane; j < deg; j += L) {
             const int32_t c = cols[r0 + j];
             if (c < 0 || c >= ne) continue;   // not an entity pattern: no out-of-range reads
-            cx<R> x0 = ld(x, c), x1 = ld(x, ne + c);
-            if (MC && mask != nullptr) {
-                if (!mask[c]) x0 = cx<R>();
-                if (!mask[ne + c]) x1 = cx<R>();
+            cx<double> x0 = ld(x, c), x1 = ld(x, ne + c);
+            if (mask != nullptr) {
+                if (!mask[c]) x0 = cx<double>();
+                if (!mask[ne + c]) x1 = cx<double>();
             }
             const int64_t p = r0 + j;
             a0 = cadd(a0, cadd(cmul(ld(vals, p), x0), cmul(ld(vals, p + deg), x1)));
             a1 = cadd(a1, cadd(cmul(ld(vals, half + p), x0), cmul(ld(vals, half + p + deg), x1)));
         }
     }
-#pragma unroll
-    for (int off = L / 2; off > 0; off >>= 1) {
-        a0.re += __shfl_xor(a0.re, off, L);
-        a0.im += __shfl_xor(a0.im, off, L);
-        a1.re += __shfl_xor(a1.re, off, L);
-        a1.im += __shfl_xor(a1.im, off, L);
-    }
+    a0 = cx<double>(lane_sum<L>(a0.re), lane_sum<L>(a0.im));
+    a1 = cx<double>(lane_sum<L>(a1.re), lane_sum<L>(a1.im));
     if (lane == 0) {
-        cx<R> v0 = k0 ? a0 : ld(x, e), v1 = k1 ? a1 : ld(x, ne + e);
+        cx<double> v0 = k0 ? a0 : ld(x, e), v1 = k1 ? a1 : ld(x, ne + e);
         if (b != nullptr) {
-            const cx<R> b0 = ld(b, e), b1 = ld(b, ne + e);
-            v0 = cx<R>(b0.re - v0.re, b0.im - v0.im);
-            v1 = cx<R>(b1.re - v1.re, b1.im - v1.im);
+            const cx<double> b0 = ld(b, e), b1 = ld(b, ne + e);
+            v0 = cx<double>(b0.re - v0.re, b0.im - v0.im);
+            v1 = cx<double>(b1.re - v1.re, b1.im - v1.im);
         }
         st(y, e, v0);
         st(y, ne + e, v1);
@@ -206,132 +188,324 @@ __global__ void __launch_bounds__(256) k_spmv_blk(int64_t ne, int64_t half, cons
 // emg_spmv_blocked, or EMG_SPMV_BLK_LANES set): EMG_SPMV_BLK_LANES (4, 8, 16 or
 // 32) if set, else 16.  Solvers tune their own (tune_spmv).
 static int spmv_blk_lanes() {
-    static int lanes = 0;
-    if (lanes == 0) {
-        const char *e = getenv("EMG_SPMV_BLK_LANES");
-        const int v = e ? atoi(e) : 16;
-        lanes = (v == 4 || v == 8 || v == 16 || v == 32) ? v : 16;
-    }
-    return lanes;
+    const char *e = getenv("EMG_SPMV_BLK_LANES");
+    const int v = e ? atoi(e) : 16;
+    return (v == 4 || v == 8 || v == 16 || v == 32) ? v : 16;
 }
 
-template <typename R>
 static void launch_spmv_blk(hipStream_t st, int64_t n, int64_t nnz, const int32_t *rowptr, const int32_t *cols,
-                            const R *vals, const uint8_t *mask, const R *x, const R *b, R *y, int L,
-                            bool mask_cols = true) {
+                            const double *vals, const uint8_t *mask, const double *x, const double *b, double *y, int L) {
     const int64_t ne = n / 2, half = nnz / 2;
     if (L != 4 && L != 8 && L != 32) L = 16;
     const unsigned grid = (unsigned)((ne * L + 255) / 256);
-#define EMG_BLK(LL, MCV) k_spmv_blk<R, LL, MCV><<<grid, 256, 0, st>>>(ne, half, rowptr, cols, vals, mask, x, b, y)
-    if (mask_cols) {
-        if (L == 4) EMG_BLK(4, true); else if (L == 8) EMG_BLK(8, true); else if (L == 32) EMG_BLK(32, true);
-        else EMG_BLK(16, true);
-    } else {
-        if (L == 4) EMG_BLK(4, false); else if (L == 8) EMG_BLK(8, false); else if (L == 32) EMG_BLK(32, false);
-        else EMG_BLK(16, false);
-    }
-#undef EMG_BLK
+    if (L == 4) k_spmv_blk<4><<<grid, 256, 0, st>>>(ne, half, rowptr, cols, vals, mask, x, b, y);
+    else if (L == 8) k_spmv_blk<8><<<grid, 256, 0, st>>>(ne, half, rowptr, cols, vals, mask, x, b, y);
+    else if (L == 32) k_spmv_blk<32><<<grid, 256, 0, st>>>(ne, half, rowptr, cols, vals, mask, x, b, y);
+    else k_spmv_blk<16><<<grid, 256, 0, st>>>(ne, half, rowptr, cols, vals, mask, x, b, y);
 }
 
 // ---------------------------------------------------------------- BLAS-1
 static constexpr int RB = 256;   // reduction block
 static constexpr int DT = 8;     // dot products per tile
 
-// partial[tile][blk][k] = sum over the block's elements of conj(V_{t*DT+k}) . w
+// Two consecutive complex values: in the solver's own vectors the two modes of an
+// entity (DOFs e and ne + e side by side), one 16-byte access in complex64.
 template <typename R>
-__global__ void __launch_bounds__(RB) k_mdot(int64_t n, int nv, const R *__restrict__ V, int64_t ldv,
-                                             const R *__restrict__ w, double *__restrict__ partial,
-                                             const double *__restrict__ run) {
-    if (run != nullptr && run[0] == 0.0) return;   // device-side skip (second Gram-Schmidt pass not needed)
-    const int tile = blockIdx.y;
-    const int i0 = tile * DT;
-    double ar[DT], ai[DT];
-#pragma unroll
-    for (int k = 0; k < DT; k++) { ar[k] = 0; ai[k] = 0; }
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n; e += (int64_t)gridDim.x * RB) {
-        const cx<R> wv = ld(w, e);
-#pragma unroll
-        for (int k = 0; k < DT; k++) {
-            if (i0 + k < nv) {
-                const cx<R> v = ld(V + (int64_t)(i0 + k) * ldv * 2, e);
-                ar[k] += (double)v.re * wv.re + (double)v.im * wv.im;
-                ai[k] += (double)v.re * wv.im - (double)v.im * wv.re;
-            }
-        }
+struct cx2 {
+    R ar, ai, br, bi;
+};
+template <typename R>
+__device__ __forceinline__ cx2<R> ld2(const R *p, int64_t i) {
+    if constexpr (sizeof(R) == 8) {
+        const double2 u = reinterpret_cast<const double2 *>(p)[2 * i], v = reinterpret_cast<const double2 *>(p)[2 * i + 1];
+        return cx2<R>{u.x, u.y, v.x, v.y};
+    } else {
+        const float4 u = reinterpret_cast<const float4 *>(p)[i];
+        return cx2<R>{u.x, u.y, u.z, u.w};
     }
-    __shared__ double sr[DT][RB / 64], si[DT][RB / 64];
-#pragma unroll
-    for (int k = 0; k < DT; k++) {
-        double r = ar[k], i = ai[k];
-        for (int off = 32; off > 0; off >>= 1) {
-            r += __shfl_xor(r, off, 64);
-            i += __shfl_xor(i, off, 64);
-        }
-        if ((threadIdx.x & 63) == 0) { sr[k][threadIdx.x >> 6] = r; si[k][threadIdx.x >> 6] = i; }
-    }
-    __syncthreads();
-    if (threadIdx.x < DT) {
-        double r = 0, i = 0;
-        for (int q = 0; q < RB / 64; q++) { r += sr[threadIdx.x][q]; i += si[threadIdx.x][q]; }
-        const int64_t o = ((int64_t)tile * gridDim.x + blockIdx.x) * DT + threadIdx.x;
-        partial[2 * o] = r;
-        partial[2 * o + 1] = i;
+}
+template <typename R>
+__device__ __forceinline__ void st2(R *p, int64_t i, cx2<R> v) {
+    if constexpr (sizeof(R) == 8) {
+        reinterpret_cast<double2 *>(p)[2 * i] = make_double2(v.ar, v.ai);
+        reinterpret_cast<double2 *>(p)[2 * i + 1] = make_double2(v.br, v.bi);
+    } else {
+        reinterpret_cast<float4 *>(p)[i] = make_float4(v.ar, v.ai, v.br, v.bi);
     }
 }
 
-// h[i] (+)= sum over blocks of the partials (complex, i < nv); one block per value
-__global__ void k_mdot_finish(int nv, int nblk, const double *__restrict__ partial, double *__restrict__ h, int accumulate,
-                              const double *__restrict__ run) {
+__device__ __forceinline__ double block_sum(double v, double *sh) {
+    v = lane_sum<64>(v);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0.0;
+    for (int q = 0; q < (int)(blockDim.x >> 6); q++) t += sh[q];
+    return t;
+}
+
+// partial[r][tile][blk][k] = sum over the block's elements of conj(V_{t*DT+k}) . w_r for RHS = 1 or 2
+// vectors w_r, two complex values per lane and vector (an odd n leaves its last value to the first
+// lane).  A tile past the last vector reads that one again and its sums are not used: a test per vector
+// instead keeps the eight loads from being in flight together.  Bound by the bytes of V, which two
+// right-hand sides share.
+template <typename R, int RHS>
+__global__ void __launch_bounds__(RB) k_mdot(int64_t n, int nv, const R *__restrict__ V, int64_t ldv,
+                                             const R *__restrict__ w, const R *__restrict__ w2,
+                                             double *__restrict__ partial) {
+    constexpr int NS = 2 * DT * RHS;   // sums: real parts, imaginary parts, of each right-hand side
+    static_assert(NS == 16 || NS == 32, "the wavefront reduction handles 16 or 32 sums");
+    __shared__ double sv[NS][RB / 64];
+    const int tile = blockIdx.y;
+    const int i0 = tile * DT;
+    double v[NS];
+#pragma unroll
+    for (int k = 0; k < NS; k++) v[k] = 0;
+    auto add = [&](double *a, const cx2<R> &x, const cx2<R> &y) {
+        a[0] += (double)x.ar * y.ar + (double)x.ai * y.ai + (double)x.br * y.br + (double)x.bi * y.bi;
+        a[DT] += (double)x.ar * y.ai - (double)x.ai * y.ar + (double)x.br * y.bi - (double)x.bi * y.br;
+    };
+    const int64_t n2 = n >> 1;
+    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n2; e += (int64_t)gridDim.x * RB) {
+        const cx2<R> wv = ld2(w, e);
+        cx2<R> wv2{};
+        if constexpr (RHS == 2) wv2 = ld2(w2, e);
+        cx2<R> x[DT];
+#pragma unroll
+        for (int k = 0; k < DT; k++) x[k] = ld2(V + (int64_t)min(i0 + k, nv - 1) * ldv * 2, e);
+#pragma unroll
+        for (int k = 0; k < DT; k++) {
+            add(v + k, x[k], wv);
+            if constexpr (RHS == 2) add(v + 2 * DT + k, x[k], wv2);
+        }
+    }
+    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+        auto last = [&](const R *a) {
+            const cx<R> u = ld(a, n - 1);
+            return cx2<R>{u.re, u.im, R(0), R(0)};
+        };
+        const cx2<R> wv = last(w);
+#pragma unroll
+        for (int k = 0; k < DT; k++) {
+            const cx2<R> x = last(V + (int64_t)min(i0 + k, nv - 1) * ldv * 2);
+            add(v + k, x, wv);
+            if constexpr (RHS == 2) add(v + 2 * DT + k, x, last(w2));
+        }
+    }
+    // the sums over the wavefront: each step hands half of the values to the partner lane and adds the
+    // other half, NS - 1 exchanges and a last add or two instead of the 6 NS shuffles of NS butterflies
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int half = NS / 2, bit = 32; half >= 1; half >>= 1, bit >>= 1) {
+#pragma unroll
+        for (int k = 0; k < half; k++) {
+            const double give = (lane & bit) ? v[k] : v[k + half], keep = (lane & bit) ? v[k + half] : v[k];
+            v[k] = keep + (bit == 8 ? dpp_mov<DPP_ROR8>(give) : bit == 2 ? dpp_mov<DPP_XOR2>(give) : __shfl_xor(give, bit, 64));
+        }
+    }
+    // value i is with lanes (64 / NS) i ...: the highest bit of the lane is the highest of i, and so on
+    if constexpr (NS == 16) v[0] += dpp_mov<DPP_XOR2>(v[0]);
+    v[0] += dpp_mov<DPP_XOR1>(v[0]);
+    if (lane % (64 / NS) == 0) sv[lane / (64 / NS)][threadIdx.x >> 6] = v[0];
+    __syncthreads();
+    if (threadIdx.x < NS) {
+        double t = 0;
+        for (int q = 0; q < RB / 64; q++) t += sv[threadIdx.x][q];
+        const int r = threadIdx.x / (2 * DT), c = (threadIdx.x / DT) & 1, k = threadIdx.x % DT;
+        const int64_t o = (((int64_t)r * gridDim.y + tile) * gridDim.x + blockIdx.x) * DT + k;
+        partial[2 * o + c] = t;
+    }
+}
+
+// h[i] = sc_i * sum over blocks of the partials (complex, i < nv); one block per value.
+// gridDim.y = 2 (k_mdot<R, 2> with the last basis vector as second right-hand side): the second sums
+// are that vector's column of the basis' Gram matrix, of which E (row length ld) keeps the deviation
+// from the identity.
+__global__ void k_mdot_finish(int nv, int nblk, const double *__restrict__ partial, const double *__restrict__ sc,
+                              double *__restrict__ h, double *__restrict__ E, int ld) {
     const int i = blockIdx.x;
     if (i >= nv) return;
-    if (run != nullptr && run[0] == 0.0) {
-        if (threadIdx.x == 0 && !accumulate) { h[2 * i] = 0.0; h[2 * i + 1] = 0.0; }
-        return;
-    }
-    const int tile = i / DT, k = i % DT;
+    const int tile = i / DT, k = i % DT, ntile = (nv + DT - 1) / DT;
     double r = 0, im = 0;
     for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-        const int64_t o = ((int64_t)tile * nblk + b) * DT + k;
+        const int64_t o = (((int64_t)blockIdx.y * ntile + tile) * nblk + b) * DT + k;
         r += partial[2 * o];
         im += partial[2 * o + 1];
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        r += __shfl_xor(r, off, 64);
-        im += __shfl_xor(im, off, 64);
-    }
+    r = lane_sum<64>(r);
+    im = lane_sum<64>(im);
     __shared__ double s[2][4];
     if ((threadIdx.x & 63) == 0) { s[0][threadIdx.x >> 6] = r; s[1][threadIdx.x >> 6] = im; }
     __syncthreads();
     if (threadIdx.x == 0) {
         r = 0; im = 0;
         for (int q = 0; q < (int)(blockDim.x >> 6); q++) { r += s[0][q]; im += s[1][q]; }
-        if (accumulate) { h[2 * i] += r; h[2 * i + 1] += im; }
-        else { h[2 * i] = r; h[2 * i + 1] = im; }
+        const double c = sc != nullptr ? sc[i] : 1.0;
+        if (blockIdx.y == 0) {
+            h[2 * i] = c * r;
+            h[2 * i + 1] = c * im;
+        } else {
+            const int l = nv - 1;
+            const double f = i == l ? 0.0 : c * sc[l];   // vectors are normalised: the diagonal deviates by rounding only
+            E[2 * ((int64_t)i * ld + l)] = f * r;
+            E[2 * ((int64_t)i * ld + l) + 1] = f * im;
+            E[2 * ((int64_t)l * ld + i)] = f * r;
+            E[2 * ((int64_t)l * ld + i) + 1] = -f * im;
+        }
     }
 }
 
-// w -= sum_i h_i V_i ; partial norm^2 of the result per block
-template <typename R>
-__global__ void __launch_bounds__(RB) k_maxpy_norm(int64_t n, int nv, const R *__restrict__ V, int64_t ldv,
-                                                   const double *__restrict__ h, R *__restrict__ w,
-                                                   double *__restrict__ partial, const double *__restrict__ run) {
-    if (run != nullptr && run[0] == 0.0) return;
+// The spaces kept from earlier refinement cycles of a solve (see gmres_cycle): cycle c holds the
+// basis vectors start[c] .. start[c + 1] - 1, of which K M maps all but the last into the range
+// C_c = V Q_c; qp_i holds the coefficients of the one direction of their span outside C_c.
+static constexpr int KEEP_MAX = 32;
+struct kept_dev {
+    int32_t t0;                    // first basis vector of the running cycle
+    int32_t ncyc;                  // kept cycles
+    int32_t start[KEEP_MAX + 1];
+};
+// h (LDS, coefficients against all basis vectors) less the components along the kept cycles' outside
+// directions: what is left projects on the ranges only.  One wavefront per cycle.
+__device__ __forceinline__ void project_kept(double *h, const kept_dev *kept, const double *qp) {
+    const int nc = kept->ncyc;
+    for (int c = threadIdx.x >> 6; c < nc; c += RB / 64) {
+        const int a = kept->start[c], b = kept->start[c + 1];
+        double sr = 0.0, si = 0.0;
+        for (int i = a + (threadIdx.x & 63); i < b; i += 64) {
+            sr += qp[2 * i] * h[2 * i] + qp[2 * i + 1] * h[2 * i + 1];
+            si += qp[2 * i] * h[2 * i + 1] - qp[2 * i + 1] * h[2 * i];
+        }
+        sr = lane_sum<64>(sr);
+        si = lane_sum<64>(si);
+        for (int i = a + (threadIdx.x & 63); i < b; i += 64) {
+            h[2 * i] -= qp[2 * i] * sr - qp[2 * i + 1] * si;
+            h[2 * i + 1] -= qp[2 * i] * si + qp[2 * i + 1] * sr;
+        }
+    }
+    __syncthreads();
+}
+
+// c = h~ - E h~ with h~ the coefficients h projected (project_kept): the coefficients that take the basis'
+// part out of a vector although the basis is orthonormal only to complex64's rounding.  V^H (w - V c)
+// is E^2 h~ where plain Gram-Schmidt leaves E h~, so the deviations E of later vectors do not
+// grow with the earlier ones, and the second pass over the basis that kept them down is not needed: this
+// reads nv^2 numbers.  (A second pass only after 99 % of the squared norm had cancelled, as
+// before, let E grow until kept spaces were useless: mixed media, 3,072 tets, degree 1: 706 steps to 1e-9
+// with it, 232 with a pass in every step.)  16 rows per block.
+__global__ void __launch_bounds__(RB) k_gram_correct(int nv, const double *__restrict__ h, const double *__restrict__ E,
+                                                     int lde, const kept_dev *__restrict__ kept,
+                                                     const double *__restrict__ qp, double *__restrict__ c) {
     __shared__ double hs[2 * 512];
     for (int i = threadIdx.x; i < 2 * nv; i += RB) hs[i] = h[i];
     __syncthreads();
+    project_kept(hs, kept, qp);
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int i = blockIdx.x * 16 + (threadIdx.x >> 6) * 4 + q;
+        double r = 0.0, im = 0.0;
+        if (i < nv)
+            for (int j = lane; j < nv; j += 64) {
+                const cx<double> e = ld(E, (int64_t)i * lde + j), x(hs[2 * j], hs[2 * j + 1]);
+                r += e.re * x.re - e.im * x.im;
+                im += e.re * x.im + e.im * x.re;
+            }
+        r = lane_sum<64>(r);
+        im = lane_sum<64>(im);
+        if (lane == 0 && i < nv) {
+            c[2 * i] = hs[2 * i] - r;
+            c[2 * i + 1] = hs[2 * i + 1] - im;
+        }
+    }
+}
+
+// w -= sum_i h_i (sc_i V_i) ; partial norm^2 of the result per block.  Two complex values per
+// lane; the vectors are read four at a time so that four loads are in flight.  S = 4 (maxpy_split:
+// problems too small to fill the GPU): four lanes share an element, each takes a quarter of the
+// vectors, so the chain of loads is a quarter as long and four times the lanes are busy (7.5 us
+// with S = 1 at 19,664 DOFs and 50 vectors).  With kept spaces (kept not NULL) h is first projected
+// (project_kept); block 0 leaves the coefficients used in hout (NULL: nowhere).
+template <typename R, int S>
+__global__ void __launch_bounds__(RB) k_maxpy_norm(int64_t n, int nv, const R *__restrict__ V, int64_t ldv,
+                                                   const double *__restrict__ h, const double *__restrict__ sc,
+                                                   R *__restrict__ w, double *__restrict__ partial,
+                                                   const kept_dev *__restrict__ kept, const double *__restrict__ qp,
+                                                   double *__restrict__ hout) {
+    __shared__ double hs[2 * 512];
+    for (int i = threadIdx.x; i < 2 * nv; i += RB) hs[i] = h[i];
+    __syncthreads();
+    if (kept != nullptr) project_kept(hs, kept, qp);
+    if (hout != nullptr && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < 2 * nv; i += RB) hout[i] = hs[i];
+    if (sc != nullptr) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < 2 * nv; i += RB) hs[i] *= sc[i >> 1];
+        __syncthreads();
+    }
     double nrm = 0;
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n; e += (int64_t)gridDim.x * RB) {
-        cx<R> wv = ld(w, e);
+    const int64_t n2 = n >> 1;
+    constexpr int EB = RB / S;                       // elements of a block's pass
+    const int part = threadIdx.x / EB, el = threadIdx.x % EB;
+    const int per = (nv + S - 1) / S, i0 = part * per, i1 = min(nv, i0 + per);
+    __shared__ double red[S > 1 ? (S - 1) * EB * 4 : 1];
+    // every lane makes the same number of passes (the barriers below need them all)
+    const int64_t passes = (n2 + (int64_t)gridDim.x * EB - 1) / ((int64_t)gridDim.x * EB);
+    for (int64_t ps = 0; ps < passes; ps++) {
+        const int64_t e = (ps * gridDim.x + blockIdx.x) * EB + el;
+        const bool in = e < n2;
+        double ar = 0, ai = 0, br = 0, bi = 0;       // sum of this lane's vectors
+        if (in) {
+            auto add = [&](int i, const cx2<R> &v) {
+                const double hr = hs[2 * i], hi = hs[2 * i + 1];
+                ar += hr * v.ar - hi * v.ai;
+                ai += hr * v.ai + hi * v.ar;
+                br += hr * v.br - hi * v.bi;
+                bi += hr * v.bi + hi * v.br;
+            };
+            int i = i0;
+            for (; i + 4 <= i1; i += 4) {
+                cx2<R> v[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[q] = ld2(V + (int64_t)(i + q) * ldv * 2, e);
+#pragma unroll
+                for (int q = 0; q < 4; q++) add(i + q, v[q]);
+            }
+            for (; i < i1; i++) add(i, ld2(V + (int64_t)i * ldv * 2, e));
+        }
+        if constexpr (S > 1) {
+            if (part > 0) {
+                double *r = red + ((part - 1) * 4) * EB + el;
+                r[0] = ar; r[EB] = ai; r[2 * EB] = br; r[3 * EB] = bi;
+            }
+            __syncthreads();
+            if (part == 0) {
+#pragma unroll
+                for (int q = 0; q < S - 1; q++) {
+                    const double *r = red + (q * 4) * EB + el;
+                    ar += r[0]; ai += r[EB]; br += r[2 * EB]; bi += r[3 * EB];
+                }
+            }
+            __syncthreads();
+        }
+        if (in && part == 0) {
+            const cx2<R> wv = ld2(w, e);
+            const cx2<R> o{(R)(wv.ar - ar), (R)(wv.ai - ai), (R)(wv.br - br), (R)(wv.bi - bi)};
+            st2(w, e, o);
+            nrm += (double)o.ar * o.ar + (double)o.ai * o.ai + (double)o.br * o.br + (double)o.bi * o.bi;
+        }
+    }
+    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+        const cx<R> wv = ld(w, n - 1);
         double wr = wv.re, wi = wv.im;
         for (int i = 0; i < nv; i++) {
-            const cx<R> v = ld(V + (int64_t)i * ldv * 2, e);
+            const cx<R> v = ld(V + (int64_t)i * ldv * 2, n - 1);
             wr -= hs[2 * i] * v.re - hs[2 * i + 1] * v.im;
             wi -= hs[2 * i] * v.im + hs[2 * i + 1] * v.re;
         }
-        st(w, e, cx<R>((R)wr, (R)wi));
+        st(w, n - 1, cx<R>((R)wr, (R)wi));
         nrm += (double)(R)wr * (double)(R)wr + (double)(R)wi * (double)(R)wi;
     }
-    for (int off = 32; off > 0; off >>= 1) nrm += __shfl_xor(nrm, off, 64);
+    nrm = lane_sum<64>(nrm);
     __shared__ double s[RB / 64];
     if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = nrm;
     __syncthreads();
@@ -340,6 +514,20 @@ __global__ void __launch_bounds__(RB) k_maxpy_norm(int64_t n, int nv, const R *_
         for (int q = 0; q < RB / 64; q++) t += s[q];
         partial[blockIdx.x] = t;
     }
+}
+
+// Lanes per element of k_maxpy_norm: four on problems of a few ten thousand DOFs, where one lane
+// per element leaves most of the GPU idle (19,664 DOFs: 7.5 us with one, 5.9 with four; 245,000 DOFs:
+// 28.8 and 31.5).
+static int maxpy_split(int64_t n) { return n < 65536 ? 4 : 1; }
+template <typename R>
+static void launch_maxpy(hipStream_t st, int nb, int64_t n, int nv, const R *V, const double *h, const double *sc, R *w,
+                         double *partial, const kept_dev *kept = nullptr, const double *qp = nullptr,
+                         double *hout = nullptr) {
+    if (maxpy_split(n) == 4)
+        k_maxpy_norm<R, 4><<<nb, RB, 0, st>>>(n, nv, V, n, h, sc, w, partial, kept, qp, hout);
+    else
+        k_maxpy_norm<R, 1><<<nb, RB, 0, st>>>(n, nv, V, n, h, sc, w, partial, kept, qp, hout);
 }
 
 // x += sum_i y_i V_i   (y on device, complex)
@@ -371,7 +559,7 @@ __global__ void __launch_bounds__(RB) k_norm2(int64_t n, const R *__restrict__ x
         const cx<R> v = ld(x, e);
         s += (double)v.re * v.re + (double)v.im * v.im;
     }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    s = lane_sum<64>(s);
     __shared__ double sh[RB / 64];
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
@@ -390,7 +578,7 @@ __global__ void __launch_bounds__(RB) k_scale_by_norm(int64_t n, const double *_
     if (threadIdx.x < 64) {
         double s = 0;
         for (int b = threadIdx.x; b < nblk; b += 64) s += partial[b];
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        s = lane_sum<64>(s);
         if (threadIdx.x == 0) {
             const double nv = sqrt(s);
             inv = nv > 0 ? 1.0 / nv : 0.0;
@@ -406,13 +594,12 @@ __global__ void __launch_bounds__(RB) k_scale_by_norm(int64_t n, const double *_
 
 // 2x2 mode-block Jacobi: z = blk^{-1} r on DOF pairs (e, e + n_ent).
 // inv holds per entity the 4 complex entries of the inverse block (row-major).
-template <typename R>
-__global__ void __launch_bounds__(RB) k_bj_apply(int64_t n_ent, const R *__restrict__ inv, const R *__restrict__ r,
-                                                 R *__restrict__ z) {
+__global__ void __launch_bounds__(RB) k_bj_apply(int64_t n_ent, const double *__restrict__ inv, const double *__restrict__ r,
+                                                 double *__restrict__ z) {
     const int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x;
     if (e >= n_ent) return;
-    const cx<R> a = ld(inv, 4 * e), b = ld(inv, 4 * e + 1), c = ld(inv, 4 * e + 2), d = ld(inv, 4 * e + 3);
-    const cx<R> r0 = ld(r, e), r1 = ld(r, e + n_ent);
+    const cx<double> a = ld(inv, 4 * e), b = ld(inv, 4 * e + 1), c = ld(inv, 4 * e + 2), d = ld(inv, 4 * e + 3);
+    const cx<double> r0 = ld(r, e), r1 = ld(r, e + n_ent);
     st(z, e, cadd(cmul(a, r0), cmul(b, r1)));
     st(z, e + n_ent, cadd(cmul(c, r0), cmul(d, r1)));
 }
@@ -476,73 +663,51 @@ __global__ void __launch_bounds__(RB) k_dsinv(int64_t np2, const double *__restr
     if (inv32) { inv32[2 * p] = (float)r; inv32[2 * p + 1] = (float)im; }
 }
 
-// t[p] = dsinv[p] * sum over row p of G^T of g * r, GL lanes per row (vertex rows of G^T
-// hold tens of entries, edge rows about ten; the solver's tuner picks GL)
-template <typename R, int GL>
+// t[p] = dsinv[p] * sum over row p of G^T of g * r, 8 lanes per row (caller's layout)
+static constexpr int GT_STD = 8;
 __global__ void __launch_bounds__(256) k_gt_apply(int64_t np2, const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                                                  const R *__restrict__ gv, const R *__restrict__ dsinv,
-                                                  const R *__restrict__ r, R *__restrict__ t) {
-    const int64_t p = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / GL;
-    const int lane = threadIdx.x % GL;
+                                                  const double *__restrict__ gv, const double *__restrict__ dsinv,
+                                                  const double *__restrict__ r, double *__restrict__ t) {
+    const int64_t p = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / GT_STD;
+    const int lane = threadIdx.x % GT_STD;
     if (p >= np2) return;
     double ar = 0.0, ai = 0.0;
-    for (int32_t e = rp[p] + lane; e < rp[p + 1]; e += GL) {
-        const cx<R> v = ld(r, ci[e]);
-        ar += (double)gv[e] * v.re;
-        ai += (double)gv[e] * v.im;
+    for (int32_t e = rp[p] + lane; e < rp[p + 1]; e += GT_STD) {
+        const cx<double> v = ld(r, ci[e]);
+        ar += gv[e] * v.re;
+        ai += gv[e] * v.im;
     }
-#pragma unroll
-    for (int off = GL / 2; off > 0; off >>= 1) {
-        ar += __shfl_xor(ar, off, GL);
-        ai += __shfl_xor(ai, off, GL);
-    }
+    ar = lane_sum<GT_STD>(ar);
+    ai = lane_sum<GT_STD>(ai);
     if (lane == 0) {
-        const cx<R> d = ld(dsinv, p);
-        st(t, p, cx<R>((R)(d.re * ar - d.im * ai), (R)(d.re * ai + d.im * ar)));
+        const cx<double> d = ld(dsinv, p);
+        st(t, p, cx<double>(d.re * ar - d.im * ai, d.re * ai + d.im * ar));
     }
 }
 
-template <typename R>
-static void launch_gt(hipStream_t st, int L, int64_t np2, const int32_t *rp, const int32_t *ci, const R *gv,
-                      const R *dsinv, const R *r, R *t) {
-    if (L != 4 && L != 16) L = 8;
-    const unsigned grid = (unsigned)((np2 * L + 255) / 256);
-    if (L == 4) k_gt_apply<R, 4><<<grid, 256, 0, st>>>(np2, rp, ci, gv, dsinv, r, t);
-    else if (L == 16) k_gt_apply<R, 16><<<grid, 256, 0, st>>>(np2, rp, ci, gv, dsinv, r, t);
-    else k_gt_apply<R, 8><<<grid, 256, 0, st>>>(np2, rp, ci, gv, dsinv, r, t);
+static void launch_gt(hipStream_t st, int64_t np2, const int32_t *rp, const int32_t *ci, const double *gv,
+                      const double *dsinv, const double *r, double *t) {
+    k_gt_apply<<<(unsigned)((np2 * GT_STD + 255) / 256), 256, 0, st>>>(np2, rp, ci, gv, dsinv, r, t);
 }
 
-// z = BJ(r) + G t, both modes of entity e per thread
-template <typename R>
-__global__ void __launch_bounds__(RB) k_bj_grad_apply(int64_t n_ent, const R *__restrict__ inv, const R *__restrict__ r,
-                                                      const int32_t *__restrict__ grp, const int32_t *__restrict__ gcol,
-                                                      const R *__restrict__ gv, const R *__restrict__ t,
-                                                      R *__restrict__ z) {
+// z = BJ(r) + G t, both modes of entity e per thread (caller's layout)
+__global__ void __launch_bounds__(RB) k_bj_grad_apply(int64_t n_ent, const double *__restrict__ inv,
+                                                      const double *__restrict__ r, const int32_t *__restrict__ grp,
+                                                      const int32_t *__restrict__ gcol, const double *__restrict__ gv,
+                                                      const double *__restrict__ t, double *__restrict__ z) {
     const int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x;
     if (e >= n_ent) return;
-    const cx<R> a = ld(inv, 4 * e), b = ld(inv, 4 * e + 1), c = ld(inv, 4 * e + 2), d = ld(inv, 4 * e + 3);
-    const cx<R> r0 = ld(r, e), r1 = ld(r, e + n_ent);
-    cx<R> z0 = cadd(cmul(a, r0), cmul(b, r1));
-    cx<R> z1 = cadd(cmul(c, r0), cmul(d, r1));
-    const int32_t q0 = grp[e], q1 = grp[e + 1], q2 = grp[e + n_ent], q3 = grp[e + n_ent + 1];
-    if (q1 - q0 == q3 - q2) {
-        // both modes' rows list the same P2 nodes in the same order (the entity's nodes less the
-        // dropped ones): one column index and one gather of t serve both rows
-        for (int32_t k = 0; k < q1 - q0; k++) {
-            const cx<R> tv = ld(t, gcol[q0 + k]);
-            const R g0 = gv[q0 + k], g1 = gv[q2 + k];
-            z0 = cx<R>(z0.re + g0 * tv.re, z0.im + g0 * tv.im);
-            z1 = cx<R>(z1.re + g1 * tv.re, z1.im + g1 * tv.im);
-        }
-    } else {
-        for (int32_t q = q0; q < q1; q++) {
-            const cx<R> tv = ld(t, gcol[q]);
-            z0 = cx<R>(z0.re + gv[q] * tv.re, z0.im + gv[q] * tv.im);
-        }
-        for (int32_t q = q2; q < q3; q++) {
-            const cx<R> tv = ld(t, gcol[q]);
-            z1 = cx<R>(z1.re + gv[q] * tv.re, z1.im + gv[q] * tv.im);
-        }
+    const cx<double> a = ld(inv, 4 * e), b = ld(inv, 4 * e + 1), c = ld(inv, 4 * e + 2), d = ld(inv, 4 * e + 3);
+    const cx<double> r0 = ld(r, e), r1 = ld(r, e + n_ent);
+    cx<double> z0 = cadd(cmul(a, r0), cmul(b, r1));
+    cx<double> z1 = cadd(cmul(c, r0), cmul(d, r1));
+    for (int32_t q = grp[e]; q < grp[e + 1]; q++) {
+        const cx<double> tv = ld(t, gcol[q]);
+        z0 = cx<double>(z0.re + gv[q] * tv.re, z0.im + gv[q] * tv.im);
+    }
+    for (int32_t q = grp[e + n_ent]; q < grp[e + n_ent + 1]; q++) {
+        const cx<double> tv = ld(t, gcol[q]);
+        z1 = cx<double>(z1.re + gv[q] * tv.re, z1.im + gv[q] * tv.im);
     }
     st(z, e, z0);
     st(z, e + n_ent, z1);
@@ -589,32 +754,6 @@ __global__ void __launch_bounds__(RB) k_bj_setup(int64_t n_ent, const int32_t *_
     }
 }
 
-__global__ void __launch_bounds__(RB) k_to_c64(int64_t n, const double *__restrict__ a, float *__restrict__ b) {
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < 2 * n; e += (int64_t)gridDim.x * RB) b[e] = (float)a[e];
-}
-// complex64 copy of the matrix values with the masked (PEC) columns set to zero
-__global__ void __launch_bounds__(RB) k_to_c64_masked(int64_t nnz, const int32_t *__restrict__ cols,
-                                                      const uint8_t *__restrict__ mask, const double *__restrict__ a,
-                                                      float *__restrict__ b) {
-    for (int64_t p = blockIdx.x * (int64_t)RB + threadIdx.x; p < nnz; p += (int64_t)gridDim.x * RB) {
-        const bool keep = mask == nullptr || mask[cols[p]];
-        b[2 * p] = keep ? (float)a[2 * p] : 0.0f;
-        b[2 * p + 1] = keep ? (float)a[2 * p + 1] : 0.0f;
-    }
-}
-__global__ void __launch_bounds__(RB) k_add_c64_to_c128(int64_t n, const float *__restrict__ d, double *__restrict__ x) {
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < 2 * n; e += (int64_t)gridDim.x * RB) x[e] += (double)d[e];
-}
-// y = x (scaled to c64) * s  (s real)
-__global__ void __launch_bounds__(RB) k_c128_to_c64_scaled(int64_t n, const double *__restrict__ a, double s, float *__restrict__ b) {
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < 2 * n; e += (int64_t)gridDim.x * RB) b[e] = (float)(a[e] * s);
-}
-
-// x (complex128) += scale * d (element type R)
-template <typename R>
-__global__ void __launch_bounds__(RB) k_add_scaled(int64_t n, const R *__restrict__ d, double scale, double *__restrict__ x) {
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < 2 * n; e += (int64_t)gridDim.x * RB) x[e] += scale * (double)d[e];
-}
 // u += z (same element type)
 template <typename R>
 __global__ void __launch_bounds__(RB) k_add(int64_t n, const R *__restrict__ z, R *__restrict__ u) {
@@ -647,17 +786,443 @@ __global__ void __launch_bounds__(RB) k_csr_find(int64_t m, const int32_t *__res
     pos[i] = find_col(cols, rowptr[r], rowptr[r + 1], qc[i]);
 }
 
+// ---------------------------------------------------------------- packed solver layout
+// The vectors of the solver's own steps hold the two modes of an entity side by side
+// (V[2 e + m] for DOF m * ne + e), and its operators are stored for that:
+//  * K as 2x2 blocks over the entity pattern in two planes, the real parts kre[4 p ..] and
+//    the imaginary parts kim[4 p ..] of entry p (p = rowptr[e] / 2 + k), the columns acol[p]
+//    once per block.  A row whose imaginary parts all vanish (lossless media: every row but
+//    those of ports and absorbing boundaries) is flagged and its kim plane is never read, so
+//    a complex64 product moves 20 instead of 36 bytes per block.  PEC columns are zeroed.
+//  * G in slices of 64 entities, transposed (slot k of the 64 lanes together): one column and
+//    both modes' values per slot; G^T in rows of (entity, both modes' values).
+static constexpr uint8_t ROW0 = 1, ROW1 = 2, ROW_CPLX = 4;   // flags: row (0, e) free, (1, e) free, kim used
+
+// acol[p] of every block (16 lanes per entity)
+__global__ void __launch_bounds__(256) k_pack_cols(int64_t ne, const int32_t *__restrict__ rowptr,
+                                                   const int32_t *__restrict__ cols, int32_t *__restrict__ acol) {
+    const int64_t e = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / SUB;
+    if (e >= ne) return;
+    const int32_t r0 = rowptr[e], deg = (rowptr[e + 1] - r0) >> 1;
+    for (int32_t k = threadIdx.x % SUB; k < deg; k += SUB) acol[(r0 >> 1) + k] = cols[r0 + k];
+}
+
+// The planes and flags of K (complex128 CSR values) in element type R.
+template <typename R>
+__global__ void __launch_bounds__(256) k_pack_matrix(int64_t ne, int64_t half, const int32_t *__restrict__ rowptr,
+                                                     const int32_t *__restrict__ acol, const double *__restrict__ vals,
+                                                     const uint8_t *__restrict__ mask, R *__restrict__ kre,
+                                                     R *__restrict__ kim, uint8_t *__restrict__ flag) {
+    const int64_t e = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / SUB;
+    const int lane = threadIdx.x % SUB;
+    if (e >= ne) return;
+    const bool m0 = mask == nullptr || mask[e], m1 = mask == nullptr || mask[ne + e];
+    const int32_t r0 = rowptr[e], deg = (rowptr[e + 1] - r0) >> 1, a0 = r0 >> 1;
+    int any = 0;
+    for (int pass = 0; pass < 2; pass++) {
+        for (int32_t k = lane; k < deg; k += SUB) {
+            const int32_t c = acol[a0 + k];
+            const bool c0 = mask == nullptr || mask[c], c1 = mask == nullptr || mask[ne + c];
+            const int64_t p = (int64_t)r0 + k;
+            cx<double> v00 = ld(vals, p), v01 = ld(vals, p + deg), v10 = ld(vals, half + p), v11 = ld(vals, half + p + deg);
+            if (!(m0 && c0)) v00 = cx<double>();
+            if (!(m0 && c1)) v01 = cx<double>();
+            if (!(m1 && c0)) v10 = cx<double>();
+            if (!(m1 && c1)) v11 = cx<double>();
+            const cx2<R> im{(R)v00.im, (R)v01.im, (R)v10.im, (R)v11.im};
+            if (pass == 0) {
+                st2(kre, a0 + k, cx2<R>{(R)v00.re, (R)v01.re, (R)v10.re, (R)v11.re});
+                // != is true of NaN too: such a row keeps its imaginary plane
+                any |= (im.ar != R(0)) | (im.ai != R(0)) | (im.br != R(0)) | (im.bi != R(0));
+            } else {
+                st2(kim, a0 + k, im);
+            }
+        }
+        if (pass == 0) {
+#pragma unroll
+            for (int off = SUB / 2; off > 0; off >>= 1) any |= __shfl_xor(any, off, SUB);
+            if (!any) break;
+        }
+    }
+    if (lane == 0) flag[e] = (uint8_t)((m0 ? ROW0 : 0) | (m1 ? ROW1 : 0) | (any ? ROW_CPLX : 0));
+}
+
+// Workgroup b of a grid as work item: XCD b % 8 takes runs of XCD_RUN consecutive items, whose rows
+// gather mostly the same parts of x, instead of every eighth (complex64 product on air: 40.1 -> 36.2 us
+// at 60 x 30 x 12 hexes, 114.6 -> 113.4 at 80 x 40 x 16; runs of 8 and 128 the same within 2 %, runs of
+// 512 slower again, an eighth of the grid per XCD 30 % slower).
+static constexpr unsigned XCD_RUN = 32;
+__device__ __forceinline__ unsigned xcd_run(unsigned b, unsigned n) {
+    const unsigned full = n / (8 * XCD_RUN) * (8 * XCD_RUN);
+    if (b >= full) return b;
+    const unsigned i = b / 8;
+    return i / XCD_RUN * (8 * XCD_RUN) + (b % 8) * XCD_RUN + i % XCD_RUN;
+}
+
+// What follows a product v = K x in the same launch:
+//   SP_Y: y = v;   SP_RESID: y = b - v;
+//   SP_POLY: p = q - c_i v, y = (i == 0 ? c_0 q : y) + c_{i+1} p (apply_prec_poly; q scaled by *qs)
+enum { SP_Y, SP_RESID, SP_POLY };
+template <typename R>
+struct sp_args {
+    const R *b;          // SP_RESID: b; SP_POLY: q (may be p)
+    R *y;
+    R *p;                // SP_POLY
+    const double *c;     // SP_POLY: the polynomial's coefficients
+    int i;               // SP_POLY
+    const double *qs;    // SP_POLY: scale of q, or NULL
+};
+
+// v = K x on the packed matrix: L lanes per entity, every lane loading the columns and blocks of
+// up to U entries before it gathers x for them, so that a row of average length (21 blocks) costs
+// two round trips to memory instead of two per L entries.  Bound by the bytes of kre, acol and (in
+// rows with losses) kim; small problems by the latency of that chain.  STD: x, y, b in the caller's
+// layout (mode * ne + e) instead of interleaved (SP_Y and SP_RESID only).
+template <typename R, int L, int EP, bool STD>
+__global__ void __launch_bounds__(256) k_spmv_pk(int64_t ne, const int32_t *__restrict__ rowptr,
+                                                 const int32_t *__restrict__ acol, const R *__restrict__ kre,
+                                                 const R *__restrict__ kim, const uint8_t *__restrict__ flag,
+                                                 const R *__restrict__ x, sp_args<R> a) {
+    constexpr int U = L <= 4 ? 4 : L == 8 ? 3 : L == 16 ? 2 : 1;
+    const int64_t e = (xcd_run(blockIdx.x, gridDim.x) * (int64_t)blockDim.x + threadIdx.x) / L;
+    const int lane = threadIdx.x % L;
+    if (e >= ne) return;
+    const uint8_t fl = flag[e];
+    const int32_t p0 = rowptr[e] >> 1, p1 = rowptr[e + 1] >> 1;
+    cx2<R> own{}, qv{}, yv{};
+    // the epilogue's operands, asked for before the row
+    if (lane == 0) {
+        auto get = [&](const R *v) {
+            if constexpr (STD) {
+                const cx<R> u0 = ld(v, e), u1 = ld(v, ne + e);
+                return cx2<R>{u0.re, u0.im, u1.re, u1.im};
+            } else {
+                return ld2(v, e);
+            }
+        };
+        if ((fl & (ROW0 | ROW1)) != (ROW0 | ROW1)) own = get(x);
+        if constexpr (EP != SP_Y) qv = get(a.b);
+        if constexpr (EP == SP_POLY)
+            if (a.i > 0) yv = get(a.y);
+    }
+    R s0r = 0, s0i = 0, s1r = 0, s1i = 0;
+    if (fl & (ROW0 | ROW1)) {
+        for (int32_t p = p0 + lane; p < p1; p += L * U) {
+            int32_t c[U];
+            cx2<R> k[U], xv[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int32_t q = p + u * L < p1 ? p + u * L : p;   // past the row's end: its own entry again, not used
+                c[u] = acol[q];
+                k[u] = ld2(kre, q);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if constexpr (STD) {
+                    cx<R> u0 = ld(x, c[u]), u1 = ld(x, ne + c[u]);
+                    if constexpr (sizeof(R) == 8) {
+                        // a caller's x may hold anything on PEC DOFs (their columns are zero, but 0 * inf is not)
+                        const uint8_t cf = flag[c[u]];
+                        if (!(cf & ROW0)) u0 = cx<R>();
+                        if (!(cf & ROW1)) u1 = cx<R>();
+                    }
+                    xv[u] = cx2<R>{u0.re, u0.im, u1.re, u1.im};
+                } else {
+                    xv[u] = ld2(x, c[u]);
+                }
+            }
+            // an entry's products are summed before they join the row's sums, as in the complex product
+            cx2<R> v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                v[u] = cx2<R>{k[u].ar * xv[u].ar + k[u].ai * xv[u].br, k[u].ar * xv[u].ai + k[u].ai * xv[u].bi,
+                              k[u].br * xv[u].ar + k[u].bi * xv[u].br, k[u].br * xv[u].ai + k[u].bi * xv[u].bi};
+            if (fl & ROW_CPLX) {
+#pragma unroll
+                for (int u = 0; u < U; u++) k[u] = ld2(kim, p + u * L < p1 ? p + u * L : p);
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    v[u].ar -= k[u].ar * xv[u].ai + k[u].ai * xv[u].bi;
+                    v[u].ai += k[u].ar * xv[u].ar + k[u].ai * xv[u].br;
+                    v[u].br -= k[u].br * xv[u].ai + k[u].bi * xv[u].bi;
+                    v[u].bi += k[u].br * xv[u].ar + k[u].bi * xv[u].br;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (p + u * L < p1) {
+                    s0r += v[u].ar;
+                    s0i += v[u].ai;
+                    s1r += v[u].br;
+                    s1i += v[u].bi;
+                }
+        }
+    }
+    s0r = lane_sum<L>(s0r);
+    s0i = lane_sum<L>(s0i);
+    s1r = lane_sum<L>(s1r);
+    s1i = lane_sum<L>(s1i);
+    if (lane != 0) return;
+    cx2<R> v{(fl & ROW0) ? s0r : own.ar, (fl & ROW0) ? s0i : own.ai, (fl & ROW1) ? s1r : own.br, (fl & ROW1) ? s1i : own.bi};
+    if constexpr (EP == SP_RESID) v = cx2<R>{qv.ar - v.ar, qv.ai - v.ai, qv.br - v.br, qv.bi - v.bi};
+    if constexpr (EP == SP_POLY) {
+        const double *cc = a.c + 2 * a.i;
+        const double cr = cc[0], ci = cc[1], nr = cc[2], ni = cc[3];
+        const double s = a.qs != nullptr ? a.qs[0] : 1.0;
+        const double q0r = s * qv.ar, q0i = s * qv.ai, q1r = s * qv.br, q1i = s * qv.bi;
+        double y0r = yv.ar, y0i = yv.ai, y1r = yv.br, y1i = yv.bi;
+        if (a.i == 0) {
+            y0r = cr * q0r - ci * q0i; y0i = cr * q0i + ci * q0r;
+            y1r = cr * q1r - ci * q1i; y1i = cr * q1i + ci * q1r;
+        }
+        const double p0r = q0r - (cr * v.ar - ci * v.ai), p0i = q0i - (cr * v.ai + ci * v.ar);
+        const double p1r = q1r - (cr * v.br - ci * v.bi), p1i = q1i - (cr * v.bi + ci * v.br);
+        st2(a.p, e, cx2<R>{(R)p0r, (R)p0i, (R)p1r, (R)p1i});
+        st2(a.y, e, cx2<R>{(R)(y0r + nr * p0r - ni * p0i), (R)(y0i + nr * p0i + ni * p0r),
+                           (R)(y1r + nr * p1r - ni * p1i), (R)(y1i + nr * p1i + ni * p1r)});
+    } else if constexpr (STD) {
+        st(a.y, e, cx<R>(v.ar, v.ai));
+        st(a.y, ne + e, cx<R>(v.br, v.bi));
+    } else {
+        st2(a.y, e, v);
+    }
+}
+
+template <typename R, int EP, bool STD>
+static void launch_spmv_pk(hipStream_t st, int L, int64_t ne, const int32_t *rowptr, const int32_t *acol, const R *kre,
+                           const R *kim, const uint8_t *flag, const R *x, const sp_args<R> &a) {
+    if (L != 4 && L != 8 && L != 32) L = 16;
+    const unsigned grid = (unsigned)((ne * L + 255) / 256);
+    if (L == 4) k_spmv_pk<R, 4, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
+    else if (L == 8) k_spmv_pk<R, 8, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
+    else if (L == 32) k_spmv_pk<R, 32, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
+    else k_spmv_pk<R, 16, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
+}
+
+// Entries of entity e's packed G row: the nodes of row e with both modes' values where rows e and
+// ne + e list the same nodes in the same order (the entity's nodes less the dropped ones), else the
+// entries of both rows one after the other, each with a zero for the other mode.
+__device__ __forceinline__ int g_entries(const int32_t *grp, const int32_t *gcol, int64_t ne, int64_t e, bool &same) {
+    const int32_t q0 = grp[e], n0 = grp[e + 1] - q0, q1 = grp[ne + e], n1 = grp[ne + e + 1] - q1;
+    same = n0 == n1;
+    for (int32_t k = 0; same && k < n0; k++) same = gcol[q0 + k] == gcol[q1 + k];
+    return same ? n0 : n0 + n1;
+}
+// width[s]: the longest packed row of the 64 entities of slice s
+__global__ void __launch_bounds__(64) k_g_width(int64_t ne, const int32_t *__restrict__ grp,
+                                                const int32_t *__restrict__ gcol, int32_t *__restrict__ width) {
+    const int64_t e = blockIdx.x * (int64_t)64 + threadIdx.x;
+    bool same;
+    int w = e < ne ? g_entries(grp, gcol, ne, e, same) : 0;
+    for (int off = 32; off > 0; off >>= 1) w = max(w, __shfl_xor(w, off, 64));
+    if (threadIdx.x == 0) width[blockIdx.x] = w;
+}
+// Where the slots of a slice begin: slices before `cut` have w0 slots per entity, the others w1 (edges
+// hold 3 nodes and come first, faces 6), so no table is read ahead of the slots.
+struct g_shape {
+    int64_t cut;
+    int w0, w1;
+    __host__ __device__ int width(int64_t s) const { return s < cut ? w0 : w1; }
+    __host__ __device__ int64_t first(int64_t s) const { return 64 * (s < cut ? s * w0 : cut * w0 + (s - cut) * w1); }
+};
+template <typename R>
+__global__ void __launch_bounds__(64) k_g_fill(int64_t ne, const int32_t *__restrict__ grp,
+                                               const int32_t *__restrict__ gcol, const double *__restrict__ gv,
+                                               g_shape sh, int32_t *__restrict__ pcol, R *__restrict__ pval) {
+    const int64_t e = blockIdx.x * (int64_t)64 + threadIdx.x;
+    const int64_t b = sh.first(blockIdx.x) + threadIdx.x;
+    const int w = sh.width(blockIdx.x);
+    bool same = true;
+    const int n = e < ne ? g_entries(grp, gcol, ne, e, same) : 0;
+    const int32_t q0 = e < ne ? grp[e] : 0, n0 = e < ne ? grp[e + 1] - q0 : 0, q1 = e < ne ? grp[ne + e] : 0;
+    for (int k = 0; k < w; k++) {
+        int32_t c = -1;
+        double v0 = 0.0, v1 = 0.0;
+        if (k < n) {
+            if (same) { c = gcol[q0 + k]; v0 = gv[q0 + k]; v1 = gv[q1 + k]; }
+            else if (k < n0) { c = gcol[q0 + k]; v0 = gv[q0 + k]; }
+            else { c = gcol[q1 + k - n0]; v1 = gv[q1 + k - n0]; }
+        }
+        pcol[b + 64 * (int64_t)k] = c;
+        st(pval, b + 64 * (int64_t)k, cx<R>((R)v0, (R)v1));
+    }
+}
+
+// Row p of G^T (DOF columns, mode 0 before mode 1 when ascending) as (entity, both modes'
+// values): the two runs merged when the row is strictly ascending, else every entry by itself
+// with a zero for the other mode.  Returns the number of entries; writes them when ocol is given.
+template <typename R>
+__device__ int gt_entries(const int32_t *ci, const double *gv, int32_t a, int32_t b, int64_t ne, int32_t *ocol, R *oval) {
+    bool asc = true;
+    int32_t m = b;
+    for (int32_t i = a; i < b; i++) {
+        if (i > a && ci[i] <= ci[i - 1]) asc = false;
+        if (m == b && ci[i] >= ne) m = i;
+    }
+    int n = 0;
+    auto put = [&](int32_t e, double v0, double v1) {
+        if (ocol != nullptr) { ocol[n] = e; st(oval, n, cx<R>((R)v0, (R)v1)); }
+        n++;
+    };
+    if (!asc) {
+        for (int32_t i = a; i < b; i++) {
+            if (ci[i] < ne) put(ci[i], gv[i], 0.0); else put((int32_t)(ci[i] - ne), 0.0, gv[i]);
+        }
+        return n;
+    }
+    int32_t i = a, j = m;
+    while (i < m || j < b) {
+        const int64_t ei = i < m ? ci[i] : INT64_MAX, ej = j < b ? ci[j] - ne : INT64_MAX;
+        if (ei == ej) { put((int32_t)ei, gv[i], gv[j]); i++; j++; }
+        else if (ei < ej) { put((int32_t)ei, gv[i], 0.0); i++; }
+        else { put((int32_t)ej, 0.0, gv[j]); j++; }
+    }
+    return n;
+}
+__global__ void __launch_bounds__(RB) k_gt_count(int64_t np2, int64_t ne, const int32_t *__restrict__ rp,
+                                                 const int32_t *__restrict__ ci, int32_t *__restrict__ cnt) {
+    const int64_t p = blockIdx.x * (int64_t)RB + threadIdx.x;
+    if (p < np2) cnt[p] = gt_entries<float>(ci, nullptr, rp[p], rp[p + 1], ne, nullptr, nullptr);
+}
+template <typename R>
+__global__ void __launch_bounds__(RB) k_gt_fill(int64_t np2, int64_t ne, const int32_t *__restrict__ rp,
+                                                const int32_t *__restrict__ ci, const double *__restrict__ gv,
+                                                const int32_t *__restrict__ prp, int32_t *__restrict__ pcol,
+                                                R *__restrict__ pval) {
+    const int64_t p = blockIdx.x * (int64_t)RB + threadIdx.x;
+    if (p < np2) gt_entries<R>(ci, gv, rp[p], rp[p + 1], ne, pcol + prp[p], pval + 2 * (int64_t)prp[p]);
+}
+
+// t = diag(G^T K G)^{-1} G^T (xs x), GL lanes per row, up to U entries of a lane loaded before
+// their gathers (a vertex row of a Kuhn mesh holds 50 entities: two round trips at 8 lanes where
+// one entry at a time took seven).  Sums in FP64.
+template <typename R, int GL>
+__global__ void __launch_bounds__(256) k_gt_pk(int64_t np2, const int32_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                               const R *__restrict__ val, const R *__restrict__ dsinv,
+                                               const R *__restrict__ x, const double *__restrict__ xs, R *__restrict__ t) {
+    constexpr int U = GL == 16 ? 2 : 4;
+    const int64_t p = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / GL;
+    const int lane = threadIdx.x % GL;
+    if (p >= np2) return;
+    const double s = xs != nullptr ? xs[0] : 1.0;
+    const cx<R> d = ld(dsinv, p);
+    double ar = 0.0, ai = 0.0;
+    const int32_t e1 = rp[p + 1];
+    for (int32_t e = rp[p] + lane; e < e1; e += GL * U) {
+        int32_t c[U];
+        cx<R> g[U];
+        cx2<R> v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int32_t q = e + u * GL < e1 ? e + u * GL : e;
+            c[u] = col[q];
+            g[u] = ld(val, q);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = ld2(x, c[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (e + u * GL < e1) {
+                ar += (double)g[u].re * v[u].ar + (double)g[u].im * v[u].br;
+                ai += (double)g[u].re * v[u].ai + (double)g[u].im * v[u].bi;
+            }
+    }
+    ar = lane_sum<GL>(ar);
+    ai = lane_sum<GL>(ai);
+    if (lane == 0) {
+        ar *= s;
+        ai *= s;
+        st(t, p, cx<R>((R)(d.re * ar - d.im * ai), (R)(d.re * ai + d.im * ar)));
+    }
+}
+
+template <typename R>
+static void launch_gt_pk(hipStream_t st, int L, int64_t np2, const int32_t *rp, const int32_t *col, const R *val,
+                         const R *dsinv, const R *x, const double *xs, R *t) {
+    if (L != 4 && L != 16) L = 8;
+    const unsigned grid = (unsigned)((np2 * L + 255) / 256);
+    if (L == 4) k_gt_pk<R, 4><<<grid, 256, 0, st>>>(np2, rp, col, val, dsinv, x, xs, t);
+    else if (L == 16) k_gt_pk<R, 16><<<grid, 256, 0, st>>>(np2, rp, col, val, dsinv, x, xs, t);
+    else k_gt_pk<R, 8><<<grid, 256, 0, st>>>(np2, rp, col, val, dsinv, x, xs, t);
+}
+
+// z = BJ(xs x) + G t (G in slices of 64 entities, gcol NULL: no gradient part), one entity per lane
+template <typename R>
+__global__ void __launch_bounds__(RB) k_bj_grad_pk(int64_t ne, const R *__restrict__ inv, const R *__restrict__ x,
+                                                   const double *__restrict__ xs, g_shape sh,
+                                                   const int32_t *__restrict__ gcol, const R *__restrict__ gval,
+                                                   const R *__restrict__ t, R *__restrict__ z) {
+    const int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x;
+    if (e >= ne) return;
+    const double s = xs != nullptr ? xs[0] : 1.0;
+    const cx2<R> i0 = ld2(inv, 2 * e), i1 = ld2(inv, 2 * e + 1);
+    cx2<R> r = ld2(x, e);
+    r = cx2<R>{(R)(s * r.ar), (R)(s * r.ai), (R)(s * r.br), (R)(s * r.bi)};
+    const cx<R> r0(r.ar, r.ai), r1(r.br, r.bi);
+    cx<R> z0 = cadd(cmul(cx<R>(i0.ar, i0.ai), r0), cmul(cx<R>(i0.br, i0.bi), r1));
+    cx<R> z1 = cadd(cmul(cx<R>(i1.ar, i1.ai), r0), cmul(cx<R>(i1.br, i1.bi), r1));
+    if (gcol != nullptr) {
+        const int64_t si = e >> 6;
+        const int w = sh.width(si);
+        const int64_t b = sh.first(si) + (e & 63);
+        constexpr int U = 3;   // edges hold 3 nodes, faces 6
+        for (int k = 0; k < w; k += U) {
+            int32_t c[U];
+            cx<R> g[U], tv[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int64_t q = b + 64 * (int64_t)(k + u < w ? k + u : k);
+                c[u] = k + u < w ? gcol[q] : -1;
+                g[u] = ld(gval, q);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) tv[u] = c[u] >= 0 ? ld(t, c[u]) : cx<R>();
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                z0 = cx<R>(z0.re + g[u].re * tv[u].re, z0.im + g[u].re * tv[u].im);
+                z1 = cx<R>(z1.re + g[u].im * tv[u].re, z1.im + g[u].im * tv[u].im);
+            }
+        }
+    }
+    st2(z, e, cx2<R>{z0.re, z0.im, z1.re, z1.im});
+}
+
+// b (interleaved, R) = s a (caller's layout, complex128)
+template <typename R>
+__global__ void __launch_bounds__(RB) k_pack_vec(int64_t ne, const double *__restrict__ a, double s, R *__restrict__ b) {
+    const int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x;
+    if (e >= ne) return;
+    const cx<double> u = ld(a, e), v = ld(a, ne + e);
+    st2(b, e, cx2<R>{(R)(u.re * s), (R)(u.im * s), (R)(v.re * s), (R)(v.im * s)});
+}
+// x (caller's layout, complex128) = (add ? x : 0) + s d (interleaved, R)
+template <typename R>
+__global__ void __launch_bounds__(RB) k_unpack_vec(int64_t ne, const R *__restrict__ d, double s, int add,
+                                                   double *__restrict__ x) {
+    const int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x;
+    if (e >= ne) return;
+    const cx2<R> v = ld2(d, e);
+    cx<double> u0, u1;
+    if (add) { u0 = ld(x, e); u1 = ld(x, ne + e); }
+    st(x, e, cx<double>(u0.re + s * (double)v.ar, u0.im + s * (double)v.ai));
+    st(x, ne + e, cx<double>(u1.re + s * (double)v.br, u1.im + s * (double)v.bi));
+}
+
 // ---------------------------------------------------------------- solver object
 struct emg_solver {
     int64_t n = 0, nnz = 0, n_ent = 0;
     int restart = 0, precision = 64;
+    int cap = 0;                    // Krylov steps the basis storage holds: restart, up to twice that in complex64
     const int32_t *rowptr = nullptr, *cols = nullptr;
     const double *vals = nullptr;   // complex128 K (caller-owned)
     const uint8_t *mask = nullptr;  // caller-owned, may be null
-    float *vals32 = nullptr;        // complex64 copy for precision 32
+    // K in the packed layout, in the precision of the solver's steps (k_pack_matrix)
+    int32_t *acol = nullptr;        // nnz / 4 column entities
+    void *kre = nullptr, *kim = nullptr;   // real and imaginary planes, nnz values each
+    uint8_t *row_flag = nullptr;    // n_ent
     double *inv64 = nullptr;
     float *inv32 = nullptr;
-    double *V = nullptr;            // (restart+1) basis vectors, element type per precision
+    double *V = nullptr;            // cap + 1 basis vectors, element type per precision
     double *w = nullptr, *z = nullptr, *r = nullptr, *d = nullptr;
     double *partial = nullptr, *h = nullptr, *nrm = nullptr;
     int nblk = 0;
@@ -666,14 +1231,20 @@ struct emg_solver {
     // updated on the device; the host reads the estimates once per chunk.
     double *arn = nullptr;        // device Arnoldi state (see arn_off)
     double *pn = nullptr;         // per-block partial norms of the new basis vector
-    double *flag = nullptr;       // [0]: 1 = run the second Gram-Schmidt pass
-    double *res_host = nullptr;   // pinned copy of the residual estimates
-    hipStream_t cap = nullptr;    // capture stream (graphs are launched on the caller's stream)
+    double *gram = nullptr;       // the basis' Gram matrix less the identity, (cap + 1)^2 complex
+    double *flag = nullptr;       // scratch of the pattern check
+    double *host = nullptr;       // pinned host memory the kernels write to and small uploads go through (host_off)
+    double *host_dev = nullptr;   // the device's address of it
+    kept_dev *kept = nullptr;     // spaces kept from the running solve's earlier refinement cycles (in arn)
+    hipStream_t cap_stream = nullptr;   // capture stream (graphs are launched on the caller's stream)
     // optional gradient correction of the smoother: G (n x np2), G^T (np2 x n)
     int64_t np2 = 0;
     const int32_t *g_rowptr = nullptr, *g_cols = nullptr, *gt_rowptr = nullptr, *gt_cols = nullptr;
     const double *g_vals = nullptr, *gt_vals = nullptr;   // caller-owned
-    float *g_vals32 = nullptr, *gt_vals32 = nullptr;      // owned copies for complex64 steps
+    // the same in the packed layout, in the precision of the solver's steps
+    g_shape g_sh{0, 0, 0};
+    int32_t *g_pcol = nullptr, *gt_prp = nullptr, *gt_pcol = nullptr;
+    void *g_pval = nullptr, *gt_pval = nullptr;
     double *dS = nullptr, *dsinv64 = nullptr, *tg = nullptr;
     float *dsinv32 = nullptr;
     // optional learned weights of the smoother (caller-owned complex128):
@@ -692,91 +1263,105 @@ struct emg_solver {
     // SpMV (gradient set), then 4, 8 or 16, with the measured milliseconds per launch
     int gt_lanes = 0;
     float gt_ms[3] = {};
-    struct graphs {
-        std::vector<hipGraphExec_t> exec;
-        const void *vals = nullptr, *inv = nullptr, *mask = nullptr;
-        int64_t np2 = 0;
-        int poly = 1;
-    } gs[2];                      // [0] complex128 steps, [1] complex64 steps
+    // captured steps by the basis vector they start from, as cycles first reach them; every buffer
+    // they name is the solver's own, so only another gradient or degree makes them stale
+    std::vector<hipGraphExec_t> exec;
+    hipGraphExec_t tail = nullptr;   // the preconditioner at a cycle's end
+    int64_t exec_np2 = 0;
+    int exec_poly = 0;
 };
 static constexpr int POLY_MAX = 16;
 
+static void drop_graphs(emg_solver *s) {
+    for (hipGraphExec_t e : s->exec)
+        if (e != nullptr) (void)hipGraphExecDestroy(e);
+    s->exec.clear();
+    if (s->tail != nullptr) (void)hipGraphExecDestroy(s->tail);
+    s->tail = nullptr;
+}
+
 static void free_solver(emg_solver *s) {
     if (!s) return;
-    for (auto &g : s->gs)
-        for (hipGraphExec_t e : g.exec) (void)hipGraphExecDestroy(e);
-    void *ps[] = {s->vals32, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial, s->h, s->nrm,
-                  s->arn, s->pn, s->flag, s->g_vals32, s->gt_vals32, s->dS, s->dsinv64, s->tg, s->dsinv32,
-                  s->poly_c, s->pp, s->pt, s->py, s->pu};
+    drop_graphs(s);
+    void *ps[] = {s->acol, s->kre, s->kim, s->row_flag, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial,
+                  s->h, s->nrm, s->arn, s->pn, s->gram, s->flag, s->g_pcol, s->gt_prp, s->gt_pcol, s->g_pval,
+                  s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32, s->poly_c, s->pp, s->pt, s->py, s->pu};
     for (void *p : ps) (void)hipFree(p);
-    if (s->res_host) (void)hipHostFree(s->res_host);
-    if (s->cap) (void)hipStreamDestroy(s->cap);
+    if (s->host) (void)hipHostFree(s->host);
+    if (s->cap_stream) (void)hipStreamDestroy(s->cap_stream);
     delete s;
 }
 
-// The smoother: 2x2 block Jacobi, plus the gradient correction when set.
-template <typename R>
-static void apply_prec(emg_solver *s, const R *inv, const R *x, R *y, hipStream_t st) {
+// The smoother in the caller's layout and complex128 (the Arnoldi probe): 2x2 block Jacobi, plus the
+// gradient correction when set.
+static void apply_prec_std(emg_solver *s, const double *x, double *y, hipStream_t st) {
     if (s->np2 > 0) {
-        const R *gv = sizeof(R) == 8 ? reinterpret_cast<const R *>(s->g_vals) : reinterpret_cast<const R *>(s->g_vals32);
-        const R *gtv = sizeof(R) == 8 ? reinterpret_cast<const R *>(s->gt_vals) : reinterpret_cast<const R *>(s->gt_vals32);
-        const R *dsi = sizeof(R) == 8 ? reinterpret_cast<const R *>(s->dsinv64) : reinterpret_cast<const R *>(s->dsinv32);
-        R *t = reinterpret_cast<R *>(s->tg);
-        launch_gt<R>(st, s->gt_lanes, s->np2, s->gt_rowptr, s->gt_cols, gtv, dsi, x, t);
-        k_bj_grad_apply<R><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, inv, x, s->g_rowptr, s->g_cols, gv, t, y);
+        launch_gt(st, s->np2, s->gt_rowptr, s->gt_cols, s->gt_vals, s->dsinv64, x, s->tg);
+        k_bj_grad_apply<<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->inv64, x, s->g_rowptr, s->g_cols,
+                                                                    s->g_vals, s->tg, y);
     } else {
-        k_bj_apply<R><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, inv, x, y);
+        k_bj_apply<<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->inv64, x, y);
     }
 }
 
-
-// y = c[0] x   (c: complex128 coefficients on the device)
+// The smoother in the solver's layout: y = M (xs x), xs a scale on the device or NULL.
 template <typename R>
-__global__ void __launch_bounds__(RB) k_poly_first(int64_t n, const double *__restrict__ c, const R *__restrict__ x,
-                                                   R *__restrict__ y) {
-    const double cr = c[0], ci = c[1];
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n; e += (int64_t)gridDim.x * RB) {
-        const cx<R> v = ld(x, e);
-        st(y, e, cx<R>((R)(cr * v.re - ci * v.im), (R)(cr * v.im + ci * v.re)));
+static void apply_prec(emg_solver *s, const R *x, const double *xs, R *y, hipStream_t st) {
+    const bool grad = s->np2 > 0;
+    const R *inv = sizeof(R) == 8 ? reinterpret_cast<const R *>(s->inv64) : reinterpret_cast<const R *>(s->inv32);
+    R *t = reinterpret_cast<R *>(s->tg);
+    if (grad) {
+        const R *dsi = sizeof(R) == 8 ? reinterpret_cast<const R *>(s->dsinv64) : reinterpret_cast<const R *>(s->dsinv32);
+        launch_gt_pk<R>(st, s->gt_lanes, s->np2, s->gt_prp, s->gt_pcol, static_cast<const R *>(s->gt_pval), dsi, x, xs, t);
     }
+    k_bj_grad_pk<R><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, inv, x, xs, s->g_sh, grad ? s->g_pcol : nullptr,
+                                                                static_cast<const R *>(s->g_pval), t, y);
 }
-// p = q - c[i] t ;  y += c[i+1] p   (q may be p)
-template <typename R>
-__global__ void __launch_bounds__(RB) k_poly_step(int64_t n, const double *__restrict__ c, int i, const R *q,
-                                                  const R *__restrict__ t, R *p, R *__restrict__ y) {
-    const double ar = c[2 * i], ai = c[2 * i + 1], br = c[2 * i + 2], bi = c[2 * i + 3];
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n; e += (int64_t)gridDim.x * RB) {
-        const cx<R> qv = ld(q, e), tv = ld(t, e), yv = ld(y, e);
-        const double pr = qv.re - (ar * tv.re - ai * tv.im), pi = qv.im - (ar * tv.im + ai * tv.re);
-        st(p, e, cx<R>((R)pr, (R)pi));
-        st(y, e, cx<R>((R)(yv.re + br * pr - bi * pi), (R)(yv.im + br * pi + bi * pr)));
+
+// A product with the packed matrix; L lanes per entity.
+template <typename R, int EP, bool STD>
+static void spmv_pk(emg_solver *s, int L, const R *x, const sp_args<R> &a, hipStream_t st) {
+    launch_spmv_pk<R, EP, STD>(st, L, s->n_ent, s->rowptr, s->acol, static_cast<const R *>(s->kre),
+                               static_cast<const R *>(s->kim), s->row_flag, x, a);
+}
+
+// Lanes per entity for vectors in the caller's layout, whose two gathers per block favour few: 8 / 16
+// lanes take 116 / 141 us (complex64, air), 185 / 193 (complex64, lossy), 208 / 237 and 318 / 346
+// (complex128) on the posts box at 80 x 40 x 16 hexes, and 8 is within 2 % of the best down to 2,000 tets.
+static constexpr int STD_LANES = 8;
+
+// y = K x, or b - K x, in complex128 and the caller's layout: the packed planes where they are
+// complex128 (precision 64), else the caller's CSR values.
+static void spmv_std(emg_solver *s, const double *x, const double *b, double *y, hipStream_t st) {
+    if (s->precision == 64) {
+        sp_args<double> a{b, y, nullptr, nullptr, 0, nullptr};
+        if (b != nullptr) spmv_pk<double, SP_RESID, true>(s, STD_LANES, x, a, st);
+        else spmv_pk<double, SP_Y, true>(s, STD_LANES, x, a, st);
+    } else {
+        launch_spmv_blk(st, s->n, s->nnz, s->rowptr, s->cols, s->vals, s->mask, x, b, y, s->lanes[0]);
     }
 }
 
 // The preconditioner: the smoother M, or with a polynomial of degree d > 1,
 // M p(K M) x evaluated as  y = c_0 x, q_0 = x;  q_{i+1} = q_i - c_i K M q_i,
 // y += c_{i+1} q_{i+1}  (i < d-1);  out = M y.  d - 1 extra SpMVs and d - 1
-// extra smoother applications per call.
+// extra smoother applications per call; the updates of q and y follow each product in
+// its own launch (SP_POLY), which at 19,664 DOFs saves the 2.7 us launch they took
+// after every product and at any size the pass over t = K M q.
 template <typename R>
-static void apply_prec_poly(emg_solver *s, const R *vals, const R *inv, const R *x, R *out, hipStream_t st) {
+static void apply_prec_poly(emg_solver *s, const R *x, const double *xs, R *out, hipStream_t st) {
     if (s->poly_deg <= 1) {
-        apply_prec<R>(s, inv, x, out, st);
+        apply_prec<R>(s, x, xs, out, st);
         return;
     }
-    const int64_t n = s->n;
-    const unsigned g = (unsigned)std::min<int64_t>((n + RB - 1) / RB, 2048);
-    R *pp = reinterpret_cast<R *>(s->pp), *pt = reinterpret_cast<R *>(s->pt);
-    R *py = reinterpret_cast<R *>(s->py), *pu = reinterpret_cast<R *>(s->pu);
-    k_poly_first<R><<<g, RB, 0, st>>>(n, s->poly_c, x, py);
-    const R *q = x;
+    R *pp = reinterpret_cast<R *>(s->pp), *py = reinterpret_cast<R *>(s->py), *pu = reinterpret_cast<R *>(s->pu);
     for (int i = 0; i < s->poly_deg - 1; i++) {
-        apply_prec<R>(s, inv, q, pu, st);
-        launch_spmv_blk<R>(st, n, s->nnz, s->rowptr, s->cols, vals, s->mask, pu, nullptr, pt, s->lanes[sizeof(R) == 4],
-                           sizeof(R) == 8);
-        k_poly_step<R><<<g, RB, 0, st>>>(n, s->poly_c, i, q, pt, pp, py);
-        q = pp;
+        const R *q = i == 0 ? x : pp;
+        const double *qs = i == 0 ? xs : nullptr;
+        apply_prec<R>(s, q, qs, pu, st);
+        spmv_pk<R, SP_POLY, false>(s, s->lanes[sizeof(R) == 4], pu, sp_args<R>{q, py, pp, s->poly_c, i, qs}, st);
     }
-    apply_prec<R>(s, inv, py, out, st);
+    apply_prec<R>(s, py, nullptr, out, st);
 }
 
 // Blocks per tile of the multi-dot: about 2048 blocks in total, so each block
@@ -784,23 +1369,48 @@ static void apply_prec_poly(emg_solver *s, const R *vals, const R *inv, const R 
 static int mdot_blocks(int64_t n, int nv) {
     const int ntile = (nv + DT - 1) / DT;
     const int64_t cap = std::max<int64_t>(64, 2048 / ntile);
-    return (int)std::max<int64_t>(1, std::min<int64_t>({(n + RB - 1) / RB, 1024, cap}));
+    return (int)std::max<int64_t>(1, std::min<int64_t>({(n / 2 + RB - 1) / RB, 1024, cap}));
 }
 
-// Offsets (in doubles) into the device Arnoldi state for restart length m.
+// Offsets (in doubles) into the device Arnoldi state for m steps.
 struct arn_off {
-    int64_t H, cs, sn, g, res, inv, total;
+    int64_t H, cs, sn, g, fin, res, sc, qp, kept, total;
     explicit arn_off(int m) {
-        H = 0;                                  // column j at 2 * j * (m + 1), rows 0..m
+        H = 0;                                  // column t at 2 t (m + 1), rows 0 .. t
         cs = 2 * (int64_t)m * (m + 1);
         sn = cs + 2 * m;
         g = sn + 2 * m;                         // m + 1 complex
-        res = g + 2 * (m + 1);                  // |g[j+1]| after step j
-        inv = res + m;                          // 1 / ||new vector|| of the last step
-        total = inv + 8;
+        fin = g + 2 * (m + 1);                  // g[t] as step t leaves it, m complex
+        res = fin + 2 * m;                      // |g[t+1]| after step t
+        sc = res + m;                           // sc[j]: basis vector j is sc[j] V_j
+        qp = sc + m + 1;                        // outside directions of the kept cycles, m + 1 complex,
+        kept = qp + 2 * (m + 1);                // then the kept_dev that says where they are (one upload)
+        total = kept + sizeof(kept_dev) / sizeof(double) + 1;
     }
 };
-static constexpr int CHUNK_IT = 10;   // Arnoldi steps per captured graph
+// Offsets (in doubles) into the pinned host memory: what k_arn_report and others tell the host (a
+// cycle's end needs no copies), then the staging of small uploads.
+struct host_off {
+    int64_t H, cs, sn, g, sc, res, h0, norm, y, qp, kept, total;
+    explicit host_off(int m) {
+        H = 0;                                  // as arn_off
+        cs = 2 * (int64_t)m * (m + 1);
+        sn = cs + 2 * m;
+        g = sn + 2 * m;
+        sc = g + 2 * (m + 1);
+        res = sc + m + 1;                       // |g[t+1]| after step t
+        h0 = res + m;                           // coefficients of a cycle's start vector in the kept spaces
+        norm = h0 + 2 * (m + 1);                // squared norms
+        y = norm + 2;
+        qp = y + 2 * (m + 1);
+        kept = qp + 2 * (m + 1);                // right behind qp, as on the device
+        total = kept + sizeof(kept_dev) / sizeof(double) + 1;
+    }
+};
+// Arnoldi steps between two looks of the host at the residual estimates.  A look costs about 20 us
+// and a cycle of about 40 steps overruns its end by half a chunk on average, so the best length is
+// about sqrt(1600 us / step): a step takes 0.1 ms at 20,000 DOFs and over 1 ms at a million.
+static int chunk_it(int64_t n) { return n < 400000 ? 4 : 2; }
 
 // Sets *bad when the CSR is not on an entity pattern (the layout k_spmv_blk and
 // the smoother rely on): rows (0, e) and (1, e) list the same column entities
@@ -842,22 +1452,38 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
     s->n = n; s->nnz = nnz; s->n_ent = n / 2; s->restart = restart; s->precision = precision;
     s->rowptr = d_rowptr; s->cols = d_cols;
     const size_t es = precision == 64 ? 16 : 8;   // bytes per complex element of the basis
-    s->nblk = (int)std::min<int64_t>((n + RB - 1) / RB, 1024);
-    const int ntile = (restart + 1 + DT - 1) / DT;
+    s->nblk = (int)std::min<int64_t>((n / 2 * maxpy_split(n) + RB - 1) / RB, 1024);
     hipError_t e = hipSuccess;
     auto A = [&](void **p, size_t bytes) { if (e == hipSuccess) e = hipMalloc(p, bytes); };
-    A((void **)&s->V, (size_t)(restart + 1) * n * es);
+    // complex64 refinement cycles keep up to two restart lengths of basis vectors (gmres_cycle), the
+    // bytes of the complex128 basis of one; where that does not fit, one
+    s->cap = precision == 32 ? std::min(2 * restart, 500) : restart;
+    A((void **)&s->V, (size_t)(s->cap + 1) * n * es);
+    if (e == hipErrorOutOfMemory && s->cap > restart) {
+        (void)hipGetLastError();
+        e = hipSuccess;
+        s->cap = restart;
+        A((void **)&s->V, (size_t)(s->cap + 1) * n * es);
+    }
+    const int ntile = (s->cap + 1 + DT - 1) / DT;
     A((void **)&s->w, n * 16); A((void **)&s->z, n * 16); A((void **)&s->r, n * 16); A((void **)&s->d, n * 16);
-    A((void **)&s->partial, (size_t)ntile * s->nblk * DT * 2 * sizeof(double) + 1024 * sizeof(double));
-    A((void **)&s->h, 3 * 2 * 512 * sizeof(double));   // h pass 1 | h pass 2 | y
+    A((void **)&s->partial, ((size_t)2 * ntile * 1024 * DT * 2 + 1024) * sizeof(double));
+    A((void **)&s->gram, (size_t)(s->cap + 1) * (s->cap + 1) * 16);
+    A((void **)&s->h, 4 * 2 * 512 * sizeof(double));   // dots | corrected | the part subtracted | y
     A((void **)&s->nrm, 4 * sizeof(double));
     A((void **)&s->inv64, s->n_ent * 4 * 16);
-    A((void **)&s->arn, arn_off(restart).total * sizeof(double));
+    A((void **)&s->arn, arn_off(s->cap).total * sizeof(double));
     A((void **)&s->pn, 1024 * sizeof(double));
     A((void **)&s->flag, 8 * sizeof(double));
-    if (e == hipSuccess) e = hipHostMalloc((void **)&s->res_host, (restart + 8) * sizeof(double), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->cap, hipStreamNonBlocking);
-    if (precision == 32) { A((void **)&s->inv32, s->n_ent * 4 * 8); A((void **)&s->vals32, nnz * 8); }
+    if (e == hipSuccess) e = hipHostMalloc((void **)&s->host, host_off(s->cap).total * sizeof(double), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->cap_stream, hipStreamNonBlocking);
+    if (precision == 32) A((void **)&s->inv32, s->n_ent * 4 * 8);
+    A((void **)&s->acol, (size_t)(nnz > 0 ? nnz : 4) / 4 * sizeof(int32_t));
+    A(&s->kre, (size_t)nnz * es / 2);
+    A(&s->kim, (size_t)nnz * es / 2);
+    A((void **)&s->row_flag, s->n_ent);
+    if (e == hipSuccess) s->kept = reinterpret_cast<kept_dev *>(s->arn + arn_off(s->cap).kept);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&s->host_dev, s->host, 0);
     A((void **)&s->poly_c, 2 * POLY_MAX * sizeof(double));
     A((void **)&s->pp, n * 16); A((void **)&s->pt, n * 16); A((void **)&s->py, n * 16); A((void **)&s->pu, n * 16);
     if (e != hipSuccess) {
@@ -888,6 +1514,14 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
                        "nnz/2 after row e); pass the full unreduced matrix and the PEC mask");
         free_solver(s);
         return -1;
+    }
+    k_pack_cols<<<(unsigned)((s->n_ent * SUB + 255) / 256), 256>>>(s->n_ent, d_rowptr, d_cols, s->acol);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) {
+        emg::set_error(std::string("emg_solver_create: packing the pattern: ") + hipGetErrorString(e));
+        free_solver(s);
+        return -2;
     }
     *out = s;
     return 0;
@@ -920,115 +1554,112 @@ __global__ void __launch_bounds__(RB) k_scale_tables(int64_t n_ent, const double
     }
 }
 
-// Autotuner of the blocked SpMV: each lanes-per-entity variant (4, 8, 16, 32) runs
-// once untimed and five times between HIP events on the solver's first matrix, in
-// the precision the solver's steps use; the fastest is kept for the solver's life
-// (the sparsity pattern fixes the row lengths that decide it).  Vectors: zeroed
-// solver work buffers.  EMG_SPMV_BLK_LANES, when set, overrides the search.
-static const int TUNE_LANES[4] = {4, 8, 16, 32};
-
-template <typename R>
-static int tune_spmv_one(emg_solver *s, const R *vals, int slot, hipStream_t st) {
+// Autotuners: each candidate shape runs eight times in a captured graph between HIP events, after one
+// untimed replay, on the solver's first matrix and zeroed work vectors, and the fastest is kept for the
+// solver's life.  Before each run goes what precedes it in a step (`lead`, whose own time is measured
+// and taken off): launched back to back by itself, a small product finds everything in the L2 it ran
+// from, or takes as long as it takes to issue, and all candidates look alike (the G^T product at 3,072
+// tets takes 5.5 us with 4 lanes and 4.1 us with 16 in the steps, and was chosen now the one way and now
+// the other).
+static constexpr int TUNE_RUNS = 8;
+template <typename LEAD, typename RUN>
+static int tune_lanes(emg_solver *s, int n, const int *cand, LEAD &&lead, RUN &&run, float *ms, int *choice,
+                      hipStream_t st) {
     hipEvent_t ev[2];
     EMG_HIP(hipEventCreate(&ev[0]));
     if (hipEventCreate(&ev[1]) != hipSuccess) {
         (void)hipEventDestroy(ev[0]);
-        emg::set_error("tune_spmv: hipEventCreate failed");
+        emg::set_error("tune_lanes: hipEventCreate failed");
         return -2;
     }
     hipError_t e = hipSuccess;
-    float best = 3.4e38f;
-    int bl = 16;
-    for (int i = 0; i < 4 && e == hipSuccess; i++) {
-        const int L = TUNE_LANES[i];
-        auto run = [&]() {
-            launch_spmv_blk<R>(st, s->n, s->nnz, s->rowptr, s->cols, vals, s->mask, reinterpret_cast<const R *>(s->z),
-                               nullptr, reinterpret_cast<R *>(s->pp), L, sizeof(R) == 8);
-        };
-        run();
-        e = hipEventRecord(ev[0], st);
-        for (int r = 0; r < 5; r++) run();
+    float base = 0.f;
+    for (int i = -1; i < n && e == hipSuccess; i++) {   // -1: the lead alone
+        hipGraph_t graph = nullptr;
+        hipGraphExec_t exec = nullptr;
+        float t = 0.f;
+        e = hipStreamBeginCapture(s->cap_stream, hipStreamCaptureModeThreadLocal);
+        if (e != hipSuccess) break;
+        for (int r = 0; r < TUNE_RUNS; r++) {
+            lead(s->cap_stream);
+            if (i >= 0) run(cand[i], s->cap_stream);
+        }
+        e = hipStreamEndCapture(s->cap_stream, &graph);
+        if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        if (graph != nullptr) (void)hipGraphDestroy(graph);
+        if (e == hipSuccess) e = hipGraphLaunch(exec, st);
+        if (e == hipSuccess) e = hipEventRecord(ev[0], st);
+        if (e == hipSuccess) e = hipGraphLaunch(exec, st);
         if (e == hipSuccess) e = hipEventRecord(ev[1], st);
         if (e == hipSuccess) e = hipEventSynchronize(ev[1]);
-        float ms = 0.f;
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev[0], ev[1]);
-        ms /= 5.f;
-        s->tune_ms[slot][i] = ms;
-        if (e == hipSuccess && ms < best) { best = ms; bl = L; }
+        if (e == hipSuccess) e = hipEventElapsedTime(&t, ev[0], ev[1]);
+        if (exec != nullptr) (void)hipGraphExecDestroy(exec);
+        t /= (float)TUNE_RUNS;
+        if (i < 0) base = t; else ms[i] = std::max(t - base, 1e-6f);
     }
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
     EMG_HIP(e);
-    s->lanes[slot] = bl;
+    *choice = cand[std::min_element(ms, ms + n) - ms];
     return 0;
 }
 
-// The smoother's G^T product with 4, 8 and 16 lanes per row, timed like the SpMV (one
-// untimed and five timed launches, in the precision of the solver's steps, on zeroed
-// vectors); EMG_GT_LANES (4, 8 or 16) overrides.  Needs the gradient correction set.
+// Lanes per entity of the solver's products: complex128 (slot 0: the packed matrix for precision 64,
+// the caller's CSR for precision 32) and complex64 (slot 1); EMG_SPMV_BLK_LANES overrides.
+static const int TUNE_LANES[4] = {4, 8, 16, 32};
+// Lanes per row of the smoother's G^T product; EMG_GT_LANES (4, 8 or 16) overrides.
 static const int GT_LANES[3] = {4, 8, 16};
 
-static int tune_gt(emg_solver *s, hipStream_t st) {
+template <typename R>
+static int tune_steps(emg_solver *s, hipStream_t st) {
+    R *z = reinterpret_cast<R *>(s->z), *pu = reinterpret_cast<R *>(s->pu), *pp = reinterpret_cast<R *>(s->pp);
+    const int slot = sizeof(R) == 4;
+    EMG_HIP(hipMemsetAsync(z, 0, s->n * 2 * sizeof(R), st));
+    auto product = [&](int L, hipStream_t rs) {
+        spmv_pk<R, SP_Y, false>(s, L, pu, sp_args<R>{nullptr, pp, nullptr, nullptr, 0, nullptr}, rs);
+    };
+    if (getenv("EMG_SPMV_BLK_LANES") != nullptr) {
+        s->lanes[slot] = spmv_blk_lanes();
+    } else {
+        auto smooth = [&](hipStream_t rs) { apply_prec<R>(s, z, nullptr, pu, rs); };
+        if (int rc = tune_lanes(s, 4, TUNE_LANES, smooth, product, s->tune_ms[slot], &s->lanes[slot], st)) return rc;
+    }
     if (s->np2 <= 0) return 0;
     if (const char *env = getenv("EMG_GT_LANES")) {
         const int v = atoi(env);
         s->gt_lanes = (v == 4 || v == 16) ? v : 8;
         return 0;
     }
-    EMG_HIP(hipMemsetAsync(s->z, 0, s->n * 16, st));
-    hipEvent_t ev[2];
-    EMG_HIP(hipEventCreate(&ev[0]));
-    if (hipEventCreate(&ev[1]) != hipSuccess) {
-        (void)hipEventDestroy(ev[0]);
-        emg::set_error("tune_gt: hipEventCreate failed");
-        return -2;
-    }
-    hipError_t e = hipSuccess;
-    float best = 3.4e38f;
-    int bl = 8;
-    for (int i = 0; i < 3 && e == hipSuccess; i++) {
-        const int L = GT_LANES[i];
-        auto run = [&]() {
-            if (s->precision == 32)
-                launch_gt<float>(st, L, s->np2, s->gt_rowptr, s->gt_cols, s->gt_vals32, s->dsinv32,
-                                 reinterpret_cast<const float *>(s->z), reinterpret_cast<float *>(s->tg));
-            else
-                launch_gt<double>(st, L, s->np2, s->gt_rowptr, s->gt_cols, s->gt_vals, s->dsinv64, s->z, s->tg);
-        };
-        run();
-        e = hipEventRecord(ev[0], st);
-        for (int r = 0; r < 5; r++) run();
-        if (e == hipSuccess) e = hipEventRecord(ev[1], st);
-        if (e == hipSuccess) e = hipEventSynchronize(ev[1]);
-        float ms = 0.f;
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev[0], ev[1]);
-        if (e == hipSuccess) e = hipGetLastError();
-        ms /= 5.f;
-        s->gt_ms[i] = ms;
-        if (e == hipSuccess && ms < best) { best = ms; bl = L; }
-    }
-    (void)hipEventDestroy(ev[0]);
-    (void)hipEventDestroy(ev[1]);
-    EMG_HIP(e);
-    s->gt_lanes = bl;
-    return 0;
+    EMG_HIP(hipMemsetAsync(pu, 0, s->n * 2 * sizeof(R), st));
+    auto before = [&](hipStream_t rs) { product(s->lanes[slot], rs); };
+    auto gt = [&](int L, hipStream_t rs) {
+        const R *dsi = slot ? reinterpret_cast<const R *>(s->dsinv32) : reinterpret_cast<const R *>(s->dsinv64);
+        launch_gt_pk<R>(rs, L, s->np2, s->gt_prp, s->gt_pcol, static_cast<const R *>(s->gt_pval), dsi, pp, nullptr,
+                        reinterpret_cast<R *>(s->tg));
+    };
+    return tune_lanes(s, 3, GT_LANES, before, gt, s->gt_ms, &s->gt_lanes, st);
 }
 
 static int tune_spmv(emg_solver *s, hipStream_t st) {
-    if (getenv("EMG_SPMV_BLK_LANES") != nullptr) {
-        s->lanes[0] = s->lanes[1] = spmv_blk_lanes();
-        return tune_gt(s, st);
-    }
-    EMG_HIP(hipMemsetAsync(s->z, 0, s->n * 16, st));
-    int rc = tune_spmv_one<double>(s, s->vals, 0, st);
-    if (rc) return rc;
-    if (s->precision == 32) {
-        rc = tune_spmv_one<float>(s, s->vals32, 1, st);
-        if (rc) return rc;
-    } else {
+    if (s->precision == 64) {
+        if (int rc = tune_steps<double>(s, st)) return rc;
         s->lanes[1] = s->lanes[0];
+        return 0;
     }
-    return tune_gt(s, st);
+    if (getenv("EMG_SPMV_BLK_LANES") != nullptr) {
+        s->lanes[0] = spmv_blk_lanes();
+    } else {
+        EMG_HIP(hipMemsetAsync(s->z, 0, s->n * 16, st));
+        EMG_HIP(hipMemsetAsync(s->r, 0, s->n * 16, st));
+        auto input = [&](hipStream_t rs) {
+            k_pack_vec<double><<<emg::grid_for(s->n_ent, RB), RB, 0, rs>>>(s->n_ent, s->r, 1.0, s->z);
+        };
+        auto csr = [&](int L, hipStream_t rs) {
+            launch_spmv_blk(rs, s->n, s->nnz, s->rowptr, s->cols, s->vals, s->mask, s->z, nullptr, s->pp, L);
+        };
+        if (int rc = tune_lanes(s, 4, TUNE_LANES, input, csr, s->tune_ms[0], &s->lanes[0], st)) return rc;
+    }
+    return tune_steps<float>(s, st);
 }
 
 extern "C" int emg_solver_smoother_tuning(emg_solver *s, int *h_lanes, float *h_ms) {
@@ -1053,7 +1684,13 @@ extern "C" int emg_solver_set_matrix(emg_solver *s, const double *d_vals, const 
     s->vals = d_vals;
     s->mask = d_mask;
     k_bj_setup<<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->rowptr, s->cols, d_vals, d_mask, s->inv64, s->inv32);
-    if (s->precision == 32) k_to_c64_masked<<<2048, RB, 0, st>>>(s->nnz, s->cols, d_mask, d_vals, s->vals32);
+    const unsigned gp = (unsigned)((s->n_ent * SUB + 255) / 256);
+    if (s->precision == 32)
+        k_pack_matrix<float><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, d_vals, d_mask,
+                                                 static_cast<float *>(s->kre), static_cast<float *>(s->kim), s->row_flag);
+    else
+        k_pack_matrix<double><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, d_vals, d_mask,
+                                                  static_cast<double *>(s->kre), static_cast<double *>(s->kim), s->row_flag);
     if (s->np2 > 0) {
         EMG_HIP(hipMemsetAsync(s->dS, 0, s->np2 * 16, st));
         k_gdiag<<<emg::grid_for(s->n, RB), RB, 0, st>>>(s->n, s->rowptr, s->cols, d_vals, d_mask, s->g_rowptr,
@@ -1085,9 +1722,9 @@ extern "C" int emg_solver_set_weights(emg_solver *s, const double *d_we, const d
 extern "C" int emg_solver_smoother_parts(emg_solver *s, const double *d_r, double *d_u, double *d_t, void *stream) {
     EMG_CHECK(s && d_r && d_u, "emg_solver_smoother_parts: null argument");
     hipStream_t st = (hipStream_t)stream;
-    k_bj_apply<double><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->inv64, d_r, d_u);
+    k_bj_apply<<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->inv64, d_r, d_u);
     if (s->np2 > 0 && d_t != nullptr)
-        launch_gt<double>(st, s->gt_lanes, s->np2, s->gt_rowptr, s->gt_cols, s->gt_vals, s->dsinv64, d_r, d_t);
+        launch_gt(st, s->np2, s->gt_rowptr, s->gt_cols, s->gt_vals, s->dsinv64, d_r, d_t);
     EMG_LAUNCH_CHECK();
     return 0;
 }
@@ -1143,13 +1780,13 @@ extern "C" int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0
         double *vj = V + (size_t)j * n * 2, *w = V + (size_t)(j + 1) * n * 2;
         const int nv = j + 1, nbm = mdot_blocks(n, nv);
         const dim3 grid(nbm, (nv + DT - 1) / DT);
-        apply_prec<double>(s, s->inv64, vj, z, st);
-        launch_spmv_blk<double>(st, n, s->nnz, s->rowptr, s->cols, s->vals, s->mask, z, nullptr, w, s->lanes[0]);
+        apply_prec_std(s, vj, z, st);
+        spmv_std(s, z, nullptr, w, st);
         double wn = 0;
         for (int pass = 0; pass < 2; pass++) {
-            k_mdot<double><<<grid, RB, 0, st>>>(n, nv, V, n, w, s->partial, nullptr);
-            k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, s->partial, s->h, 0, nullptr);
-            k_maxpy_norm<double><<<nb, RB, 0, st>>>(n, nv, V, n, s->h, w, s->pn, nullptr);
+            k_mdot<double, 1><<<grid, RB, 0, st>>>(n, nv, V, n, w, nullptr, s->partial);
+            k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, s->partial, nullptr, s->h, nullptr, 0);
+            launch_maxpy<double>(st, nb, n, nv, V, s->h, nullptr, w, s->pn);
             EMG_HIP(hipMemcpyAsync(hh.data(), s->h, 2 * nv * sizeof(double), hipMemcpyDeviceToHost, st));
             wn = host_norm(s->pn);
             for (int i = 0; i < nv; i++) {
@@ -1166,8 +1803,56 @@ extern "C" int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0
     return 0;
 }
 
-__global__ void __launch_bounds__(RB) k_f64_to_f32(int64_t n, const double *__restrict__ a, float *__restrict__ b) {
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n; e += (int64_t)gridDim.x * RB) b[e] = (float)a[e];
+// off[i] = sum of cnt[0 .. i) for i <= n, through the host (once per gradient)
+static int prefix_on_host(const int32_t *d_cnt, int64_t n, int32_t **d_off, int64_t *total, hipStream_t st) {
+    std::vector<int32_t> c(n), o(n + 1, 0);
+    EMG_HIP(hipMemcpyAsync(c.data(), d_cnt, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    EMG_HIP(hipStreamSynchronize(st));
+    int64_t t = 0;
+    for (int64_t i = 0; i < n; i++) {
+        t += c[i];
+        EMG_CHECK(t < ((int64_t)1 << 31), "emg_solver_set_gradient: too many entries");
+        o[i + 1] = (int32_t)t;
+    }
+    EMG_HIP(hipMalloc((void **)d_off, (n + 1) * sizeof(int32_t)));
+    EMG_HIP(hipMemcpyAsync(*d_off, o.data(), (n + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    EMG_HIP(hipStreamSynchronize(st));
+    *total = t;
+    return 0;
+}
+
+template <typename R>
+static int pack_gradient(emg_solver *s, int64_t np2, const int32_t *grp, const int32_t *gcol, const double *gv,
+                         const int32_t *tp, const int32_t *tcol, const double *tv, int32_t *cnt, hipStream_t st) {
+    const int64_t ne = s->n_ent, ns = (ne + 63) / 64;
+    int64_t total = 0;
+    k_g_width<<<(unsigned)ns, 64, 0, st>>>(ne, grp, gcol, cnt);
+    EMG_LAUNCH_CHECK();
+    // the cut between two runs of slices, each as wide as its widest, that leaves the fewest slots
+    std::vector<int32_t> wd(ns), after_max(ns + 1, 0);
+    EMG_HIP(hipMemcpyAsync(wd.data(), cnt, ns * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    EMG_HIP(hipStreamSynchronize(st));
+    for (int64_t i = ns - 1; i >= 0; i--) after_max[i] = std::max(after_max[i + 1], wd[i]);
+    int64_t best = INT64_MAX;
+    int32_t before_max = 0;
+    for (int64_t c = 0; c <= ns; c++) {
+        const int64_t size = c * before_max + (ns - c) * after_max[c];
+        if (size < best) { best = size; s->g_sh = g_shape{c, before_max, after_max[c]}; }
+        if (c < ns) before_max = std::max(before_max, wd[c]);
+    }
+    const int64_t slots = std::max<int64_t>(s->g_sh.first(ns), 1);
+    EMG_HIP(hipMalloc((void **)&s->g_pcol, slots * sizeof(int32_t)));
+    EMG_HIP(hipMalloc(&s->g_pval, slots * 2 * sizeof(R)));
+    k_g_fill<R><<<(unsigned)ns, 64, 0, st>>>(ne, grp, gcol, gv, s->g_sh, s->g_pcol, static_cast<R *>(s->g_pval));
+    k_gt_count<<<emg::grid_for(np2, RB), RB, 0, st>>>(np2, ne, tp, tcol, cnt);
+    EMG_LAUNCH_CHECK();
+    if (int rc = prefix_on_host(cnt, np2, &s->gt_prp, &total, st)) return rc;
+    EMG_HIP(hipMalloc((void **)&s->gt_pcol, std::max<int64_t>(total, 1) * sizeof(int32_t)));
+    EMG_HIP(hipMalloc(&s->gt_pval, std::max<int64_t>(total, 1) * 2 * sizeof(R)));
+    k_gt_fill<R><<<emg::grid_for(np2, RB), RB, 0, st>>>(np2, ne, tp, tcol, tv, s->gt_prp, s->gt_pcol,
+                                                        static_cast<R *>(s->gt_pval));
+    EMG_LAUNCH_CHECK();
+    return 0;
 }
 
 extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t *d_g_rowptr, const int32_t *d_g_cols,
@@ -1189,276 +1874,425 @@ extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t
     EMG_CHECK(nnz_g <= G_ROW_MAX * s->n, "emg_solver_set_gradient: more than 8 entries per row of G");
     // captured step graphs hold the old gradient buffers: drop them before the buffers go
     EMG_HIP(hipStreamSynchronize(st));
-    for (auto &g : s->gs) {
-        for (hipGraphExec_t e : g.exec) (void)hipGraphExecDestroy(e);
-        g.exec.clear();
-    }
-    void *old[] = {s->g_vals32, s->gt_vals32, s->dS, s->dsinv64, s->tg, s->dsinv32};
+    drop_graphs(s);
+    void *old[] = {s->g_pcol, s->g_pval, s->gt_prp, s->gt_pcol, s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32};
     for (void *p : old) (void)hipFree(p);
-    s->g_vals32 = s->gt_vals32 = nullptr;
+    s->g_pcol = s->gt_prp = s->gt_pcol = nullptr;
+    s->g_pval = s->gt_pval = nullptr;
     s->dS = s->dsinv64 = s->tg = nullptr;
     s->dsinv32 = nullptr;
     s->np2 = 0;
-    EMG_HIP(hipMalloc((void **)&s->g_vals32, (size_t)nnz_g * sizeof(float)));
-    EMG_HIP(hipMalloc((void **)&s->gt_vals32, (size_t)nnz_g * sizeof(float)));
     EMG_HIP(hipMalloc((void **)&s->dS, (size_t)np2 * 16));
     EMG_HIP(hipMalloc((void **)&s->dsinv64, (size_t)np2 * 16));
     EMG_HIP(hipMalloc((void **)&s->dsinv32, (size_t)np2 * 8));
     EMG_HIP(hipMalloc((void **)&s->tg, (size_t)np2 * 16));
-    k_f64_to_f32<<<1024, RB, 0, st>>>(nnz_g, d_g_vals, s->g_vals32);
-    k_f64_to_f32<<<1024, RB, 0, st>>>(nnz_g, d_gt_vals, s->gt_vals32);
-    EMG_LAUNCH_CHECK();
+    {
+        int32_t *cnt = nullptr;
+        EMG_HIP(hipMalloc((void **)&cnt, std::max<int64_t>(np2, s->n_ent / 64 + 1) * sizeof(int32_t)));
+        int rc = s->precision == 32 ? pack_gradient<float>(s, np2, d_g_rowptr, d_g_cols, d_g_vals, d_gt_rowptr, d_gt_cols,
+                                                           d_gt_vals, cnt, st)
+                                    : pack_gradient<double>(s, np2, d_g_rowptr, d_g_cols, d_g_vals, d_gt_rowptr, d_gt_cols,
+                                                            d_gt_vals, cnt, st);
+        const hipError_t e = hipStreamSynchronize(st);   // cnt is read by kernels in flight
+        (void)hipFree(cnt);
+        if (rc) return rc;
+        EMG_HIP(e);
+    }
     s->g_rowptr = d_g_rowptr; s->g_cols = d_g_cols; s->g_vals = d_g_vals;
     s->gt_rowptr = d_gt_rowptr; s->gt_cols = d_gt_cols; s->gt_vals = d_gt_vals;
     s->np2 = np2;
     return 0;
 }
 
-// ---- one restarted GMRES solve of K u = rhs (element type R), right preconditioned.
-// On return u holds the solution; returns the iteration count through *iters and
-// the final residual estimate relative to |rhs| through *rel.
 // ---------------------------------------------------------------- device Arnoldi bookkeeping
-__device__ __forceinline__ double block_sum(double v, double *sh) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double t = 0.0;
-    for (int q = 0; q < (int)(blockDim.x >> 6); q++) t += sh[q];
-    return t;
+// A cycle whose first basis vector is t0: g[t0] = beta = *nrm, V_t0 is stored normalised.
+__global__ void k_arn_init(int t0, const double *__restrict__ nrm, double *__restrict__ arn, arn_off o) {
+    if (threadIdx.x == 0) {
+        arn[o.g + 2 * t0] = nrm[0];
+        arn[o.g + 2 * t0 + 1] = 0.0;
+        arn[o.sc + t0] = 1.0;
+    }
 }
 
-// g = (beta, 0, ...), residual estimates cleared; beta = *nrm.
-__global__ void __launch_bounds__(RB) k_arn_init(int m, const double *__restrict__ nrm, double *__restrict__ arn,
-                                                 arn_off o) {
-    for (int i = threadIdx.x; i < 2 * (m + 1); i += RB) arn[o.g + i] = (i == 0) ? nrm[0] : 0.0;
-    for (int i = threadIdx.x; i < m; i += RB) arn[o.res + i] = 0.0;
-}
-
-// Second Gram-Schmidt pass only if the first removed more than 99% of the
-// vector's squared norm (||w after|| < 0.1 ||w before||, with
-// ||w before||^2 = ||w after||^2 + ||h||^2).  The 0.707 threshold of the
-// classical test reorthogonalised nearly every step of these solves without
-// changing their iteration counts; 0.1 keeps the second pass for real
-// cancellation only.
-__global__ void __launch_bounds__(RB) k_arn_check(int nb, const double *__restrict__ pn, const double *__restrict__ h,
-                                                  int nv, double *__restrict__ flag) {
+// out = sum of nb partial sums (one block)
+__global__ void __launch_bounds__(RB) k_sum_partials(int nb, const double *__restrict__ p, double *__restrict__ out) {
     __shared__ double sh[RB / 64];
-    double a = 0.0, b = 0.0;
-    for (int i = threadIdx.x; i < nb; i += RB) a += pn[i];
-    for (int i = threadIdx.x; i < 2 * nv; i += RB) b += h[i] * h[i];
+    double a = 0.0;
+    for (int i = threadIdx.x; i < nb; i += RB) a += p[i];
     a = block_sum(a, sh);
-    b = block_sum(b, sh);
-    if (threadIdx.x == 0) flag[0] = (a < 0.01 * (a + b)) ? 1.0 : 0.0;
+    if (threadIdx.x == 0) *out = a;
 }
 
-// Hessenberg column j = h1 + h2 with ||new vector||, previous rotations, the
-// new rotation, g update, residual estimate |g[j+1]| and 1/||new vector||.
-// The column and the rotations are staged in LDS by the whole block; the
-// rotation chain itself is sequential and runs in registers of one lane.
-__global__ void __launch_bounds__(RB) k_arn_givens(int j, int m, int nb, const double *__restrict__ pn,
-                                                   const double *__restrict__ h1, const double *__restrict__ h2,
+// x -> a x + b, complex: the maps whose composition carries a column through the rotations
+struct affine {
+    cx<double> a, b;
+};
+__device__ __forceinline__ affine after(const affine &l, const affine &e) {   // l after e
+    return affine{cmul(l.a, e.a), cadd(cmul(l.a, e.b), l.b)};
+}
+__device__ __forceinline__ affine shfl_up(const affine &v, int off) {
+    return affine{cx<double>(__shfl_up(v.a.re, off, 64), __shfl_up(v.a.im, off, 64)),
+                  cx<double>(__shfl_up(v.b.re, off, 64), __shfl_up(v.b.im, off, 64))};
+}
+
+// Step t of the cycle that began at basis vector t0: the column h with ||new vector||; rows below t0 (the kept spaces) are stored as they are, the rows of
+// the cycle after the previous rotations; then the new rotation, the update of g, the residual
+// estimate |g[t+1]| and the new vector's scale 1 / norm.
+// The rotations carry x_{i+1} = -s_i x_i + c_i y_{i+1} down the column: a chain of maps x -> a x + b,
+// composed by a scan over the block, two per lane (all |s_i| <= 1: the compositions stay bounded).
+// One lane walking the chain took 70 ns a rotation, 4.8 us a step on average at 31 steps per cycle.
+__global__ void __launch_bounds__(RB) k_arn_givens(int t, int m, int nb, const double *__restrict__ pn,
+                                                   const double *__restrict__ h, const kept_dev *__restrict__ kept,
                                                    double *__restrict__ arn, arn_off o) {
     __shared__ double sh[RB / 64];
-    __shared__ double2 col[512], rot[2 * 512];
+    __shared__ double tot[RB / 64][4];
+    static_assert(2 * RB >= 512, "two rotations per lane cover the longest restart");
+    const int t0 = kept->t0, j = t - t0;   // j rotations
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    double *Hc = arn + o.H + 2 * (int64_t)t * (m + 1);
+    double *cs = arn + o.cs + 2 * t0, *sn = arn + o.sn + 2 * t0, *g = arn + o.g;
+    auto col = [&](int i) { return ld(h, i); };   // row i of the column, of all basis vectors
     double a = 0.0;
     for (int i = threadIdx.x; i < nb; i += RB) a += pn[i];
-    for (int i = threadIdx.x; i <= j; i += RB) col[i] = make_double2(h1[2 * i] + h2[2 * i], h1[2 * i + 1] + h2[2 * i + 1]);
-    const double *cs = arn + o.cs, *sn = arn + o.sn;
-    for (int i = threadIdx.x; i < j; i += RB) {
-        rot[2 * i] = make_double2(cs[2 * i], cs[2 * i + 1]);
-        rot[2 * i + 1] = make_double2(sn[2 * i], sn[2 * i + 1]);
+    for (int i = threadIdx.x; i < t0; i += RB) {
+        const cx<double> v = col(i);
+        Hc[2 * i] = v.re;
+        Hc[2 * i + 1] = v.im;
     }
-    a = block_sum(a, sh);          // contains __syncthreads: col / rot are visible after it
+    cx<double> c[2], s[2], y[2];
+    affine f[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int i = 2 * threadIdx.x + q;
+        f[q] = affine{cx<double>(1.0, 0.0), cx<double>()};
+        if (i < j) {
+            c[q] = cx<double>(cs[2 * i], cs[2 * i + 1]);
+            s[q] = cx<double>(sn[2 * i], sn[2 * i + 1]);
+            y[q] = col(t0 + i + 1);
+            f[q] = affine{cx<double>(-s[q].re, -s[q].im), cmul(c[q], y[q])};
+        }
+    }
+    const cx<double> x0 = col(t0), g0(g[2 * t], g[2 * t + 1]);
+    affine v = after(f[1], f[0]);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const affine u = shfl_up(v, off);
+        if (lane >= off) v = after(v, u);
+    }
+    if (lane == 63) { tot[wave][0] = v.a.re; tot[wave][1] = v.a.im; tot[wave][2] = v.b.re; tot[wave][3] = v.b.im; }
+    affine before = shfl_up(v, 1);
+    if (lane == 0) before = affine{cx<double>(1.0, 0.0), cx<double>()};
+    a = block_sum(a, sh);          // contains __syncthreads: tot is visible after it
+    cx<double> x = x0, last = x0;
+    for (int w = 0; w < RB / 64; w++) {
+        last = cadd(cmul(cx<double>(tot[w][0], tot[w][1]), last), cx<double>(tot[w][2], tot[w][3]));
+        if (w + 1 == wave) x = last;
+    }
+    x = cadd(cmul(before.a, x), before.b);
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int i = 2 * threadIdx.x + q;
+        if (i < j) {   // conj(c) x + conj(s) y
+            Hc[2 * (t0 + i)] = c[q].re * x.re + c[q].im * x.im + s[q].re * y[q].re + s[q].im * y[q].im;
+            Hc[2 * (t0 + i) + 1] = c[q].re * x.im - c[q].im * x.re + s[q].re * y[q].im - s[q].im * y[q].re;
+            x = cadd(cmul(f[q].a, x), f[q].b);
+        }
+    }
     if (threadIdx.x != 0) return;
-    const double hn = sqrt(a);
-    // carry = current entry i of the column after rotations 0..i-1
-    double xr = col[0].x, xi = col[0].y;
-    for (int i = 0; i < j; i++) {
-        const double2 c = rot[2 * i], sv = rot[2 * i + 1], y = col[i + 1];
-        // col[i] = conj(c) x + conj(s) y ; carry = -s x + c y
-        col[i] = make_double2(c.x * xr + c.y * xi + sv.x * y.x + sv.y * y.y,
-                              c.x * xi - c.y * xr + sv.x * y.y - sv.y * y.x);
-        const double nr = -(sv.x * xr - sv.y * xi) + (c.x * y.x - c.y * y.y);
-        const double ni = -(sv.x * xi + sv.y * xr) + (c.x * y.y + c.y * y.x);
-        xr = nr;
-        xi = ni;
-    }
+    const double hn = sqrt(a), xr = last.re, xi = last.im;
     // new rotation from (x, hn)
     const double den = sqrt(xr * xr + xi * xi + hn * hn);
-    double cr = 1.0, ci = 0.0, sr = 0.0, si = 0.0;
+    double cr = 1.0, ci = 0.0, sr = 0.0;
     if (den > 0.0) { cr = xr / den; ci = xi / den; sr = hn / den; }
-    double *Hc = arn + o.H + 2 * (int64_t)j * (m + 1);
-    for (int i = 0; i < j; i++) { Hc[2 * i] = col[i].x; Hc[2 * i + 1] = col[i].y; }
-    Hc[2 * j] = cr * xr + ci * xi + sr * hn;          // conj(c) x + conj(s) hn
-    Hc[2 * j + 1] = cr * xi - ci * xr;
-    Hc[2 * j + 2] = 0.0;
-    Hc[2 * j + 3] = 0.0;
-    double *csw = arn + o.cs, *snw = arn + o.sn, *g = arn + o.g;
-    csw[2 * j] = cr; csw[2 * j + 1] = ci;
-    snw[2 * j] = sr; snw[2 * j + 1] = si;
-    const double gr = g[2 * j], gi = g[2 * j + 1];
-    g[2 * j + 2] = -(sr * gr - si * gi);
-    g[2 * j + 3] = -(sr * gi + si * gr);
-    g[2 * j] = cr * gr + ci * gi;
-    g[2 * j + 1] = cr * gi - ci * gr;
-    arn[o.res + j] = sqrt(g[2 * j + 2] * g[2 * j + 2] + g[2 * j + 3] * g[2 * j + 3]);
-    arn[o.inv] = hn > 0.0 ? 1.0 / hn : 0.0;
+    Hc[2 * t] = cr * xr + ci * xi + sr * hn;          // conj(c) x + conj(s) hn
+    Hc[2 * t + 1] = cr * xi - ci * xr;
+    cs[2 * j] = cr;
+    cs[2 * j + 1] = ci;
+    sn[2 * j] = sr;
+    sn[2 * j + 1] = 0.0;
+    const double er = -sr * g0.re, ei = -sr * g0.im;
+    g[2 * t + 2] = er;
+    g[2 * t + 3] = ei;
+    double *fin = arn + o.fin + 2 * t;   // g[t] after its rotation
+    fin[0] = cr * g0.re + ci * g0.im;
+    fin[1] = cr * g0.im - ci * g0.re;
+    arn[o.sc + t + 1] = hn > 0.0 ? 1.0 / hn : 0.0;
+    arn[o.res + t] = sqrt(er * er + ei * ei);
 }
 
-template <typename R>
-__global__ void __launch_bounds__(RB) k_scale_inv(int64_t n, const double *__restrict__ inv, R *__restrict__ v) {
-    const double s = inv[0];
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n; e += (int64_t)gridDim.x * RB) {
-        const cx<R> a = ld(v, e);
-        st(v, e, cx<R>((R)(a.re * s), (R)(a.im * s)));
+// What the host wants to know of steps t .. t + gridDim.x - 1, one block each, into pinned memory.
+// One launch per look: written by each step, the stores across PCIe held up every one by 2.5 us.
+__global__ void __launch_bounds__(RB) k_arn_report(int t, int m, const double *__restrict__ arn, arn_off o,
+                                                   double *__restrict__ hst, host_off ho) {
+    t += blockIdx.x;
+    const int64_t c = 2 * (int64_t)t * (m + 1);
+    for (int i = threadIdx.x; i < 2 * (t + 1); i += RB) hst[ho.H + c + i] = arn[o.H + c + i];
+    if (threadIdx.x < 2) {
+        const int i = 2 * t + threadIdx.x;
+        hst[ho.cs + i] = arn[o.cs + i];
+        hst[ho.sn + i] = arn[o.sn + i];
+        hst[ho.g + i] = arn[o.fin + i];
     }
+    if (threadIdx.x == 2) hst[ho.sc + t + 1] = arn[o.sc + t + 1];
+    if (threadIdx.x == 3) hst[ho.res + t] = arn[o.res + t];
 }
 
-// One Arnoldi step j: v_{j+1} = K M^{-1} v_j, CGS (second pass decided on the
-// device), Hessenberg/Givens update, normalisation.  Only kernel launches, so
-// it can be captured.
+// Takes the parts along the nv basis vectors (of kept cycles: along their ranges) out of w, after
+// bringing the last vector's Gram column up: coefficients in h, partial squared norms of what is left.
 template <typename R>
-static void enqueue_step(emg_solver *s, const R *vals, const R *inv, int j, hipStream_t st) {
+static void orthogonalise(emg_solver *s, int nv, R *w, double *norms, double *h, hipStream_t st) {
     const int64_t n = s->n;
-    const int m = s->restart, nb = s->nblk, nv = j + 1;
+    const arn_off o(s->cap);
+    const double *sc = s->arn + o.sc, *qp = s->arn + o.qp;
+    const R *V = reinterpret_cast<const R *>(s->V);
+    const int nbm = mdot_blocks(n, nv), ldg = s->cap + 1;
+    double *dots = s->h, *c = s->h + 2 * 512;
+    k_mdot<R, 2><<<dim3(nbm, (nv + DT - 1) / DT), RB, 0, st>>>(n, nv, V, n, w, V + (size_t)(nv - 1) * n * 2, s->partial);
+    k_mdot_finish<<<dim3(nv, 2), 256, 0, st>>>(nv, nbm, s->partial, sc, dots, s->gram, ldg);
+    k_gram_correct<<<(nv + 15) / 16, RB, 0, st>>>(nv, dots, s->gram, ldg, s->kept, qp, c);
+    launch_maxpy<R>(st, s->nblk, n, nv, V, c, sc, w, norms, s->kept, qp, h);
+}
+
+// One Arnoldi step t: v_{t+1} = K M^{-1} v_t, classical Gram-Schmidt with the basis' Gram matrix
+// (k_gram_correct) and the Hessenberg/Givens update.  Basis vector i is kept as it came out of the
+// projection, with its scale sc[i] = 1 / norm beside it: every reader multiplies by it, and the
+// pass over the new vector that normalised it is gone.  Only kernel launches, so it can be
+// captured: 23 of them at degree 6 with the gradient correction (33 before, at 19,664 DOFs 174 us
+// of kernels that take 2.5 us and more each whatever their size).
+template <typename R>
+static void enqueue_step(emg_solver *s, int t, hipStream_t st) {
+    const int64_t n = s->n;
+    const int m = s->cap, nb = s->nblk, nv = t + 1;
     R *V = reinterpret_cast<R *>(s->V);
     R *z = reinterpret_cast<R *>(s->z);
-    R *vj = V + (size_t)j * n * 2, *vn = V + (size_t)(j + 1) * n * 2;
-    double *h1 = s->h, *h2 = s->h + 2 * 512;
+    R *vt = V + (size_t)t * n * 2, *vn = V + (size_t)(t + 1) * n * 2;
     const arn_off o(m);
-    const int nbm = mdot_blocks(n, nv);
-    const dim3 grid(nbm, (nv + DT - 1) / DT);
-    apply_prec_poly<R>(s, vals, inv, vj, z, st);
-    // the complex64 copy has its masked columns zeroed (k_to_c64_masked)
-    launch_spmv_blk<R>(st, n, s->nnz, s->rowptr, s->cols, vals, s->mask, z, nullptr, vn, s->lanes[sizeof(R) == 4],
-                       sizeof(R) == 8);
-    k_mdot<R><<<grid, RB, 0, st>>>(n, nv, V, n, vn, s->partial, nullptr);
-    k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, s->partial, h1, 0, nullptr);
-    k_maxpy_norm<R><<<nb, RB, 0, st>>>(n, nv, V, n, h1, vn, s->pn, nullptr);
-    k_arn_check<<<1, RB, 0, st>>>(nb, s->pn, h1, nv, s->flag);
-    k_mdot<R><<<grid, RB, 0, st>>>(n, nv, V, n, vn, s->partial, s->flag);
-    k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, s->partial, h2, 0, s->flag);
-    k_maxpy_norm<R><<<nb, RB, 0, st>>>(n, nv, V, n, h2, vn, s->pn, s->flag);
-    k_arn_givens<<<1, RB, 0, st>>>(j, m, nb, s->pn, h1, h2, s->arn, o);
-    k_scale_inv<R><<<nb, RB, 0, st>>>(n, s->arn + o.inv, vn);
+    apply_prec_poly<R>(s, vt, s->arn + o.sc + t, z, st);
+    spmv_pk<R, SP_Y, false>(s, s->lanes[sizeof(R) == 4], z, sp_args<R>{nullptr, vn, nullptr, nullptr, 0, nullptr}, st);
+    double *h = s->h + 4 * 512;
+    orthogonalise<R>(s, nv, vn, s->pn, h, st);
+    k_arn_givens<<<1, RB, 0, st>>>(t, m, nb, s->pn, h, s->kept, s->arn, o);
 }
 
-// Capture the m steps of a restart cycle as graphs of CHUNK_IT steps (once per
-// solver, precision and matrix/preconditioner/mask buffers).
-template <typename R>
-static int ensure_graphs(emg_solver *s, const R *vals, const R *inv) {
-    auto &g = s->gs[sizeof(R) == 8 ? 0 : 1];
-    if (!g.exec.empty() && g.vals == vals && g.inv == inv && g.mask == s->mask && g.np2 == s->np2 &&
-        g.poly == s->poly_deg)
-        return 0;
-    for (hipGraphExec_t e : g.exec) (void)hipGraphExecDestroy(e);
-    g.exec.clear();
-    const int m = s->restart;
-    for (int c0 = 0; c0 < m; c0 += CHUNK_IT) {
-        EMG_HIP(hipStreamBeginCapture(s->cap, hipStreamCaptureModeThreadLocal));
-        for (int j = c0; j < std::min(m, c0 + CHUNK_IT); j++) enqueue_step<R>(s, vals, inv, j, s->cap);
-        hipGraph_t graph = nullptr;
-        EMG_HIP(hipStreamEndCapture(s->cap, &graph));
-        hipGraphExec_t exec = nullptr;
-        const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        EMG_HIP(e);
-        g.exec.push_back(exec);
-    }
-    g.vals = vals;
-    g.inv = inv;
-    g.mask = s->mask;
-    g.np2 = s->np2;
-    g.poly = s->poly_deg;
+// Captures what `fill` enqueues as one graph.
+template <typename FN>
+static int capture(emg_solver *s, FN &&fill, hipGraphExec_t *out) {
+    *out = nullptr;
+    EMG_HIP(hipStreamBeginCapture(s->cap_stream, hipStreamCaptureModeThreadLocal));
+    fill(s->cap_stream);
+    hipGraph_t graph = nullptr;
+    EMG_HIP(hipStreamEndCapture(s->cap_stream, &graph));
+    const hipError_t e = hipGraphInstantiate(out, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    if (e != hipSuccess) *out = nullptr;
+    EMG_HIP(e);
     return 0;
 }
 
+// Step t as a graph, captured when a cycle first gets to it (few get to the end of the basis), or
+// with t = -1 the preconditioner that closes a cycle: z = M p(K M) w.
 template <typename R>
-static int gmres_core(emg_solver *s, const R *vals, const R *inv, const R *rhs, R *u, double tol, int maxiter,
-                      int *iters, double *rel, hipStream_t st) {
-    const int64_t n = s->n;
-    const int m = s->restart;
-    const int nb = s->nblk;
-    const arn_off o(m);
-    R *V = reinterpret_cast<R *>(s->V);
-    R *w = reinterpret_cast<R *>(s->w);
-    R *z = reinterpret_cast<R *>(s->z);
-    auto prec = [&](const R *x, R *y) { apply_prec_poly<R>(s, vals, inv, x, y, st); };
-    double bnorm = 0;
-    {
-        k_norm2<R><<<nb, RB, 0, st>>>(n, rhs, s->partial);
-        std::vector<double> p(nb);
-        EMG_HIP(hipMemcpyAsync(p.data(), s->partial, nb * sizeof(double), hipMemcpyDeviceToHost, st));
-        EMG_HIP(hipStreamSynchronize(st));
-        for (double v : p) bnorm += v;
-        bnorm = std::sqrt(bnorm);
+static int step_graph(emg_solver *s, int t, hipGraphExec_t *out) {
+    if (s->exec_np2 != s->np2 || s->exec_poly != s->poly_deg) drop_graphs(s);
+    s->exec_np2 = s->np2;
+    s->exec_poly = s->poly_deg;
+    s->exec.resize(s->cap, nullptr);
+    hipGraphExec_t &g = t >= 0 ? s->exec[t] : s->tail;
+    if (g == nullptr) {
+        const int rc = capture(s, [&](hipStream_t cs) {
+            if (t >= 0) enqueue_step<R>(s, t, cs);
+            else apply_prec_poly<R>(s, reinterpret_cast<const R *>(s->w), nullptr, reinterpret_cast<R *>(s->z), cs);
+        }, &g);
+        if (rc) return rc;
     }
+    *out = g;
+    return 0;
+}
+
+// The cycles of one solve that share the basis storage, as the host sees them: basis vectors
+// t0 .. t0 + k with k columns each, the upper triangular factor over all of them and the rotations.
+struct kept_host {
+    using C = std::complex<double>;
+    int m;
+    struct cyc { int t0, k; };
+    std::vector<cyc> cycles;
+    std::vector<C> R, cs, sn, g;      // R: column t at t * (m + 1)
+    std::vector<double> sc;
+    explicit kept_host(int m_) : m(m_), R((size_t)m_ * (m_ + 1)), cs(m_), sn(m_), g(m_ + 1), sc(m_ + 1) {}
+    int used() const { return cycles.empty() ? 0 : cycles.back().t0 + cycles.back().k + 1; }
+    C &r(int i, int t) { return R[(size_t)t * (m + 1) + i]; }
+    // rows t0 .. t0 + k of a column through the rotations of cycle c
+    void rotate(const cyc &c, C *col) const {
+        C x = col[c.t0];
+        for (int i = c.t0; i < c.t0 + c.k; i++) {
+            const C y = col[i + 1];
+            col[i] = std::conj(cs[i]) * x + std::conj(sn[i]) * y;
+            x = -sn[i] * x + cs[i] * y;
+        }
+        col[c.t0 + c.k] = x;
+    }
+};
+
+// Residual reduction at which a complex64 cycle ends.  With the spaces kept a new cycle costs little
+// (an FP64 residual and three passes over the basis), and the sooner the residual is formed anew the
+// less complex64 rounding the estimates carry: 200 / 241 / 263 steps to 3e-13 at 1e-1 / 3e-2 / 1e-2 on
+// the posts box at 40 x 20 x 8 hexes.
+static constexpr double CYCLE_CUT = 1e-1;
+static constexpr int CYCLE_ROOM = 12;       // basis vectors worth starting another kept cycle for
+
+// What the device knows of the kept cycles: their spans, and where the next cycle begins.  (The
+// staging is not written again before the stream has been waited for.)
+static int upload_kept(emg_solver *s, const kept_host &kh, hipStream_t st) {
+    kept_dev *kd = reinterpret_cast<kept_dev *>(s->host + host_off(s->cap).kept);
+    kd->t0 = kh.used();
+    kd->ncyc = (int32_t)kh.cycles.size();
+    for (size_t c = 0; c < kh.cycles.size(); c++) kd->start[c] = kh.cycles[c].t0;
+    kd->start[kh.cycles.size()] = kd->t0;
+    // with the outside direction of the last cycle, which lies before it (gmres_cycle)
+    const host_off ho(s->cap);
+    const int64_t from = kh.cycles.empty() ? ho.kept - ho.qp : 2 * kh.cycles.back().t0;
+    EMG_HIP(hipMemcpyAsync(s->arn + arn_off(s->cap).qp + from, s->host + ho.qp + from,
+                           (ho.total - ho.qp - from) * sizeof(double), hipMemcpyHostToDevice, st));
+    return 0;
+}
+
+// One cycle of GMRES on K u = w (right preconditioned), beginning at the free end of the basis:
+// until the residual estimate relative to `unit` is at most tol, at most maxiter steps, or the basis is
+// full.  On entry s->w holds w; on return s->z holds u.  iters: steps done; rel: the last estimate
+// relative to `unit`.
+//
+// With cycles kept in kh (the refinement cycles of one mixed-precision solve) the operator is
+// projected off their ranges, as GCRO does: the cycle minimises over the kept spaces and its own
+// together, so in exact arithmetic the cycles continue ONE unrestarted GMRES although each starts
+// from a residual that was formed anew in FP64.  A cycle that forgets the others pays their first steps
+// again: the posts box at 40 x 20 x 8 hexes took 425 steps in 7 cycles to 3e-13, where complex128
+// GMRES, which never restarts on the way, takes 155.  The ranges are not stored: C_c = V Q_c is applied
+// through the basis vectors and the rotations of cycle c (project_kept), and what the projections
+// take away enters the triangular factor of the least-squares problem.  When the basis is nearly full
+// everything is forgotten (the caller clears kh).
+template <typename R>
+static int gmres_cycle(emg_solver *s, double unit, double tol, int maxiter, kept_host &kh, int *iters, double *rel,
+                       hipStream_t st) {
+    using C = std::complex<double>;
+    const int64_t n = s->n;
+    const int m = s->cap, nb = s->nblk, t0 = kh.used();
+    const arn_off o(m);
+    const host_off ho(m);
+    R *V = reinterpret_cast<R *>(s->V), *w = reinterpret_cast<R *>(s->w), *vt = V + (size_t)t0 * n * 2;
     *iters = 0;
-    *rel = 0;
+    if (t0 > 0) {
+        // the kept ranges' part of w is solved by them: coefficients to the host, w projected
+        orthogonalise<R>(s, t0, w, s->pn, s->host_dev + ho.h0, st);
+    } else {
+        k_norm2<R><<<nb, RB, 0, st>>>(n, w, s->pn);
+    }
+    k_scale_by_norm<R><<<nb, RB, 0, st>>>(n, s->pn, nb, w, vt, s->nrm);
+    k_arn_init<<<1, 64, 0, st>>>(t0, s->nrm, s->arn, o);
+    EMG_LAUNCH_CHECK();
+    const int len = chunk_it(n), most = std::min({m - t0, s->restart, maxiter});
+    int k = 0;
+    for (bool done = false; !done && k < most;) {
+        const int k1 = std::min(k + len, most);
+        for (int q = k; q < k1; q++) {
+            hipGraphExec_t graph = nullptr;
+            if (int rc = step_graph<R>(s, t0 + q, &graph)) return rc;
+            EMG_HIP(hipGraphLaunch(graph, st));
+        }
+        k_arn_report<<<k1 - k, RB, 0, st>>>(t0 + k, m, s->arn, o, s->host_dev, ho);
+        EMG_HIP(hipStreamSynchronize(st));
+        for (; k < k1; k++) {   // steps of the chunk past the one that reaches tol serve too
+            const double e = s->host[ho.res + t0 + k] / unit;
+            if (!std::isfinite(e)) { done = true; break; }
+            *rel = e;
+            if (e <= tol) done = true;
+        }
+    }
+    *iters = k;
+    if (k == 0) { *rel = std::numeric_limits<double>::quiet_NaN(); return 0; }
+    // the new columns of the triangular factor, then y = R^{-1} g over all kept columns
+    auto from_host = [&](int64_t off, int64_t i) { return C(s->host[off + 2 * i], s->host[off + 2 * i + 1]); };
+    std::vector<C> g(m + 1), y(m + 1);
+    for (int i = 0; i < t0; i++) g[i] = from_host(ho.h0, i);
+    for (int t = t0; t < t0 + k; t++) {
+        kh.cs[t] = from_host(ho.cs, t);
+        kh.sn[t] = from_host(ho.sn, t);
+        g[t] = from_host(ho.g, t);
+        for (int i = 0; i <= t; i++) kh.r(i, t) = from_host(ho.H + 2 * (int64_t)t * (m + 1), i);
+        for (const auto &c : kh.cycles) kh.rotate(c, &kh.r(0, t));
+    }
+    kh.sc[t0] = 1.0;
+    for (int t = t0 + 1; t <= t0 + k; t++) kh.sc[t] = s->host[ho.sc + t];
+    for (const auto &c : kh.cycles) kh.rotate(c, g.data());
+    kh.cycles.push_back({t0, k});
+    for (int c = (int)kh.cycles.size() - 1; c >= 0; c--) {
+        const auto &cy = kh.cycles[c];
+        for (int i = cy.t0 + cy.k - 1; i >= cy.t0; i--) {
+            const C *r = &kh.r(0, i);
+            // a zero pivot is a breakdown: the columns past it add nothing
+            const C yi = r[i] == C(0.0) ? C(0.0) : g[i] / r[i];
+            y[i] = yi;
+            for (int q = 0; q < i; q++)   // the rows of the cycles' last vectors are not read again
+                g[q] -= C(r[q].real() * yi.real() - r[q].imag() * yi.imag(), r[q].real() * yi.imag() + r[q].imag() * yi.real());
+        }
+    }
+    const int nv = t0 + k;
+    C *ys = reinterpret_cast<C *>(s->host + ho.y), *qs = reinterpret_cast<C *>(s->host + ho.qp + 2 * t0);
+    for (int i = 0; i < nv; i++) ys[i] = y[i] * kh.sc[i];   // a cycle's last vector has no column: y = 0
+    double *yd = s->h + 6 * 512;
+    EMG_HIP(hipMemcpyAsync(yd, ys, nv * sizeof(C), hipMemcpyHostToDevice, st));
+    k_mcomb<R><<<nb, RB, 0, st>>>(n, nv, V, n, yd, w, 1);
+    EMG_LAUNCH_CHECK();
+    hipGraphExec_t graph = nullptr;
+    if (int rc = step_graph<R>(s, -1, &graph)) return rc;
+    EMG_HIP(hipGraphLaunch(graph, st));
+    // the direction of the cycle's span outside its range, Q e_{k+1}, back through the rotations; it
+    // stays in the staging for the next upload_kept
+    for (int i = 0; i < k; i++) qs[i] = 0.0;
+    qs[k] = 1.0;
+    for (int i = k - 1; i >= 0; i--) {
+        const C a = qs[i], b = qs[i + 1], cc = kh.cs[t0 + i], ss = kh.sn[t0 + i];
+        qs[i] = cc * a - std::conj(ss) * b;
+        qs[i + 1] = ss * a + std::conj(cc) * b;
+    }
+    return 0;
+}
+
+// sqrt of the sum of |v|^2 (waits for the stream)
+static int norm_to_host(emg_solver *s, const double *v, int slot, double *out, hipStream_t st) {
+    const host_off ho(s->cap);
+    k_norm2<double><<<s->nblk, RB, 0, st>>>(s->n, v, s->partial);
+    k_sum_partials<<<1, RB, 0, st>>>(s->nblk, s->partial, s->host_dev + ho.norm + slot);
+    EMG_HIP(hipStreamSynchronize(st));
+    *out = std::sqrt(s->host[ho.norm + slot]);
+    return 0;
+}
+
+// ---- restarted GMRES solve of K u = rhs in complex128: u holds the initial guess and the solution;
+// *iters the steps done.
+static int gmres_full(emg_solver *s, const double *rhs, double *u, double tol, int maxiter, int *iters, hipStream_t st) {
+    const int64_t n = s->n;
+    *iters = 0;
+    double bnorm = 0, beta = 0;
+    if (int rc = norm_to_host(s, rhs, 0, &bnorm, st)) return rc;
     if (bnorm == 0) {
-        EMG_HIP(hipMemsetAsync(u, 0, n * 2 * sizeof(R), st));
+        EMG_HIP(hipMemsetAsync(u, 0, n * 2 * sizeof(double), st));
         return 0;
     }
-    if (int rc = ensure_graphs<R>(s, vals, inv)) return rc;
-    const auto &graphs = s->gs[sizeof(R) == 8 ? 0 : 1].exec;
-    std::vector<double> Hh, gh(2 * (m + 1));
-    std::vector<std::complex<double>> y(m);
-    int total = 0;
-    double resid = 1.0;
+    kept_host kh(s->cap);
     while (true) {
-        // r = rhs - K u  ->  v0 = r / |r|
-        launch_spmv_blk<R>(st, n, s->nnz, s->rowptr, s->cols, vals, s->mask, u, rhs, w, s->lanes[sizeof(R) == 4],
-                           sizeof(R) == 8);
-        k_norm2<R><<<nb, RB, 0, st>>>(n, w, s->partial);
-        k_scale_by_norm<R><<<nb, RB, 0, st>>>(n, s->partial, nb, w, V, s->nrm);
-        double beta;
-        EMG_HIP(hipMemcpyAsync(&beta, s->nrm, sizeof(double), hipMemcpyDeviceToHost, st));
-        EMG_HIP(hipStreamSynchronize(st));
-        resid = beta / bnorm;
-        if (resid <= tol || total >= maxiter || !(beta > 0) || !std::isfinite(beta)) break;
-        k_arn_init<<<1, RB, 0, st>>>(m, s->nrm, s->arn, o);
-        int k = 0;
-        bool done = false;
-        for (int c = 0; c < (int)graphs.size() && !done; c++) {
-            const int j0 = c * CHUNK_IT, j1 = std::min(m, j0 + CHUNK_IT);
-            EMG_HIP(hipGraphLaunch(graphs[c], st));
-            EMG_HIP(hipMemcpyAsync(s->res_host + j0, s->arn + o.res + j0, (j1 - j0) * sizeof(double),
-                                   hipMemcpyDeviceToHost, st));
-            EMG_HIP(hipStreamSynchronize(st));
-            for (int j = j0; j < j1; j++) {
-                k = j + 1;
-                resid = s->res_host[j] / bnorm;
-                if (!std::isfinite(resid) || resid <= tol || total + k >= maxiter) { done = true; break; }
-            }
-        }
-        total += k;
-        // y = R^{-1} g (upper triangular after the rotations) ; u += M^{-1} V y
-        Hh.resize(2 * (size_t)k * (m + 1));
-        EMG_HIP(hipMemcpyAsync(Hh.data(), s->arn + o.H, Hh.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-        EMG_HIP(hipMemcpyAsync(gh.data(), s->arn + o.g, 2 * (m + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
-        EMG_HIP(hipStreamSynchronize(st));
-        auto Hc = [&](int i, int q) { return std::complex<double>(Hh[2 * ((size_t)q * (m + 1) + i)], Hh[2 * ((size_t)q * (m + 1) + i) + 1]); };
-        for (int i = k - 1; i >= 0; i--) {
-            std::complex<double> acc(gh[2 * i], gh[2 * i + 1]);
-            for (int q = i + 1; q < k; q++) acc -= Hc(i, q) * y[q];
-            y[i] = acc / Hc(i, i);
-        }
-        std::vector<double> yb(2 * k);
-        for (int i = 0; i < k; i++) { yb[2 * i] = y[i].real(); yb[2 * i + 1] = y[i].imag(); }
-        double *yd = s->h + 4 * 512;
-        if (k > 0) {
-            EMG_HIP(hipMemcpyAsync(yd, yb.data(), 2 * k * sizeof(double), hipMemcpyHostToDevice, st));
-            k_mcomb<R><<<nb, RB, 0, st>>>(n, k, V, n, yd, w, 1);
-            prec(w, z);
-            k_add<R><<<nb, RB, 0, st>>>(n, z, u);
-        }
-        EMG_HIP(hipStreamSynchronize(st));
-        if (!std::isfinite(resid)) break;
+        spmv_pk<double, SP_RESID, false>(s, s->lanes[0], u, sp_args<double>{rhs, s->w, nullptr, nullptr, 0, nullptr}, st);
+        if (int rc = norm_to_host(s, s->w, 0, &beta, st)) return rc;
+        if (beta / bnorm <= tol || *iters >= maxiter || !(beta > 0) || !std::isfinite(beta)) return 0;
+        kh.cycles.clear();
+        if (int rc = upload_kept(s, kh, st)) return rc;
+        int it = 0;
+        double rel = 0;
+        if (int rc = gmres_cycle<double>(s, bnorm, tol, maxiter - *iters, kh, &it, &rel, st)) return rc;
+        *iters += it;
+        if (it > 0) k_add<double><<<s->nblk, RB, 0, st>>>(n, s->z, u);
+        EMG_HIP(hipStreamSynchronize(st));   // the upload staging is written again
+        if (it == 0 || !std::isfinite(rel)) return 0;
     }
-    *iters = total;
-    *rel = resid;
-    return 0;
 }
 
 extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, double tol, int maxiter, int max_refine,
@@ -1466,69 +2300,79 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
     EMG_CHECK(s && d_b && d_x && info, "emg_solver_solve: null argument");
     EMG_CHECK(s->vals != nullptr, "emg_solver_solve: emg_solver_set_matrix was not called");
     hipStream_t st = (hipStream_t)stream;
-    const int64_t n = s->n;
-    const int nb = s->nblk;
     memset(info, 0, sizeof(*info));
-    auto true_resid = [&](double *out_rel, double *bn) -> int {
+    double bn = -1.0;   // ||b||, formed with the first residual
+    auto true_resid = [&](double *out_rel) -> int {
         // r = b - K x in complex128 (masked)
-        launch_spmv_blk<double>(st, n, s->nnz, s->rowptr, s->cols, s->vals, s->mask, d_x, d_b, s->r, s->lanes[0]);
-        k_norm2<double><<<nb, RB, 0, st>>>(n, s->r, s->partial);
-        k_norm2<double><<<nb, RB, 0, st>>>(n, d_b, s->partial + 1024);
-        std::vector<double> p(2048);
-        EMG_HIP(hipMemcpyAsync(p.data(), s->partial, nb * sizeof(double), hipMemcpyDeviceToHost, st));
-        EMG_HIP(hipMemcpyAsync(p.data() + 1024, s->partial + 1024, nb * sizeof(double), hipMemcpyDeviceToHost, st));
-        EMG_HIP(hipStreamSynchronize(st));
-        double rn = 0, b2 = 0;
-        for (int i = 0; i < nb; i++) { rn += p[i]; b2 += p[1024 + i]; }
-        *bn = std::sqrt(b2);
-        *out_rel = *bn > 0 ? std::sqrt(rn) / *bn : 0.0;
+        double rn = 0;
+        if (bn < 0)
+            if (int rc = norm_to_host(s, d_b, 0, &bn, st)) return rc;
+        spmv_std(s, d_x, d_b, s->r, st);
+        if (int rc = norm_to_host(s, s->r, 1, &rn, st)) return rc;
+        *out_rel = bn > 0 ? rn / bn : 0.0;
         return 0;
     };
-    double rel, bn;
+    double rel;
     if (s->precision == 64) {
         int it;
-        double est;
-        int rc = gmres_core<double>(s, s->vals, s->inv64, d_b, d_x, tol, maxiter, &it, &est, st);
+        k_pack_vec<double><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, d_b, 1.0, s->r);
+        k_pack_vec<double><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, d_x, 1.0, s->d);
+        int rc = gmres_full(s, s->r, s->d, tol, maxiter, &it, st);
         if (rc) return rc;
+        k_unpack_vec<double><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->d, 1.0, 0, d_x);
         info->iterations = it;
         info->refinements = 0;
-        rc = true_resid(&rel, &bn);
+        rc = true_resid(&rel);
         if (rc) return rc;
         info->residual = rel;
     } else {
-        // Mixed-precision restarted GMRES: every restart cycle runs in complex64
-        // on K d = r / |r|, then x += d and r = b - K x are formed in FP64, so
-        // complex64 never has to resolve more than one cycle's reduction.
-        float *r32 = reinterpret_cast<float *>(s->d);
-        float *d32 = reinterpret_cast<float *>(s->d) + 2 * n;
-        int rc = true_resid(&rel, &bn);
+        // Mixed-precision GMRES: every cycle runs in complex64 on K d = r / |r|, then x += d and
+        // r = b - K x are formed in FP64.
+        int rc = true_resid(&rel);
         if (rc) return rc;
         int total = 0, ref = 0;
         const int limit = max_refine > 0 ? max_refine : (1 << 30);
         int stall = 0;
+        kept_host kh(s->cap);
+        rc = upload_kept(s, kh, st);
+        if (rc) return rc;
         while (rel > tol && ref < limit && total < maxiter) {
             const double rs = 1.0 / (rel * bn);
-            k_c128_to_c64_scaled<<<1024, RB, 0, st>>>(n, s->r, rs, r32);
-            EMG_HIP(hipMemsetAsync(d32, 0, n * 8, st));
-            // A cycle stops once complex64 GMRES has reduced its residual 100-fold (or
-            // reached what tol needs): each FP64 update then starts a short cycle
-            // on a small Krylov basis (posts box, 201 points, polynomial degree 6:
-            // sweep 24.5 s with a 1e-7 floor, 15.9 s with 1e-2).
-            const double inner_tol = std::max(0.5 * tol / rel, 1e-2);
-            int it;
-            double est;
-            rc = gmres_core<float>(s, s->vals32, s->inv32, r32, d32, inner_tol,
-                                   std::min(s->restart, maxiter - total), &it, &est, st);
+            k_pack_vec<float><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->r, rs, reinterpret_cast<float *>(s->w));
+            // A cycle stops once complex64 GMRES has reduced its residual by CYCLE_CUT (or
+            // reached what tol needs), so that complex64 never has to resolve more than that.
+            const double inner_tol = std::max(0.5 * tol / rel, CYCLE_CUT);
+            int it = 0;
+            double est = 0;
+            rc = gmres_cycle<float>(s, 1.0, inner_tol, maxiter - total, kh, &it, &est, st);
             if (rc) return rc;
+            if (it == 0 && kh.cycles.empty()) break;
             total += it;
             ref++;
-            k_add_scaled<float><<<1024, RB, 0, st>>>(n, d32, 1.0 / rs, d_x);
+            if (it > 0)
+                k_unpack_vec<float><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(
+                    s->n_ent, reinterpret_cast<const float *>(s->z), 1.0 / rs, 1, d_x);
             const double prev = rel;
-            rc = true_resid(&rel, &bn);
+            rc = true_resid(&rel);
             if (rc) return rc;
-            if (it == 0) break;
+            if (it > 0 && !(rel <= 2.0 * prev)) {
+                // the kept spaces no longer fit the operator in complex64: take the step back and forget
+                k_unpack_vec<float><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(
+                    s->n_ent, reinterpret_cast<const float *>(s->z), -1.0 / rs, 1, d_x);
+                rc = true_resid(&rel);
+                if (rc) return rc;
+                if (kh.cycles.size() == 1) break;   // nothing was kept: complex64 cannot do better here
+                it = 0;
+            }
             stall = (rel > 0.999 * prev) ? stall + 1 : 0;
             if (stall >= 3) break;   // no progress in complex64: stop (caller sees converged = 0)
+            // A full basis, or two cycles without progress, end the memory of the cycles before.  One
+            // such cycle does not: rounding of a large correction can undo its gain, which the next
+            // cycles of the same space make up in a few steps (posts box at 2.2 GHz: 244 steps to 1e-9,
+            // 500 when it forgot there).
+            if (it == 0 || s->cap - kh.used() < CYCLE_ROOM || (int)kh.cycles.size() == KEEP_MAX || stall >= 2) kh.cycles.clear();
+            rc = upload_kept(s, kh, st);
+            if (rc) return rc;
         }
         info->iterations = total;
         info->refinements = ref;
@@ -1569,7 +2413,7 @@ extern "C" int emg_scatter_add(int64_t m, const int32_t *d_pos, const double *d_
 extern "C" int emg_spmv(int64_t n, const int32_t *d_rowptr, const int32_t *d_cols, const double *d_vals,
                         const uint8_t *d_mask, const double *d_x, double *d_y, void *stream) {
     EMG_CHECK(d_rowptr && d_cols && d_vals && d_x && d_y, "emg_spmv: null argument");
-    launch_spmv<double>((hipStream_t)stream, n, d_rowptr, d_cols, d_vals, d_mask, d_x, nullptr, d_y);
+    launch_spmv((hipStream_t)stream, n, d_rowptr, d_cols, d_vals, d_mask, d_x, d_y);
     EMG_LAUNCH_CHECK();
     return 0;
 }
@@ -1579,7 +2423,7 @@ extern "C" int emg_spmv_blocked(int64_t n, int64_t nnz, const int32_t *d_rowptr,
                                 void *stream) {
     EMG_CHECK(d_rowptr && d_cols && d_vals && d_x && d_y, "emg_spmv_blocked: null argument");
     EMG_CHECK(n > 0 && n % 2 == 0 && nnz % 2 == 0, "emg_spmv_blocked: n and nnz must be even");
-    launch_spmv_blk<double>((hipStream_t)stream, n, nnz, d_rowptr, d_cols, d_vals, d_mask, d_x, nullptr, d_y,
+    launch_spmv_blk((hipStream_t)stream, n, nnz, d_rowptr, d_cols, d_vals, d_mask, d_x, nullptr, d_y,
                             spmv_blk_lanes());
     EMG_LAUNCH_CHECK();
     return 0;
@@ -1593,18 +2437,19 @@ extern "C" int emg_solver_apply(emg_solver *s, int precision, const void *d_x, v
     EMG_CHECK(s->vals != nullptr, "emg_solver_apply: no matrix set");
     hipStream_t st = (hipStream_t)stream;
     if (precision == 64) {
-        launch_spmv_blk<double>(st, s->n, s->nnz, s->rowptr, s->cols, s->vals, s->mask,
-                                static_cast<const double *>(d_x), nullptr, static_cast<double *>(d_y), s->lanes[0]);
+        spmv_std(s, static_cast<const double *>(d_x), nullptr, static_cast<double *>(d_y), st);
     } else {
         EMG_CHECK(precision == 32 && s->precision == 32, "emg_solver_apply: precision 32 needs a precision-32 solver");
-        launch_spmv_blk<float>(st, s->n, s->nnz, s->rowptr, s->cols, s->vals32, s->mask,
-                               static_cast<const float *>(d_x), nullptr, static_cast<float *>(d_y), s->lanes[1], false);
+        spmv_pk<float, SP_Y, true>(s, STD_LANES, static_cast<const float *>(d_x),
+                                   sp_args<float>{nullptr, static_cast<float *>(d_y), nullptr, nullptr, 0, nullptr}, st);
     }
     EMG_LAUNCH_CHECK();
     return 0;
 }
 
-static int nblk_for(int64_t n) { return (int)std::min<int64_t>((n + RB - 1) / RB, 1024); }
+static int nblk_for(int64_t n) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>((n / 2 * maxpy_split(n) + RB - 1) / RB, 1024));
+}
 
 // d_h[i] = sum_k conj(V_i[k]) w[k], i < nv; V holds nv vectors of n entries back to back.
 // d_work: at least ceil(nv/8) * 1024 * 16 + 16 doubles.
@@ -1613,8 +2458,8 @@ extern "C" int emg_mdotc(int64_t n, int nv, const double *d_V, const double *d_w
     EMG_CHECK(d_V && d_w && d_h && d_work && nv > 0 && nv <= 512, "emg_mdotc: bad argument");
     hipStream_t st = (hipStream_t)stream;
     const int nbm = mdot_blocks(n, nv);
-    k_mdot<double><<<dim3(nbm, (nv + DT - 1) / DT), RB, 0, st>>>(n, nv, d_V, n, d_w, d_work, nullptr);
-    k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, d_work, d_h, 0, nullptr);
+    k_mdot<double, 1><<<dim3(nbm, (nv + DT - 1) / DT), RB, 0, st>>>(n, nv, d_V, n, d_w, nullptr, d_work);
+    k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, d_work, nullptr, d_h, nullptr, 0);
     EMG_LAUNCH_CHECK();
     return 0;
 }
@@ -1625,7 +2470,7 @@ extern "C" int emg_maxpy(int64_t n, int nv, const double *d_V, const double *d_h
     EMG_CHECK(d_V && d_h && d_w && d_norm && d_work && nv >= 0 && nv <= 512, "emg_maxpy: bad argument");
     hipStream_t st = (hipStream_t)stream;
     const int nb = nblk_for(n);
-    k_maxpy_norm<double><<<nb, RB, 0, st>>>(n, nv, d_V, n, d_h, d_w, d_work, nullptr);
+    launch_maxpy<double>(st, nb, n, nv, d_V, d_h, nullptr, d_w, d_work);
     k_scale_by_norm<double><<<1, RB, 0, st>>>(0, d_work, nb, d_w, d_w, d_norm);   // n = 0: norm only
     EMG_LAUNCH_CHECK();
     return 0;
@@ -1643,10 +2488,8 @@ __global__ void __launch_bounds__(256) k_csr_real(int64_t nrows, const int32_t *
         ar += av[e] * x[2 * ci[e]];
         ai += av[e] * x[2 * ci[e] + 1];
     }
-    for (int off = SUB / 2; off > 0; off >>= 1) {
-        ar += __shfl_xor(ar, off, SUB);
-        ai += __shfl_xor(ai, off, SUB);
-    }
+    ar = lane_sum<SUB>(ar);
+    ai = lane_sum<SUB>(ai);
     if (lane == 0) {
         if (accumulate) { y[2 * r] += ar; y[2 * r + 1] += ai; }
         else { y[2 * r] = ar; y[2 * r + 1] = ai; }

@@ -161,16 +161,16 @@ int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0, double *h
 int emg_solver_apply(emg_solver *s, int precision, const void *d_x, void *d_y, void *stream);
 
 /* The solver's autotuned SpMV shape: on its first emg_solver_set_matrix the solver times
- * the blocked SpMV with 4, 8, 16 and 32 lanes per entity (HIP events, 5 launches each, in
- * complex128 and, for precision 32, complex64) and keeps the fastest.  h_lanes[2]: the
- * chosen lanes (complex128, complex64); h_ms[8]: the measured milliseconds per launch
- * (4 per precision, in the order 4, 8, 16, 32).  EMG_SPMV_BLK_LANES overrides the search.
- * No reference counterpart (PARDISO has no shape to tune).                              */
+ * its product with 4, 8, 16 and 32 lanes per entity (HIP events around graphs of 8 runs, each
+ * after what precedes it in a step; in complex128 and, for precision 32, complex64) and keeps the
+ * fastest.  h_lanes[2]: the chosen lanes (complex128, complex64); h_ms[8]: the measured
+ * milliseconds per launch (4 per precision, in the order 4, 8, 16, 32).  EMG_SPMV_BLK_LANES
+ * overrides the search.  No reference counterpart (PARDISO has no shape to tune).         */
 int emg_solver_spmv_tuning(emg_solver *s, int *h_lanes, float *h_ms);
 
 /* The solver's autotuned smoother shape: with the gradient correction set, the first
  * emg_solver_set_matrix also times the smoother's G^T product with 4, 8 and 16 lanes per
- * row (HIP events, 5 launches each, in the precision of the solver's steps) and keeps the
+ * row (as the SpMV's, in the precision of the solver's steps) and keeps the
  * fastest.  h_lanes[1]: the choice (0 before tuning or without a gradient: 8 is used);
  * h_ms[3]: milliseconds per launch for 4, 8, 16.  EMG_GT_LANES overrides the search.
  * No reference counterpart (its solvers are direct).                                     */
