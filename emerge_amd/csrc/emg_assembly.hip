@@ -70,7 +70,8 @@ struct emg_pattern {
     double *tet_rec = nullptr;       // nt * REC: per-tet Gram records (fused-path workspace)
     double *tet_rec_batch = nullptr; // rec_batch_cap * nt * REC: the records of a batch of meshes
     int rec_batch_cap = 0;
-    uint8_t *recipes = nullptr;      // 100 * RECIPE_BYTES
+    uint8_t *recipes = nullptr;      // 2 * 100 * RECIPE_BYTES: symmetric Gram indices, then full ones (tensors)
+    double *tensor_rec = nullptr;    // nt * TREC: per-tet records of the tensor path (workspace)
     int wg_per_cu = 0;               // fused launch: workgroups per CU, 0 until tuned (first fused assembly)
     float wg_ms[5] = {};             // measured ms per assembly for ASM_WG[i]
 };
@@ -88,7 +89,7 @@ static constexpr int CHUNK_TMAX = 128;
 static constexpr int CHUNK_NMAX = 2048;  // incidences per chunk handled by the tet-list builder
 static constexpr int RECIPE_BYTES = 48;
 
-static void build_recipes(uint8_t *out);
+static void build_recipes(uint8_t *out, bool full);
 __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int32_t *__restrict__ chunk_tets,
                                                       int32_t *__restrict__ chunk_ntets, uint16_t *__restrict__ inc_local,
                                                       uint16_t *__restrict__ chunk_perm, int *__restrict__ overflow);
@@ -267,11 +268,12 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
         // two spare codes: the fused kernel reads the codes as 32-bit words
         TRY(hipMalloc(&pat->inc_local, (size_t)(n_inc + 2) * sizeof(uint16_t)));
         TRY(hipMalloc(&pat->chunk_perm, (size_t)pat->nchunk * pat->chunk * sizeof(uint16_t)));
-        TRY(hipMalloc(&pat->recipes, 100 * RECIPE_BYTES));
+        TRY(hipMalloc(&pat->recipes, 2 * 100 * RECIPE_BYTES));
         TRY(hipMalloc(&d_over, sizeof(int)));
         TRY(hipMemsetAsync(d_over, 0, sizeof(int), st));
-        uint8_t host_rec[100 * RECIPE_BYTES];
-        build_recipes(host_rec);
+        uint8_t host_rec[2 * 100 * RECIPE_BYTES];
+        build_recipes(host_rec, false);
+        build_recipes(host_rec + 100 * RECIPE_BYTES, true);
         TRY(hipMemcpyAsync(pat->recipes, host_rec, sizeof(host_rec), hipMemcpyHostToDevice, st));
         k_chunk_tets<<<(unsigned)pat->nchunk, CHUNK, 0, st>>>(*pat, pat->chunk_tets, pat->chunk_ntets, pat->inc_local,
                                                              pat->chunk_perm, d_over);
@@ -331,6 +333,7 @@ extern "C" void emg_pattern_destroy(emg_pattern *pat) {
     hfree(pat->tet_rec);
     hfree(pat->tet_rec_batch);
     hfree(pat->recipes);
+    hfree(pat->tensor_rec);
     delete pat;
 }
 
@@ -361,20 +364,6 @@ __device__ __forceinline__ double c4(int w, int x, int y, int z) {
     }
     return r;
 }
-
-template <bool C>
-struct Num;
-template <>
-struct Num<false> {
-    using T = double;
-};
-template <>
-struct Num<true> {
-    using T = cplx;
-};
-
-__device__ __forceinline__ double dmul(double a, double b) { return a * b; }
-__device__ __forceinline__ cplx dmul(cplx a, double b) { return a * b; }
 
 struct V3 {
     double x, y, z;
@@ -412,12 +401,13 @@ struct Stage {
     }
 };
 
-template <bool TENSOR>
+// One lane per adjacency entry, every tet's products formed anew per incidence: meshes without chunk
+// tables, and EMG_FORCE_TWO_PHASE.  Bound by its registers (198 and a spill: 2 waves per SIMD) and the
+// repeated work: 1430 us at 49,680 tets, where the staged path takes 289.
 __global__ void __launch_bounds__(ABLK) k_assemble(const emg_pattern pat, const double *__restrict__ nodes,
                                                    const int32_t *__restrict__ tets, const cplx *__restrict__ mat_m,
                                                    const cplx *__restrict__ mat_s, int exact_face_mass,
                                                    cplx *__restrict__ E, cplx *__restrict__ B) {
-    using T = typename Num<TENSOR>::T;
     __shared__ double lds[24 * ABLK];
     Stage st{lds, (int)threadIdx.x};
     const int64_t k = blockIdx.x * (int64_t)ABLK + threadIdx.x;
@@ -434,7 +424,7 @@ __global__ void __launch_bounds__(ABLK) k_assemble(const emg_pattern pat, const 
         // The reference mirrors its edge-face blocks by transposition
         // (fem/mth/tet.py:997-1004); with non-symmetric tensors the face-row /
         // edge-column entries are therefore the edge-row / face-column formula.
-        const bool swp = TENSOR && (s >= 6) && (s2 < 6);
+        const bool swp = (s >= 6) && (s2 < 6);
         if (swp) { int tmp = s; s = s2; s2 = tmp; }
         const int4 tv = reinterpret_cast<const int4 *>(tets)[t];
         V3 P[4];
@@ -475,34 +465,24 @@ __global__ void __launch_bounds__(ABLK) k_assemble(const emg_pattern pat, const 
                                   {fi ? -2.0 : 0.0, fi ? -1.0 : -3.0, fi ? 1.0 : 0.0}};
         const double cfj[2][3] = {{fj ? -1.0 : -3.0, fj ? -2.0 : 0.0, fj ? -1.0 : 0.0},
                                   {fj ? -2.0 : 0.0, fj ? -1.0 : -3.0, fj ? 1.0 : 0.0}};
-        T H[3][3], Gb[3][3];
-        const cplx *Mm = TENSOR ? mat_m + 9 * (int64_t)t : nullptr;
-        const cplx *Ms = TENSOR ? mat_s + 9 * (int64_t)t : nullptr;
+        cplx H[3][3], Gb[3][3];
+        const cplx *Mm = mat_m + 9 * (int64_t)t, *Ms = mat_s + 9 * (int64_t)t;
         cplx mmt[9], mst[9];
-        if constexpr (TENSOR) {
 #pragma unroll
-            for (int i = 0; i < 9; i++) { mmt[i] = Mm[i]; mst[i] = Ms[i]; }
-        }
+        for (int i = 0; i < 9; i++) { mmt[i] = Mm[i]; mst[i] = Ms[i]; }
 #pragma unroll
         for (int x = 0; x < 3; x++)
 #pragma unroll
             for (int y = 0; y < 3; y++) {
                 const double w = (tvi[x] == tvj[y]) ? 2.0 : 1.0;
-                if constexpr (TENSOR) {
-                    H[x][y] = qform(Ki[x], mst, Kj[y]) * w;
-                    Gb[x][y] = qform(Gi[x], mmt, Gj[y]);
-                } else {
-                    H[x][y] = dot(Ki[x], Kj[y]) * w;
-                    Gb[x][y] = dot(Gi[x], Gj[y]);
-                }
+                H[x][y] = qform(Ki[x], mst, Kj[y]) * w;
+                Gb[x][y] = qform(Gi[x], mmt, Gj[y]);
             }
         // Basis (p, q, r): r = a always; edge mode 1 (a, b, a), edge mode 2
         // (b, b, a), face mode 1 (b, c, a), face mode 2 (c, b, a).  q sits at
         // position c only for face mode 1.
         const double dscale = 1.0 / (120.0 * V6 * V6 * V6);
         const double fscale = 1.0 / (5040.0 * V6);
-        cplx cm = TENSOR ? cplx(1.0) : mat_m[t];
-        cplx cs = TENSOR ? cplx(1.0) : mat_s[t];
 #pragma unroll
         for (int m = 0; m < 2; m++) {
             const int p = (m == 0) ? (fi ? ib : ia) : (fi ? ic : ib);
@@ -515,34 +495,27 @@ __global__ void __launch_bounds__(ABLK) k_assemble(const emg_pattern pat, const 
                 const int q2 = (m2 == 0 && fj) ? jc : jb;
                 const int r2 = ja;
                 const bool qc2 = (m2 == 0 && fj);
-                const T g_rq = qc2 ? Gb[0][2] : Gb[0][1];
-                const T g_qr = qc ? Gb[2][0] : Gb[1][0];
-                const T g_qq = qc ? (qc2 ? Gb[2][2] : Gb[2][1]) : (qc2 ? Gb[1][2] : Gb[1][1]);
+                const cplx g_rq = qc2 ? Gb[0][2] : Gb[0][1];
+                const cplx g_qr = qc ? Gb[2][0] : Gb[1][0];
+                const cplx g_qq = qc ? (qc2 ? Gb[2][2] : Gb[2][1]) : (qc2 ? Gb[1][2] : Gb[1][1]);
                 // curl-curl
-                T d = T(0.0);
+                cplx d;
 #pragma unroll
                 for (int x = 0; x < 3; x++) {
-                    T row = T(0.0);
+                    cplx row;
 #pragma unroll
-                    for (int y = 0; y < 3; y++) row += dmul(H[x][y], cfj[m2][y]);
-                    d += dmul(row, cfi[m][x]);
+                    for (int y = 0; y < 3; y++) row += H[x][y] * cfj[m2][y];
+                    d += row * cfi[m][x];
                 }
                 // mass (second coefficient: reference index choice unless exact)
                 double c2 = c4(p, qq, p2, r2);
                 if (!exact_face_mass && fi && fj && m2 == 0) c2 = c4(ib, r2, p2, q2);
-                T f = dmul(Gb[0][0], c4(p, qq, p2, q2));
-                f += dmul(g_rq, -c2);
-                f += dmul(g_qr, -c4(p, r, p2, q2));
-                f += dmul(g_qq, c4(p, r, p2, r2));
+                cplx f = Gb[0][0] * c4(p, qq, p2, q2);
+                f += g_rq * (-c2);
+                f += g_qr * (-c4(p, r, p2, q2));
+                f += g_qq * c4(p, r, p2, r2);
                 const double sij = si[m] * sj[m2];
-                cplx dv, fv;
-                if constexpr (TENSOR) {
-                    dv = d * (sij * dscale);
-                    fv = f * (sij * fscale);
-                } else {
-                    dv = cs * (d * sij * dscale);
-                    fv = cm * (f * sij * fscale);
-                }
+                const cplx dv = d * (sij * dscale), fv = f * (sij * fscale);
                 const int a0 = swp ? m2 : m, a1 = swp ? m : m2;
                 accD[a0][a1] += dv;
                 accF[a0][a1] += fv;
@@ -751,6 +724,7 @@ __global__ void __launch_bounds__(256) k_gather_iso(const emg_pattern pat, const
 // Recipe of an ordered slot pair (s, s'), RECIPE_BYTES bytes:
 //   [0..8]   H index (symmetric 6x6 over canonical edges) of block (x, y)
 //   [9..17]  G index (symmetric 4x4 over vertices) of block (x, y)
+//            (full: row-major 6x6 and 4x4, whose entries a tensor need not mirror)
 //   [18..19] bit x*3+y: paired curl vertices coincide (integral weight 2)
 //   [20..35] per (m, m') the moments of the 4 mass terms (exact)
 //   [36..39] per (m, m') the second mass moment as the reference indexes it
@@ -759,7 +733,7 @@ __global__ void __launch_bounds__(256) k_gather_iso(const emg_pattern pat, const
 __host__ __device__ constexpr int sym4(int a, int b) { return a <= b ? a * 4 - a * (a - 1) / 2 + (b - a) : sym4(b, a); }
 __host__ __device__ constexpr int sym6(int a, int b) { return a <= b ? a * 6 - a * (a - 1) / 2 + (b - a) : sym6(b, a); }
 
-static void build_recipes(uint8_t *out) {
+static void build_recipes(uint8_t *out, bool full) {
     for (int s = 0; s < 10; s++)
         for (int s2 = 0; s2 < 10; s2++) {
             uint8_t *R = out + (s * 10 + s2) * RECIPE_BYTES;
@@ -774,8 +748,8 @@ static void build_recipes(uint8_t *out) {
             int w = 0;
             for (int x = 0; x < 3; x++)
                 for (int y = 0; y < 3; y++) {
-                    R[x * 3 + y] = (uint8_t)sym6(ki[x], kj[y]);
-                    R[9 + x * 3 + y] = (uint8_t)sym4(vi[x], vj[y]);
+                    R[x * 3 + y] = (uint8_t)(full ? 6 * ki[x] + kj[y] : sym6(ki[x], kj[y]));
+                    R[9 + x * 3 + y] = (uint8_t)(full ? 4 * vi[x] + vj[y] : sym4(vi[x], vj[y]));
                     if (tvi[x] == tvj[y]) w |= 1 << (x * 3 + y);
                 }
             R[18] = (uint8_t)(w & 255);
@@ -1334,21 +1308,246 @@ static void launch_staged(const emg_pattern *pat, dim3 grid, hipStream_t st, con
         k_assemble_staged<CHUNK_TMAX, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride);
 }
 
-static int g_num_cus = 0;
+// ------------------------------------------------------------ tensor materials
+// Record of a tet, TREC doubles: the 36 products X_k . Ms X_l of its edge cross products
+// X_k = g_a x g_b, scaled (complex, row-major), the 16 products g_a . Mm g_b, scaled, and the
+// 6 edge lengths: what every entry of its element matrices is a short combination of.
+static constexpr int T_H = 0, T_G = 72, T_L = 104, T_FIELDS = 110;
+static constexpr int TREC = 112;   // 896 bytes: seven whole 128-byte lines
 
-template <bool TENSOR>
-static int assemble(const emg_pattern *pat, const double *d_nodes, const int32_t *d_tets, const double *d_m,
-                    const double *d_s, int flags, double *d_E, double *d_B, void *stream) {
-    EMG_CHECK(pat && d_nodes && d_tets && d_m && d_s && d_E && d_B, "emg_assemble: null argument");
-    EMG_CHECK(!(flags & EMG_REFERENCE_GEOMETRY), "emg_assemble_tensor: EMG_REFERENCE_GEOMETRY is isotropic-only");
-    hipStream_t st = (hipStream_t)stream;
-    unsigned grid = (unsigned)((pat->nnz_ent + ABLK - 1) / ABLK);
-    k_assemble<TENSOR><<<grid, ABLK, 0, st>>>(*pat, d_nodes, d_tets, reinterpret_cast<const cplx *>(d_m),
-                                              reinterpret_cast<const cplx *>(d_s), (flags & EMG_EXACT_FACE_MASS) ? 1 : 0,
-                                              reinterpret_cast<cplx *>(d_E), reinterpret_cast<cplx *>(d_B));
-    EMG_LAUNCH_CHECK();
-    return 0;
+__global__ void __launch_bounds__(64) k_tet_tensor(int64_t nt, const double *__restrict__ nodes,
+                                                   const int32_t *__restrict__ tets, const cplx *__restrict__ mat_m,
+                                                   const cplx *__restrict__ mat_s, double *__restrict__ rec) {
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t >= nt) return;
+    const int4 tv = reinterpret_cast<const int4 *>(tets)[t];
+    const int vid[4] = {tv.x, tv.y, tv.z, tv.w};
+    V3 P[4], gr[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) P[i] = {nodes[3 * (int64_t)vid[i]], nodes[3 * (int64_t)vid[i] + 1], nodes[3 * (int64_t)vid[i] + 2]};
+    const V3 e1 = sub(P[1], P[0]), e2 = sub(P[2], P[0]), e3 = sub(P[3], P[0]);
+    gr[1] = crs(e2, e3);
+    gr[2] = crs(e3, e1);
+    gr[3] = crs(e1, e2);
+    gr[0] = {-(gr[1].x + gr[2].x + gr[3].x), -(gr[1].y + gr[2].y + gr[3].y), -(gr[1].z + gr[2].z + gr[3].z)};
+    const double V6 = fabs(dot(e1, gr[1]));
+    const double fscale = 1.0 / (5040.0 * V6), dscale = 1.0 / (120.0 * V6 * V6 * V6);
+    constexpr int EU[6] = {0, 0, 0, 1, 1, 2}, EV[6] = {1, 2, 3, 2, 3, 3};
+    double2 *out = reinterpret_cast<double2 *>(rec + t * TREC);
+    // M b for a complex 3x3 tensor, times s
+    auto apply = [](const cplx *M, V3 b, double s, cplx (&v)[3]) {
+        const double x = b.x * s, y = b.y * s, z = b.z * s;
+#pragma unroll
+        for (int i = 0; i < 3; i++) v[i] = x * M[3 * i] + y * M[3 * i + 1] + z * M[3 * i + 2];
+    };
+    cplx M[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) M[i] = mat_m[9 * t + i];
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        cplx v[3];
+        apply(M, gr[b], fscale, v);
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const cplx r = gr[a].x * v[0] + gr[a].y * v[1] + gr[a].z * v[2];
+            out[T_G / 2 + 4 * a + b] = make_double2(r.re, r.im);
+        }
+    }
+    V3 X[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) X[k] = crs(gr[EU[k]], gr[EV[k]]);
+#pragma unroll
+    for (int i = 0; i < 9; i++) M[i] = mat_s[9 * t + i];
+#pragma unroll
+    for (int l = 0; l < 6; l++) {
+        cplx v[3];
+        apply(M, X[l], dscale, v);
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            const cplx r = X[k].x * v[0] + X[k].y * v[1] + X[k].z * v[2];
+            out[T_H / 2 + 6 * k + l] = make_double2(r.re, r.im);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        out[T_L / 2 + k] = make_double2(nrm(sub(P[EV[2 * k]], P[EU[2 * k]])), nrm(sub(P[EV[2 * k + 1]], P[EU[2 * k + 1]])));
+    out[T_FIELDS / 2] = make_double2(0.0, 0.0);
 }
+
+// One incidence v = (local tet << 8) | (s << 4) | s': adds the 2x2 blocks of D and F of the slot
+// pair (s, s').  The reference mirrors its edge-face blocks by transposition (fem/mth/tet.py:997-1004),
+// so a face row / edge column takes the block of the pair swapped, transposed.
+template <int TS>
+__device__ __forceinline__ void tensor_incidence(const uint32_t *rcp, const double *td, uint32_t v, int exact_face_mass,
+                                                 cplx (&aD)[2][2], cplx (&aF)[2][2]) {
+    const int s = (int)((v >> 4) & 15u), s2 = (int)(v & 15u);
+    const bool swp = s >= 6 && s2 < 6;
+    const int sp = swp ? s2 * 10 + s : s * 10 + s2;
+    uint32_t w[12];
+    const uint4 *R4 = reinterpret_cast<const uint4 *>(rcp + sp * (RECIPE_BYTES / 4));
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const uint4 u = R4[i];
+        w[4 * i] = u.x; w[4 * i + 1] = u.y; w[4 * i + 2] = u.z; w[4 * i + 3] = u.w;
+    }
+    const double *T = td + (int)(v >> 8);
+    auto at = [&](int f) { return cplx(T[f * TS], T[(f + 1) * TS]); };
+    const uint32_t wm = rbyte(w, 18) | (rbyte(w, 19) << 8);
+    const uint32_t fl = rbyte(w, 44);
+    const bool fi = fl & 1u, fj = fl & 2u;
+    const double cfi[2][3] = {{fi ? -1.0 : -3.0, fi ? -2.0 : 0.0, fi ? -1.0 : 0.0},
+                              {fi ? -2.0 : 0.0, fi ? -1.0 : -3.0, fi ? 1.0 : 0.0}};
+    const double cfj[2][3] = {{fj ? -1.0 : -3.0, fj ? -2.0 : 0.0, fj ? -1.0 : 0.0},
+                              {fj ? -2.0 : 0.0, fj ? -1.0 : -3.0, fj ? 1.0 : 0.0}};
+    const double si[2] = {(fi ? -1.0 : 1.0) * T[(T_L + rbyte(w, 40)) * TS], T[(T_L + rbyte(w, 41)) * TS]};
+    const double sj[2] = {(fj ? -1.0 : 1.0) * T[(T_L + rbyte(w, 42)) * TS], T[(T_L + rbyte(w, 43)) * TS]};
+    cplx d[2][2];
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+        cplx h[3], r[2];
+#pragma unroll
+        for (int y = 0; y < 3; y++) {
+            h[y] = at(T_H + 2 * (int)rbyte(w, x * 3 + y));
+            if ((wm >> (x * 3 + y)) & 1u) h[y] = 2.0 * h[y];
+        }
+#pragma unroll
+        for (int m2 = 0; m2 < 2; m2++) r[m2] = cfj[m2][0] * h[0] + cfj[m2][1] * h[1] + cfj[m2][2] * h[2];
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int m2 = 0; m2 < 2; m2++) d[m][m2] += cfi[m][x] * r[m2];
+    }
+    auto g = [&](int x, int y) { return at(T_G + 2 * (int)rbyte(w, 9 + x * 3 + y)); };
+    const cplx g00 = g(0, 0);
+    cplx f[2][2];
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        const int qi = (m == 0 && fi) ? 2 : 1;   // position of q among (a, b, c)
+        const cplx gq0 = at(T_G + 2 * (int)(qi == 2 ? rbyte(w, 9 + 6) : rbyte(w, 9 + 3)));
+#pragma unroll
+        for (int m2 = 0; m2 < 2; m2++) {
+            const bool qc2 = m2 == 0 && fj;
+            const cplx g0q = at(T_G + 2 * (int)(qc2 ? rbyte(w, 9 + 2) : rbyte(w, 9 + 1)));
+            const uint32_t iq = qi == 2 ? (qc2 ? rbyte(w, 9 + 8) : rbyte(w, 9 + 7)) : (qc2 ? rbyte(w, 9 + 5) : rbyte(w, 9 + 4));
+            const cplx gqq = at(T_G + 2 * (int)iq);
+            const int o = 20 + 4 * (m * 2 + m2);
+            const double c1 = (double)(exact_face_mass ? rbyte(w, o + 1) : rbyte(w, 36 + m * 2 + m2));
+            f[m][m2] = (double)rbyte(w, o) * g00 - c1 * g0q - (double)rbyte(w, o + 2) * gq0 + (double)rbyte(w, o + 3) * gqq;
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int m2 = 0; m2 < 2; m2++) {
+            const cplx dv = (si[m] * sj[m2]) * d[m][m2], fv = (si[m] * sj[m2]) * f[m][m2];
+            if (m == m2) {
+                aD[m][m] += dv;
+                aF[m][m] += fv;
+            } else {
+                const cplx zero;
+                aD[m][m2] += swp ? zero : dv;
+                aD[m2][m] += swp ? dv : zero;
+                aF[m][m2] += swp ? zero : fv;
+                aF[m2][m] += swp ? fv : zero;
+            }
+        }
+}
+
+// Numeric assembly with tensor materials: one workgroup per chunk of CHUNK adjacency entries, the
+// records of its distinct tets (k_tet_tensor) and its index data in LDS, lanes in the chunk's order of
+// descending incidence count, values through LDS into entry order (as k_assemble_staged, without the
+// staging of the next chunk: a workgroup that waits for its records leaves the CU to the others).
+// Bound by the latency of that start and by the CSR writes: 245 us at 49,680 tets (460 MB, 1.9 TB/s),
+// with the records' 36 us 289 us where one lane per entry took 1430.
+template <int TS>
+__global__ void __launch_bounds__(CHUNK)
+    k_assemble_tensor_staged(const emg_pattern pat, const double *__restrict__ rec, int exact_face_mass,
+                             cplx *__restrict__ E, cplx *__restrict__ B) {
+    constexpr int TSP = TS + 1;
+    constexpr int TD = T_FIELDS * TSP, SD = 2 * 4 * CHUNK;
+    constexpr int NID = CHUNK_NMAX / 2 + 1;
+    __shared__ __align__(16) uint32_t rcp[100 * RECIPE_BYTES / 4];
+    __shared__ __align__(16) double td[TD > SD ? TD : SD];
+    __shared__ int32_t s_row[CHUNK + 2];
+    __shared__ uint32_t s_inc[NID];
+    __shared__ int2 s_out[CHUNK];
+    const int tid = threadIdx.x;
+    const int64_t c = blockIdx.x, k0 = c * CHUNK;
+    const int np = (int)(pat.nnz_ent - k0 < CHUNK ? pat.nnz_ent - k0 : CHUNK);
+    const int nT = pat.chunk_ntets[c];
+    const int32_t q0 = pat.pair_ptr[k0], ninc = pat.pair_ptr[k0 + np] - q0;
+    const int32_t r0 = pat.chunk_row0[c], nr = pat.chunk_row0[c + 1] - r0 + 2;
+    // eight lanes per record, seven pairs of doubles each
+    for (int slot = tid >> 3; slot < nT; slot += CHUNK / 8) {
+        const double2 *src = reinterpret_cast<const double2 *>(rec + (int64_t)pat.chunk_tets[c * CHUNK_TMAX + slot] * TREC);
+        double2 v[7];
+#pragma unroll
+        for (int q = 0; q < 7; q++) v[q] = src[(tid & 7) + 8 * q];
+#pragma unroll
+        for (int q = 0; q < 7; q++) {
+            const int f = 2 * ((tid & 7) + 8 * q);
+            if (f < T_FIELDS) {
+                td[f * TSP + slot] = v[q].x;
+                td[(f + 1) * TSP + slot] = v[q].y;
+            }
+        }
+    }
+    const uint32_t *recipe = reinterpret_cast<const uint32_t *>(pat.recipes + 100 * RECIPE_BYTES);
+    for (int i = tid; i < 100 * RECIPE_BYTES / 4; i += CHUNK) rcp[i] = recipe[i];
+    for (int i = tid; i < nr && i < CHUNK + 2; i += CHUNK) s_row[i] = pat.ent_ptr[r0 + i];
+    const int32_t ioff = q0 & 1;
+    for (int i = tid; i < (ioff + ninc + 1) / 2; i += CHUNK)
+        s_inc[i] = reinterpret_cast<const uint32_t *>(pat.inc_local)[(q0 >> 1) + i];
+    const int lk = pat.chunk_perm[k0 + tid];
+    const bool act = lk < np;
+    const int qa = act ? pat.pair_ptr[k0 + lk] - q0 + ioff : 0, qb = act ? pat.pair_ptr[k0 + lk + 1] - q0 + ioff : 0;
+    __syncthreads();
+    cplx aD[2][2], aF[2][2];
+    int32_t p0 = 0, deg = 0;
+    if (act) {
+        const int64_t k = k0 + lk;
+        int lo = 0, hi = nr - 2;   // the row of k: last i with s_row[i] <= k
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (s_row[mid] <= k) lo = mid; else hi = mid - 1;
+        }
+        p0 = s_row[lo];
+        deg = s_row[lo + 1] - p0;
+        const uint16_t *inc16 = reinterpret_cast<const uint16_t *>(s_inc);
+#pragma unroll 1
+        for (int q = qa; q < qb; q++) tensor_incidence<TSP>(rcp, td, inc16[q], exact_face_mass, aD, aF);
+    }
+    cplx *stg = reinterpret_cast<cplx *>(td);
+    int2 o = make_int2(0, 0);
+#pragma unroll
+    for (int mat = 0; mat < 2; mat++) {
+        __syncthreads();   // records, then the first matrix' blocks, no longer read
+        if (act) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) stg[m * CHUNK + lk] = mat == 0 ? aD[m >> 1][m & 1] : aF[m >> 1][m & 1];
+            if (mat == 0) s_out[lk] = make_int2(p0, deg);
+        }
+        __syncthreads();
+        if (tid < np) {
+            if (mat == 0) o = s_out[tid];
+            cplx *out = mat == 0 ? E : B;
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+                out[(int64_t)(m >> 1) * 2 * pat.nnz_ent + o.x + (int64_t)(m & 1) * o.y + k0 + tid] = stg[m * CHUNK + tid];
+        }
+    }
+}
+
+static void launch_tensor_staged(const emg_pattern *pat, hipStream_t st, int efm, cplx *oE, cplx *oB) {
+    const unsigned grid = (unsigned)pat->nchunk;
+    const int tm = pat->chunk_tmax;
+    if (tm <= 48) k_assemble_tensor_staged<48><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
+    else if (tm <= 64) k_assemble_tensor_staged<64><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
+    else if (tm <= 96) k_assemble_tensor_staged<96><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
+    else k_assemble_tensor_staged<CHUNK_TMAX><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
+}
+
+static int g_num_cus = 0;
 
 // Autotuner of the fused launch's grid: workgroups per CU.  A grid-stride workgroup owns
 // whole chunks, so every grid gives the same values bit for bit; the grid only decides how
@@ -1497,5 +1696,20 @@ extern "C" int emg_assemble_iso_batched(const emg_pattern *pat, int nbatch, int6
 extern "C" int emg_assemble_tensor(const emg_pattern *pat, const double *d_nodes, const int32_t *d_tets,
                                    const double *d_mm, const double *d_ms, int flags, double *d_E, double *d_B,
                                    void *stream) {
-    return assemble<true>(pat, d_nodes, d_tets, d_mm, d_ms, flags, d_E, d_B, stream);
+    EMG_CHECK(pat && d_nodes && d_tets && d_mm && d_ms && d_E && d_B, "emg_assemble: null argument");
+    EMG_CHECK(!(flags & EMG_REFERENCE_GEOMETRY), "emg_assemble_tensor: EMG_REFERENCE_GEOMETRY is isotropic-only");
+    hipStream_t st = (hipStream_t)stream;
+    const int efm = (flags & EMG_EXACT_FACE_MASS) ? 1 : 0;
+    const cplx *cm = reinterpret_cast<const cplx *>(d_mm), *cs = reinterpret_cast<const cplx *>(d_ms);
+    cplx *oE = reinterpret_cast<cplx *>(d_E), *oB = reinterpret_cast<cplx *>(d_B);
+    if (pat->fused_ok && !(flags & EMG_FORCE_TWO_PHASE)) {
+        emg_pattern *mp = const_cast<emg_pattern *>(pat);
+        if (!mp->tensor_rec) EMG_HIP(hipMalloc(&mp->tensor_rec, (size_t)pat->nt * TREC * sizeof(double)));
+        k_tet_tensor<<<emg::grid_for(pat->nt, 64), 64, 0, st>>>(pat->nt, d_nodes, d_tets, cm, cs, mp->tensor_rec);
+        launch_tensor_staged(pat, st, efm, oE, oB);
+    } else {
+        k_assemble<<<emg::grid_for(pat->nnz_ent, ABLK), ABLK, 0, st>>>(*pat, d_nodes, d_tets, cm, cs, efm, oE, oB);
+    }
+    EMG_LAUNCH_CHECK();
+    return 0;
 }
