@@ -42,17 +42,29 @@ __device__ __forceinline__ void stc(double *p, int64_t i, c2 v) {
 }
 
 constexpr int RES_BLOCK = 256;
-constexpr int ROW_LANES = 64;        // one wavefront per entity (two CSR rows)
+constexpr int ROW_LANES = 32;        // half a wavefront per entity (two CSR rows)
 constexpr int MAX_VEC = 16;
-constexpr int RES_GRID_MAX = 4096;   // persistent grid: partial sums per block
+constexpr int RES_GRID_MAX = 1024;   // persistent grid, 4 blocks per CU: partial sums per block
 
-// One wavefront per entity e of the pattern (emg_pattern_csr: DOF = mode * ne +
-// entity; rows (0, e) and (1, e) list the same column entities e'_k, a row's
-// (1, e'_k) entries deg after its (0, e'_k) ones, row (1, e) half = rowptr[ne]
-// entries after row (0, e)).  Lane l handles vector j = l % NV over the
-// column entities l / NV, l / NV + 64 / NV, ...: the two NV-vector runs of x
-// gathered for e'_k serve four matrix entries, and E, B and the column index
-// of an entry are loaded once per group of NV lanes and shared by the NV vectors.
+// Half a wavefront per entity e of the pattern (emg_pattern_csr: DOF = mode * ne + entity; rows (0, e)
+// and (1, e) list the same column entities e'_k, a row's (1, e'_k) entries deg after its (0, e'_k)
+// ones, row (1, e) half = rowptr[ne] entries after row (0, e)).  Lane (part, jl) takes the column
+// entities part, part + PARTS, ... for the vectors jl, jl + LPE, ...: the NV-vector runs of x gathered
+// for e'_k serve four matrix entries.  The columns of the next entity's first 32 entries and its row
+// offsets are loaded while this entity's are worked on, so an entry's gathers wait for one load only.
+//
+// What bounds it: every lane of an entry loads its E and B values, so with one vector per lane the
+// vector cache's return path (64 bytes per clock and CU) alone took 0.74 ms of 1.20; two vectors per lane from
+// NV = 8 halve those loads (four: 190 registers, 2 waves per SIMD, slower).  What is left is latency at
+// 4 waves per SIMD: two entities per wavefront halve the chain of loads, sums and results that an
+// entity costs.  At 16 pairs, 849,804 DOFs: 1.20 ms with a wavefront per entity, one vector per lane
+// and no loads ahead; 0.98 with two vectors, 0.84 with the columns ahead, 0.80 with half a wavefront
+// (4 vectors: 0.62 -> 0.38).  Slower: E and B staged through LDS (1.28; 2 waves per SIMD with loads ahead: 1.9),
+// a contiguous eighth of the entities per XCD (1.10 against 0.84), 768 or 1,280 blocks in place of
+// the 1,024 that the chip holds at once (0.93, 1.15).
+template <int NV>
+constexpr int res_vpl = NV >= 8 ? 2 : 1;   // vectors per lane
+
 template <int NV>
 __global__ void __launch_bounds__(RES_BLOCK)
     k_sweep_residual(int64_t ne, const int32_t *__restrict__ rowptr, const int32_t *__restrict__ cols,
@@ -61,71 +73,112 @@ __global__ void __launch_bounds__(RES_BLOCK)
                      const int32_t *__restrict__ qidx, const double *__restrict__ c,
                      const int32_t *__restrict__ prow_of_row, const double *__restrict__ Zp,
                      double *__restrict__ R, double *__restrict__ partial) {
-    constexpr int SPLIT = ROW_LANES / NV;   // entry strides per vector
+    constexpr int VPL = res_vpl<NV>, LPE = NV / VPL, PARTS = ROW_LANES / LPE;
     const int lane = threadIdx.x % ROW_LANES;
-    const int j = lane % NV;
-    const int part = lane / NV;
-    const double sj = s[j];
-    const int qj = qidx[j];
-    const c2 cj = ldc(c, j);
+    const int jl = lane % LPE, part = lane / LPE;
+    double sj[VPL];
+#pragma unroll
+    for (int v = 0; v < VPL; v++) sj[v] = s[jl + v * LPE];
     const int64_t n = 2 * ne;
     const int64_t half = rowptr[ne];
-    double rr = 0.0, bb = 0.0;
+    double rr[VPL], bb[VPL];
+#pragma unroll
+    for (int v = 0; v < VPL; v++) rr[v] = bb[v] = 0.0;
     const int64_t groups = (int64_t)gridDim.x * (RES_BLOCK / ROW_LANES);
-    for (int64_t e = blockIdx.x * (int64_t)(RES_BLOCK / ROW_LANES) + threadIdx.x / ROW_LANES; e < ne; e += groups) {
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};   // row (0, e) re, im; row (1, e) re, im
-        const int32_t r0 = rowptr[e];
-        const int32_t deg = (rowptr[e + 1] - r0) >> 1;
-        for (int32_t k = part; k < deg; k += SPLIT) {
-            const int32_t col = cols[r0 + k];
+    // blocks go round the 8 XCDs: each XCD takes consecutive entities, whose columns share its L2
+    const int64_t blk = gridDim.x % 8 == 0 ? (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+    int64_t e = blk * (RES_BLOCK / ROW_LANES) + threadIdx.x / ROW_LANES;
+    int32_t r0 = 0, r1 = 0, cn = -1;
+    if (e < ne) {
+        r0 = rowptr[e];
+        r1 = rowptr[e + 1];
+        cn = lane < ((r1 - r0) >> 1) ? cols[r0 + lane] : -1;
+    }
+    while (e < ne) {
+        double acc[VPL][4];   // row (0, e) re, im; row (1, e) re, im
+#pragma unroll
+        for (int v = 0; v < VPL; v++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[v][q] = 0.0;
+        const int64_t en = e + groups;
+        const int32_t rs = r0, deg = (r1 - r0) >> 1;
+        int32_t cv = cn;
+        if (en < ne) {   // the next entity's offsets, while this one's entries are on their way
+            r0 = rowptr[en];
+            r1 = rowptr[en + 1];
+        }
+        for (int32_t kb = 0; kb < deg; kb += PARTS) {
+            if (kb > 0 && (kb & (ROW_LANES - 1)) == 0) cv = kb + lane < deg ? cols[rs + kb + lane] : -1;
+            const int32_t k = kb + part;
+            const int32_t col = __shfl(cv, (kb & (ROW_LANES - 1)) + part, ROW_LANES);
             if (col < 0 || col >= ne) continue;   // not an entity pattern: no out-of-range reads
-            const c2 x0 = ldc(X, (int64_t)col * NV + j), x1 = ldc(X, (int64_t)(ne + col) * NV + j);
-            const int64_t pos[4] = {r0 + k, r0 + k + deg, half + r0 + k, half + r0 + k + deg};
+            c2 x0[VPL], x1[VPL];
+#pragma unroll
+            for (int v = 0; v < VPL; v++) {
+                x0[v] = ldc(X, (int64_t)col * NV + jl + v * LPE);
+                x1[v] = ldc(X, (int64_t)(ne + col) * NV + jl + v * LPE);
+            }
+            const int64_t pos[4] = {rs + k, rs + k + deg, half + rs + k, half + rs + k + deg};
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const c2 ev = ldc(E, pos[q]), bv = ldc(B, pos[q]);
-                const c2 x = (q & 1) ? x1 : x0;
-                const double kre = ev.re - sj * bv.re, kim = ev.im - sj * bv.im;
-                acc[(q >> 1) * 2] += kre * x.re - kim * x.im;
-                acc[(q >> 1) * 2 + 1] += kre * x.im + kim * x.re;
+#pragma unroll
+                for (int v = 0; v < VPL; v++) {
+                    const c2 x = (q & 1) ? x1[v] : x0[v];
+                    const double kre = ev.re - sj[v] * bv.re, kim = ev.im - sj[v] * bv.im;
+                    acc[v][(q >> 1) * 2] += kre * x.re - kim * x.im;
+                    acc[v][(q >> 1) * 2 + 1] += kre * x.im + kim * x.re;
+                }
             }
         }
 #pragma unroll
-        for (int off = ROW_LANES / 2; off >= NV; off >>= 1)
+        for (int off = ROW_LANES / 2; off >= LPE; off >>= 1)
 #pragma unroll
-            for (int q = 0; q < 4; q++) acc[q] += __shfl_xor(acc[q], off, ROW_LANES);
-        if (part == 0) {
+            for (int v = 0; v < VPL; v++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int64_t row = h * ne + e;
-                double are = acc[2 * h], aim = acc[2 * h + 1];
-                const int32_t pr = prow_of_row ? prow_of_row[row] : -1;
+                for (int q = 0; q < 4; q++) acc[v][q] += __shfl_xor(acc[v][q], off, ROW_LANES);
+        if (en < ne) cn = lane < ((r1 - r0) >> 1) ? cols[r0 + lane] : -1;
+        if (part < 2) {   // part h finishes row (h, e)
+            const int64_t row = part * ne + e;
+            const int32_t pr = prow_of_row ? prow_of_row[row] : -1;
+            const bool keep = mask == nullptr || mask[row];
+#pragma unroll
+            for (int v = 0; v < VPL; v++) {
+                const int j = jl + v * LPE;
+                double are = part ? acc[v][2] : acc[v][0], aim = part ? acc[v][3] : acc[v][1];
                 if (pr >= 0) {
                     const c2 z = ldc(Zp, (int64_t)pr * NV + j);
                     are += z.re;
                     aim += z.im;
                 }
                 double rre = 0.0, rim = 0.0;
-                if (mask == nullptr || mask[row]) {
-                    const c2 q = ldc(Q, (int64_t)qj * n + row);
+                if (keep) {
+                    const c2 q = ldc(Q, (int64_t)qidx[j] * n + row), cj = ldc(c, j);
                     const double bre = cj.re * q.re - cj.im * q.im, bim = cj.re * q.im + cj.im * q.re;
                     rre = bre - are;
                     rim = bim - aim;
-                    rr += rre * rre + rim * rim;
-                    bb += bre * bre + bim * bim;
+                    rr[v] += rre * rre + rim * rim;
+                    bb[v] += bre * bre + bim * bim;
                 }
                 if (R != nullptr) stc(R, row * NV + j, c2{rre, rim});
             }
         }
+        e = en;
     }
-    // block reduction of (rr, bb) per vector
-    __shared__ double sr[RES_BLOCK], sb[RES_BLOCK];
-    sr[threadIdx.x] = (part == 0) ? rr : 0.0;
-    sb[threadIdx.x] = (part == 0) ? bb : 0.0;
+    // block reduction of (rr, bb) per vector: [wave][row][vector]
+    __shared__ double sr[RES_BLOCK / ROW_LANES * 2 * NV], sb[RES_BLOCK / ROW_LANES * 2 * NV];
+    if (part < 2) {
+#pragma unroll
+        for (int v = 0; v < VPL; v++) {
+            const int at = (threadIdx.x / ROW_LANES * 2 + part) * NV + jl + v * LPE;
+            sr[at] = rr[v];
+            sb[at] = bb[v];
+        }
+    }
     __syncthreads();
     if (threadIdx.x < NV) {
         double a = 0.0, d = 0.0;
-        for (int t = threadIdx.x; t < RES_BLOCK; t += ROW_LANES) {
+        for (int t = threadIdx.x; t < RES_BLOCK / ROW_LANES * 2 * NV; t += NV) {
             a += sr[t];
             d += sb[t];
         }
@@ -171,19 +224,30 @@ __global__ void __launch_bounds__(256) k_port_apply(int64_t nprow, int nv, const
     stc(Zp, i * nv + j, c2{are, aim});
 }
 
-// X[row, j] = sum_i V[i, row] * Y[j, i]   (Y staged in LDS)
+// X[row, j] = sum_i V[i, row] * Y[j, i], a row per lane, Y in LDS.  HBM-bound: V is read and X written
+// once.  A lane's NV results lie 16 * NV bytes from its neighbour's, so a store of one vector would
+// touch a line per lane: the results go through LDS, 8 vectors at a time, and leave as whole lines
+// (849,804 DOFs, m = 14, NV = 16: 127 -> 100 us for 408 MB).
 constexpr int COMB_MAX = 2048;   // nvec * m complex entries held in LDS (32 KB)
+constexpr int COMB_BLOCK = 256;   // at most; half of it where the results and Y would not fit 64 KB of LDS
 template <int NV>
-__global__ void __launch_bounds__(256) k_basis_combine(int64_t n, int m, const double *__restrict__ V,
-                                                       const double *__restrict__ Y, double *__restrict__ X) {
-    __shared__ double2 sy[COMB_MAX];
+__global__ void __launch_bounds__(COMB_BLOCK) k_basis_combine(int64_t n, int m, const double *__restrict__ V,
+                                                              const double *__restrict__ Y, double *__restrict__ X) {
+    // a wavefront's results of WV vectors, to leave as whole lines
+    constexpr int WV = NV < 8 ? NV : 8;
+    extern __shared__ double2 comb_lds[];
+    double2 *const sy = comb_lds, *const sx = comb_lds + NV * m + (threadIdx.x / 64) * 64 * (WV + 1);
     for (int t = threadIdx.x; t < NV * m; t += blockDim.x) sy[t] = reinterpret_cast<const double2 *>(Y)[t];
     __syncthreads();
-    const int64_t row = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (row >= n) return;
+    const int lane = threadIdx.x % 64;
+    const int64_t row0 = blockIdx.x * (int64_t)blockDim.x + (threadIdx.x / 64) * 64;
+    if (row0 >= n) return;
+    const int64_t row = row0 + lane < n ? row0 + lane : n - 1;
+    const int64_t left = n - row0 < 64 ? n - row0 : 64;
     double are[NV], aim[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) { are[j] = 0.0; aim[j] = 0.0; }
+#pragma unroll 2
     for (int i = 0; i < m; i++) {
         const c2 v = ldc(V, (int64_t)i * n + row);
 #pragma unroll
@@ -194,7 +258,19 @@ __global__ void __launch_bounds__(256) k_basis_combine(int64_t n, int m, const d
         }
     }
 #pragma unroll
-    for (int j = 0; j < NV; j++) stc(X, row * NV + j, c2{are[j], aim[j]});
+    for (int h = 0; h < NV; h += WV) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < WV; j++) sx[lane * (WV + 1) + j] = make_double2(are[h + j], aim[h + j]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = 0; t < WV; t++) {
+            const int i = t * 64 + lane, r = i / WV, j = i % WV;
+            if (r < left) reinterpret_cast<double2 *>(X)[(row0 + r) * NV + h + j] = sx[r * (WV + 1) + j];
+        }
+    }
 }
 
 template <int NV>
@@ -208,7 +284,15 @@ void launch_residual(hipStream_t st, int grid, int64_t n, const int32_t *rowptr,
 
 template <int NV>
 void launch_combine(hipStream_t st, int64_t n, int m, const double *V, const double *Y, double *X) {
-    k_basis_combine<NV><<<emg::grid_for(n, 256), 256, 0, st>>>(n, m, V, Y, X);
+    constexpr int WV = NV < 8 ? NV : 8;
+    const auto lds = [&](int block) { return ((size_t)NV * m + (size_t)block * (WV + 1)) * sizeof(double2); };
+    const int block = lds(COMB_BLOCK) <= 64 * 1024 ? COMB_BLOCK : COMB_BLOCK / 2;
+    k_basis_combine<NV><<<emg::grid_for(n, block), block, lds(block), st>>>(n, m, V, Y, X);
+}
+
+int residual_grid(int64_t n) {
+    constexpr int per_block = RES_BLOCK / ROW_LANES;
+    return (int)std::min<int64_t>(RES_GRID_MAX, (n / 2 + per_block - 1) / per_block);
 }
 
 bool valid_nvec(int nv) { return nv == 1 || nv == 2 || nv == 4 || nv == 8 || nv == 16; }
@@ -226,8 +310,7 @@ extern "C" int emg_sweep_residual(int64_t n, const int32_t *d_rowptr, const int3
     EMG_CHECK((d_prow_of_row == nullptr) == (d_Zp == nullptr), "emg_sweep_residual: port rows need Zp");
     hipStream_t st = (hipStream_t)stream;
     EMG_CHECK(n % 2 == 0, "emg_sweep_residual: n must be 2 * entities (an entity pattern)");
-    constexpr int ents_per_block = RES_BLOCK / ROW_LANES;
-    const int grid = (int)std::min<int64_t>(RES_GRID_MAX, (n / 2 + ents_per_block - 1) / ents_per_block);
+    const int grid = residual_grid(n);
     switch (nvec) {
         case 1: launch_residual<1>(st, grid, n, d_rowptr, d_cols, d_E, d_B, d_mask, d_s, d_X, d_Q, d_qidx, d_c, d_prow_of_row, d_Zp, d_R, d_work); break;
         case 2: launch_residual<2>(st, grid, n, d_rowptr, d_cols, d_E, d_B, d_mask, d_s, d_X, d_Q, d_qidx, d_c, d_prow_of_row, d_Zp, d_R, d_work); break;
@@ -248,7 +331,7 @@ extern "C" int emg_sweep_residual(int64_t n, const int32_t *d_rowptr, const int3
 // hipGetSymbolAddress and cached.  Every block of the residual kernel writes
 // its own partial entries before k_sweep_norms reads them, so the array needs
 // no clearing between calls; calls that overlap on one device race on it.
-constexpr int64_t NOALLOC_SCRATCH_DOUBLES = (int64_t)RES_GRID_MAX * MAX_VEC * 2;   // 1 MiB
+constexpr int64_t NOALLOC_SCRATCH_DOUBLES = (int64_t)RES_GRID_MAX * MAX_VEC * 2;   // 256 KiB
 __device__ __align__(256) double scratch[NOALLOC_SCRATCH_DOUBLES];
 
 namespace {
@@ -279,10 +362,8 @@ extern "C" int emg_sweep_residual_noalloc(int64_t n, const int32_t *d_rowptr, co
                                           const double *d_Zp, double *d_R, double *d_norms, void *stream) {
     EMG_CHECK(valid_nvec(nvec), "emg_sweep_residual_noalloc: nvec must be 1, 2, 4, 8 or 16");
     EMG_CHECK(n > 0 && n % 2 == 0, "emg_sweep_residual_noalloc: n must be 2 * entities (an entity pattern)");
-    constexpr int ents_per_block = RES_BLOCK / ROW_LANES;
-    const int64_t grid = std::min<int64_t>(RES_GRID_MAX, (n / 2 + ents_per_block - 1) / ents_per_block);
-    EMG_CHECK(grid * nvec * 2 <= NOALLOC_SCRATCH_DOUBLES,
-              "emg_sweep_residual_noalloc: partial sums exceed the 1 MiB scratch array");
+    EMG_CHECK((int64_t)residual_grid(n) * nvec * 2 <= NOALLOC_SCRATCH_DOUBLES,
+              "emg_sweep_residual_noalloc: partial sums exceed the scratch array");
     double *work = nullptr;
     const int rc = scratch_for_current_device(&work);
     if (rc != 0) return rc;

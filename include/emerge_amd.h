@@ -368,7 +368,7 @@ int emg_sweep_residual(int64_t n, const int32_t *d_rowptr, const int32_t *d_cols
                        const double *d_Q, const int32_t *d_qidx, const double *d_c, const int32_t *d_prow_of_row,
                        const double *d_Zp, double *d_R, double *d_norms, double *d_work, void *stream);
 /* The same residual with no workspace argument and no allocation: the
- * per-block partial sums live in the library's static 1 MiB device array
+ * per-block partial sums live in the library's static 256 KiB device array
  * (one per GPU, held until the process ends).  No counterpart in the
  * reference: it is for callers that cannot allocate (code under HIP stream
  * capture, tight serving loops).  Limits as emg_sweep_residual (nvec <= 16);
