@@ -878,20 +878,38 @@ __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int
 }
 
 static constexpr int TD_FIELDS = 41;  // H(21) G(10) L(6) eps(2) nu(2)
+static constexpr int REC = 48;        // doubles of a tet's record: 384 bytes, three whole 128-byte lines
+
+// Eight pairs of doubles of every lane's record (pairs p0 .. p0 + 7 of rows of `pairs` pairs, lane's row
+// row0 + lane) through LDS, so that eight lanes write one whole line of a record where each lane by itself
+// would write its own lines piece by piece.  One wavefront per workgroup.
+static constexpr int ROW_LDS = 64 * 9;
+__device__ __forceinline__ void put_lines(double2 *lds, const double2 *v, double *rec, int64_t row0, int64_t rows, int pairs,
+                                          int p0) {
+    const int lane = threadIdx.x;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 8; q++) lds[lane * 9 + q] = v[q];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int r = i * 8 + (lane >> 3), q = lane & 7;
+        if (row0 + r < rows) reinterpret_cast<double2 *>(rec)[(row0 + r) * pairs + p0 + q] = lds[r * 9 + q];
+    }
+}
 
 __device__ __forceinline__ uint32_t rbyte(const uint32_t *w, int i) { return (w[i >> 2] >> ((i & 3) * 8)) & 255u; }
 
-// Gram record of a tet (vertices P, materials ev, nv): field f at dst[f * S].
+// Gram record of a tet (vertices P, materials ev, nv): field f at dst[f].
 // Fields: H = (grad x grad) products of the 6 edges (0..20), G = grad.grad of
 // the 4 vertices (21..30), the 6 edge lengths (31..36), eps (37, 38), nu (39, 40).
-template <int S>
 __device__ __forceinline__ void fused_tet_gram(const V3 (&P)[4], const V3 (&gr)[4], double V6, cplx ev, cplx nv,
-                                               double *dst) {
+                                               double (&dst)[REC]) {
     const double fscale = 1.0 / (5040.0 * V6);
     const double dscale = 1.0 / (120.0 * V6 * V6 * V6);
     constexpr int EU[6] = {0, 0, 0, 1, 1, 2}, EV[6] = {1, 2, 3, 2, 3, 3};
 #pragma unroll
-    for (int k = 0; k < 6; k++) dst[(31 + k) * S] = nrm(sub(P[EV[k]], P[EU[k]]));
+    for (int k = 0; k < 6; k++) dst[31 + k] = nrm(sub(P[EV[k]], P[EU[k]]));
     // H_kl = (g_a x g_b).(g_c x g_d) = G_ac G_bd - G_ad G_bc (Binet-Cauchy) with
     // G = the Gram matrix of the vertex gradients: no edge cross products held.
     double G[4][4];
@@ -901,19 +919,19 @@ __device__ __forceinline__ void fused_tet_gram(const V3 (&P)[4], const V3 (&gr)[
         for (int b = a; b < 4; b++) {
             G[a][b] = dot(gr[a], gr[b]);
             G[b][a] = G[a][b];
-            dst[(21 + sym4(a, b)) * S] = G[a][b] * fscale;
+            dst[21 + sym4(a, b)] = G[a][b] * fscale;
         }
 #pragma unroll
     for (int k = 0; k < 6; k++)
 #pragma unroll
         for (int l = k; l < 6; l++) {
             const int a = EU[k], b = EV[k], c = EU[l], d = EV[l];
-            dst[sym6(k, l) * S] = (G[a][c] * G[b][d] - G[a][d] * G[b][c]) * dscale;
+            dst[sym6(k, l)] = (G[a][c] * G[b][d] - G[a][d] * G[b][c]) * dscale;
         }
-    dst[37 * S] = ev.re;
-    dst[38 * S] = ev.im;
-    dst[39 * S] = nv.re;
-    dst[40 * S] = nv.im;
+    dst[37] = ev.re;
+    dst[38] = ev.im;
+    dst[39] = nv.re;
+    dst[40] = nv.im;
 }
 
 // One incidence v = (local tet << 8) | (s << 4) | s' of an adjacency entry:
@@ -978,9 +996,9 @@ __device__ __forceinline__ void fused_incidence(const uint32_t *rcp, const doubl
 }
 
 // Gram record of every tet (REC doubles each, fields as fused_tet_gram, the
-// rest padding): the first step of the numeric assembly, so each tet's geometry
-// is computed once.  48 doubles = 384 bytes = three whole 128-byte lines.
-static constexpr int REC = 48;
+// rest zero): the first step of the numeric assembly, so each tet's geometry
+// is computed once.  Bound by the records' bytes (385 MB at 1,005,000 tets): 168 us with every lane
+// storing its own record field by field, 85 (4.5 TB/s) through put_lines.
 // The reference's vertex-gradient cofactors and volume from absolute coordinates
 // (fem/mth/optimized.py:343-369), term for term and left to right with no fused
 // multiply-adds, so the cancellation they suffer away from the origin is the
@@ -1016,12 +1034,12 @@ __device__ __attribute__((noinline)) void reference_bcd(const V3 (&Q)[4], double
 // blockIdx.y selects the mesh of a batch sharing the tets (strides in doubles / complex
 // values between consecutive meshes' nodes, materials and records; 0 for one mesh).
 template <bool REF_GEOM>
-__global__ void __launch_bounds__(256) k_tet_gram(int64_t nt, const double *__restrict__ nodes,
+__global__ void __launch_bounds__(64) k_tet_gram(int64_t nt, const double *__restrict__ nodes,
                                                   const int32_t *__restrict__ tets, const cplx *__restrict__ eps,
                                                   const cplx *__restrict__ nu, double *__restrict__ rec,
                                                   int64_t node_stride, int64_t mat_stride, int64_t rec_stride) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= nt) return;
+    __shared__ __align__(16) double2 lds[ROW_LDS];
+    const int64_t row0 = blockIdx.x * (int64_t)64, t = min(row0 + threadIdx.x, nt - 1);
     nodes += blockIdx.y * node_stride;
     eps += blockIdx.y * mat_stride;
     nu += blockIdx.y * mat_stride;
@@ -1072,7 +1090,15 @@ __global__ void __launch_bounds__(256) k_tet_gram(int64_t nt, const double *__re
         gr[0] = {-(gr[1].x + gr[2].x + gr[3].x), -(gr[1].y + gr[2].y + gr[3].y), -(gr[1].z + gr[2].z + gr[3].z)};
         V6 = fabs(dot(e1, gr[1]));
     }
-    fused_tet_gram<1>(P, gr, V6, eps[t], nu[t], rec + t * REC);
+    double f[REC] = {};
+    fused_tet_gram(P, gr, V6, eps[t], nu[t], f);
+#pragma unroll
+    for (int g = 0; g < REC / 16; g++) {
+        double2 v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = make_double2(f[16 * g + 2 * q], f[16 * g + 2 * q + 1]);
+        put_lines(lds, v, rec, row0, nt, REC / 2, 8 * g);
+    }
 }
 
 // Numeric assembly, one workgroup of CH lanes per chunk of CH consecutive
@@ -1309,17 +1335,18 @@ static void launch_staged(const emg_pattern *pat, dim3 grid, hipStream_t st, con
 }
 
 // ------------------------------------------------------------ tensor materials
-// Record of a tet, TREC doubles: the 36 products X_k . Ms X_l of its edge cross products
-// X_k = g_a x g_b, scaled (complex, row-major), the 16 products g_a . Mm g_b, scaled, and the
-// 6 edge lengths: what every entry of its element matrices is a short combination of.
-static constexpr int T_H = 0, T_G = 72, T_L = 104, T_FIELDS = 110;
+// Record of a tet, TREC doubles: the 16 products g_a . Mm g_b, scaled (complex, row-major), the 36
+// products X_k . Ms X_l of its edge cross products X_k = g_a x g_b, scaled, and the 6 edge lengths: what
+// every entry of its element matrices is a short combination of.  Bound by the records' bytes
+// (45 MB at 49,680 tets): 36 us with every lane storing its own record, 17 through put_lines.
+static constexpr int T_G = 0, T_H = 32, T_L = 104, T_FIELDS = 110;
 static constexpr int TREC = 112;   // 896 bytes: seven whole 128-byte lines
 
 __global__ void __launch_bounds__(64) k_tet_tensor(int64_t nt, const double *__restrict__ nodes,
                                                    const int32_t *__restrict__ tets, const cplx *__restrict__ mat_m,
                                                    const cplx *__restrict__ mat_s, double *__restrict__ rec) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= nt) return;
+    __shared__ __align__(16) double2 lds[ROW_LDS];
+    const int64_t row0 = blockIdx.x * (int64_t)64, t = min(row0 + threadIdx.x, nt - 1);
     const int4 tv = reinterpret_cast<const int4 *>(tets)[t];
     const int vid[4] = {tv.x, tv.y, tv.z, tv.w};
     V3 P[4], gr[4];
@@ -1333,25 +1360,27 @@ __global__ void __launch_bounds__(64) k_tet_tensor(int64_t nt, const double *__r
     const double V6 = fabs(dot(e1, gr[1]));
     const double fscale = 1.0 / (5040.0 * V6), dscale = 1.0 / (120.0 * V6 * V6 * V6);
     constexpr int EU[6] = {0, 0, 0, 1, 1, 2}, EV[6] = {1, 2, 3, 2, 3, 3};
-    double2 *out = reinterpret_cast<double2 *>(rec + t * TREC);
-    // M b for a complex 3x3 tensor, times s
+    double2 row[TREC / 2];
+    // b^T M for a complex 3x3 tensor, times s
     auto apply = [](const cplx *M, V3 b, double s, cplx (&v)[3]) {
         const double x = b.x * s, y = b.y * s, z = b.z * s;
 #pragma unroll
-        for (int i = 0; i < 3; i++) v[i] = x * M[3 * i] + y * M[3 * i + 1] + z * M[3 * i + 2];
+        for (int j = 0; j < 3; j++) v[j] = x * M[j] + y * M[3 + j] + z * M[6 + j];
     };
+    auto put = [&](int g) { put_lines(lds, row + 8 * g, rec, row0, nt, TREC / 2, 8 * g); };
     cplx M[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) M[i] = mat_m[9 * t + i];
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
+    for (int a = 0; a < 4; a++) {
         cplx v[3];
-        apply(M, gr[b], fscale, v);
+        apply(M, gr[a], fscale, v);
 #pragma unroll
-        for (int a = 0; a < 4; a++) {
-            const cplx r = gr[a].x * v[0] + gr[a].y * v[1] + gr[a].z * v[2];
-            out[T_G / 2 + 4 * a + b] = make_double2(r.re, r.im);
+        for (int b = 0; b < 4; b++) {
+            const cplx r = gr[b].x * v[0] + gr[b].y * v[1] + gr[b].z * v[2];
+            row[T_G / 2 + 4 * a + b] = make_double2(r.re, r.im);
         }
+        if (a & 1) put(a >> 1);
     }
     V3 X[6];
 #pragma unroll
@@ -1359,19 +1388,22 @@ __global__ void __launch_bounds__(64) k_tet_tensor(int64_t nt, const double *__r
 #pragma unroll
     for (int i = 0; i < 9; i++) M[i] = mat_s[9 * t + i];
 #pragma unroll
-    for (int l = 0; l < 6; l++) {
+    for (int k = 0; k < 6; k++) {
         cplx v[3];
-        apply(M, X[l], dscale, v);
+        apply(M, X[k], dscale, v);
 #pragma unroll
-        for (int k = 0; k < 6; k++) {
-            const cplx r = X[k].x * v[0] + X[k].y * v[1] + X[k].z * v[2];
-            out[T_H / 2 + 6 * k + l] = make_double2(r.re, r.im);
+        for (int l = 0; l < 6; l++) {
+            const cplx r = X[l].x * v[0] + X[l].y * v[1] + X[l].z * v[2];
+            const int at = T_H / 2 + 6 * k + l;
+            row[at] = make_double2(r.re, r.im);
+            if (at % 8 == 7) put(at / 8);
         }
     }
 #pragma unroll
     for (int k = 0; k < 3; k++)
-        out[T_L / 2 + k] = make_double2(nrm(sub(P[EV[2 * k]], P[EU[2 * k]])), nrm(sub(P[EV[2 * k + 1]], P[EU[2 * k + 1]])));
-    out[T_FIELDS / 2] = make_double2(0.0, 0.0);
+        row[T_L / 2 + k] = make_double2(nrm(sub(P[EV[2 * k]], P[EU[2 * k]])), nrm(sub(P[EV[2 * k + 1]], P[EU[2 * k + 1]])));
+    row[T_FIELDS / 2] = make_double2(0.0, 0.0);
+    put(6);
 }
 
 // One incidence v = (local tet << 8) | (s << 4) | s': adds the 2x2 blocks of D and F of the slot
@@ -1458,7 +1490,7 @@ __device__ __forceinline__ void tensor_incidence(const uint32_t *rcp, const doub
 // descending incidence count, values through LDS into entry order (as k_assemble_staged, without the
 // staging of the next chunk: a workgroup that waits for its records leaves the CU to the others).
 // Bound by the latency of that start and by the CSR writes: 245 us at 49,680 tets (460 MB, 1.9 TB/s),
-// with the records' 36 us 289 us where one lane per entry took 1430.
+// with the records' 17 us 265 us where one lane per entry took 1430.
 template <int TS>
 __global__ void __launch_bounds__(CHUNK)
     k_assemble_tensor_staged(const emg_pattern pat, const double *__restrict__ rec, int exact_face_mass,
@@ -1620,10 +1652,10 @@ extern "C" int emg_assemble_iso(const emg_pattern *pat, const double *d_nodes, c
         if (!mp->tet_rec) EMG_HIP(hipMalloc(&mp->tet_rec, (size_t)pat->nt * REC * sizeof(double)));
         auto run = [&](int wg) {
             if (flags & EMG_REFERENCE_GEOMETRY)
-                k_tet_gram<true><<<emg::grid_for(pat->nt, 256), 256, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn,
+                k_tet_gram<true><<<emg::grid_for(pat->nt, 64), 64, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn,
                                                                              mp->tet_rec, 0, 0, 0);
             else
-                k_tet_gram<false><<<emg::grid_for(pat->nt, 256), 256, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn,
+                k_tet_gram<false><<<emg::grid_for(pat->nt, 64), 64, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn,
                                                                               mp->tet_rec, 0, 0, 0);
             const int64_t grid = std::min<int64_t>(pat->nchunk, (int64_t)g_num_cus * wg);
             launch_staged<CHUNK>(pat, dim3((unsigned)grid), st, mp->tet_rec, efm, oE, oB);
@@ -1683,11 +1715,11 @@ extern "C" int emg_assemble_iso_batched(const emg_pattern *pat, int nbatch, int6
     const cplx *ce = reinterpret_cast<const cplx *>(d_eps), *cn = reinterpret_cast<const cplx *>(d_nu);
     cplx *oE = reinterpret_cast<cplx *>(d_E), *oB = reinterpret_cast<cplx *>(d_B);
     const int64_t nvs = 3 * nv, rs = pat->nt * (int64_t)REC, os = 4 * pat->nnz_ent;
-    const dim3 gg(emg::grid_for(pat->nt, 256), (unsigned)nbatch);
+    const dim3 gg(emg::grid_for(pat->nt, 64), (unsigned)nbatch);
     if (flags & EMG_REFERENCE_GEOMETRY)
-        k_tet_gram<true><<<gg, 256, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn, mp->tet_rec_batch, nvs, pat->nt, rs);
+        k_tet_gram<true><<<gg, 64, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn, mp->tet_rec_batch, nvs, pat->nt, rs);
     else
-        k_tet_gram<false><<<gg, 256, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn, mp->tet_rec_batch, nvs, pat->nt, rs);
+        k_tet_gram<false><<<gg, 64, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn, mp->tet_rec_batch, nvs, pat->nt, rs);
     launch_staged<CHUNK>(pat, dim3((unsigned)gx, (unsigned)nbatch), st, mp->tet_rec_batch, efm, oE, oB, rs, os);
     EMG_LAUNCH_CHECK();
     return 0;
