@@ -63,10 +63,11 @@ struct emg_pattern {
     int fused_ok = 0;
     int32_t *chunk_row0 = nullptr;   // nchunk + 1, row of each chunk's first entry (last: n_ent - 1)
     int32_t *chunk_tets = nullptr;   // nchunk * CHUNK_TMAX
-    int32_t *chunk_ntets = nullptr;  // nchunk
-    int chunk_tmax = 0;              // largest chunk_ntets of this mesh (sizes the fused kernel's LDS)
+    int32_t *chunk_desc = nullptr;   // nchunk * DESC: what a chunk's workgroup needs to know (DESC_*)
+    int chunk_tmax = 0;              // most tets of a chunk (sizes the fused kernel's LDS)
     uint16_t *inc_local = nullptr;   // n_inc: (local tet << 8) | (s << 4) | s'
-    uint16_t *chunk_perm = nullptr;  // nchunk * CHUNK: chunk-local entries by descending incidence count
+    uint32_t *chunk_ent = nullptr;   // nchunk * CHUNK: the chunk's entries by kind and descending incidence count (ENT_*)
+    uint8_t *chunk_cnt = nullptr;    // nchunk * CHUNK: their incidences, 0 past the last entry
     double *tet_rec = nullptr;       // nt * REC: per-tet Gram records (fused-path workspace)
     double *tet_rec_batch = nullptr; // rec_batch_cap * nt * REC: the records of a batch of meshes
     int rec_batch_cap = 0;
@@ -88,11 +89,23 @@ static constexpr int CHUNK = 512;
 static constexpr int CHUNK_TMAX = 128;
 static constexpr int CHUNK_NMAX = 2048;  // incidences per chunk handled by the tet-list builder
 static constexpr int RECIPE_BYTES = 48;
+// A chunk's values leave in the order of the CSR rows, 2 * CHUNK values of each row mode: of every row's
+// part in the chunk the mode-0 columns, then the mode-1 columns.  A word of chunk_ent: the place of the
+// entry's mode-0 column among them (10 bits), the entries of its row in the chunk (10 bits: its mode-1
+// column is that much further), its first incidence counted from the chunk's first even one (12 bits).
+static constexpr int ENT_ROW = 10, ENT_START = 20;
+static_assert(CHUNK <= 512 && CHUNK_NMAX < 1 << (32 - ENT_START), "a chunk's entries fit their words");
+static_assert(CHUNK_TMAX < 256, "an entry's incidences, each of another tet, fit chunk_cnt");
+// chunk_desc: first 32-bit word of incidence codes and their number, distinct tets, then where the values
+// go: value u of chunk c belongs at 2 c CHUNK + u + (u < N1 ? D0 : u < 2 N1 ? D1 : u >= U4 ? D4 : 0) of its
+// row mode's half (the chunk's first and last row may lie partly in its neighbours).
+enum { DESC_W0, DESC_NW, DESC_NT, DESC_N1, DESC_U4, DESC_D0, DESC_D1, DESC_D4, DESC };
 
 static void build_recipes(uint8_t *out, bool full);
 __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int32_t *__restrict__ chunk_tets,
-                                                      int32_t *__restrict__ chunk_ntets, uint16_t *__restrict__ inc_local,
-                                                      uint16_t *__restrict__ chunk_perm, int *__restrict__ overflow);
+                                                      int32_t *__restrict__ chunk_desc, uint16_t *__restrict__ inc_local,
+                                                      uint32_t *__restrict__ chunk_ent, uint8_t *__restrict__ chunk_cnt,
+                                                      int *__restrict__ overflow);
 
 // ------------------------------------------------------------------ symbolic
 __global__ void k_make_keys(const int32_t *__restrict__ tet_ent, int64_t nt, int bits,
@@ -264,10 +277,11 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
     {
         int *d_over = nullptr;
         TRY(hipMalloc(&pat->chunk_tets, (size_t)pat->nchunk * CHUNK_TMAX * sizeof(int32_t)));
-        TRY(hipMalloc(&pat->chunk_ntets, (size_t)pat->nchunk * sizeof(int32_t)));
+        TRY(hipMalloc(&pat->chunk_desc, (size_t)pat->nchunk * DESC * sizeof(int32_t)));
+        TRY(hipMalloc(&pat->chunk_cnt, (size_t)pat->nchunk * pat->chunk));
         // two spare codes: the fused kernel reads the codes as 32-bit words
         TRY(hipMalloc(&pat->inc_local, (size_t)(n_inc + 2) * sizeof(uint16_t)));
-        TRY(hipMalloc(&pat->chunk_perm, (size_t)pat->nchunk * pat->chunk * sizeof(uint16_t)));
+        TRY(hipMalloc(&pat->chunk_ent, (size_t)pat->nchunk * pat->chunk * sizeof(uint32_t)));
         TRY(hipMalloc(&pat->recipes, 2 * 100 * RECIPE_BYTES));
         TRY(hipMalloc(&d_over, sizeof(int)));
         TRY(hipMemsetAsync(d_over, 0, sizeof(int), st));
@@ -275,18 +289,18 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
         build_recipes(host_rec, false);
         build_recipes(host_rec + 100 * RECIPE_BYTES, true);
         TRY(hipMemcpyAsync(pat->recipes, host_rec, sizeof(host_rec), hipMemcpyHostToDevice, st));
-        k_chunk_tets<<<(unsigned)pat->nchunk, CHUNK, 0, st>>>(*pat, pat->chunk_tets, pat->chunk_ntets, pat->inc_local,
-                                                             pat->chunk_perm, d_over);
+        k_chunk_tets<<<(unsigned)pat->nchunk, CHUNK, 0, st>>>(*pat, pat->chunk_tets, pat->chunk_desc, pat->inc_local,
+                                                             pat->chunk_ent, pat->chunk_cnt, d_over);
         TRY(hipGetLastError());
         int over = 0;
         TRY(hipMemcpyAsync(&over, d_over, sizeof(int), hipMemcpyDeviceToHost, st));
-        std::vector<int32_t> cnt((size_t)pat->nchunk);
-        TRY(hipMemcpyAsync(cnt.data(), pat->chunk_ntets, cnt.size() * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+        std::vector<int32_t> desc((size_t)pat->nchunk * DESC);
+        TRY(hipMemcpyAsync(desc.data(), pat->chunk_desc, desc.size() * sizeof(int32_t), hipMemcpyDeviceToHost, st));
         TRY(hipStreamSynchronize(st));
         hfree(d_over);
         pat->fused_ok = over ? 0 : 1;
         pat->chunk_tmax = 0;
-        for (int32_t v : cnt) pat->chunk_tmax = std::max(pat->chunk_tmax, (int)v);
+        for (size_t i = DESC_NT; i < desc.size(); i += DESC) pat->chunk_tmax = std::max(pat->chunk_tmax, (int)desc[i]);
     }
     TRY(hipStreamSynchronize(st));
     hfree(uniq);
@@ -326,9 +340,10 @@ extern "C" void emg_pattern_destroy(emg_pattern *pat) {
     hfree(pat->blk_row0);
     hfree(pat->tet_blocks);
     hfree(pat->chunk_tets);
-    hfree(pat->chunk_ntets);
+    hfree(pat->chunk_desc);
+    hfree(pat->chunk_cnt);
     hfree(pat->inc_local);
-    hfree(pat->chunk_perm);
+    hfree(pat->chunk_ent);
     hfree(pat->chunk_row0);
     hfree(pat->tet_rec);
     hfree(pat->tet_rec_batch);
@@ -748,8 +763,8 @@ static void build_recipes(uint8_t *out, bool full) {
             int w = 0;
             for (int x = 0; x < 3; x++)
                 for (int y = 0; y < 3; y++) {
-                    R[x * 3 + y] = (uint8_t)(full ? 6 * ki[x] + kj[y] : sym6(ki[x], kj[y]));
-                    R[9 + x * 3 + y] = (uint8_t)(full ? 4 * vi[x] + vj[y] : sym4(vi[x], vj[y]));
+                    R[x * 3 + y] = (uint8_t)(full ? 6 * ki[x] + kj[y] : 8 * sym6(ki[x], kj[y]));
+                    R[9 + x * 3 + y] = (uint8_t)(full ? 4 * vi[x] + vj[y] : 8 * sym4(vi[x], vj[y]));
                     if (tvi[x] == tvj[y]) w |= 1 << (x * 3 + y);
                 }
             R[18] = (uint8_t)(w & 255);
@@ -767,18 +782,23 @@ static void build_recipes(uint8_t *out, bool full) {
                     c[3] = (uint8_t)moment(p, r, p2, r2);
                     R[36 + m * 2 + m2] = (fi && fj && m2 == 0) ? (uint8_t)moment(vi[1], r2, p2, q2) : c[1];
                 }
-            R[40] = (uint8_t)(fi ? edge_index(vi[0], vi[2]) : edge_index(vi[0], vi[1]));
-            R[41] = (uint8_t)edge_index(vi[0], vi[1]);
-            R[42] = (uint8_t)(fj ? edge_index(vj[0], vj[2]) : edge_index(vj[0], vj[1]));
-            R[43] = (uint8_t)edge_index(vj[0], vj[1]);
+            const int ls = full ? 1 : 8;
+            R[40] = (uint8_t)(ls * (fi ? edge_index(vi[0], vi[2]) : edge_index(vi[0], vi[1])));
+            R[41] = (uint8_t)(ls * edge_index(vi[0], vi[1]));
+            R[42] = (uint8_t)(ls * (fj ? edge_index(vj[0], vj[2]) : edge_index(vj[0], vj[1])));
+            R[43] = (uint8_t)(ls * edge_index(vj[0], vj[1]));
             R[44] = (uint8_t)((fi ? 1 : 0) | (fj ? 2 : 0));
         }
 }
 
+// Kind of the entry an incidence (.. | s << 4 | s') belongs to: edge-edge 0, edge-face 1, face-edge 2, face-face 3.
+__device__ __forceinline__ int pair_kind(uint32_t v) { return ((v >> 4) & 15u) >= 6 ? ((v & 15u) >= 6 ? 3 : 2) : ((v & 15u) >= 6 ? 1 : 0); }
+
 // Distinct tets of every chunk, and chunk-local incidence codes.
 __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int32_t *__restrict__ chunk_tets,
-                                                      int32_t *__restrict__ chunk_ntets, uint16_t *__restrict__ inc_local,
-                                                      uint16_t *__restrict__ chunk_perm, int *__restrict__ overflow) {
+                                                      int32_t *__restrict__ chunk_desc, uint16_t *__restrict__ inc_local,
+                                                      uint32_t *__restrict__ chunk_ent, uint8_t *__restrict__ chunk_cnt,
+                                                      int *__restrict__ overflow) {
     __shared__ uint32_t key[CHUNK_NMAX];
     __shared__ uint32_t uq[CHUNK_NMAX];
     __shared__ int hist[256], base[256];       // entries per key, and those with a smaller key
@@ -790,15 +810,16 @@ __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int
     const int64_t k0 = c * ch, k1 = (k0 + ch < pat.nnz_ent) ? k0 + ch : pat.nnz_ent;
     const int32_t q0 = pat.pair_ptr[k0], q1 = pat.pair_ptr[k1];
     const int n = q1 - q0;
-    // Lane order of the fused kernel: the chunk's entries sorted (stably) by
-    // descending incidence count, so a wavefront's lanes loop a similar number
-    // of times.  Position r of the chunk holds local entry chunk_perm[k0 + r].
+    // Lane order of the fused kernels: the chunk's entries sorted (stably) by kind
+    // and descending incidence count, so a wavefront's lanes run the same formulas
+    // a similar number of times.  Position r of the chunk is described by chunk_ent[k0 + r] and chunk_cnt[k0 + r].
     const int np = (int)(k1 - k0);
     const bool has = tid < np;
-    int myk = 255;
+    int myk = 255, my_cnt = 0;
     if (has) {
-        const int cnt = pat.pair_ptr[k0 + tid + 1] - pat.pair_ptr[k0 + tid];
-        myk = 255 - (cnt < 255 ? cnt : 255);
+        const int32_t qk = pat.pair_ptr[k0 + tid];
+        my_cnt = pat.pair_ptr[k0 + tid + 1] - qk;
+        myk = pair_kind(pat.inc[qk]) * 64 + 63 - (my_cnt < 63 ? my_cnt : 63);
     }
     // Stable counting rank: the entries with a smaller key, the entries with my key in
     // earlier wavefronts, and those earlier in my wavefront.  A wavefront walks only the
@@ -829,12 +850,38 @@ __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int
     if (has) {
         int rank = base[myk] + before;
         for (int w = 0; w < wave; w++) rank += wcnt[w][myk];
-        if (rank < ch) chunk_perm[k0 + rank] = (uint16_t)tid;
+        // the entry's row: the last one that starts at or before it
+        int32_t lo = pat.chunk_row0[c], hi = pat.chunk_row0[c + 1];
+        while (lo < hi) {
+            const int32_t mid = (lo + hi + 1) >> 1;
+            if (pat.ent_ptr[mid] <= k0 + tid) lo = mid; else hi = mid - 1;
+        }
+        const int64_t a = max((int64_t)pat.ent_ptr[lo], k0), b = min((int64_t)pat.ent_ptr[lo + 1], k1);
+        const int place = (int)(2 * (a - k0) + (k0 + tid - a));
+        if (rank < ch) {
+            chunk_ent[k0 + rank] = (uint32_t)place | (uint32_t)(b - a) << ENT_ROW | (uint32_t)(pat.pair_ptr[k0 + tid] - (q0 & ~1)) << ENT_START;
+            chunk_cnt[k0 + rank] = (uint8_t)(my_cnt < 255 ? my_cnt : 255);
+        }
+        int32_t *d = chunk_desc + c * DESC;
+        const int64_t row_a = pat.ent_ptr[lo], row_n = pat.ent_ptr[lo + 1] - row_a;
+        if (tid == 0) {
+            d[DESC_W0] = q0 >> 1;
+            d[DESC_NW] = ((q1 + 1) >> 1) - (q0 >> 1);
+            d[DESC_N1] = (int32_t)(b - a);
+            d[DESC_D0] = (int32_t)(row_a - k0);
+            d[DESC_D1] = (int32_t)(row_a + row_n - k0 - (b - a));
+        }
+        if (tid == np - 1) {
+            const bool one = a == k0;   // also the chunk's first row
+            d[DESC_U4] = one ? 2 * np : (int32_t)(2 * np - (b - a));
+            d[DESC_D4] = one ? 0 : (int32_t)(2 * (row_a - k0) + row_n - 2 * np + (b - a));
+        }
     } else if (tid < ch) {
-        chunk_perm[k0 + tid] = (uint16_t)tid;
+        chunk_ent[k0 + tid] = 0;
+        chunk_cnt[k0 + tid] = 0;
     }
     if (n > CHUNK_NMAX * ch / CHUNK) {   // the fused kernel stages at most this many incidences
-        if (tid == 0) { atomicOr(overflow, 1); chunk_ntets[c] = -1; }
+        if (tid == 0) { atomicOr(overflow, 1); chunk_desc[c * DESC + DESC_NT] = -1; }
         return;
     }
     for (int i = tid; i < CHUNK_NMAX; i += CHUNK) key[i] = (i < n) ? (pat.inc[q0 + i] >> 8) : 0xFFFFFFFFu;
@@ -860,11 +907,11 @@ __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int
     __syncthreads();
     const int m = nuniq;
     if (m > CHUNK_TMAX) {
-        if (tid == 0) { atomicOr(overflow, 1); chunk_ntets[c] = -1; }
+        if (tid == 0) { atomicOr(overflow, 1); chunk_desc[c * DESC + DESC_NT] = -1; }
         return;
     }
     for (int i = tid; i < m; i += CHUNK) chunk_tets[c * CHUNK_TMAX + i] = (int32_t)uq[i];
-    if (tid == 0) chunk_ntets[c] = m;
+    if (tid == 0) chunk_desc[c * DESC + DESC_NT] = m;
     for (int i = tid; i < n; i += CHUNK) {
         const uint32_t v = pat.inc[q0 + i];
         const uint32_t t = v >> 8;
@@ -936,11 +983,14 @@ __device__ __forceinline__ void fused_tet_gram(const V3 (&P)[4], const V3 (&gr)[
 
 // One incidence v = (local tet << 8) | (s << 4) | s' of an adjacency entry:
 // adds nu_t * D_t and eps_t * F_t of the slot pair (s, s') (2x2 each) into aD, aF.
-template <int TS>
-__device__ __forceinline__ void fused_incidence(const uint32_t *rcp, const double *td, uint32_t v,
+// FI, FJ: s, s' are faces (the edges' formulas have one curl product, one length and a quarter of
+// the mass terms of the faces').  An entry of a face row and an edge column takes the block of the
+// pair swapped, which is its own transposed: the caller swaps s and s' and transposes at the end.
+// T: the records, TDW doubles each; recipe bytes hold byte offsets into them.
+static constexpr int TDW = TD_FIELDS + 1;
+template <bool FI, bool FJ>
+__device__ __forceinline__ void fused_incidence(const uint32_t *rcp, const double *td, uint32_t tl, uint32_t sp,
                                                 int exact_face_mass, cplx (&aD)[2][2], cplx (&aF)[2][2]) {
-    const int tl = (int)(v >> 8);
-    const int sp = (int)(((v >> 4) & 15u) * 10 + (v & 15u));
     uint32_t w[12];
     const uint4 *R4 = reinterpret_cast<const uint4 *>(rcp + sp * (RECIPE_BYTES / 4));
 #pragma unroll
@@ -948,49 +998,56 @@ __device__ __forceinline__ void fused_incidence(const uint32_t *rcp, const doubl
         const uint4 u = R4[i];
         w[4 * i] = u.x; w[4 * i + 1] = u.y; w[4 * i + 2] = u.z; w[4 * i + 3] = u.w;
     }
-    const double *T = td + tl;
-    const uint32_t wm = rbyte(w, 18) | (rbyte(w, 19) << 8);
-    double h[3][3], g[3][3];
+    const char *T = reinterpret_cast<const char *>(td + tl * TDW);
+    auto at = [&](int field, int byte) { return *reinterpret_cast<const double *>(T + 8 * field + rbyte(w, byte)); };
+    auto field = [&](int f) { return reinterpret_cast<const double *>(T)[f]; };
+    const cplx ct(field(37), field(38)), nt_(field(39), field(40));
+    constexpr int NX = FI ? 3 : 2, NY = FJ ? 3 : 2;
+    // curl products: an edge's first two are the same, up to the integral's weight
+    double h[NX][NY];
 #pragma unroll
-    for (int x = 0; x < 3; x++)
+    for (int x = 0; x < NX; x++)
 #pragma unroll
-        for (int y = 0; y < 3; y++) {
-            const double hv = T[rbyte(w, x * 3 + y) * TS];
-            h[x][y] = ((wm >> (x * 3 + y)) & 1u) ? 2.0 * hv : hv;
-            g[x][y] = T[(21 + rbyte(w, 9 + x * 3 + y)) * TS];
+        for (int y = 0; y < NY; y++) {
+            const double hv = at(0, (FI ? x : 0) * 3 + (FJ ? y : 0));
+            const int b = x * 3 + y;
+            h[x][y] = ((b < 8 ? w[4] >> (16 + b) : w[4] >> 24) & 1u) ? 2.0 * hv : hv;
         }
-    const uint32_t fl = rbyte(w, 44);
-    const bool fi = fl & 1u, fj = fl & 2u;
-    const double cfi[2][3] = {{fi ? -1.0 : -3.0, fi ? -2.0 : 0.0, fi ? -1.0 : 0.0},
-                              {fi ? -2.0 : 0.0, fi ? -1.0 : -3.0, fi ? 1.0 : 0.0}};
-    const double cfj[2][3] = {{fj ? -1.0 : -3.0, fj ? -2.0 : 0.0, fj ? -1.0 : 0.0},
-                              {fj ? -2.0 : 0.0, fj ? -1.0 : -3.0, fj ? 1.0 : 0.0}};
-    const double si[2] = {(fi ? -1.0 : 1.0) * T[(31 + rbyte(w, 40)) * TS], T[(31 + rbyte(w, 41)) * TS]};
-    const double sj[2] = {(fj ? -1.0 : 1.0) * T[(31 + rbyte(w, 42)) * TS], T[(31 + rbyte(w, 43)) * TS]};
-    const cplx ct(T[37 * TS], T[38 * TS]), nt_(T[39 * TS], T[40 * TS]);
-    double hc[3][2];
+    double hc[NX][2];   // along s'
 #pragma unroll
-    for (int x = 0; x < 3; x++)
+    for (int x = 0; x < NX; x++) {
+        if constexpr (FJ) {
+            hc[x][0] = -h[x][0] - 2.0 * h[x][1] - h[x][2];
+            hc[x][1] = -2.0 * h[x][0] - h[x][1] + h[x][2];
+        } else {
+            hc[x][0] = -3.0 * h[x][0];
+            hc[x][1] = -3.0 * h[x][1];
+        }
+    }
+    const double si[2] = {FI ? -at(31, 40) : at(31, 41), at(31, 41)};
+    const double sj[2] = {FJ ? -at(31, 42) : at(31, 43), at(31, 43)};
 #pragma unroll
-        for (int m2 = 0; m2 < 2; m2++)
-            hc[x][m2] = h[x][0] * cfj[m2][0] + h[x][1] * cfj[m2][1] + h[x][2] * cfj[m2][2];
-#pragma unroll
-    for (int m = 0; m < 2; m++) {
-        const bool qc = (m == 0) && fi;
-        const double g_q0 = qc ? g[2][0] : g[1][0];
+    for (int m = 0; m < 2; m++)
 #pragma unroll
         for (int m2 = 0; m2 < 2; m2++) {
-            const bool qc2 = (m2 == 0) && fj;
-            const double g_0q = qc2 ? g[0][2] : g[0][1];
-            const double g_qq = qc ? (qc2 ? g[2][2] : g[2][1]) : (qc2 ? g[1][2] : g[1][1]);
+            double d;
+            if constexpr (FI) d = m == 0 ? -hc[0][m2] - 2.0 * hc[1][m2] - hc[2][m2] : -2.0 * hc[0][m2] - hc[1][m2] + hc[2][m2];
+            else d = -3.0 * hc[m][m2];
+            aD[m][m2] += nt_ * ((si[m] * sj[m2]) * d);
+        }
+    __builtin_amdgcn_sched_barrier(0);   // the curl products' registers serve the mass terms
+    auto g = [&](int x, int y) { return at(21, 9 + x * 3 + y); };
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        const int q = FI && m == 0 ? 2 : 1;
+#pragma unroll
+        for (int m2 = 0; m2 < 2; m2++) {
+            const int q2 = FJ && m2 == 0 ? 2 : 1;
             const int o = 20 + 4 * (m * 2 + m2);
-            const double c1 = (double)(exact_face_mass ? rbyte(w, o + 1) : rbyte(w, 36 + m * 2 + m2));
-            const double f = (double)rbyte(w, o) * g[0][0] - c1 * g_0q - (double)rbyte(w, o + 2) * g_q0 +
-                             (double)rbyte(w, o + 3) * g_qq;
-            const double d = cfi[m][0] * hc[0][m2] + cfi[m][1] * hc[1][m2] + cfi[m][2] * hc[2][m2];
-            const double sij = si[m] * sj[m2];
-            aD[m][m2] += nt_ * (sij * d);
-            aF[m][m2] += ct * (sij * f);
+            const uint32_t c1 = FI && FJ && !exact_face_mass ? rbyte(w, 36 + m * 2 + m2) : rbyte(w, o + 1);
+            const double f = (double)rbyte(w, o) * g(0, 0) - (double)c1 * g(0, q2) - (double)rbyte(w, o + 2) * g(q, 0) +
+                             (double)rbyte(w, o + 3) * g(q, q2);
+            aF[m][m2] += ct * ((si[m] * sj[m2]) * f);
         }
     }
 }
@@ -1101,237 +1158,220 @@ __global__ void __launch_bounds__(64) k_tet_gram(int64_t nt, const double *__res
     }
 }
 
+// Lane's value i (0 or 1) of the 2 CH values of a row mode whose half of the matrix begins at `half`: u, shifted
+// so that eight consecutive lanes hold one aligned 128-byte line wherever the chunk's values are consecutive.
+template <int CH>
+__device__ __forceinline__ int out_value(const cplx *half, int i) {
+    const int u = i * CH + (int)threadIdx.x - (int)((reinterpret_cast<uintptr_t>(half) >> 4) & 7);
+    return u < 0 ? u + 2 * CH : u;
+}
+__device__ __forceinline__ int out_shift(int u, int n1, int u4, int d0, int d1, int d4) {
+    return u < n1 ? d0 : u < 2 * n1 ? d1 : u >= u4 ? d4 : 0;
+}
+
 // Numeric assembly, one workgroup of CH lanes per chunk of CH consecutive
 // adjacency entries (grid-stride over chunks).  Per chunk:
-//  * its index data (entry offsets into the incidences, the offsets of the rows
-//    it spans, the incidence codes, the lane order) and the Gram records of its
-//    distinct tets (k_tet_gram) are loaded into registers while the previous
-//    chunk writes its output (the tet ids one step earlier, while it runs its
-//    incidence loop), and put into LDS when the chunk starts: no global load is
-//    waited for on the chunk's critical path, and the incidence loop reads only LDS;
-//  * lane r accumulates entry chunk_perm[r] (entries by descending incidence
-//    count, so the lanes of a wavefront loop a similar number of times);
-//  * the 2x2 blocks go back through LDS (reusing the Gram area) and are written
-//    in entry order, coalesced.
-// The wavefront taking the heaviest entries rotates with the chunk, so no SIMD
-// always gets them.  Launch bound: 4 waves per SIMD (3 for the widest LDS layout).
+//  * the Gram records of its distinct tets (k_tet_gram) and its incidence codes are in LDS, so the
+//    incidence loop reads only LDS;
+//  * lane r accumulates entry chunk_ent[r] (entries by kind and descending incidence
+//    count, so the lanes of a wavefront run the same formulas a similar number of times);
+//  * the 2x2 blocks go through LDS into the order of the CSR rows and leave as whole lines.
+// What bounds it is the CSR writes, and the reads among them: at 1,005,000 tets (8.6 GB written, 1.2 read)
+// 2.31 ms, 2.22 without the incidence loop, 1.45 without the stores.  What counts for them (2.89 ms before):
+//  * whole lines per store: rows of 37 values per mode, stored as they lie in the entries' order, split
+//    a line between two stores at every row's end (a store-only kernel of that shape 2.07 ms, 1.46 with lines);
+//  * runs of 32 chunks per XCD: workgroups that step through the whole grid drift apart, and the stores
+//    in flight spread over too much memory (store-only, 512 resident workgroups: 1.75 ms, 1.45 in runs);
+//  * the next loads issued before the stores, so that waiting for them does not wait for the stores;
+//  * an entry's place, row and incidences in five bytes, where the search for its row took nine steps in LDS;
+//  * formulas by kind: with edge pairs, edge-face pairs and face pairs in wavefronts of their own the
+//    incidence loop takes 118, 140 and 182 vector instructions where the common one took 190.
+// 128 registers, so 4 waves per SIMD, two workgroups per CU.  Slower: one chunk per workgroup with 4, 5 or
+// 6 waves per SIMD and no loads ahead (3.5 - 3.8 ms), non-temporal stores (3.6), 256-entry chunks (2.57),
+// fewer vector instructions at the price of longer chains of them in the loop (2.45).
 template <int TS, int CH>
-__global__ void __launch_bounds__(CH, TS <= 96 ? 4 : 3)
+__global__ void __launch_bounds__(CH, TS <= 96 ? 4 : 2)
     k_assemble_staged(const emg_pattern pat, const double *__restrict__ rec, int exact_face_mass,
-                      cplx *__restrict__ E, cplx *__restrict__ B, int64_t rec_stride, int64_t out_stride) {
+                      cplx *__restrict__ E, cplx *__restrict__ B, int64_t rec_stride, int64_t out_stride, int run) {
     // blockIdx.y: the mesh of a batch (its records and output values at these strides)
     rec += blockIdx.y * rec_stride;
     E += blockIdx.y * out_stride;
     B += blockIdx.y * out_stride;
-    constexpr int TSP = TS + 1;             // odd field stride of the Gram data: fewer LDS bank conflicts
-    constexpr int TD = TD_FIELDS * TSP;     // doubles of Gram data
-    constexpr int SD = 2 * 4 * CH;          // doubles of one staged matrix: 4 blocks x CH complex
-    constexpr int NINC = CHUNK_NMAX * CH / CHUNK;
-    constexpr int NID = NINC / 2 + 1;       // incidence codes as 32-bit words (first one may be half used)
-    constexpr int RI = (NID + CH - 1) / CH; // words per lane
+    constexpr int NID = CHUNK_NMAX * CH / CHUNK / 2 + 1;   // incidence codes as 32-bit words (first one may be half used)
     constexpr int NW = CH / 64;
-    constexpr int SPR = CH / 8;             // tet records per round: 8 lanes per record, 7 of them load 6 doubles
-    constexpr int RR = (TS + SPR - 1) / SPR;
-    static_assert(7 * 6 >= TD_FIELDS && 7 * 6 <= REC, "7 lanes of 6 doubles cover a record");
-    static_assert(RR * SPR <= CHUNK_TMAX, "tet_ids reads slots below CHUNK_TMAX only");
-    __shared__ uint32_t rcp[100 * RECIPE_BYTES / 4];
-    __shared__ __align__(16) double td[TD > SD ? TD : SD];
-    __shared__ int32_t s_pp[CH + 1];        // entry -> first incidence (absolute)
-    __shared__ int32_t s_row[CH + 2];       // ent_ptr of the rows the chunk spans
+    constexpr int SPR = CH / 8;             // tet records loaded ahead: 8 lanes per record, 7 of them load 6 doubles
+    static_assert(7 * 6 == TDW && TDW <= REC, "7 lanes of 6 doubles cover a record");
+    static_assert(SPR <= CHUNK_TMAX, "look_up reads slots below CHUNK_TMAX only");
+    __shared__ __align__(16) uint32_t rcp[100 * RECIPE_BYTES / 4];
+    __shared__ __align__(16) double td[TS * TDW];
+    __shared__ __align__(16) double stage_lds[2 * 4 * CH];
     __shared__ uint32_t s_inc[NID];         // the chunk's incidence codes (16-bit), from an even index
-    __shared__ uint16_t s_perm[CH];         // lane order
-    __shared__ int2 s_out[CH];              // per entry: (row start, row length)
+    cplx *const stg = reinterpret_cast<cplx *>(stage_lds);   // one matrix' values, 2 CH of either row mode
     const int tid = threadIdx.x;
-    const int rs = tid >> 3, rsub = tid & 7;   // record slot within a round, 6-double part of the record
+    const int rs = tid >> 3, rsub = tid & 7;   // record slot, 6-double part of the record
     for (int i = tid; i < 100 * RECIPE_BYTES / 4; i += CH) rcp[i] = reinterpret_cast<const uint32_t *>(pat.recipes)[i];
-    cplx *stg = reinterpret_cast<cplx *>(td);
-    // registers holding the next chunk's data; every one is assigned on every
-    // path, so none stays live through the incidence loop
-    int32_t f_q0 = 0, f_ninc = 0, f_nr = 0, f_nt = 0;              // uniform
-    int32_t g_nt = 0;                                               // uniform
-    int32_t g_u = 0;   // lanes 0-3 of each wave: the next chunk's first and end incidence, first and end row
-    int32_t f_pp[2], f_row[2], g_t[RR];
-    uint32_t f_inc[RI];
-    int f_perm = 0;
-    double2 f_rec[RR][3];
-    // The chunk's tet ids and its uniform offsets, issued before the incidence loop.
-    // Unconditional loads (the chunk index clamped, every slot below CHUNK_TMAX in
-    // bounds): nothing here depends on a loaded value, so nothing waits for these
-    // loads before prefetch uses them; slots at or past the tet count are never used.
-    auto tet_ids = [&](int64_t cc) {
-        const int64_t cl = cc < pat.nchunk ? cc : pat.nchunk - 1;
-        const int64_t kl = cl * CH;
-        g_nt = pat.chunk_ntets[cl];
-        // one gather, lane by lane, so the values stay in vector registers until
-        // prefetch reads them (a uniform load would be moved to a scalar register,
-        // which waits for it at once)
-        const int32_t *src = (tid & 3) == 0   ? pat.pair_ptr + kl
-                             : (tid & 3) == 1 ? pat.pair_ptr + (pat.nnz_ent - kl < CH ? pat.nnz_ent : kl + CH)
-                             : (tid & 3) == 2 ? pat.chunk_row0 + cl
-                                              : pat.chunk_row0 + cl + 1;
-        g_u = *src;
-#pragma unroll
-        for (int h = 0; h < RR; h++) g_t[h] = pat.chunk_tets[cl * CHUNK_TMAX + h * SPR + rs];
+    const uint16_t *inc16 = reinterpret_cast<const uint16_t *>(s_inc);
+    // registers holding the next chunk's data and, one step further ahead, what its loads need
+    int32_t f_desc[DESC] = {};   // uniform
+    uint32_t f_inc = 0, f_ent = 0;
+    int f_cnt = 0;
+    double2 f_rec0 = make_double2(0.0, 0.0), f_rec1 = f_rec0, f_rec2 = f_rec0;
+    int32_t g_desc = 0, g_t = 0;   // g_desc: lane i of each eight holds word i of the descriptor
+    // A chunk's descriptor and tet ids: unconditional loads (the chunk index clamped, slots below
+    // CHUNK_TMAX in bounds), the descriptor lane by lane, so that it stays in a vector register until
+    // prefetch reads it (a uniform load would be moved to scalar registers, which waits for it at once).
+    auto look_up = [&](int64_t cl) {
+        g_desc = pat.chunk_desc[cl * DESC + rsub];
+        g_t = pat.chunk_tets[cl * CHUNK_TMAX + rs];
     };
-    auto prefetch = [&](int64_t cc) {
-        f_q0 = 0; f_ninc = 0; f_nr = 0; f_perm = 0; f_nt = 0;
+    auto prefetch = [&](int64_t cl) {
 #pragma unroll
-        for (int h = 0; h < 2; h++) { f_pp[h] = 0; f_row[h] = 0; }
-#pragma unroll
-        for (int h = 0; h < RI; h++) f_inc[h] = 0;
-#pragma unroll
-        for (int h = 0; h < RR; h++)
-#pragma unroll
-            for (int q = 0; q < 3; q++) f_rec[h][q] = make_double2(0.0, 0.0);
-        if (cc >= pat.nchunk) return;
-        f_nt = g_nt;
-        const int64_t kk = cc * CH;
-        const int npp = (int)(pat.nnz_ent - kk < CH ? pat.nnz_ent - kk : CH);
-        f_q0 = __builtin_amdgcn_readlane(g_u, 0);
-        f_ninc = __builtin_amdgcn_readlane(g_u, 1) - f_q0;
-        const int32_t r0 = __builtin_amdgcn_readlane(g_u, 2);
-        f_nr = __builtin_amdgcn_readlane(g_u, 3) - r0 + 2;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int i = tid + h * CH;
-            if (i <= npp) f_pp[h] = pat.pair_ptr[kk + i];
-            if (i < f_nr) f_row[h] = pat.ent_ptr[r0 + i];
-        }
-        const int64_t w0 = f_q0 >> 1;
-        const int nwords = (int)(((int64_t)f_q0 + f_ninc + 1) / 2 - w0);
-#pragma unroll
-        for (int h = 0; h < RI; h++) {
-            const int i = tid + h * CH;
-            if (i < nwords) f_inc[h] = reinterpret_cast<const uint32_t *>(pat.inc_local)[w0 + i];
-        }
-        f_perm = pat.chunk_perm[kk + tid];
-#pragma unroll
-        for (int h = 0; h < RR; h++)
-            if (h * SPR + rs < f_nt && rsub < 7) {
-                const double2 *r = reinterpret_cast<const double2 *>(rec + (int64_t)g_t[h] * REC + rsub * 6);
-#pragma unroll
-                for (int q = 0; q < 3; q++) f_rec[h][q] = r[q];
-            }
+        for (int i = 0; i < DESC; i++) f_desc[i] = __builtin_amdgcn_readlane(g_desc, i);
+        f_inc = reinterpret_cast<const uint32_t *>(pat.inc_local)[f_desc[DESC_W0] + (tid < f_desc[DESC_NW] ? tid : 0)];
+        // wave hw takes the first (heaviest) 64 positions of the chunk's order, another one in every chunk
+        const int hw = (int)((cl + NW / 2) % NW);
+        const int64_t at = cl * CH + (((tid >> 6) - hw + NW) % NW) * 64 + (tid & 63);
+        f_ent = pat.chunk_ent[at];
+        f_cnt = pat.chunk_cnt[at];
+        const double2 *r = reinterpret_cast<const double2 *>(rec + (int64_t)(rs < f_desc[DESC_NT] ? g_t : 0) * REC + (rsub < 7 ? rsub * 6 : 0));
+        f_rec0 = r[0];
+        f_rec1 = r[1];
+        f_rec2 = r[2];
     };
-    // the prefetched registers of chunk cc into LDS; the chunk's row count and first
-    // incidence index stay in cur_nr / cur_qb
-    int32_t cur_nr = 0, cur_qb = 0;
+    // the chunk in the registers into LDS, with what they do not hold
+    uint32_t ent = 0;
+    int cnt = 0;
+    int32_t n1 = 0, u4 = 0, d0 = 0, d1 = 0, d4 = 0;
     auto stage = [&](int64_t cc) {
-        const int64_t kk = cc * CH;
-        const int npp = cc < pat.nchunk ? (int)(pat.nnz_ent - kk < CH ? pat.nnz_ent - kk : CH) : 0;
-        const int32_t ioff = f_q0 & 1, nr = f_nr, nT = f_nt;
+        const int nt = f_desc[DESC_NT], nw = f_desc[DESC_NW];
+        double2 *t2 = reinterpret_cast<double2 *>(td);
+        if (rs < nt && rsub < 7) {
+            t2[rs * (TDW / 2) + rsub * 3] = f_rec0;
+            t2[rs * (TDW / 2) + rsub * 3 + 1] = f_rec1;
+            t2[rs * (TDW / 2) + rsub * 3 + 2] = f_rec2;
+        }
+        for (int slot = rs + SPR; slot < nt; slot += SPR)
+            if (rsub < 7) {
+                const double2 *r = reinterpret_cast<const double2 *>(rec + (int64_t)pat.chunk_tets[cc * CHUNK_TMAX + slot] * REC + rsub * 6);
 #pragma unroll
-        for (int h = 0; h < RR; h++) {
-            const int slot = h * SPR + rs;
-            if (slot < nT && rsub < 7) {
-#pragma unroll
-                for (int q = 0; q < 6; q++) {
-                    const int f = rsub * 6 + q;
-                    if (f < TD_FIELDS) td[f * TSP + slot] = (q & 1) ? f_rec[h][q >> 1].y : f_rec[h][q >> 1].x;
-                }
+                for (int q = 0; q < 3; q++) t2[slot * (TDW / 2) + rsub * 3 + q] = r[q];
             }
-        }
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int i = tid + h * CH;
-            if (i <= npp) s_pp[i] = f_pp[h];
-            if (i < nr) s_row[i] = f_row[h];
-        }
-        {
-            const int nwords = (ioff + f_ninc + 1) / 2;
-#pragma unroll
-            for (int h = 0; h < RI; h++) {
-                const int i = tid + h * CH;
-                if (i < nwords) s_inc[i] = f_inc[h];
-            }
-        }
-        s_perm[tid] = (uint16_t)f_perm;
-        cur_nr = nr;
-        cur_qb = f_q0 - ioff;   // incidence index of s_inc's first 16-bit half
+        if (tid < nw) s_inc[tid] = f_inc;
+        for (int i = tid + CH; i < nw; i += CH)
+            s_inc[i] = reinterpret_cast<const uint32_t *>(pat.inc_local)[f_desc[DESC_W0] + i];
+        ent = f_ent;
+        cnt = f_cnt;
+        n1 = f_desc[DESC_N1]; u4 = f_desc[DESC_U4];
+        d0 = f_desc[DESC_D0]; d1 = f_desc[DESC_D1]; d4 = f_desc[DESC_D4];
     };
-    tet_ids(blockIdx.x);
-    prefetch(blockIdx.x);
-    stage(blockIdx.x);
-    for (int64_t c = blockIdx.x; c < pat.nchunk; c += gridDim.x) {
-        __syncthreads();   // the chunk's index data and Gram records are in LDS
-        const int64_t k0 = c * CH;
-        const int np = (int)(pat.nnz_ent - k0 < CH ? pat.nnz_ent - k0 : CH);
-        const int32_t nr = cur_nr, qb = cur_qb;
-        tet_ids(c + gridDim.x);
-        const int hw = (int)((c + NW / 2) % NW);   // wave hw takes the first (heaviest) 64 lane-order positions
-        const int lk = s_perm[(((tid >> 6) - hw + NW) % NW) * 64 + (tid & 63)];
-        const bool act = lk < np;
+    // Chunk l of this workgroup's XCD (workgroup b is on XCD b % 8), clamped to its last one: the XCDs take
+    // runs of 1 << run consecutive chunks in turn.
+    const int64_t xcd = blockIdx.x % 8, all = pat.nchunk >> run >> 3;
+    const int64_t rest = pat.nchunk - (all << run << 3) - (xcd << run), most = (int64_t)1 << run;
+    const int64_t mine = (all << run) + (rest < 0 ? 0 : rest < most ? rest : most);
+    auto chunk_at = [&](int64_t l) {
+        if (l >= mine) l = mine - 1;
+        return (((l >> run << 3) + xcd) << run) + (l & (most - 1));
+    };
+    const int64_t step = (gridDim.x + 7 - xcd) / 8;
+    int64_t l = blockIdx.x / 8;
+    if (l >= mine) return;
+    look_up(chunk_at(l));
+    prefetch(chunk_at(l));
+    look_up(chunk_at(l + step));
+    stage(chunk_at(l));
+    prefetch(chunk_at(l + step));
+    look_up(chunk_at(l + 2 * step));
+    for (; l < mine; l += step) {
+        const int64_t c = chunk_at(l);
+        __syncthreads();   // the chunk's incidence codes and Gram records are in LDS
+        const int qa = (int)(ent >> ENT_START), qe = qa + cnt;
         cplx aD[2][2], aF[2][2];
-        int32_t p0 = 0, deg = 0;
-        if (act) {
-            const int64_t k = k0 + lk;
-            int lo = 0, hi = nr - 2;   // the row of k: last i with s_row[i] <= k
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (s_row[mid] <= k) lo = mid; else hi = mid - 1;
-            }
-            p0 = s_row[lo];
-            deg = s_row[lo + 1] - p0;
-            const int q1 = s_pp[lk + 1] - qb;
-            const uint16_t *inc16 = reinterpret_cast<const uint16_t *>(s_inc);
+        uint32_t vn = inc16[qa];   // the next incidence's code
+        const int kind = cnt > 0 ? pair_kind(vn) : 4;   // of every incidence of the entry
+        if (kind == 0) {
 #pragma unroll 1
-            for (int q = s_pp[lk] - qb; q < q1; q++) fused_incidence<TSP>(rcp, td, inc16[q], exact_face_mass, aD, aF);
+            for (int q = qa; q < qe; q++) {
+                const uint32_t v = vn;
+                vn = inc16[q + 1];
+                fused_incidence<false, false>(rcp, td, v >> 8, ((v >> 4) & 15u) * 10 + (v & 15u), 0, aD, aF);
+            }
+        } else if (kind == 3) {
+#pragma unroll 1
+            for (int q = qa; q < qe; q++) {
+                const uint32_t v = vn;
+                vn = inc16[q + 1];
+                fused_incidence<true, true>(rcp, td, v >> 8, ((v >> 4) & 15u) * 10 + (v & 15u), exact_face_mass, aD, aF);
+            }
+        } else if (kind < 4) {
+#pragma unroll 1
+            for (int q = qa; q < qe; q++) {
+                const uint32_t v = vn, a = (v >> 4) & 15u, b = v & 15u;
+                vn = inc16[q + 1];
+                fused_incidence<false, true>(rcp, td, v >> 8, kind == 1 ? a * 10 + b : b * 10 + a, 0, aD, aF);
+            }
         }
-        __syncthreads();   // Gram data no longer read: td becomes the output stage
-        prefetch(c + gridDim.x);
-        if (act) {
-#pragma unroll
-            for (int m = 0; m < 4; m++) stg[m * CH + lk] = aD[m >> 1][m & 1];
-            s_out[lk] = make_int2(p0, deg);
+        // where the values go: of row mode 0 and 1, the mode-1 columns `next` further; an entry of a face
+        // row and an edge column has its block transposed
+        cplx *const s00 = stg + (ent & ((1 << ENT_ROW) - 1));
+        const int next = (int)(ent >> ENT_ROW) & ((1 << (ENT_START - ENT_ROW)) - 1);
+        const int o01 = kind == 2 ? 2 * CH : next, o10 = kind == 2 ? next : 2 * CH;
+        if (cnt > 0) {
+            s00[0] = aD[0][0];
+            s00[o01] = aD[0][1];
+            s00[o10] = aD[1][0];
+            s00[2 * CH + next] = aD[1][1];
         }
-        __syncthreads();
-        // the blocks in entry order into registers, through the stage
-        int2 o = make_int2(0, 0);
-        cplx ev[4], bv[4];
-        if (tid < np) {
-            o = s_out[tid];
-#pragma unroll
-            for (int m = 0; m < 4; m++) ev[m] = stg[m * CH + tid];
-        }
-        __syncthreads();
-        if (act) {
-#pragma unroll
-            for (int m = 0; m < 4; m++) stg[m * CH + lk] = aF[m >> 1][m & 1];
-        }
-        __syncthreads();
-        if (tid < np) {
-#pragma unroll
-            for (int m = 0; m < 4; m++) bv[m] = stg[m * CH + tid];
-        }
-        __syncthreads();   // LDS free: the next chunk's data goes in before this chunk's stores
-        // are issued, so waiting for the prefetched loads does not wait for the stores
-        // (loads and stores share one counter); the stores drain during the next chunk
-        stage(c + gridDim.x);
-        if (tid < np) {
+        const int32_t cn1 = n1, cu4 = u4, cd0 = d0, cd1 = d1, cd4 = d4;
+        const bool act = cnt > 0;
+        const int64_t k0 = c * CH, half = 2 * pat.nnz_ent;
+        const int n2 = 2 * (int)(pat.nnz_ent - k0 < CH ? pat.nnz_ent - k0 : CH);
+        auto leave = [&](cplx *out) {
 #pragma unroll
             for (int m = 0; m < 4; m++) {
-                const int64_t a = (int64_t)(m >> 1) * 2 * pat.nnz_ent + o.x + (int64_t)(m & 1) * o.y + k0 + tid;
-                E[a] = ev[m];
-                B[a] = bv[m];
+                cplx *const o = out + 2 * k0 + (m >> 1) * half;
+                const int u = out_value<CH>(o, m & 1);
+                if (u < n2) o[u + out_shift(u, cn1, cu4, cd0, cd1, cd4)] = stg[(m >> 1) * 2 * CH + u];
             }
+        };
+        __syncthreads();
+        // the next chunk into LDS and the loads of the one after it before this chunk's stores: loads and
+        // stores share one counter, so a wait for loads issued after them would wait for the stores
+        stage(chunk_at(l + step));
+        prefetch(chunk_at(l + 2 * step));
+        look_up(chunk_at(l + 3 * step));
+        leave(E);
+        __syncthreads();
+        if (act) {
+            s00[0] = aF[0][0];
+            s00[o01] = aF[0][1];
+            s00[o10] = aF[1][0];
+            s00[2 * CH + next] = aF[1][1];
         }
+        __syncthreads();
+        leave(B);
     }
 }
 
+// Chunks (a power of two) that an XCD takes in a run: 32, but of at least 16 runs per XCD, so that the XCDs
+// get equal shares (1,005,000 tets: 2.40 ms with runs of 8 or 32, 2.43 with 256, 2.49 with 2,048, 2.62 with 1).
+static constexpr int ASM_RUN = 5;
 template <int CH>
 static void launch_staged(const emg_pattern *pat, dim3 grid, hipStream_t st, const double *rec, int efm, cplx *oE,
                           cplx *oB, int64_t rec_stride = 0, int64_t out_stride = 0) {
     const int tm = pat->chunk_tmax;
+    int run = 0;
+    while (run < ASM_RUN && pat->nchunk >> (run + 8) > 0) run++;   // 2^run * 8 XCDs * 16 runs at most nchunk
     if (tm <= 32)
-        k_assemble_staged<32, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride);
+        k_assemble_staged<32, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride, run);
     else if (tm <= 48)
-        k_assemble_staged<48, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride);
+        k_assemble_staged<48, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride, run);
     else if (tm <= 64)
-        k_assemble_staged<64, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride);
+        k_assemble_staged<64, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride, run);
     else if (tm <= 96)
-        k_assemble_staged<96, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride);
+        k_assemble_staged<96, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride, run);
     else
-        k_assemble_staged<CHUNK_TMAX, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride);
+        k_assemble_staged<CHUNK_TMAX, CH><<<grid, CH, 0, st>>>(*pat, rec, efm, oE, oB, rec_stride, out_stride, run);
 }
 
 // ------------------------------------------------------------ tensor materials
@@ -1489,10 +1529,10 @@ __device__ __forceinline__ void tensor_incidence(const uint32_t *rcp, const doub
 // records of its distinct tets (k_tet_tensor) and its index data in LDS, lanes in the chunk's order of
 // descending incidence count, values through LDS into entry order (as k_assemble_staged, without the
 // staging of the next chunk: a workgroup that waits for its records leaves the CU to the others).
-// Bound by the latency of that start and by the CSR writes: 245 us at 49,680 tets (460 MB, 1.9 TB/s),
-// with the records' 17 us 265 us where one lane per entry took 1430.
+// Bound by the latency of that start and by the CSR writes: 234 us at 49,680 tets (460 MB, 2.0 TB/s),
+// with the records' 17 us 250 us where one lane per entry took 1430.
 template <int TS>
-__global__ void __launch_bounds__(CHUNK)
+__global__ void __launch_bounds__(CHUNK, TS <= 64 ? 4 : 2)
     k_assemble_tensor_staged(const emg_pattern pat, const double *__restrict__ rec, int exact_face_mass,
                              cplx *__restrict__ E, cplx *__restrict__ B) {
     constexpr int TSP = TS + 1;
@@ -1500,15 +1540,11 @@ __global__ void __launch_bounds__(CHUNK)
     constexpr int NID = CHUNK_NMAX / 2 + 1;
     __shared__ __align__(16) uint32_t rcp[100 * RECIPE_BYTES / 4];
     __shared__ __align__(16) double td[TD > SD ? TD : SD];
-    __shared__ int32_t s_row[CHUNK + 2];
     __shared__ uint32_t s_inc[NID];
-    __shared__ int2 s_out[CHUNK];
     const int tid = threadIdx.x;
     const int64_t c = blockIdx.x, k0 = c * CHUNK;
-    const int np = (int)(pat.nnz_ent - k0 < CHUNK ? pat.nnz_ent - k0 : CHUNK);
-    const int nT = pat.chunk_ntets[c];
-    const int32_t q0 = pat.pair_ptr[k0], ninc = pat.pair_ptr[k0 + np] - q0;
-    const int32_t r0 = pat.chunk_row0[c], nr = pat.chunk_row0[c + 1] - r0 + 2;
+    const int32_t *d = pat.chunk_desc + c * DESC;
+    const int nT = d[DESC_NT], nw = d[DESC_NW], w0 = d[DESC_W0];
     // eight lanes per record, seven pairs of doubles each
     for (int slot = tid >> 3; slot < nT; slot += CHUNK / 8) {
         const double2 *src = reinterpret_cast<const double2 *>(rec + (int64_t)pat.chunk_tets[c * CHUNK_TMAX + slot] * TREC);
@@ -1526,46 +1562,33 @@ __global__ void __launch_bounds__(CHUNK)
     }
     const uint32_t *recipe = reinterpret_cast<const uint32_t *>(pat.recipes + 100 * RECIPE_BYTES);
     for (int i = tid; i < 100 * RECIPE_BYTES / 4; i += CHUNK) rcp[i] = recipe[i];
-    for (int i = tid; i < nr && i < CHUNK + 2; i += CHUNK) s_row[i] = pat.ent_ptr[r0 + i];
-    const int32_t ioff = q0 & 1;
-    for (int i = tid; i < (ioff + ninc + 1) / 2; i += CHUNK)
-        s_inc[i] = reinterpret_cast<const uint32_t *>(pat.inc_local)[(q0 >> 1) + i];
-    const int lk = pat.chunk_perm[k0 + tid];
-    const bool act = lk < np;
-    const int qa = act ? pat.pair_ptr[k0 + lk] - q0 + ioff : 0, qb = act ? pat.pair_ptr[k0 + lk + 1] - q0 + ioff : 0;
+    for (int i = tid; i < nw; i += CHUNK) s_inc[i] = reinterpret_cast<const uint32_t *>(pat.inc_local)[w0 + i];
+    const uint32_t ent = pat.chunk_ent[k0 + tid];
+    const int qa = (int)(ent >> ENT_START), qb = qa + pat.chunk_cnt[k0 + tid];
     __syncthreads();
     cplx aD[2][2], aF[2][2];
-    int32_t p0 = 0, deg = 0;
-    if (act) {
-        const int64_t k = k0 + lk;
-        int lo = 0, hi = nr - 2;   // the row of k: last i with s_row[i] <= k
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (s_row[mid] <= k) lo = mid; else hi = mid - 1;
-        }
-        p0 = s_row[lo];
-        deg = s_row[lo + 1] - p0;
-        const uint16_t *inc16 = reinterpret_cast<const uint16_t *>(s_inc);
+    const uint16_t *inc16 = reinterpret_cast<const uint16_t *>(s_inc);
 #pragma unroll 1
-        for (int q = qa; q < qb; q++) tensor_incidence<TSP>(rcp, td, inc16[q], exact_face_mass, aD, aF);
-    }
-    cplx *stg = reinterpret_cast<cplx *>(td);
-    int2 o = make_int2(0, 0);
+    for (int q = qa; q < qb; q++) tensor_incidence<TSP>(rcp, td, inc16[q], exact_face_mass, aD, aF);
+    cplx *const stg = reinterpret_cast<cplx *>(td), *const s00 = stg + (ent & ((1 << ENT_ROW) - 1));
+    const int next = (int)(ent >> ENT_ROW) & ((1 << (ENT_START - ENT_ROW)) - 1);
+    const int n2 = 2 * (int)(pat.nnz_ent - k0 < CHUNK ? pat.nnz_ent - k0 : CHUNK);
 #pragma unroll
     for (int mat = 0; mat < 2; mat++) {
         __syncthreads();   // records, then the first matrix' blocks, no longer read
-        if (act) {
-#pragma unroll
-            for (int m = 0; m < 4; m++) stg[m * CHUNK + lk] = mat == 0 ? aD[m >> 1][m & 1] : aF[m >> 1][m & 1];
-            if (mat == 0) s_out[lk] = make_int2(p0, deg);
+        if (qb > qa) {
+            s00[0] = mat == 0 ? aD[0][0] : aF[0][0];
+            s00[next] = mat == 0 ? aD[0][1] : aF[0][1];
+            s00[2 * CHUNK] = mat == 0 ? aD[1][0] : aF[1][0];
+            s00[2 * CHUNK + next] = mat == 0 ? aD[1][1] : aF[1][1];
         }
         __syncthreads();
-        if (tid < np) {
-            if (mat == 0) o = s_out[tid];
-            cplx *out = mat == 0 ? E : B;
 #pragma unroll
-            for (int m = 0; m < 4; m++)
-                out[(int64_t)(m >> 1) * 2 * pat.nnz_ent + o.x + (int64_t)(m & 1) * o.y + k0 + tid] = stg[m * CHUNK + tid];
+        for (int m = 0; m < 4; m++) {
+            cplx *const o = (mat == 0 ? E : B) + 2 * k0 + (m >> 1) * 2 * pat.nnz_ent;
+            const int u = out_value<CHUNK>(o, m & 1);
+            if (u < n2)
+                o[u + out_shift(u, d[DESC_N1], d[DESC_U4], d[DESC_D0], d[DESC_D1], d[DESC_D4])] = stg[(m >> 1) * 2 * CHUNK + u];
         }
     }
 }
@@ -1587,6 +1610,7 @@ static int g_num_cus = 0;
 // assembly on a pattern runs each candidate once untimed and twice between HIP events (so it
 // synchronises the stream once) and keeps the fastest for the pattern's life;
 // EMG_ASM_WG_PER_CU (one of the candidates) overrides the search.
+static constexpr int BATCH_WG = 4;   // workgroups per CU of a batch on an untuned pattern
 static const int ASM_WG[5] = {4, 8, 16, 32, 64};
 
 template <typename RUN>
@@ -1706,11 +1730,11 @@ extern "C" int emg_assemble_iso_batched(const emg_pattern *pat, int nbatch, int6
         EMG_HIP(hipMalloc(&mp->tet_rec_batch, (size_t)nbatch * pat->nt * REC * sizeof(double)));
         mp->rec_batch_cap = nbatch;
     }
-    // every mesh gets the single-mesh grid (the tuned workgroups per CU, else 32): the batch is the
-    // single launches back to back without their gaps, and small meshes, whose own launch
-    // cannot fill the GPU, fill it together
-    const int64_t gx = std::max<int64_t>(1, std::min<int64_t>(pat->nchunk,
-                                                              (int64_t)g_num_cus * (pat->wg_per_cu ? pat->wg_per_cu : 32)));
+    // the tuned workgroups per CU, or 4, shared out among the meshes: of small meshes every workgroup
+    // still steps through several chunks, whose loads it issues ahead (32 meshes of 864 tets: 82 us with a
+    // workgroup per chunk, 77 with 4 workgroups per CU, 78 and 79 with 2 and 8)
+    const int64_t per_mesh = ((int64_t)g_num_cus * (pat->wg_per_cu ? pat->wg_per_cu : BATCH_WG) / nbatch + 7) / 8 * 8;
+    const int64_t gx = std::max<int64_t>(1, std::min<int64_t>(pat->nchunk, per_mesh));
     const int efm = (flags & EMG_EXACT_FACE_MASS) ? 1 : 0;
     const cplx *ce = reinterpret_cast<const cplx *>(d_eps), *cn = reinterpret_cast<const cplx *>(d_nu);
     cplx *oE = reinterpret_cast<cplx *>(d_E), *oB = reinterpret_cast<cplx *>(d_B);

@@ -1,0 +1,58 @@
+"""The fused assembly's chunks of 512 entries at their edges, against the two-phase kernels: a row longer
+than a chunk (a fan of tets round one edge), chunks that begin and end inside rows, a last chunk with a
+remainder, several chunks per run, and value arrays at every 16-byte place within a 128-byte line."""
+import numpy as np
+import pytest
+
+from emerge_amd import _lib, meshgen
+from emerge_amd.assembly import EXACT_FACE_MASS, FORCE_TWO_PHASE, GPUPattern
+from emerge_amd.mesh import Mesh3D
+
+pytestmark = pytest.mark.gpu
+
+
+def _fan(n):
+    """n tets round the edge (0, 1): its row holds 1 + 3 n edges and 3 n faces."""
+    a = 2 * np.pi * np.arange(n) / n
+    nodes = np.concatenate([[[0, 0], [0, 0], [-1, 1]], np.stack([np.cos(a), np.sin(a), 0.1 * np.cos(3 * a)])], axis=1)
+    ring = 2 + np.arange(n)
+    return Mesh3D(nodes, np.stack([np.zeros(n, int), np.ones(n, int), ring, np.roll(ring, -1)]))
+
+
+MESHES = {"fan 120": lambda: _fan(120), "fan 30": lambda: _fan(30),
+          "1 hex": lambda: meshgen.structured_box(1, 1, 1, jitter=0.0, seed=0),
+          "5x4x3": lambda: meshgen.structured_box(5, 4, 3, jitter=0.1, seed=3),
+          "13x11x10": lambda: meshgen.structured_box(13, 11, 10, jitter=0.1, seed=4)}
+
+
+@pytest.mark.parametrize("name", list(MESHES))
+@pytest.mark.parametrize("flags", [0, EXACT_FACE_MASS])
+def test_chunks_equal_two_phase(cuda, name, flags):
+    """Both paths sum the same terms, at most 9 per curl and 4 per mass entry and tet and at most 128
+    tets, in another order: within 128 * 13 * 4 unit roundoffs of the largest element entry, which the
+    largest assembled entry bounds to within the cancellation between tets (a factor 16)."""
+    import torch
+    mesh = MESHES[name]()
+    pat = GPUPattern(mesh)
+    rng = np.random.default_rng(mesh.n_tets)
+    eps, nu = (torch.from_numpy(rng.uniform(1, 4, mesh.n_tets) * (1 - 0.1j * rng.uniform(0, 1, mesh.n_tets))).to(cuda)
+               for _ in range(2))
+    L = _lib.load()
+
+    def run(f, offset):
+        vals = [torch.full((pat.nnz + 16,), complex(7.0, -7.0), dtype=torch.complex128, device=cuda) for _ in range(2)]
+        E, B = (v[o:o + pat.nnz] for v, o in zip(vals, (offset, (3 * offset) % 8)))
+        _lib.check(L.emg_assemble_iso(pat.handle, _lib.ptr(pat.nodes), _lib.ptr(pat.tets), _lib.ptr(eps), _lib.ptr(nu),
+                                      f, _lib.ptr(E), _lib.ptr(B), _lib.stream_ptr()), "emg_assemble_iso")
+        for v, o in zip(vals, (offset, (3 * offset) % 8)):   # nothing beside the values is written
+            assert torch.all(v[:o] == complex(7.0, -7.0)) and torch.all(v[o + pat.nnz:] == complex(7.0, -7.0))
+        return E, B
+
+    print(f"chunks {name} flags={flags} nnz={pat.nnz}", flush=True)
+    ref = run(flags | FORCE_TWO_PHASE, 0)
+    first = run(flags, 0)
+    for a, r in zip(first, ref):
+        assert float((a - r).abs().max()) <= 128 * 13 * 4 * 16 * 2.0 ** -53 * float(r.abs().max())
+    for offset in range(1, 8):
+        for a, b in zip(run(flags, offset), first):
+            assert torch.equal(a, b)
