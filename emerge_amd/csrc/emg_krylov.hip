@@ -1146,7 +1146,8 @@ static void launch_gt_pk(hipStream_t st, int L, int64_t np2, const int32_t *rp, 
     else k_gt_pk<R, 8><<<grid, 256, 0, st>>>(np2, rp, col, val, dsinv, x, xs, t);
 }
 
-// z = BJ(xs x) + G t (G in slices of 64 entities, gcol NULL: no gradient part), one entity per lane
+// z = BJ(xs x) + G t (G in slices of 64 entities, gcol NULL: no gradient part; inv NULL: x in place of BJ(xs x)),
+// one entity per lane
 template <typename R>
 __global__ void __launch_bounds__(RB) k_bj_grad_pk(int64_t ne, const R *__restrict__ inv, const R *__restrict__ x,
                                                    const double *__restrict__ xs, g_shape sh,
@@ -1154,13 +1155,16 @@ __global__ void __launch_bounds__(RB) k_bj_grad_pk(int64_t ne, const R *__restri
                                                    const R *__restrict__ t, R *__restrict__ z) {
     const int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x;
     if (e >= ne) return;
-    const double s = xs != nullptr ? xs[0] : 1.0;
-    const cx2<R> i0 = ld2(inv, 2 * e), i1 = ld2(inv, 2 * e + 1);
     cx2<R> r = ld2(x, e);
-    r = cx2<R>{(R)(s * r.ar), (R)(s * r.ai), (R)(s * r.br), (R)(s * r.bi)};
-    const cx<R> r0(r.ar, r.ai), r1(r.br, r.bi);
-    cx<R> z0 = cadd(cmul(cx<R>(i0.ar, i0.ai), r0), cmul(cx<R>(i0.br, i0.bi), r1));
-    cx<R> z1 = cadd(cmul(cx<R>(i1.ar, i1.ai), r0), cmul(cx<R>(i1.br, i1.bi), r1));
+    cx<R> z0(r.ar, r.ai), z1(r.br, r.bi);
+    if (inv != nullptr) {
+        const double s = xs != nullptr ? xs[0] : 1.0;
+        const cx2<R> i0 = ld2(inv, 2 * e), i1 = ld2(inv, 2 * e + 1);
+        r = cx2<R>{(R)(s * r.ar), (R)(s * r.ai), (R)(s * r.br), (R)(s * r.bi)};
+        const cx<R> r0(r.ar, r.ai), r1(r.br, r.bi);
+        z0 = cadd(cmul(cx<R>(i0.ar, i0.ai), r0), cmul(cx<R>(i0.br, i0.bi), r1));
+        z1 = cadd(cmul(cx<R>(i1.ar, i1.ai), r0), cmul(cx<R>(i1.br, i1.bi), r1));
+    }
     if (gcol != nullptr) {
         const int64_t si = e >> 6;
         const int w = sh.width(si);
@@ -1185,6 +1189,414 @@ __global__ void __launch_bounds__(RB) k_bj_grad_pk(int64_t ne, const R *__restri
         }
     }
     st2(z, e, cx2<R>{z0.re, z0.im, z1.re, z1.im});
+}
+
+// ---------------------------------------------------------------- one launch per smoother application and product
+// With M = L + G D G^T (L the 2x2 block inverses, D the inverted diagonal) and t = D G^T q,
+//   K M q = K (L q) + (K G) t   and   G^T (K M q) = (G^T K) (L q) + (G^T K G) t,
+// so with the matrices KG = K G, H = G^T K and HG = G^T K G at hand the polynomial's recurrence on q carries
+// G^T q along and needs one launch per product where smoother and product take three (G^T, then L and G, then
+// K).  KG's rows are the entities', with the P2 nodes of their columns' rows of G; H's and HG's are the nodes',
+// with the columns of the entities in their rows of G^T and the nodes of those' KG rows.  They are formed in
+// complex128 and kept in complex64 beside K.
+
+// The distinct values that GEN(row, put) puts, ascending: their number to cnt, or with out the values
+// themselves at out[ptr[row]].  A row with more than CAND candidates or UNIQ values sets *over.
+static constexpr int FUSE_CAND = 8192, FUSE_UNIQ = 512;
+template <typename GEN>
+__global__ void __launch_bounds__(256) k_distinct(GEN gen, int32_t *__restrict__ cnt, const int32_t *__restrict__ ptr,
+                                                  int32_t *__restrict__ out, int *__restrict__ over) {
+    __shared__ int32_t cand[FUSE_CAND];
+    __shared__ uint8_t first[FUSE_CAND];
+    __shared__ int found, kept;
+    const int64_t row = blockIdx.x;
+    if (threadIdx.x == 0) { found = 0; kept = 0; }
+    __syncthreads();
+    gen(row, [&](int32_t v) {
+        const int i = atomicAdd(&found, 1);
+        if (i < FUSE_CAND) cand[i] = v;
+    });
+    __syncthreads();
+    const int n = min(found, FUSE_CAND);
+    for (int i = threadIdx.x; i < n; i += 256) {
+        bool f = true;
+        for (int j = 0; f && j < i; j++) f = cand[j] != cand[i];
+        first[i] = f;
+        if (f) atomicAdd(&kept, 1);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && (found > FUSE_CAND || kept > FUSE_UNIQ)) *over = 1;
+    if (out == nullptr) {
+        if (threadIdx.x == 0) cnt[row] = kept;
+        return;
+    }
+    for (int i = threadIdx.x; i < n; i += 256) {
+        if (!first[i]) continue;
+        int rank = 0;
+        for (int j = 0; j < n; j++) rank += first[j] && cand[j] < cand[i];
+        out[ptr[row] + rank] = cand[i];
+    }
+}
+struct gen_kg {   // the nodes of the G rows of entity row's columns
+    int64_t ne;
+    const int32_t *rowptr, *acol, *grp, *gcol;
+    template <typename PUT>
+    __device__ void operator()(int64_t e, PUT &&put) const {
+        const int32_t a0 = rowptr[e] >> 1, deg = (rowptr[e + 1] >> 1) - a0;
+        for (int k = threadIdx.x; k < 2 * deg; k += 256) {
+            const int64_t d = (k & 1 ? ne : 0) + acol[a0 + (k >> 1)];
+            for (int32_t q = grp[d]; q < grp[d + 1]; q++) put(gcol[q]);
+        }
+    }
+};
+struct gen_of_nodes {   // what the rows (of rp and col, at rp[i] >> shift) of the entities in node row's row of G^T list
+    int64_t ne;
+    const int32_t *trp, *tcol, *rp, *col;
+    int shift;
+    template <typename PUT>
+    __device__ void operator()(int64_t p, PUT &&put) const {
+        for (int32_t q = trp[p]; q < trp[p + 1]; q++) {
+            const int64_t e = tcol[q] % ne;
+            for (int32_t k = (rp[e] >> shift) + threadIdx.x; k < rp[e + 1] >> shift; k += 256) put(col[k]);
+        }
+    }
+};
+
+// KG: a wavefront per entity, a node per lane; sums in the order of the row.
+__global__ void __launch_bounds__(64) k_kg_values(int64_t ne, int64_t half, const int32_t *__restrict__ rowptr,
+                                                  const int32_t *__restrict__ acol, const double *__restrict__ vals,
+                                                  const uint8_t *__restrict__ mask, const int32_t *__restrict__ grp,
+                                                  const int32_t *__restrict__ gcol, const double *__restrict__ gv,
+                                                  const int32_t *__restrict__ kgp, const int32_t *__restrict__ kgc,
+                                                  float *__restrict__ kgv) {
+    const int64_t e = blockIdx.x;
+    const int32_t r0 = rowptr[e], deg = (rowptr[e + 1] - r0) >> 1;
+    const bool m0 = mask == nullptr || mask[e], m1 = mask == nullptr || mask[ne + e];
+    for (int32_t k0 = kgp[e]; k0 < kgp[e + 1]; k0 += 64) {
+        const int32_t k = k0 + (int)threadIdx.x, p = k < kgp[e + 1] ? kgc[k] : -1;
+        cx<double> a, b;
+        for (int32_t j = 0; j < deg; j++) {
+            const int64_t c = acol[(r0 >> 1) + j];
+            for (int m = 0; m < 2; m++) {
+                const int64_t d = m * ne + c;
+                if (mask != nullptr && !mask[d]) continue;
+                double g = 0.0;
+                for (int32_t q = grp[d]; q < grp[d + 1]; q++)
+                    if (gcol[q] == p) g += gv[q];
+                const cx<double> u = ld(vals, (int64_t)r0 + j + m * deg), v = ld(vals, half + r0 + j + m * deg);
+                a = cx<double>(a.re + g * u.re, a.im + g * u.im);
+                b = cx<double>(b.re + g * v.re, b.im + g * v.im);
+            }
+        }
+        // a masked row of K is the identity's: G's own row
+        for (int m = 0; m < 2; m++) {
+            if (m == 0 ? m0 : m1) continue;
+            double g = 0.0;
+            for (int32_t q = grp[m * ne + e]; q < grp[m * ne + e + 1]; q++)
+                if (gcol[q] == p) g += gv[q];
+            (m == 0 ? a : b) = cx<double>(g, 0.0);
+        }
+        if (p >= 0) st2(kgv, k, cx2<float>{(float)a.re, (float)a.im, (float)b.re, (float)b.im});
+    }
+}
+
+__device__ __forceinline__ int place_of(const int32_t *list, int n, int32_t v) {
+    int lo = 0;
+    for (int hi = n - 1; lo < hi;) {
+        const int mid = (lo + hi) >> 1;
+        if (list[mid] < v) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+}
+// H (FROM_KG false: rows of K) or HG (rows of KG): a wavefront per node, one entry of its row of G^T after the
+// other, whose distinct columns go to different lanes; sums in LDS in the order of the row.
+template <bool FROM_KG>
+__global__ void __launch_bounds__(64) k_node_values(int64_t ne, int64_t half, const int32_t *__restrict__ rowptr,
+                                                    const int32_t *__restrict__ acol, const double *__restrict__ vals,
+                                                    const uint8_t *__restrict__ mask, const int32_t *__restrict__ kgp,
+                                                    const int32_t *__restrict__ kgc, const float *__restrict__ kgv,
+                                                    const int32_t *__restrict__ trp, const int32_t *__restrict__ tcol,
+                                                    const double *__restrict__ tv, const int32_t *__restrict__ ptr,
+                                                    const int32_t *__restrict__ col, float *__restrict__ out) {
+    __shared__ int32_t list[FUSE_UNIQ];
+    __shared__ double acc[FUSE_UNIQ][4];
+    const int64_t p = blockIdx.x;
+    const int lane = threadIdx.x, n = min(ptr[p + 1] - ptr[p], FUSE_UNIQ);
+    for (int i = lane; i < n; i += 64) {
+        list[i] = col[ptr[p] + i];
+        for (int q = 0; q < 4; q++) acc[i][q] = 0.0;
+    }
+    __syncthreads();
+    for (int32_t q = trp[p]; q < trp[p + 1]; q++) {
+        const int64_t d = tcol[q], e = d % ne;
+        const int r = d >= ne;
+        const double g = tv[q];
+        if constexpr (FROM_KG) {
+            for (int32_t k = kgp[e] + lane; k < kgp[e + 1]; k += 64) {
+                const cx2<float> v = ld2(kgv, k);
+                double *a = acc[place_of(list, n, kgc[k])];
+                a[0] += g * (r ? v.br : v.ar);
+                a[1] += g * (r ? v.bi : v.ai);
+            }
+        } else if (mask != nullptr && !mask[d]) {
+            if (lane == 0) acc[place_of(list, n, (int32_t)e)][2 * r] += g;
+        } else {
+            const int32_t r0 = rowptr[e], deg = (rowptr[e + 1] - r0) >> 1;
+            const int64_t b = (int64_t)r * half + r0;
+            for (int32_t j = lane; j < deg; j += 64) {
+                const int32_t c = acol[(r0 >> 1) + j];
+                const bool c0 = mask == nullptr || mask[c], c1 = mask == nullptr || mask[ne + c];
+                const cx<double> u = ld(vals, b + j), v = ld(vals, b + j + deg);
+                double *a = acc[place_of(list, n, c)];
+                if (c0) { a[0] += g * u.re; a[1] += g * u.im; }
+                if (c1) { a[2] += g * v.re; a[3] += g * v.im; }
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = lane; i < n; i += 64) {
+        if constexpr (FROM_KG) st(out, (int64_t)ptr[p] + i, cx<float>((float)acc[i][0], (float)acc[i][1]));
+        else st2(out, (int64_t)ptr[p] + i, cx2<float>{(float)acc[i][0], (float)acc[i][1], (float)acc[i][2], (float)acc[i][3]});
+    }
+}
+
+// The matrices of the fused steps and the vectors they work on.
+struct fuse_mat {
+    int64_t ne, np2;
+    const int32_t *rowptr, *acol;
+    const float *kre, *kim;
+    const uint8_t *flag;
+    const int32_t *kgp, *kgc, *hp, *hc, *hgp, *hgc;
+    const float *kgv, *hv, *hgv;
+    const float *inv, *dsinv;   // L and D
+    double *s, *sy;             // G^T q and G^T y, complex
+};
+
+// Start of a step: yl = L (xs x), s = G^T (xs x), t = D s.  One lane per entity, then 16 per node.
+__global__ void __launch_bounds__(256) k_fuse_start(fuse_mat f, unsigned eblocks, const int32_t *__restrict__ trp,
+                                                    const int32_t *__restrict__ tcol, const float *__restrict__ tval,
+                                                    const float *__restrict__ x, const double *__restrict__ xs,
+                                                    float *__restrict__ yl, float *__restrict__ t) {
+    const double sc = xs != nullptr ? xs[0] : 1.0;
+    if (blockIdx.x < eblocks) {
+        const int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x;
+        if (e >= f.ne) return;
+        const cx2<float> i0 = ld2(f.inv, 2 * e), i1 = ld2(f.inv, 2 * e + 1);
+        const cx2<float> r = ld2(x, e);
+        const cx<float> r0((float)(sc * r.ar), (float)(sc * r.ai)), r1((float)(sc * r.br), (float)(sc * r.bi));
+        const cx<float> z0 = cadd(cmul(cx<float>(i0.ar, i0.ai), r0), cmul(cx<float>(i0.br, i0.bi), r1));
+        const cx<float> z1 = cadd(cmul(cx<float>(i1.ar, i1.ai), r0), cmul(cx<float>(i1.br, i1.bi), r1));
+        st2(yl, e, cx2<float>{z0.re, z0.im, z1.re, z1.im});
+        return;
+    }
+    const int64_t p = ((blockIdx.x - eblocks) * (int64_t)256 + threadIdx.x) / 16;
+    const int lane = threadIdx.x % 16;
+    if (p >= f.np2) return;
+    const cx<float> d = ld(f.dsinv, p);
+    double ar = 0.0, ai = 0.0;
+    const int32_t q1 = trp[p + 1];
+    for (int32_t q = trp[p] + lane; q < q1; q += 32) {
+        const bool two = q + 16 < q1;
+        const int32_t qb = two ? q + 16 : q;
+        const cx<float> ga = ld(tval, q), gb = ld(tval, qb);
+        const cx2<float> va = ld2(x, tcol[q]), vb = ld2(x, tcol[qb]);
+        ar += (double)ga.re * va.ar + (double)ga.im * va.br;
+        ai += (double)ga.re * va.ai + (double)ga.im * va.bi;
+        if (two) {
+            ar += (double)gb.re * vb.ar + (double)gb.im * vb.br;
+            ai += (double)gb.re * vb.ai + (double)gb.im * vb.bi;
+        }
+    }
+    ar = lane_sum<16>(ar) * sc;
+    ai = lane_sum<16>(ai) * sc;
+    if (lane == 0) {
+        st(f.s, p, cx<double>(ar, ai));
+        st(t, p, cx<float>((float)(d.re * ar - d.im * ai), (float)(d.re * ai + d.im * ar)));
+    }
+}
+
+// v = K M q from yl = L q and t = D G^T q, on the rows of K and (END false) of G^T K, and what follows it:
+// END false: p = q - c_i v, y = (i == 0 ? c_0 q : y) + c_{i+1} p and the same for s = G^T q and sy = G^T y, then
+// yl2 = L p, t2 = D s (last: of y and sy, for the product that ends the step).  END true: y = v.
+// L lanes per entity, then LN per node, each lane with all its loads of a trip in flight: an edge's 37 blocks
+// and 27 nodes, or a vertex' 220 entities and 65 nodes, take one trip or four.  Bound by the latency of a launch
+// and of its chain of loads: 7.7 us at 21,000 DOFs where the three launches it replaces took 3.9 (G^T), 4.0
+// (L and G) and 4.1 (K); a step 121 -> 90 us.  (8 or 32 lanes per entity, 16 or 64 per node: 2 - 8 % slower.)
+struct fuse_args {
+    const float *q, *yl, *t;
+    float *y, *p, *yl2, *t2;
+    const double *c, *qs;
+    int i, last;
+};
+template <int L, int LN, bool END>
+__global__ void __launch_bounds__(256) k_fuse_step(fuse_mat f, unsigned eblocks, fuse_args a) {
+    if (blockIdx.x < eblocks) {
+        constexpr int UK = 48 / L, UG = UK;   // blocks of K and nodes of a lane whose loads are in flight together
+        const int64_t e = (blockIdx.x * (int64_t)256 + threadIdx.x) / L;
+        const int lane = threadIdx.x % L;
+        if (e >= f.ne) return;
+        const uint8_t fl = f.flag[e];
+        const int32_t p0 = f.rowptr[e] >> 1, p1 = f.rowptr[e + 1] >> 1, g0 = f.kgp[e], g1 = f.kgp[e + 1];
+        const int32_t gs = g0 < g1 ? g0 : 0;   // a slot to read in place of none
+        cx2<float> own{}, qv{}, yv{}, i0{}, i1{};
+        if (lane == 0) {
+            if ((fl & (ROW0 | ROW1)) != (ROW0 | ROW1)) own = ld2(a.yl, e);
+            if constexpr (!END) {
+                qv = ld2(a.q, e);
+                i0 = ld2(f.inv, 2 * e);
+                i1 = ld2(f.inv, 2 * e + 1);
+                if (a.i > 0) yv = ld2(a.y, e);
+            }
+        }
+        float s0r = 0, s0i = 0, s1r = 0, s1i = 0;
+        const int32_t none = fl & (ROW0 | ROW1) ? p1 : p0;   // end of the row's blocks of K
+        for (int32_t o = lane; p0 + o < none || g0 + o < g1; o += L * UK) {
+            int32_t c[UK], n[UG];
+            cx2<float> k[UK], xv[UK], kg[UG], v[UK];
+            cx<float> t[UG];
+#pragma unroll
+            for (int u = 0; u < UK; u++) {
+                const int32_t q = p0 + o + u * L < none ? p0 + o + u * L : p0;
+                c[u] = f.acol[q];
+                k[u] = ld2(f.kre, q);
+            }
+#pragma unroll
+            for (int u = 0; u < UG; u++) {
+                const int32_t q = g0 + o + u * L < g1 ? g0 + o + u * L : gs;
+                n[u] = f.kgc[q];
+                kg[u] = ld2(f.kgv, q);
+            }
+#pragma unroll
+            for (int u = 0; u < UK; u++) xv[u] = ld2(a.yl, c[u]);
+#pragma unroll
+            for (int u = 0; u < UG; u++) t[u] = ld(a.t, n[u]);
+#pragma unroll
+            for (int u = 0; u < UK; u++)
+                v[u] = cx2<float>{k[u].ar * xv[u].ar + k[u].ai * xv[u].br, k[u].ar * xv[u].ai + k[u].ai * xv[u].bi,
+                                  k[u].br * xv[u].ar + k[u].bi * xv[u].br, k[u].br * xv[u].ai + k[u].bi * xv[u].bi};
+            if (fl & ROW_CPLX) {
+#pragma unroll
+                for (int u = 0; u < UK; u++) k[u] = ld2(f.kim, p0 + o + u * L < none ? p0 + o + u * L : p0);
+#pragma unroll
+                for (int u = 0; u < UK; u++) {
+                    v[u].ar -= k[u].ar * xv[u].ai + k[u].ai * xv[u].bi;
+                    v[u].ai += k[u].ar * xv[u].ar + k[u].ai * xv[u].br;
+                    v[u].br -= k[u].br * xv[u].ai + k[u].bi * xv[u].bi;
+                    v[u].bi += k[u].br * xv[u].ar + k[u].bi * xv[u].br;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < UK; u++)
+                if (p0 + o + u * L < none) {
+                    s0r += v[u].ar;
+                    s0i += v[u].ai;
+                    s1r += v[u].br;
+                    s1i += v[u].bi;
+                }
+#pragma unroll
+            for (int u = 0; u < UG; u++)
+                if (g0 + o + u * L < g1) {
+                    s0r += kg[u].ar * t[u].re - kg[u].ai * t[u].im;
+                    s0i += kg[u].ar * t[u].im + kg[u].ai * t[u].re;
+                    s1r += kg[u].br * t[u].re - kg[u].bi * t[u].im;
+                    s1i += kg[u].br * t[u].im + kg[u].bi * t[u].re;
+                }
+        }
+        // a masked row of K is the identity's (its entries are zero, its KG row is G's)
+        s0r = lane_sum<L>(s0r);
+        s0i = lane_sum<L>(s0i);
+        s1r = lane_sum<L>(s1r);
+        s1i = lane_sum<L>(s1i);
+        if (lane != 0) return;
+        cx2<float> v{s0r, s0i, s1r, s1i};
+        if (!(fl & ROW0)) { v.ar += own.ar; v.ai += own.ai; }
+        if (!(fl & ROW1)) { v.br += own.br; v.bi += own.bi; }
+        if constexpr (END) {
+            st2(a.y, e, v);
+        } else {
+            const double *cc = a.c + 2 * a.i;
+            const double cr = cc[0], ci = cc[1], nr = cc[2], ni = cc[3];
+            const double s = a.qs != nullptr ? a.qs[0] : 1.0;
+            const double q0r = s * qv.ar, q0i = s * qv.ai, q1r = s * qv.br, q1i = s * qv.bi;
+            double y0r = yv.ar, y0i = yv.ai, y1r = yv.br, y1i = yv.bi;
+            if (a.i == 0) {
+                y0r = cr * q0r - ci * q0i; y0i = cr * q0i + ci * q0r;
+                y1r = cr * q1r - ci * q1i; y1i = cr * q1i + ci * q1r;
+            }
+            const double p0r = q0r - (cr * v.ar - ci * v.ai), p0i = q0i - (cr * v.ai + ci * v.ar);
+            const double p1r = q1r - (cr * v.br - ci * v.bi), p1i = q1i - (cr * v.bi + ci * v.br);
+            const cx2<float> pn{(float)p0r, (float)p0i, (float)p1r, (float)p1i};
+            const cx2<float> yn{(float)(y0r + nr * p0r - ni * p0i), (float)(y0i + nr * p0i + ni * p0r),
+                                (float)(y1r + nr * p1r - ni * p1i), (float)(y1i + nr * p1i + ni * p1r)};
+            if (!a.last) {
+                st2(a.p, e, pn);
+                st2(a.y, e, yn);
+            }
+            const cx2<float> w = a.last ? yn : pn;
+            const cx<float> r0(w.ar, w.ai), r1(w.br, w.bi);
+            const cx<float> z0 = cadd(cmul(cx<float>(i0.ar, i0.ai), r0), cmul(cx<float>(i0.br, i0.bi), r1));
+            const cx<float> z1 = cadd(cmul(cx<float>(i1.ar, i1.ai), r0), cmul(cx<float>(i1.br, i1.bi), r1));
+            st2(a.yl2, e, cx2<float>{z0.re, z0.im, z1.re, z1.im});
+        }
+        return;
+    }
+    if constexpr (!END) {
+        const int64_t p = ((blockIdx.x - eblocks) * (int64_t)256 + threadIdx.x) / LN;
+        const int lane = threadIdx.x % LN;
+        if (p >= f.np2) return;
+        const int32_t h0 = f.hp[p], h1 = f.hp[p + 1], g0 = f.hgp[p], g1 = f.hgp[p + 1];
+        const int32_t hs = h0 < h1 ? h0 : 0, gs = g0 < g1 ? g0 : 0;
+        cx<float> d;
+        cx<double> sv, yv;
+        if (lane == 0) {
+            d = ld(f.dsinv, p);
+            sv = ld(f.s, p);
+            if (a.i > 0) yv = ld(f.sy, p);
+        }
+        double zr = 0.0, zi = 0.0;
+        constexpr int UH = 2;
+        for (int32_t o = lane; h0 + o < h1 || g0 + o < g1; o += UH * LN) {
+            int32_t c[UH], n[UH];
+            cx2<float> hv[UH], xv[UH];
+            cx<float> gv[UH], tv[UH];
+#pragma unroll
+            for (int u = 0; u < UH; u++) {
+                const int32_t q = h0 + o + u * LN < h1 ? h0 + o + u * LN : hs, r = g0 + o + u * LN < g1 ? g0 + o + u * LN : gs;
+                c[u] = f.hc[q];
+                hv[u] = ld2(f.hv, q);
+                n[u] = f.hgc[r];
+                gv[u] = ld(f.hgv, r);
+            }
+#pragma unroll
+            for (int u = 0; u < UH; u++) {
+                xv[u] = ld2(a.yl, c[u]);
+                tv[u] = ld(a.t, n[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < UH; u++) {
+                if (h0 + o + u * LN < h1) {
+                    zr += (double)hv[u].ar * xv[u].ar - (double)hv[u].ai * xv[u].ai + (double)hv[u].br * xv[u].br - (double)hv[u].bi * xv[u].bi;
+                    zi += (double)hv[u].ar * xv[u].ai + (double)hv[u].ai * xv[u].ar + (double)hv[u].br * xv[u].bi + (double)hv[u].bi * xv[u].br;
+                }
+                if (g0 + o + u * LN < g1) {
+                    zr += (double)gv[u].re * tv[u].re - (double)gv[u].im * tv[u].im;
+                    zi += (double)gv[u].re * tv[u].im + (double)gv[u].im * tv[u].re;
+                }
+            }
+        }
+        zr = lane_sum<LN>(zr);
+        zi = lane_sum<LN>(zi);
+        if (lane != 0) return;
+        const double *cc = a.c + 2 * a.i;
+        const double cr = cc[0], ci = cc[1], nr = cc[2], ni = cc[3];
+        if (a.i == 0) yv = cx<double>(cr * sv.re - ci * sv.im, cr * sv.im + ci * sv.re);
+        const cx<double> sn(sv.re - (cr * zr - ci * zi), sv.im - (cr * zi + ci * zr));
+        const cx<double> yn(yv.re + nr * sn.re - ni * sn.im, yv.im + nr * sn.im + ni * sn.re);
+        st(f.s, p, sn);
+        st(f.sy, p, yn);
+        const cx<double> w = a.last ? yn : sn;
+        st(a.t2, p, cx<float>((float)(d.re * w.re - d.im * w.im), (float)(d.re * w.im + d.im * w.re)));
+    }
 }
 
 // b (interleaved, R) = s a (caller's layout, complex128)
@@ -1247,6 +1659,12 @@ struct emg_solver {
     void *g_pval = nullptr, *gt_pval = nullptr;
     double *dS = nullptr, *dsinv64 = nullptr, *tg = nullptr;
     float *dsinv32 = nullptr;
+    // the matrices of the fused steps (fuse_pattern), all or none
+    bool fused = false;
+    int32_t *kg_ptr = nullptr, *kg_col = nullptr, *h_ptr = nullptr, *h_col = nullptr, *hg_ptr = nullptr, *hg_col = nullptr;
+    void *kg_val = nullptr, *h_val = nullptr, *hg_val = nullptr;
+    double *fuse_s = nullptr;       // G^T q and G^T y, np2 complex each
+    float *fuse_t = nullptr;        // two buffers of t, np2 complex each
     // optional learned weights of the smoother (caller-owned complex128):
     // w_e per entity scales its 2x2 block inverse, w_p per P2 node its diagonal
     const double *w_e = nullptr, *w_p = nullptr;
@@ -1280,9 +1698,21 @@ static void drop_graphs(emg_solver *s) {
     s->tail = nullptr;
 }
 
+static void drop_fused(emg_solver *s) {
+    void *ps[] = {s->kg_ptr, s->kg_col, s->h_ptr, s->h_col, s->hg_ptr, s->hg_col, s->kg_val, s->h_val, s->hg_val,
+                  s->fuse_s, s->fuse_t};
+    for (void *p : ps) (void)hipFree(p);
+    s->kg_ptr = s->kg_col = s->h_ptr = s->h_col = s->hg_ptr = s->hg_col = nullptr;
+    s->kg_val = s->h_val = s->hg_val = nullptr;
+    s->fuse_s = nullptr;
+    s->fuse_t = nullptr;
+    s->fused = false;
+}
+
 static void free_solver(emg_solver *s) {
     if (!s) return;
     drop_graphs(s);
+    drop_fused(s);
     void *ps[] = {s->acol, s->kre, s->kim, s->row_flag, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial,
                   s->h, s->nrm, s->arn, s->pn, s->gram, s->flag, s->g_pcol, s->gt_prp, s->gt_pcol, s->g_pval,
                   s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32, s->poly_c, s->pp, s->pt, s->py, s->pu};
@@ -1348,8 +1778,14 @@ static void spmv_std(emg_solver *s, const double *x, const double *b, double *y,
 // extra smoother applications per call; the updates of q and y follow each product in
 // its own launch (SP_POLY), which at 19,664 DOFs saves the 2.7 us launch they took
 // after every product and at any size the pass over t = K M q.
+static void apply_fused(emg_solver *s, const float *vt, const double *xs, float *out, bool product, hipStream_t st);
 template <typename R>
 static void apply_prec_poly(emg_solver *s, const R *x, const double *xs, R *out, hipStream_t st) {
+    if constexpr (sizeof(R) == 4)
+        if (s->fused) {
+            apply_fused(s, x, xs, out, false, st);
+            return;
+        }
     if (s->poly_deg <= 1) {
         apply_prec<R>(s, x, xs, out, st);
         return;
@@ -1362,6 +1798,38 @@ static void apply_prec_poly(emg_solver *s, const R *x, const double *xs, R *out,
         spmv_pk<R, SP_POLY, false>(s, s->lanes[sizeof(R) == 4], pu, sp_args<R>{q, py, pp, s->poly_c, i, qs}, st);
     }
     apply_prec<R>(s, py, nullptr, out, st);
+}
+
+// out = K M p(K M) (xs vt) or, with product false, M p(K M) (xs vt) through the fused steps (complex64): a launch
+// to start and one per product.
+static constexpr int FUSE_L = 16, FUSE_LN = 32;
+static void apply_fused(emg_solver *s, const float *vt, const double *xs, float *out, bool product, hipStream_t st) {
+    const int64_t ne = s->n_ent, np2 = s->np2;
+    fuse_mat f{ne, np2, s->rowptr, s->acol, static_cast<const float *>(s->kre), static_cast<const float *>(s->kim), s->row_flag,
+               s->kg_ptr, s->kg_col, s->h_ptr, s->h_col, s->hg_ptr, s->hg_col,
+               static_cast<const float *>(s->kg_val), static_cast<const float *>(s->h_val), static_cast<const float *>(s->hg_val),
+               s->inv32, s->dsinv32, s->fuse_s, s->fuse_s + 2 * np2};
+    float *pp = reinterpret_cast<float *>(s->pp), *py = reinterpret_cast<float *>(s->py);
+    float *yl[2] = {reinterpret_cast<float *>(s->pu), reinterpret_cast<float *>(s->pu) + 2 * s->n};
+    float *t[2] = {s->fuse_t, s->fuse_t + 2 * np2};
+    const unsigned eb = emg::grid_for(ne, 256);
+    k_fuse_start<<<eb + emg::grid_for(np2 * 16, 256), 256, 0, st>>>(f, eb, s->gt_prp, s->gt_pcol, static_cast<const float *>(s->gt_pval),
+                                                                   vt, xs, yl[0], t[0]);
+    const int d = std::max(1, s->poly_deg);
+    const unsigned el = emg::grid_for(ne * FUSE_L, 256), nl = emg::grid_for(np2 * FUSE_LN, 256);
+    for (int i = 0; i < d - 1; i++) {
+        fuse_args a{i == 0 ? vt : pp, yl[i & 1], t[i & 1], py, pp, yl[(i + 1) & 1], t[(i + 1) & 1], s->poly_c, i == 0 ? xs : nullptr,
+                    i, i == d - 2};
+        k_fuse_step<FUSE_L, FUSE_LN, false><<<el + nl, 256, 0, st>>>(f, el, a);
+    }
+    const float *ye = yl[(d - 1) & 1], *te = t[(d - 1) & 1];
+    if (product) {
+        fuse_args a{nullptr, ye, te, out, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
+        k_fuse_step<FUSE_L, FUSE_LN, true><<<el, 256, 0, st>>>(f, el, a);
+    } else {
+        k_bj_grad_pk<float><<<emg::grid_for(ne, RB), RB, 0, st>>>(ne, nullptr, ye, nullptr, s->g_sh, s->g_pcol,
+                                                                  static_cast<const float *>(s->g_pval), te, out);
+    }
 }
 
 // Blocks per tile of the multi-dot: about 2048 blocks in total, so each block
@@ -1697,6 +2165,18 @@ extern "C" int emg_solver_set_matrix(emg_solver *s, const double *d_vals, const 
                                                          s->g_cols, s->g_vals, s->dS);
         k_dsinv<<<emg::grid_for(s->np2, RB), RB, 0, st>>>(s->np2, s->dS, s->dsinv64, s->dsinv32);
     }
+    if (s->fused) {
+        const int64_t ne = s->n_ent, half = s->nnz / 2;
+        float *kgv = static_cast<float *>(s->kg_val);
+        k_kg_values<<<(unsigned)ne, 64, 0, st>>>(ne, half, s->rowptr, s->acol, d_vals, d_mask, s->g_rowptr, s->g_cols, s->g_vals,
+                                                 s->kg_ptr, s->kg_col, kgv);
+        k_node_values<false><<<(unsigned)s->np2, 64, 0, st>>>(ne, half, s->rowptr, s->acol, d_vals, d_mask, s->kg_ptr, s->kg_col, kgv,
+                                                              s->gt_rowptr, s->gt_cols, s->gt_vals, s->h_ptr, s->h_col,
+                                                              static_cast<float *>(s->h_val));
+        k_node_values<true><<<(unsigned)s->np2, 64, 0, st>>>(ne, half, s->rowptr, s->acol, d_vals, d_mask, s->kg_ptr, s->kg_col, kgv,
+                                                             s->gt_rowptr, s->gt_cols, s->gt_vals, s->hg_ptr, s->hg_col,
+                                                             static_cast<float *>(s->hg_val));
+    }
     if (s->w_e != nullptr || (s->w_p != nullptr && s->np2 > 0)) {
         const int64_t nmax = std::max<int64_t>(s->n_ent, s->np2);
         k_scale_tables<<<emg::grid_for(nmax, RB), RB, 0, st>>>(s->n_ent, s->w_e, s->inv64, s->inv32, s->np2,
@@ -1855,6 +2335,64 @@ static int pack_gradient(emg_solver *s, int64_t np2, const int32_t *grp, const i
     return 0;
 }
 
+// The patterns of KG, H and HG and room for their values: *fits false (and nothing kept) where a row is too long
+// or the memory does not suffice.
+template <typename GEN>
+static int fuse_rows(int64_t rows, const GEN &gen, int32_t *cnt, int *d_over, int32_t **ptr, int32_t **col, void **val,
+                     size_t bytes, bool *fits, hipStream_t st) {
+    EMG_HIP(hipMemsetAsync(d_over, 0, sizeof(int), st));
+    k_distinct<<<(unsigned)rows, 256, 0, st>>>(gen, cnt, nullptr, nullptr, d_over);
+    EMG_LAUNCH_CHECK();
+    int over = 0;
+    EMG_HIP(hipMemcpyAsync(&over, d_over, sizeof(int), hipMemcpyDeviceToHost, st));
+    int64_t total = 0;
+    if (int rc = prefix_on_host(cnt, rows, ptr, &total, st)) return rc;
+    if (over) { *fits = false; return 0; }
+    hipError_t e = hipMalloc((void **)col, std::max<int64_t>(total, 1) * sizeof(int32_t));
+    if (e == hipSuccess) e = hipMalloc(val, std::max<int64_t>(total, 1) * bytes);
+    if (e == hipErrorOutOfMemory) { (void)hipGetLastError(); *fits = false; return 0; }
+    EMG_HIP(e);
+    k_distinct<<<(unsigned)rows, 256, 0, st>>>(gen, nullptr, *ptr, *col, d_over);
+    EMG_LAUNCH_CHECK();
+    return 0;
+}
+static int fuse_pattern(emg_solver *s, int64_t np2, const int32_t *grp, const int32_t *gcol, const int32_t *trp, const int32_t *tcol,
+                        int32_t *cnt, hipStream_t st) {
+    int *d_over = reinterpret_cast<int *>(s->flag);
+    bool fits = true;
+    int rc = fuse_rows(s->n_ent, gen_kg{s->n_ent, s->rowptr, s->acol, grp, gcol}, cnt, d_over, &s->kg_ptr, &s->kg_col, &s->kg_val, 16,
+                       &fits, st);
+    if (rc == 0 && fits)
+        rc = fuse_rows(np2, gen_of_nodes{s->n_ent, trp, tcol, s->rowptr, s->acol, 1}, cnt, d_over, &s->h_ptr, &s->h_col, &s->h_val, 16,
+                       &fits, st);
+    if (rc == 0 && fits)
+        rc = fuse_rows(np2, gen_of_nodes{s->n_ent, trp, tcol, s->kg_ptr, s->kg_col, 0}, cnt, d_over, &s->hg_ptr, &s->hg_col, &s->hg_val,
+                       8, &fits, st);
+    if (rc == 0 && fits) {
+        hipError_t e = hipMalloc((void **)&s->fuse_s, (size_t)np2 * 32);
+        if (e == hipSuccess) e = hipMalloc((void **)&s->fuse_t, (size_t)np2 * 16);
+        if (e != hipSuccess) { (void)hipGetLastError(); fits = false; }
+    }
+    if (rc == 0 && fits) s->fused = true;
+    if (rc != 0 || !fits) {
+        (void)hipStreamSynchronize(st);
+        drop_fused(s);
+    }
+    return rc;
+}
+
+// Where the fused steps are used.  KG, H and HG hold about as many bytes as K, so they pay while a launch
+// costs more than its bytes: posts box with 3,072 / 4,800 / 8,640 / 14,112 tets (20,000 / 34,000 / 60,000 / 96,000
+// DOFs), air: 124 -> 90, 123 -> 99, 134 -> 125, 158 -> 169 us per step at degree 6; lossy: 124 -> 90, 130 -> 100,
+// 140 -> 133, 178 -> 179; 38,400 tets: 258 -> 360.  Complex64 only: complex128 steps are mostly above it.
+// EMG_FUSED_STEPS overrides (0: never, else wherever the rows fit).
+static constexpr int64_t FUSE_MAX_N = 50000;
+static bool fuse_wanted(const emg_solver *s) {
+    if (s->precision != 32) return false;
+    if (const char *env = getenv("EMG_FUSED_STEPS")) return atoi(env) != 0;
+    return s->n <= FUSE_MAX_N;
+}
+
 extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t *d_g_rowptr, const int32_t *d_g_cols,
                                        const double *d_g_vals, const int32_t *d_gt_rowptr, const int32_t *d_gt_cols,
                                        const double *d_gt_vals, void *stream) {
@@ -1862,6 +2400,7 @@ extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t
     hipStream_t st = (hipStream_t)stream;
     if (np2 == 0) {
         s->np2 = 0;
+        s->fused = false;
         return 0;
     }
     EMG_CHECK(d_g_rowptr && d_g_cols && d_g_vals && d_gt_rowptr && d_gt_cols && d_gt_vals,
@@ -1877,6 +2416,7 @@ extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t
     drop_graphs(s);
     void *old[] = {s->g_pcol, s->g_pval, s->gt_prp, s->gt_pcol, s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32};
     for (void *p : old) (void)hipFree(p);
+    drop_fused(s);
     s->g_pcol = s->gt_prp = s->gt_pcol = nullptr;
     s->g_pval = s->gt_pval = nullptr;
     s->dS = s->dsinv64 = s->tg = nullptr;
@@ -1888,11 +2428,13 @@ extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t
     EMG_HIP(hipMalloc((void **)&s->tg, (size_t)np2 * 16));
     {
         int32_t *cnt = nullptr;
-        EMG_HIP(hipMalloc((void **)&cnt, std::max<int64_t>(np2, s->n_ent / 64 + 1) * sizeof(int32_t)));
+        const bool fuse = fuse_wanted(s);
+        EMG_HIP(hipMalloc((void **)&cnt, std::max<int64_t>(np2, fuse ? s->n_ent : s->n_ent / 64 + 1) * sizeof(int32_t)));
         int rc = s->precision == 32 ? pack_gradient<float>(s, np2, d_g_rowptr, d_g_cols, d_g_vals, d_gt_rowptr, d_gt_cols,
                                                            d_gt_vals, cnt, st)
                                     : pack_gradient<double>(s, np2, d_g_rowptr, d_g_cols, d_g_vals, d_gt_rowptr, d_gt_cols,
                                                             d_gt_vals, cnt, st);
+        if (rc == 0 && fuse) rc = fuse_pattern(s, np2, d_g_rowptr, d_g_cols, d_gt_rowptr, d_gt_cols, cnt, st);
         const hipError_t e = hipStreamSynchronize(st);   // cnt is read by kernels in flight
         (void)hipFree(cnt);
         if (rc) return rc;
@@ -2057,8 +2599,8 @@ static void orthogonalise(emg_solver *s, int nv, R *w, double *norms, double *h,
 // (k_gram_correct) and the Hessenberg/Givens update.  Basis vector i is kept as it came out of the
 // projection, with its scale sc[i] = 1 / norm beside it: every reader multiplies by it, and the
 // pass over the new vector that normalised it is gone.  Only kernel launches, so it can be
-// captured: 23 of them at degree 6 with the gradient correction (33 before, at 19,664 DOFs 174 us
-// of kernels that take 2.5 us and more each whatever their size).
+// captured: 23 of them at degree 6 with the gradient correction, 12 with the fused steps (33 before, at
+// 19,664 DOFs 174 us of kernels that take 2.5 us and more each whatever their size).
 template <typename R>
 static void enqueue_step(emg_solver *s, int t, hipStream_t st) {
     const int64_t n = s->n;
@@ -2067,8 +2609,16 @@ static void enqueue_step(emg_solver *s, int t, hipStream_t st) {
     R *z = reinterpret_cast<R *>(s->z);
     R *vt = V + (size_t)t * n * 2, *vn = V + (size_t)(t + 1) * n * 2;
     const arn_off o(m);
-    apply_prec_poly<R>(s, vt, s->arn + o.sc + t, z, st);
-    spmv_pk<R, SP_Y, false>(s, s->lanes[sizeof(R) == 4], z, sp_args<R>{nullptr, vn, nullptr, nullptr, 0, nullptr}, st);
+    bool done = false;
+    if constexpr (sizeof(R) == 4)
+        if (s->fused) {
+            apply_fused(s, vt, s->arn + o.sc + t, vn, true, st);
+            done = true;
+        }
+    if (!done) {
+        apply_prec_poly<R>(s, vt, s->arn + o.sc + t, z, st);
+        spmv_pk<R, SP_Y, false>(s, s->lanes[sizeof(R) == 4], z, sp_args<R>{nullptr, vn, nullptr, nullptr, 0, nullptr}, st);
+    }
     double *h = s->h + 4 * 512;
     orthogonalise<R>(s, nv, vn, s->pn, h, st);
     k_arn_givens<<<1, RB, 0, st>>>(t, m, nb, s->pn, h, s->kept, s->arn, o);
