@@ -134,6 +134,12 @@ def ptr(t) -> ctypes.c_void_p:
 
 
 def stream_ptr(stream=None) -> ctypes.c_void_p:
+    """The HIP stream handle of a torch stream (the current device's current one by default)."""
     import torch
-    s = torch.cuda.current_stream() if stream is None else stream
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is None:
+        # the handle by itself where torch gives it: building the Stream object around it takes 4 us a call
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None and torch.cuda.is_initialized():
+            return ctypes.c_void_p(raw(torch._C._cuda_getDevice()))
+        stream = torch.cuda.current_stream()
+    return ctypes.c_void_p(stream.cuda_stream)

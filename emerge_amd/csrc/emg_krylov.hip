@@ -573,7 +573,7 @@ __global__ void __launch_bounds__(RB) k_norm2(int64_t n, const R *__restrict__ x
 // y = alpha * x (alpha real, on device as 1/sqrt(norm2 sum) when from_norm)
 template <typename R>
 __global__ void __launch_bounds__(RB) k_scale_by_norm(int64_t n, const double *__restrict__ partial, int nblk,
-                                                      const R *__restrict__ x, R *__restrict__ y, double *__restrict__ out_norm) {
+                                                      const R *x, R *y, double *__restrict__ out_norm) {   // x may be y
     __shared__ double inv;
     if (threadIdx.x < 64) {
         double s = 0;
@@ -2224,10 +2224,6 @@ extern "C" int emg_solver_set_poly(emg_solver *s, int degree, const double *h_co
     return 0;
 }
 
-__global__ void __launch_bounds__(RB) k_scale_c128(int64_t n, double a, double *__restrict__ x) {
-    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < 2 * n; e += (int64_t)gridDim.x * RB) x[e] *= a;
-}
-
 // d steps of Arnoldi (complex128, two classical Gram-Schmidt passes) on K M
 // (M = the smoother without polynomial, K masked) from d_v0; writes the
 // (d + 1) x d Hessenberg matrix column-major as complex128 to h_out (host).
@@ -2243,42 +2239,40 @@ extern "C" int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0
     const int nb = s->nblk;
     double *V = s->V;   // d + 1 complex128 vectors
     double *z = s->z;
-    std::vector<double> H(2 * (size_t)(d + 1) * d, 0.0), pn(nb), hh(2 * (d + 1));
-    auto host_norm = [&](const double *partial) -> double {
-        EMG_HIP(hipMemcpyAsync(pn.data(), partial, nb * sizeof(double), hipMemcpyDeviceToHost, st));
-        EMG_HIP(hipStreamSynchronize(st));
-        double t = 0;
-        for (double v : pn) t += v;
-        return std::sqrt(t);
-    };
+    // Everything stays on the device until the end (two waits per pass took a third of the probe's time at
+    // 20,000 DOFs): norms, then the coefficients of pass 0 and 1 of every column.
+    constexpr int PROBE_H = POLY_MAX + 2;   // POLY_MAX + 1 norms
+    static_assert(PROBE_H % 2 == 0 && PROBE_H + 4 * POLY_MAX * (POLY_MAX + 1) <= 4 * 2 * 512, "the probe's results fit s->h");
+    double *norms = s->h, *coef = s->h + PROBE_H;
+    const int ldc = 2 * (d + 1);
     EMG_HIP(hipMemcpyAsync(V, d_v0, n * 16, hipMemcpyDeviceToDevice, st));
     k_norm2<double><<<nb, RB, 0, st>>>(n, V, s->partial);
-    const double b0 = host_norm(s->partial);
-    EMG_CHECK(b0 > 0 && std::isfinite(b0), "emg_solver_arnoldi_probe: zero or non-finite start vector");
-    k_scale_c128<<<nb, RB, 0, st>>>(n, 1.0 / b0, V);
+    k_scale_by_norm<double><<<nb, RB, 0, st>>>(n, s->partial, nb, V, V, norms);
     for (int j = 0; j < d; j++) {
         double *vj = V + (size_t)j * n * 2, *w = V + (size_t)(j + 1) * n * 2;
         const int nv = j + 1, nbm = mdot_blocks(n, nv);
         const dim3 grid(nbm, (nv + DT - 1) / DT);
         apply_prec_std(s, vj, z, st);
         spmv_std(s, z, nullptr, w, st);
-        double wn = 0;
         for (int pass = 0; pass < 2; pass++) {
+            double *h = coef + (2 * j + pass) * ldc;
             k_mdot<double, 1><<<grid, RB, 0, st>>>(n, nv, V, n, w, nullptr, s->partial);
-            k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, s->partial, nullptr, s->h, nullptr, 0);
-            launch_maxpy<double>(st, nb, n, nv, V, s->h, nullptr, w, s->pn);
-            EMG_HIP(hipMemcpyAsync(hh.data(), s->h, 2 * nv * sizeof(double), hipMemcpyDeviceToHost, st));
-            wn = host_norm(s->pn);
-            for (int i = 0; i < nv; i++) {
-                H[2 * ((size_t)j * (d + 1) + i)] += hh[2 * i];
-                H[2 * ((size_t)j * (d + 1) + i) + 1] += hh[2 * i + 1];
-            }
+            k_mdot_finish<<<nv, 256, 0, st>>>(nv, nbm, s->partial, nullptr, h, nullptr, 0);
+            launch_maxpy<double>(st, nb, n, nv, V, h, nullptr, w, s->pn);
         }
-        H[2 * ((size_t)j * (d + 1) + j + 1)] = wn;
-        EMG_CHECK(wn > 0 && std::isfinite(wn), "emg_solver_arnoldi_probe: breakdown");
-        k_scale_c128<<<nb, RB, 0, st>>>(n, 1.0 / wn, w);
+        k_scale_by_norm<double><<<nb, RB, 0, st>>>(n, s->pn, nb, w, w, norms + j + 1);
     }
+    EMG_LAUNCH_CHECK();
+    std::vector<double> got(PROBE_H + (size_t)2 * d * ldc), H(2 * (size_t)(d + 1) * d, 0.0);
+    EMG_HIP(hipMemcpyAsync(got.data(), s->h, got.size() * sizeof(double), hipMemcpyDeviceToHost, st));
     EMG_HIP(hipStreamSynchronize(st));
+    EMG_CHECK(got[0] > 0 && std::isfinite(got[0]), "emg_solver_arnoldi_probe: zero or non-finite start vector");
+    for (int j = 0; j < d; j++) {
+        const double *h = got.data() + PROBE_H + (size_t)2 * j * ldc, wn = got[j + 1];
+        EMG_CHECK(wn > 0 && std::isfinite(wn), "emg_solver_arnoldi_probe: breakdown");
+        for (int i = 0; i < 2 * (j + 1); i++) H[(size_t)2 * j * (d + 1) + i] = h[i] + h[ldc + i];
+        H[2 * ((size_t)j * (d + 1) + j + 1)] = wn;
+    }
     memcpy(h_out, H.data(), H.size() * sizeof(double));
     return 0;
 }

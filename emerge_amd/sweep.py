@@ -146,6 +146,9 @@ class BasisSweep:
         self.nq = 0
         self.Qq = np.zeros((len(self.ports), qmax), dtype=np.complex128)
         self.u = torch.empty(N, dtype=torch.complex128, device=dev)
+        # what _project leaves on the device: norm before and after each pass, coefficients of the passes
+        self.proj = torch.empty(4 + 4 * max(qmax, max_basis), dtype=torch.float64, device=dev)
+        self.qq = torch.zeros((self.ncol, 2 * len(self.ports)), dtype=torch.float64, device=dev)
 
     # ------------------------------------------------------------ primitives
     def _spmv(self, vals, x, y):
@@ -153,26 +156,26 @@ class BasisSweep:
         _lib.check(self.L.emg_spmv(p.N, _lib.ptr(p.pat.rowptr), _lib.ptr(p.pat.cols), _lib.ptr(vals), _lib.ptr(p.mask),
                                    _lib.ptr(x), _lib.ptr(y), _lib.stream_ptr()), "emg_spmv")
 
-    def _mdotc(self, V, nv, w) -> np.ndarray:
-        """conj(V_i) . w for i < nv (in calls of at most MAX_MULTI vectors)."""
-        out = np.zeros(nv, dtype=np.complex128)
-        for i0 in range(0, nv, MAX_MULTI):
-            k = min(MAX_MULTI, nv - i0)
-            _lib.check(self.L.emg_mdotc(self.p.N, k, _lib.ptr(V[i0:i0 + k]), _lib.ptr(w), _lib.ptr(self.h),
-                                        _lib.ptr(self.work), _lib.stream_ptr()), "emg_mdotc")
-            hv = self.h[: 2 * k].cpu().numpy()
-            out[i0:i0 + k] = hv[0::2] + 1j * hv[1::2]
-        return out
+    def _project(self, V, nv, w):
+        """w less its parts along V_i, i < nv, in two Gram-Schmidt passes, without a wait between them (in
+        calls of at most MAX_MULTI vectors): the coefficients taken out and ||w|| before and after."""
+        N, buf, work, st = self.p.N, self.proj, _lib.ptr(self.work), _lib.stream_ptr()
 
-    def _maxpy(self, V, nv, coef: np.ndarray, w) -> float:
-        """w -= sum_i coef_i V_i; returns ||w|| (in calls of at most MAX_MULTI vectors)."""
-        for i0 in range(0, max(nv, 1), MAX_MULTI):
-            k = min(MAX_MULTI, nv - i0)
-            if k > 0:
-                self.h[: 2 * k].copy_(self.torch.from_numpy(_c128_to_f64(coef[i0:i0 + k])))
-            _lib.check(self.L.emg_maxpy(self.p.N, k, _lib.ptr(V[i0:i0 + max(k, 1)]), _lib.ptr(self.h), _lib.ptr(w),
-                                        _lib.ptr(self.nrm), _lib.ptr(self.work), _lib.stream_ptr()), "emg_maxpy")
-        return float(self.nrm[0].item())
+        def maxpy(i0, k, h, norm):
+            _lib.check(self.L.emg_maxpy(N, k, _lib.ptr(V[i0:i0 + max(k, 1)]), _lib.ptr(h), _lib.ptr(w),
+                                        _lib.ptr(buf[norm:]), work, st), "emg_maxpy")
+        maxpy(0, 0, buf, 0)
+        runs = [(i0, min(MAX_MULTI, nv - i0)) for i0 in range(0, nv, MAX_MULTI)]
+        for q in range(2):
+            h = buf[4 + 2 * nv * q:]
+            for i0, k in runs:
+                _lib.check(self.L.emg_mdotc(N, k, _lib.ptr(V[i0:i0 + k]), _lib.ptr(w), _lib.ptr(h[2 * i0:]), work, st),
+                           "emg_mdotc")
+            for i0, k in runs:
+                maxpy(i0, k, h[2 * i0:], 1)
+        out = buf[: 4 + 4 * nv].cpu().numpy()
+        h = out[4:].view(np.complex128).reshape(2, nv).sum(axis=0)
+        return h, float(out[0]), float(out[1] if nv > 0 else out[0])
 
     def _comb(self, V, nv, coef: np.ndarray, out):
         self.h[: 2 * nv].copy_(self.torch.from_numpy(_c128_to_f64(coef)))
@@ -186,14 +189,7 @@ class BasisSweep:
         m = self.m
         w = self.x
         w.copy_(x)
-        xn = self._maxpy(self.V, 0, np.zeros(0), w)
-        y = np.zeros(m, dtype=np.complex128)
-        r = xn
-        if m > 0:
-            for _ in range(2):
-                h = self._mdotc(self.V, m, w)
-                r = self._maxpy(self.V, m, h, w)
-                y += h
+        y, xn, r = self._project(self.V, m, w)
         if r <= 1e-13 * xn:
             return y
         if m >= self.max_basis:
@@ -204,6 +200,7 @@ class BasisSweep:
         # the columns of K(f) v for every frequency: E v, B v, P_t v (masked operator)
         self.Vpd[m] = v[self.pdofs_d].cpu().numpy()
         u = self.u
+        self._new_cols = [None] * self.ncol
         for k in range(self.ncol):
             if k == 0:
                 self._spmv(self.p.E, v, u)
@@ -212,28 +209,30 @@ class BasisSweep:
             else:
                 u.zero_()
                 u[self.pdofs_d] = self.torch.from_numpy(self.P_pd[k - 2] @ self.Vpd[m]).to(self.p.dev)
-            self._add_column(u, m * self.ncol + k)
+            self._add_column(u, m * self.ncol + k, k)
+        qq = self.qq.cpu().numpy().view(np.complex128)     # (ncol, nports): conj(q_p) . Q of the new directions
+        for k, col in enumerate(self._new_cols):
+            if col is not None:
+                self.Qq[:, col] = qq[k].conj()
         self.Fb.append(self.sampler.fields(v[None, :])[0])
         self.m = m + 1
         return np.append(y, r)
 
-    def _add_column(self, u, col: int):
-        """CGS2 of u against Q; records u = Q R[:, col], extending Q when u adds a direction."""
+    def _add_column(self, u, col: int, k: int):
+        """CGS2 of u against Q; records u = Q R[:, col], extending Q when u adds a direction (column k of
+        this basis vector: its products with the port sources stay on the device, in qq[k])."""
         nq = self.nq
-        un = self._maxpy(self.Q, 0, np.zeros(0), u)
-        h = np.zeros(nq, dtype=np.complex128)
-        rho = un
-        if nq > 0:
-            for _ in range(2):
-                hh = self._mdotc(self.Q, nq, u)
-                rho = self._maxpy(self.Q, nq, hh, u)
-                h += hh
+        h, un, rho = self._project(self.Q, nq, u)
         self.R[:nq, col] = h
         if rho > 1e-14 * un and nq < self.Q.shape[0]:
             self._comb(u[None, :], 1, np.array([1.0 / rho], dtype=np.complex128), self.Q[nq])
             self.R[nq, col] = rho
-            for pi in range(len(self.ports)):
-                self.Qq[pi, nq] = self._mdotc(self.Q[nq:nq + 1], 1, self.qsrc[pi])[0]
+            for i0 in range(0, len(self.ports), MAX_MULTI):
+                i1 = min(len(self.ports), i0 + MAX_MULTI)
+                _lib.check(self.L.emg_mdotc(self.p.N, i1 - i0, _lib.ptr(self.qsrc[i0:i1]), _lib.ptr(self.Q[nq]),
+                                            _lib.ptr(self.qq[k, 2 * i0:]), _lib.ptr(self.work), _lib.stream_ptr()),
+                           "emg_mdotc")
+            self._new_cols[k] = nq
             self.nq = nq + 1
 
     def trial(self, freq: float, port_index: int) -> np.ndarray:
