@@ -63,11 +63,11 @@ struct emg_pattern {
     int fused_ok = 0;
     int32_t *chunk_row0 = nullptr;   // nchunk + 1, row of each chunk's first entry (last: n_ent - 1)
     int32_t *chunk_tets = nullptr;   // nchunk * CHUNK_TMAX
-    int32_t *chunk_desc = nullptr;   // nchunk * DESC: what a chunk's workgroup needs to know (DESC_*)
+    int32_t *chunk_desc = nullptr;   // nchunk * DESC: what a chunk's workgroup needs to know (DESC_*); behind chunk_tets
     int chunk_tmax = 0;              // most tets of a chunk (sizes the fused kernel's LDS)
     uint16_t *inc_local = nullptr;   // n_inc: (local tet << 8) | (s << 4) | s'
     uint32_t *chunk_ent = nullptr;   // nchunk * CHUNK: the chunk's entries by kind and descending incidence count (ENT_*)
-    uint8_t *chunk_cnt = nullptr;    // nchunk * CHUNK: their incidences, 0 past the last entry
+    uint8_t *chunk_cnt = nullptr;    // nchunk * CHUNK: their incidences, 0 past the last entry; behind chunk_ent
     double *tet_rec = nullptr;       // nt * REC: per-tet Gram records (fused-path workspace)
     double *tet_rec_batch = nullptr; // rec_batch_cap * nt * REC: the records of a batch of meshes
     int rec_batch_cap = 0;
@@ -276,12 +276,12 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
                                                                      pat->chunk_row0);
     {
         int *d_over = nullptr;
-        TRY(hipMalloc(&pat->chunk_tets, (size_t)pat->nchunk * CHUNK_TMAX * sizeof(int32_t)));
-        TRY(hipMalloc(&pat->chunk_desc, (size_t)pat->nchunk * DESC * sizeof(int32_t)));
-        TRY(hipMalloc(&pat->chunk_cnt, (size_t)pat->nchunk * pat->chunk));
+        TRY(hipMalloc(&pat->chunk_tets, (size_t)pat->nchunk * (CHUNK_TMAX + DESC) * sizeof(int32_t)));
+        pat->chunk_desc = pat->chunk_tets + pat->nchunk * CHUNK_TMAX;
         // two spare codes: the fused kernel reads the codes as 32-bit words
         TRY(hipMalloc(&pat->inc_local, (size_t)(n_inc + 2) * sizeof(uint16_t)));
-        TRY(hipMalloc(&pat->chunk_ent, (size_t)pat->nchunk * pat->chunk * sizeof(uint32_t)));
+        TRY(hipMalloc(&pat->chunk_ent, (size_t)pat->nchunk * pat->chunk * (sizeof(uint32_t) + 1)));
+        pat->chunk_cnt = reinterpret_cast<uint8_t *>(pat->chunk_ent + pat->nchunk * pat->chunk);
         TRY(hipMalloc(&pat->recipes, 2 * 100 * RECIPE_BYTES));
         TRY(hipMalloc(&d_over, sizeof(int)));
         TRY(hipMemsetAsync(d_over, 0, sizeof(int), st));
@@ -340,8 +340,6 @@ extern "C" void emg_pattern_destroy(emg_pattern *pat) {
     hfree(pat->blk_row0);
     hfree(pat->tet_blocks);
     hfree(pat->chunk_tets);
-    hfree(pat->chunk_desc);
-    hfree(pat->chunk_cnt);
     hfree(pat->inc_local);
     hfree(pat->chunk_ent);
     hfree(pat->chunk_row0);
