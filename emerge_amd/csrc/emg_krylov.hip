@@ -889,14 +889,46 @@ struct sp_args {
 // two round trips to memory instead of two per L entries.  Bound by the bytes of kre, acol and (in
 // rows with losses) kim; small problems by the latency of that chain.  STD: x, y, b in the caller's
 // layout (mode * ne + e) instead of interleaved (SP_Y and SP_RESID only).
-template <typename R, int L, int EP, bool STD>
-__global__ void __launch_bounds__(256) k_spmv_pk(int64_t ne, const int32_t *__restrict__ rowptr,
+// LOC: a workgroup first gathers x for the distinct columns of its LOC_ROWS rows into LDS (loc_tab: the columns, and
+// in acol's place 16-bit places among them).  The gathers of the other form take a line of the L2 each, 21 of them
+// per row and no two lanes of a row the same; 64 rows share theirs 3.3 times, and an index is 2 bytes.  Products of
+// the posts box: complex64 on air at 1,947,698 DOFs 114 -> 90 us (4.7 TB/s), with losses at 831,972 70 -> 63 (5.3),
+// complex128 on air at 883,652 91 -> 71 (5.1).  (8 lanes per row, which is 512 of them: 92, 61, 79; 32, 96 or 128
+// rows: 96, 66, 85; 113, 65, 86; 93, 65, 74; 2, 3 or 6 blocks in flight per lane: 95, 69, 73; 96, 68, 73; 93, 63, 89.)
+static constexpr int LOC_ROWS = 64, LOC_L = 4, LOC_MAX = 1024, LOC_CAND = 8192;
+static constexpr int LOC_LANES = LOC_ROWS * LOC_L;
+struct loc_tab {
+    const int32_t *ptr, *col;
+    const uint16_t *idx;
+};
+template <typename R, int L, int EP, bool STD, bool LOC>
+__global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, const int32_t *__restrict__ rowptr,
                                                  const int32_t *__restrict__ acol, const R *__restrict__ kre,
                                                  const R *__restrict__ kim, const uint8_t *__restrict__ flag,
-                                                 const R *__restrict__ x, sp_args<R> a) {
+                                                 const R *__restrict__ x, sp_args<R> a, loc_tab loc) {
     constexpr int U = L <= 4 ? 4 : L == 8 ? 3 : L == 16 ? 2 : 1;
-    const int64_t e = (xcd_run(blockIdx.x, gridDim.x) * (int64_t)blockDim.x + threadIdx.x) / L;
+    __shared__ __align__(16) R xs[LOC ? 4 * LOC_MAX : 4];
+    const int64_t blk = xcd_run(blockIdx.x, gridDim.x);
+    const int64_t e = (blk * blockDim.x + threadIdx.x) / L;
     const int lane = threadIdx.x % L;
+    if constexpr (LOC) {
+        const int32_t b = loc.ptr[blk], nu = loc.ptr[blk + 1] - b;
+        for (int i = threadIdx.x; i < nu; i += LOC_LANES) {
+            const int32_t c = loc.col[b + i];
+            if constexpr (STD) {
+                cx<R> u0 = ld(x, c), u1 = ld(x, ne + c);
+                if constexpr (sizeof(R) == 8) {
+                    const uint8_t cf = flag[c];
+                    if (!(cf & ROW0)) u0 = cx<R>();
+                    if (!(cf & ROW1)) u1 = cx<R>();
+                }
+                st2(xs, i, cx2<R>{u0.re, u0.im, u1.re, u1.im});
+            } else {
+                st2(xs, i, ld2(x, c));
+            }
+        }
+        __syncthreads();
+    }
     if (e >= ne) return;
     const uint8_t fl = flag[e];
     const int32_t p0 = rowptr[e] >> 1, p1 = rowptr[e + 1] >> 1;
@@ -924,12 +956,14 @@ __global__ void __launch_bounds__(256) k_spmv_pk(int64_t ne, const int32_t *__re
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int32_t q = p + u * L < p1 ? p + u * L : p;   // past the row's end: its own entry again, not used
-                c[u] = acol[q];
+                c[u] = LOC ? loc.idx[q] : acol[q];
                 k[u] = ld2(kre, q);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                if constexpr (STD) {
+                if constexpr (LOC) {
+                    xv[u] = ld2(xs, c[u]);
+                } else if constexpr (STD) {
                     cx<R> u0 = ld(x, c[u]), u1 = ld(x, ne + c[u]);
                     if constexpr (sizeof(R) == 8) {
                         // a caller's x may hold anything on PEC DOFs (their columns are zero, but 0 * inf is not)
@@ -959,14 +993,23 @@ __global__ void __launch_bounds__(256) k_spmv_pk(int64_t ne, const int32_t *__re
                     v[u].bi += k[u].br * xv[u].ar + k[u].bi * xv[u].br;
                 }
             }
+            // pairwise, then to the row's sums: the shorter chains keep few lanes per row as accurate as many
 #pragma unroll
             for (int u = 0; u < U; u++)
-                if (p + u * L < p1) {
-                    s0r += v[u].ar;
-                    s0i += v[u].ai;
-                    s1r += v[u].br;
-                    s1i += v[u].bi;
+                if (p + u * L >= p1) v[u] = cx2<R>{0, 0, 0, 0};
+#pragma unroll
+            for (int h = 1; h < U; h *= 2)
+#pragma unroll
+                for (int u = 0; u + h < U; u += 2 * h) {
+                    v[u].ar += v[u + h].ar;
+                    v[u].ai += v[u + h].ai;
+                    v[u].br += v[u + h].br;
+                    v[u].bi += v[u + h].bi;
                 }
+            s0r += v[0].ar;
+            s0i += v[0].ai;
+            s1r += v[0].br;
+            s1i += v[0].bi;
         }
     }
     s0r = lane_sum<L>(s0r);
@@ -1001,13 +1044,86 @@ __global__ void __launch_bounds__(256) k_spmv_pk(int64_t ne, const int32_t *__re
 
 template <typename R, int EP, bool STD>
 static void launch_spmv_pk(hipStream_t st, int L, int64_t ne, const int32_t *rowptr, const int32_t *acol, const R *kre,
-                           const R *kim, const uint8_t *flag, const R *x, const sp_args<R> &a) {
+                           const R *kim, const uint8_t *flag, const R *x, const sp_args<R> &a, const loc_tab &loc) {
+    if (loc.ptr != nullptr) {
+        k_spmv_pk<R, LOC_L, EP, STD, true><<<(unsigned)((ne + LOC_ROWS - 1) / LOC_ROWS), LOC_LANES, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
+        return;
+    }
     if (L != 4 && L != 8 && L != 32) L = 16;
     const unsigned grid = (unsigned)((ne * L + 255) / 256);
-    if (L == 4) k_spmv_pk<R, 4, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
-    else if (L == 8) k_spmv_pk<R, 8, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
-    else if (L == 32) k_spmv_pk<R, 32, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
-    else k_spmv_pk<R, 16, EP, STD><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a);
+    if (L == 4) k_spmv_pk<R, 4, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
+    else if (L == 8) k_spmv_pk<R, 8, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
+    else if (L == 32) k_spmv_pk<R, 32, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
+    else k_spmv_pk<R, 16, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
+}
+
+// The distinct columns of every LOC_ROWS rows, ascending, and every block's 16-bit place among them: counts first
+// (idx NULL), then with their prefix the lists and places.  *over where a workgroup's rows hold more than LOC_CAND
+// blocks or LOC_MAX distinct columns.
+__global__ void __launch_bounds__(512) k_loc_columns(int64_t ne, const int32_t *__restrict__ rowptr,
+                                                     const int32_t *__restrict__ acol, const int32_t *__restrict__ ptr,
+                                                     int32_t *__restrict__ cnt, int32_t *__restrict__ col,
+                                                     uint16_t *__restrict__ idx, int *__restrict__ over) {
+    __shared__ int32_t key[LOC_CAND];
+    __shared__ int32_t wsum[8];
+    const int tid = threadIdx.x;
+    const int64_t e0 = blockIdx.x * (int64_t)LOC_ROWS, e1 = min(e0 + LOC_ROWS, ne);
+    const int32_t p0 = rowptr[e0] >> 1, n = (rowptr[e1] >> 1) - p0;
+    if (n > LOC_CAND) {
+        if (tid == 0) { *over = 1; if (cnt) cnt[blockIdx.x] = 0; }
+        return;
+    }
+    int size = 512;
+    while (size < n) size <<= 1;
+    for (int i = tid; i < size; i += 512) key[i] = i < n ? acol[p0 + i] : INT32_MAX;
+    __syncthreads();
+    for (int len = 2; len <= size; len <<= 1)
+        for (int stride = len >> 1; stride > 0; stride >>= 1) {
+            for (int i = tid; i < size; i += 512) {
+                const int j = i ^ stride;
+                if (j > i) {
+                    const bool asc = (i & len) == 0;
+                    const int32_t a = key[i], b = key[j];
+                    if ((a > b) == asc) { key[i] = b; key[j] = a; }
+                }
+            }
+            __syncthreads();
+        }
+    // each lane's stretch of the sorted keys: how many are first of their value
+    const int per = size / 512, s0 = tid * per;
+    int mine = 0;
+    for (int i = s0; i < s0 + per; i++) mine += i < n && (i == 0 || key[i] != key[i - 1]);
+    int pre = mine;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(pre, off, 64);
+        if ((tid & 63) >= off) pre += v;
+    }
+    if ((tid & 63) == 63) wsum[tid >> 6] = pre;
+    __syncthreads();
+    int total = 0, before = pre - mine;
+    for (int w = 0; w < 8; w++) {
+        if (w < tid >> 6) before += wsum[w];
+        total += wsum[w];
+    }
+    if (total > LOC_MAX && tid == 0) *over = 1;
+    if (idx == nullptr) {
+        if (tid == 0) cnt[blockIdx.x] = total;
+        return;
+    }
+    const int32_t b = ptr[blockIdx.x];
+    for (int i = s0; i < s0 + per; i++)
+        if (i < n && (i == 0 || key[i] != key[i - 1])) col[b + before++] = key[i];
+    __syncthreads();
+    __threadfence_block();
+    for (int i = tid; i < n; i += 512) {
+        const int32_t c = acol[p0 + i];
+        int lo = 0, hi = total - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (col[b + mid] < c) lo = mid + 1; else hi = mid;
+        }
+        idx[p0 + i] = (uint16_t)lo;
+    }
 }
 
 // Entries of entity e's packed G row: the nodes of row e with both modes' values where rows e and
@@ -1643,6 +1759,8 @@ struct emg_solver {
     int32_t *acol = nullptr;        // nnz / 4 column entities
     void *kre = nullptr, *kim = nullptr;   // real and imaginary planes, nnz values each
     uint8_t *row_flag = nullptr;    // n_ent
+    int32_t *loc_ptr = nullptr, *loc_col = nullptr;   // distinct columns of every LOC_ROWS rows (k_loc_columns) or NULL
+    uint16_t *loc_idx = nullptr;
     double *inv64 = nullptr;
     float *inv32 = nullptr;
     double *V = nullptr;            // cap + 1 basis vectors, element type per precision
@@ -1726,7 +1844,8 @@ static void free_solver(emg_solver *s) {
     drop_fused(s);
     void *ps[] = {s->acol, s->kre, s->kim, s->row_flag, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial,
                   s->h, s->nrm, s->arn, s->pn, s->gram, s->flag, s->g_pcol, s->gt_prp, s->gt_pcol, s->g_pval,
-                  s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32, s->poly_c, s->pp, s->pt, s->py, s->pu};
+                  s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32, s->poly_c, s->pp, s->pt, s->py, s->pu, s->loc_ptr,
+                  s->loc_col, s->loc_idx};
     for (void *p : ps) (void)hipFree(p);
     if (s->host) (void)hipHostFree(s->host);
     if (s->cap_stream) (void)hipStreamDestroy(s->cap_stream);
@@ -1763,7 +1882,7 @@ static void apply_prec(emg_solver *s, const R *x, const double *xs, R *y, hipStr
 template <typename R, int EP, bool STD>
 static void spmv_pk(emg_solver *s, int L, const R *x, const sp_args<R> &a, hipStream_t st) {
     launch_spmv_pk<R, EP, STD>(st, L, s->n_ent, s->rowptr, s->acol, static_cast<const R *>(s->kre),
-                               static_cast<const R *>(s->kim), s->row_flag, x, a);
+                               static_cast<const R *>(s->kim), s->row_flag, x, a, loc_tab{s->loc_ptr, s->loc_col, s->loc_idx});
 }
 
 // Lanes per entity for vectors in the caller's layout, whose two gathers per block favour few: 8 / 16
@@ -1921,6 +2040,66 @@ __global__ void __launch_bounds__(256) k_check_entity_pattern(int64_t ne, int64_
     }
 }
 
+// off[i] = sum of cnt[0 .. i) for i <= n, through the host (once per solver or gradient)
+static int prefix_on_host(const int32_t *d_cnt, int64_t n, int32_t **d_off, int64_t *total, hipStream_t st) {
+    std::vector<int32_t> c(n), o(n + 1, 0);
+    EMG_HIP(hipMemcpyAsync(c.data(), d_cnt, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    EMG_HIP(hipStreamSynchronize(st));
+    int64_t t = 0;
+    for (int64_t i = 0; i < n; i++) {
+        t += c[i];
+        EMG_CHECK(t < ((int64_t)1 << 31), "emg_solver: too many entries");
+        o[i + 1] = (int32_t)t;
+    }
+    EMG_HIP(hipMalloc((void **)d_off, (n + 1) * sizeof(int32_t)));
+    EMG_HIP(hipMemcpyAsync(*d_off, o.data(), (n + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    EMG_HIP(hipStreamSynchronize(st));
+    *total = t;
+    return 0;
+}
+
+// Where products take k_spmv_pk's LOC form: with fewer rows its workgroups, 64 rows each, leave CUs idle between
+// their gathers and their sums.  Complex64 and complex128 products, air then losses: 250,000 DOFs 12.9 -> 12.0,
+// 18.7 -> 20.0, 20.4 -> 18.7 and 29.9 -> 31.2 us, 96,000 DOFs 5.4 -> 4.5, 7.1 -> 7.9, 9.6 -> 7.9 and 13.5 -> 13.0; a solve's
+// step at 60,000 DOFs 134 -> 140 us, at 250,000 257 -> 255; above it see k_spmv_pk.  EMG_LOCAL_COLUMNS overrides (0: never,
+// else wherever the rows fit).
+static constexpr int64_t LOC_MIN_N = 400000;
+// The tables of the LOC form, or none where a workgroup's rows exceed it or the memory does not suffice.
+static int local_columns(emg_solver *s) {
+    const char *env = getenv("EMG_LOCAL_COLUMNS");
+    if (env != nullptr ? atoi(env) == 0 : s->n < LOC_MIN_N) return 0;
+    const int64_t nb = (s->n_ent + LOC_ROWS - 1) / LOC_ROWS;
+    int32_t *cnt = nullptr;
+    int *d_over = reinterpret_cast<int *>(s->flag), over = 0;
+    int64_t total = 0;
+    EMG_HIP(hipMalloc((void **)&cnt, nb * sizeof(int32_t)));
+    hipError_t e = hipMemset(d_over, 0, sizeof(int));
+    if (e == hipSuccess) {
+        k_loc_columns<<<(unsigned)nb, 512>>>(s->n_ent, s->rowptr, s->acol, nullptr, cnt, nullptr, nullptr, d_over);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(&over, d_over, sizeof(int), hipMemcpyDeviceToHost);
+    const int rc = e != hipSuccess || over ? 0 : prefix_on_host(cnt, nb, &s->loc_ptr, &total, nullptr);
+    (void)hipFree(cnt);
+    EMG_HIP(e);
+    if (over || rc) return rc;
+    e = hipMalloc((void **)&s->loc_col, std::max<int64_t>(total, 1) * sizeof(int32_t));
+    if (e == hipSuccess) e = hipMalloc((void **)&s->loc_idx, s->nnz / 4 * sizeof(uint16_t));
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        void *ps[] = {s->loc_ptr, s->loc_col, s->loc_idx};
+        for (void *p : ps) (void)hipFree(p);
+        s->loc_ptr = s->loc_col = nullptr;
+        s->loc_idx = nullptr;
+        return 0;
+    }
+    EMG_HIP(e);
+    k_loc_columns<<<(unsigned)nb, 512>>>(s->n_ent, s->rowptr, s->acol, s->loc_ptr, nullptr, s->loc_col, s->loc_idx, d_over);
+    EMG_LAUNCH_CHECK();
+    EMG_HIP(hipStreamSynchronize(nullptr));
+    return 0;
+}
+
 extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr, const int32_t *d_cols, int restart,
                                  int precision, emg_solver **out) {
     EMG_CHECK(out && d_rowptr && d_cols, "emg_solver_create: null argument");
@@ -2001,6 +2180,10 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
         emg::set_error(std::string("emg_solver_create: packing the pattern: ") + hipGetErrorString(e));
         free_solver(s);
         return -2;
+    }
+    if (int rc = local_columns(s)) {
+        free_solver(s);
+        return rc;
     }
     *out = s;
     return 0;
@@ -2285,24 +2468,6 @@ extern "C" int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0
         H[2 * ((size_t)j * (d + 1) + j + 1)] = wn;
     }
     memcpy(h_out, H.data(), H.size() * sizeof(double));
-    return 0;
-}
-
-// off[i] = sum of cnt[0 .. i) for i <= n, through the host (once per gradient)
-static int prefix_on_host(const int32_t *d_cnt, int64_t n, int32_t **d_off, int64_t *total, hipStream_t st) {
-    std::vector<int32_t> c(n), o(n + 1, 0);
-    EMG_HIP(hipMemcpyAsync(c.data(), d_cnt, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    EMG_HIP(hipStreamSynchronize(st));
-    int64_t t = 0;
-    for (int64_t i = 0; i < n; i++) {
-        t += c[i];
-        EMG_CHECK(t < ((int64_t)1 << 31), "emg_solver_set_gradient: too many entries");
-        o[i + 1] = (int32_t)t;
-    }
-    EMG_HIP(hipMalloc((void **)d_off, (n + 1) * sizeof(int32_t)));
-    EMG_HIP(hipMemcpyAsync(*d_off, o.data(), (n + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    EMG_HIP(hipStreamSynchronize(st));
-    *total = t;
     return 0;
 }
 
