@@ -1264,15 +1264,16 @@ __global__ void __launch_bounds__(CH, TS <= 96 ? 4 : 2)
     };
     // Chunk l of this workgroup's XCD (workgroup b is on XCD b % 8), clamped to its last one: the XCDs take
     // runs of 1 << run consecutive chunks in turn.
-    const int64_t xcd = blockIdx.x % 8, all = pat.nchunk >> run >> 3;
-    const int64_t rest = pat.nchunk - (all << run << 3) - (xcd << run), most = (int64_t)1 << run;
+    const int nx = gridDim.x < 8 ? (int)gridDim.x : 8;   // fewer workgroups than XCDs share all chunks too
+    const int64_t xcd = blockIdx.x % nx, all = (pat.nchunk >> run) / nx;
+    const int64_t rest = pat.nchunk - ((all * nx + xcd) << run), most = (int64_t)1 << run;
     const int64_t mine = (all << run) + (rest < 0 ? 0 : rest < most ? rest : most);
     auto chunk_at = [&](int64_t l) {
         if (l >= mine) l = mine - 1;
-        return (((l >> run << 3) + xcd) << run) + (l & (most - 1));
+        return (((l >> run) * nx + xcd) << run) + (l & (most - 1));
     };
-    const int64_t step = (gridDim.x + 7 - xcd) / 8;
-    int64_t l = blockIdx.x / 8;
+    const int64_t step = (gridDim.x + nx - 1 - xcd) / nx;
+    int64_t l = blockIdx.x / nx;
     if (l >= mine) return;
     look_up(chunk_at(l));
     prefetch(chunk_at(l));
@@ -1732,7 +1733,7 @@ extern "C" int emg_assemble_iso_batched(const emg_pattern *pat, int nbatch, int6
     // still steps through several chunks, whose loads it issues ahead (32 meshes of 864 tets: 82 us with a
     // workgroup per chunk, 77 with 4 workgroups per CU, 78 and 79 with 2 and 8)
     const int64_t per_mesh = ((int64_t)g_num_cus * (pat->wg_per_cu ? pat->wg_per_cu : BATCH_WG) / nbatch + 7) / 8 * 8;
-    const int64_t gx = std::max<int64_t>(1, std::min<int64_t>(pat->nchunk, per_mesh));
+    const int64_t gx = std::min<int64_t>(pat->nchunk, std::max<int64_t>(8, per_mesh));
     const int efm = (flags & EMG_EXACT_FACE_MASS) ? 1 : 0;
     const cplx *ce = reinterpret_cast<const cplx *>(d_eps), *cn = reinterpret_cast<const cplx *>(d_nu);
     cplx *oE = reinterpret_cast<cplx *>(d_E), *oB = reinterpret_cast<cplx *>(d_B);

@@ -56,3 +56,21 @@ def test_chunks_equal_two_phase(cuda, name, flags):
     for offset in range(1, 8):
         for a, b in zip(run(flags, offset), first):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("batch", [3, 300, 1100])
+def test_batches_share_the_workgroups(cuda, batch):
+    """The workgroups per mesh fall as a batch grows, to the least there are: every chunk of every mesh is
+    still written, with the single assembly's values bit for bit."""
+    import torch
+    mesh = meshgen.structured_box(3, 3, 2, jitter=0.1, seed=7)
+    pat = GPUPattern(mesh)
+    rng = np.random.default_rng(batch)
+    eps, nu = (torch.from_numpy(rng.uniform(1, 4, (batch, mesh.n_tets)) + 0j).to(cuda) for _ in range(2))
+    nodes = torch.from_numpy(np.ascontiguousarray(np.broadcast_to(mesh.nodes.T, (batch,) + mesh.nodes.T.shape))).to(cuda)
+    print(f"batch of {batch}", flush=True)
+    E, B = pat.assemble_iso_batched(nodes, eps, nu)
+    Es, Bs = torch.empty_like(E[0]), torch.empty_like(B[0])
+    for i in (0, 1, batch // 2, batch - 1):
+        pat.assemble_iso_device(eps[i].contiguous(), nu[i].contiguous(), 0, Es, Bs)
+        assert torch.equal(E[i], Es) and torch.equal(B[i], Bs)
