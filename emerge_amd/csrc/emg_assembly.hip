@@ -89,6 +89,11 @@ static constexpr int CHUNK = 512;
 static constexpr int CHUNK_TMAX = 128;
 static constexpr int CHUNK_NMAX = 2048;  // incidences per chunk handled by the tet-list builder
 static constexpr int RECIPE_BYTES = 48;
+// Doubles of a tet's record, isotropic (384 bytes, three whole 128-byte lines) and with tensors (896, seven).
+static constexpr int REC = 48, TREC = 112;
+// Up to this many tets (64 MB) the pattern build's sort buffers stay as the records' workspaces, where freeing
+// them and allocating those on the first assembly took 0.25 ms; larger meshes allocate what they use.
+static constexpr int64_t KEEP_REC_TETS = 50000;
 // A chunk's values leave in the order of the CSR rows, 2 * CHUNK values of each row mode: of every row's
 // part in the chunk the mode-0 columns, then the mode-1 columns.  A word of chunk_ent: the place of the
 // entry's mode-0 column among them (10 bits), the entries of its row in the chunk (10 bits: its mode-1
@@ -219,8 +224,11 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
         }                                                                         \
     } while (0)
     TRY(hipMalloc(&keys, n_inc * sizeof(uint64_t)));
-    TRY(hipMalloc(&keys_s, n_inc * sizeof(uint64_t)));
+    const bool keep = nt <= KEEP_REC_TETS;
+    TRY(hipMalloc(&keys_s, keep ? nt * TREC * sizeof(double) : n_inc * sizeof(uint64_t)));
     TRY(hipMalloc(&vals, n_inc * sizeof(uint32_t)));
+    static_assert(TREC * sizeof(double) >= 100 * sizeof(uint64_t) && REC * sizeof(double) <= 100 * sizeof(uint32_t),
+                  "the sorted keys fit the tensor records, the isotropic records the counts");
     TRY(hipMalloc(&pat->inc, n_inc * sizeof(uint32_t)));
     k_make_keys<<<emg::grid_for(nt, 256), 256, 0, st>>>(d_tet_ent, nt, bits, keys, vals);
     TRY(hipGetLastError());
@@ -304,8 +312,13 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
     }
     TRY(hipStreamSynchronize(st));
     hfree(uniq);
-    hfree(counts);
-    hfree(keys_s);
+    if (keep && pat->fused_ok) {
+        pat->tet_rec = reinterpret_cast<double *>(counts);
+        pat->tensor_rec = reinterpret_cast<double *>(keys_s);
+    } else {
+        hfree(counts);
+        hfree(keys_s);
+    }
     hfree(tmp);
     hfree(d_nruns);
 #undef TRY
@@ -923,7 +936,6 @@ __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int
 }
 
 static constexpr int TD_FIELDS = 41;  // H(21) G(10) L(6) eps(2) nu(2)
-static constexpr int REC = 48;        // doubles of a tet's record: 384 bytes, three whole 128-byte lines
 
 // Eight pairs of doubles of every lane's record (pairs p0 .. p0 + 7 of rows of `pairs` pairs, lane's row
 // row0 + lane) through LDS, so that eight lanes write one whole line of a record where each lane by itself
@@ -1174,8 +1186,9 @@ __device__ __forceinline__ int out_shift(int u, int n1, int u4, int d0, int d1, 
 //  * lane r accumulates entry chunk_ent[r] (entries by kind and descending incidence
 //    count, so the lanes of a wavefront run the same formulas a similar number of times);
 //  * the 2x2 blocks go through LDS into the order of the CSR rows and leave as whole lines.
-// What bounds it is the CSR writes, and the reads among them: at 1,005,000 tets (8.6 GB written, 1.2 read)
-// 2.31 ms, 2.22 without the incidence loop, 1.45 without the stores.  What counts for them (2.89 ms before):
+// What bounds it is the CSR writes, and the reads among them: at 1,005,000 tets (9.0 GB written, 2.2 read by the
+// counters: 4.8 TB/s, where a copy reaches 4.89) 2.31 ms, 2.22 without the incidence loop, 1.45 without the
+// stores.  What counts for them (2.89 ms before):
 //  * whole lines per store: rows of 37 values per mode, stored as they lie in the entries' order, split
 //    a line between two stores at every row's end (a store-only kernel of that shape 2.07 ms, 1.46 with lines);
 //  * runs of 32 chunks per XCD: workgroups that step through the whole grid drift apart, and the stores
@@ -1379,7 +1392,6 @@ static void launch_staged(const emg_pattern *pat, dim3 grid, hipStream_t st, con
 // every entry of its element matrices is a short combination of.  Bound by the records' bytes
 // (45 MB at 49,680 tets): 36 us with every lane storing its own record, 17 through put_lines.
 static constexpr int T_G = 0, T_H = 32, T_L = 104, T_FIELDS = 110;
-static constexpr int TREC = 112;   // 896 bytes: seven whole 128-byte lines
 
 __global__ void __launch_bounds__(64) k_tet_tensor(int64_t nt, const double *__restrict__ nodes,
                                                    const int32_t *__restrict__ tets, const cplx *__restrict__ mat_m,
