@@ -26,15 +26,15 @@ METRIC = "sweep freq-pts/s at ≤1e-8 FP64 residual, learned vs plain GPU; assem
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per numeric assembly (k_tet_gram + k_assemble_staged) on the
 # 1,005,000-tet workload, from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE
-# runs of this benchmark (--sweep none --no-eigen --copy-calibration): FETCH (53,747 +
-# 1,301,548) KiB x 2 + WRITE (430,714 + 8,764,685) KiB x 1, the factors a 2 GiB
+# runs of this benchmark (--sweep none --no-eigen --copy-calibration): FETCH (48,300 +
+# 1,064,000) KiB x 2 + WRITE (376,900 + 8,758,000) KiB x 1, the factors a 2 GiB
 # device-to-device copy in the same runs gives.
-ASSEMBLY_TRAFFIC_BYTES = ((53_747 + 1_301_548) * 2 + 430_714 + 8_764_685) * 1024
-# HBM bytes per launch of the sweep's complex64 SpMV (k_spmv_blk<float,16,false>) on the
+ASSEMBLY_TRAFFIC_BYTES = ((48_300 + 1_064_000) * 2 + 376_900 + 8_758_000) * 1024
+# HBM bytes per launch of the sweep's complex64 product (k_spmv_pk) on the
 # posts box, from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs of this benchmark
-# (--spmv-kernel-only --copy-calibration): FETCH 602,184 KiB x 2 + WRITE 17,228 KiB x 1,
+# (--spmv-kernel-only --copy-calibration): FETCH 252,900 KiB x 2 + WRITE 15,220 KiB x 1,
 # with the factors the 2 GiB copy in the same runs gives (FETCH 1,048,612 KiB, WRITE 2,097,152 KiB).
-SPMV_TRAFFIC_BYTES = (602_184 * 2 + 17_228) * 1024
+SPMV_TRAFFIC_BYTES = (252_900 * 2 + 15_220) * 1024
 FP64_PEAK_TFLOPS = 78.6
 # FP64 flop convention per tet for the dense contraction of the closed form
 FLOP_PER_TET = 15449
@@ -357,13 +357,13 @@ def eigen_oracle(sigma: float, k: int) -> dict:
 
 
 def spmv_kernel_roofline(mesh, ports, freq, reps: int = 50):
-    """The sweep's dominant kernel, the complex64 entity-blocked SpMV of the
-    mixed-precision GMRES steps (k_spmv_blk<float,L,false> with the lanes L the
-    solver's autotuner picked, emg_solver_apply precision 32), timed with HIP
-    events on its stream.  Algorithmic bytes per
-    launch (complex64 CSR, int32 indices, one read of x and one write of y):
-    12 nnz + 20 N; the blocked format itself moves about 9 nnz + 20 N (one
-    column index per four entries)."""
+    """The sweep's dominant kernel, the complex64 product on the packed matrix
+    (k_spmv_pk through emg_solver_apply precision 32), timed with HIP events on
+    its stream.  Algorithmic bytes per launch: the values that are not zero by
+    construction -- 4 per entry of an entity row without an imaginary part, 8
+    of one with losses --, a 2-byte place per 2 x 2 block, and N (x and y 8 each,
+    row pointers 2, flags 0.5); the lists of distinct columns add to the format
+    what the 32-bit columns of the smaller problems would."""
     import torch
     from emerge_amd import _lib
     from emerge_amd.fdsolve import GPUSolver
@@ -391,12 +391,17 @@ def spmv_kernel_roofline(mesh, ports, freq, reps: int = 50):
         ev[i][1].record(stream)
     torch.cuda.synchronize()
     ms = float(np.mean([a.elapsed_time(b) for a, b in ev]))
-    alg = 12 * nnz + 20 * n
-    fmt = 9 * nnz + 20 * n
+    lossy = (prob.system(freq).imag != 0).to(torch.float32)
+    row = torch.repeat_interleave(torch.arange(n, device=prob.dev), prob.pat.rowptr[1:] - prob.pat.rowptr[:-1])
+    any_row = torch.zeros(n, device=prob.dev).index_add_(0, row, lossy) > 0
+    any_ent = (any_row[: n // 2] | any_row[n // 2:]).repeat(2)
+    nnz_lossy = int((any_ent.to(torch.int64) * (prob.pat.rowptr[1:] - prob.pat.rowptr[:-1])).sum())
+    alg = 4 * (nnz + nnz_lossy) + nnz // 2 + int(18.5 * n)
+    fmt = alg + nnz // 2 if n < 400_000 else alg + int(0.3 * nnz)
     ach = alg / (ms * 1e-3) / 1e9
     tuning = solver.spmv_tuning()
-    return {"kernel": f"k_spmv_blk<float,{tuning['lanes_c64']},false>", "autotune": tuning,
-            "smoother_autotune": solver.smoother_tuning(), "rows": n, "nnz": nnz,
+    return {"kernel": "k_spmv_pk<float>", "autotune": tuning,
+            "smoother_autotune": solver.smoother_tuning(), "rows": n, "nnz": nnz, "nnz_lossy_rows": nnz_lossy,
             "kernel_ms": ms, "alg_bytes": alg,
             "format_bytes": fmt, "bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": ach / HBM_PEAK_GBS, "format_frac": fmt / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS,

@@ -107,7 +107,12 @@ int emg_assemble_tensor(const emg_pattern *pat, const double *d_nodes, const int
  * precision 64: complex128 GMRES.  precision 32: complex64 GMRES inside FP64
  * iterative refinement; the returned residual is always the FP64
  * ||b - K x|| / ||b|| over the free DOFs.  Preconditioner: inverse 2x2 blocks
- * coupling the two modes of every edge / face (entity e <-> e + N/2).       */
+ * coupling the two modes of every edge / face (entity e <-> e + N/2).
+ * Forms chosen by size, with environment overrides read when they are set up
+ * (0: never, else wherever the rows fit): products that gather x for 64 rows
+ * at a time from 400,000 DOFs (EMG_LOCAL_COLUMNS, emg_solver_create), and
+ * complex64 steps with one launch per smoother application and product up to
+ * 50,000 (EMG_FUSED_STEPS, emg_solver_set_gradient).                        */
 typedef struct emg_solver emg_solver;
 typedef struct {
     int iterations;   /* Krylov iterations over all restarts / refinements */
