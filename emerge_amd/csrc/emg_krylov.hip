@@ -2535,9 +2535,9 @@ static int fuse_rows(int64_t rows, const GEN &gen, int32_t *cnt, int *d_over, in
     EMG_HIP(hipMemcpyAsync(&over, d_over, sizeof(int), hipMemcpyDeviceToHost, st));
     int64_t total = 0;
     if (int rc = prefix_on_host(cnt, rows, ptr, &total, st)) return rc;
-    if (over) { *fits = false; return 0; }
-    hipError_t e = hipMalloc((void **)col, std::max<int64_t>(total, 1) * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(val, std::max<int64_t>(total, 1) * bytes);
+    if (over || total == 0) { *fits = false; return 0; }   // the steps read slot 0 in place of none
+    hipError_t e = hipMalloc((void **)col, total * sizeof(int32_t));
+    if (e == hipSuccess) e = hipMalloc(val, total * bytes);
     if (e == hipErrorOutOfMemory) { (void)hipGetLastError(); *fits = false; return 0; }
     EMG_HIP(e);
     k_distinct<<<(unsigned)rows, 256, 0, st>>>(gen, nullptr, *ptr, *col, d_over);
