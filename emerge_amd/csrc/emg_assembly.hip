@@ -28,6 +28,7 @@
 
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <algorithm>
 #include <type_traits>
@@ -47,6 +48,14 @@ void set_error(const std::string &msg) { g_err = msg; }
 }  // namespace emg
 
 extern "C" const char *emg_last_error(void) { return emg::g_err.c_str(); }
+
+// Per-tet records of the tensor path and who may write them next: a call's two launches begin after `done`
+// of the call before, whatever streams the two are on.
+struct tensor_work {
+    std::mutex mu;
+    double *rec = nullptr;       // nt * TREC
+    hipEvent_t done = nullptr;   // recorded behind the launch that reads the records
+};
 
 struct emg_pattern {
     int64_t nt = 0, n_ent = 0, nnz_ent = 0, n_inc = 0, nblk = 0;
@@ -72,7 +81,7 @@ struct emg_pattern {
     double *tet_rec_batch = nullptr; // rec_batch_cap * nt * REC: the records of a batch of meshes
     int rec_batch_cap = 0;
     uint8_t *recipes = nullptr;      // 2 * 100 * RECIPE_BYTES: symmetric Gram indices, then full ones (tensors)
-    double *tensor_rec = nullptr;    // nt * TREC: per-tet records of the tensor path (workspace)
+    tensor_work *tensor = nullptr;
     int wg_per_cu = 0;               // fused launch: workgroups per CU, 0 until tuned (first fused assembly)
     float wg_ms[5] = {};             // measured ms per assembly for ASM_WG[i]
 };
@@ -209,6 +218,7 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
     pat->n_ent = n_ent;
     pat->n_inc = n_inc;
     pat->bits = bits;
+    pat->tensor = new tensor_work();
     int rc = 0;
     auto fail = [&](int code) {
         hfree(keys); hfree(keys_s); hfree(vals); hfree(uniq); hfree(counts); hfree(tmp); hfree(d_nruns);
@@ -314,7 +324,7 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
     hfree(uniq);
     if (keep && pat->fused_ok) {
         pat->tet_rec = reinterpret_cast<double *>(counts);
-        pat->tensor_rec = reinterpret_cast<double *>(keys_s);
+        pat->tensor->rec = reinterpret_cast<double *>(keys_s);
     } else {
         hfree(counts);
         hfree(keys_s);
@@ -359,7 +369,9 @@ extern "C" void emg_pattern_destroy(emg_pattern *pat) {
     hfree(pat->tet_rec);
     hfree(pat->tet_rec_batch);
     hfree(pat->recipes);
-    hfree(pat->tensor_rec);
+    hfree(pat->tensor->rec);
+    if (pat->tensor->done != nullptr) (void)hipEventDestroy(pat->tensor->done);
+    delete pat->tensor;
     delete pat;
 }
 
@@ -428,7 +440,7 @@ struct Stage {
 };
 
 // One lane per adjacency entry, every tet's products formed anew per incidence: meshes without chunk
-// tables, and EMG_FORCE_TWO_PHASE.  Bound by its registers (198 and a spill: 2 waves per SIMD) and the
+// tables, EMG_FORCE_TWO_PHASE, and calls that may not use the pattern's records (tensor_records).  Bound by its registers (198 and a spill: 2 waves per SIMD) and the
 // repeated work: 1430 us at 49,680 tets, where the staged path takes 289.
 __global__ void __launch_bounds__(ABLK) k_assemble(const emg_pattern pat, const double *__restrict__ nodes,
                                                    const int32_t *__restrict__ tets, const cplx *__restrict__ mat_m,
@@ -1607,10 +1619,43 @@ __global__ void __launch_bounds__(CHUNK, TS <= 64 ? 4 : 2)
 static void launch_tensor_staged(const emg_pattern *pat, hipStream_t st, int efm, cplx *oE, cplx *oB) {
     const unsigned grid = (unsigned)pat->nchunk;
     const int tm = pat->chunk_tmax;
-    if (tm <= 48) k_assemble_tensor_staged<48><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
-    else if (tm <= 64) k_assemble_tensor_staged<64><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
-    else if (tm <= 96) k_assemble_tensor_staged<96><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
-    else k_assemble_tensor_staged<CHUNK_TMAX><<<grid, CHUNK, 0, st>>>(*pat, pat->tensor_rec, efm, oE, oB);
+    const double *rec = pat->tensor->rec;
+    if (tm <= 48) k_assemble_tensor_staged<48><<<grid, CHUNK, 0, st>>>(*pat, rec, efm, oE, oB);
+    else if (tm <= 64) k_assemble_tensor_staged<64><<<grid, CHUNK, 0, st>>>(*pat, rec, efm, oE, oB);
+    else if (tm <= 96) k_assemble_tensor_staged<96><<<grid, CHUNK, 0, st>>>(*pat, rec, efm, oE, oB);
+    else k_assemble_tensor_staged<CHUNK_TMAX><<<grid, CHUNK, 0, st>>>(*pat, rec, efm, oE, oB);
+}
+
+// Whether a call on st may use the pattern's records, with st waiting for their last reader.  Not where
+// st is being captured, since a graph replays later, on any stream, with nothing to order it after other calls;
+// nor where there is no memory for the records.  Those calls take k_assemble, which needs none.  The event
+// and the wait take 2.6 us of 253 at 49,680 tets (a stream's handle may come back as another stream's, so
+// equal handles do not show that the order is there already).
+static int tensor_records(const emg_pattern *pat, hipStream_t st, bool *usable) {
+    tensor_work *w = pat->tensor;
+    *usable = false;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    if (w->rec == nullptr) {
+        // an allocation must not end a capture that runs on another stream
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        EMG_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t e = hipMalloc((void **)&w->rec, (size_t)pat->nt * TREC * sizeof(double));
+        EMG_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            w->rec = nullptr;
+            return 0;
+        }
+        EMG_HIP(e);
+    }
+    if (w->done == nullptr) EMG_HIP(hipEventCreateWithFlags(&w->done, hipEventDisableTiming));
+    else EMG_HIP(hipStreamWaitEvent(st, w->done, 0));
+    *usable = true;
+    return 0;
 }
 
 static int g_num_cus = 0;
@@ -1770,13 +1815,18 @@ extern "C" int emg_assemble_tensor(const emg_pattern *pat, const double *d_nodes
     const cplx *cm = reinterpret_cast<const cplx *>(d_mm), *cs = reinterpret_cast<const cplx *>(d_ms);
     cplx *oE = reinterpret_cast<cplx *>(d_E), *oB = reinterpret_cast<cplx *>(d_B);
     if (pat->fused_ok && !(flags & EMG_FORCE_TWO_PHASE)) {
-        emg_pattern *mp = const_cast<emg_pattern *>(pat);
-        if (!mp->tensor_rec) EMG_HIP(hipMalloc(&mp->tensor_rec, (size_t)pat->nt * TREC * sizeof(double)));
-        k_tet_tensor<<<emg::grid_for(pat->nt, 64), 64, 0, st>>>(pat->nt, d_nodes, d_tets, cm, cs, mp->tensor_rec);
-        launch_tensor_staged(pat, st, efm, oE, oB);
-    } else {
-        k_assemble<<<emg::grid_for(pat->nnz_ent, ABLK), ABLK, 0, st>>>(*pat, d_nodes, d_tets, cm, cs, efm, oE, oB);
+        std::lock_guard<std::mutex> lock(pat->tensor->mu);
+        bool usable = false;
+        if (int rc = tensor_records(pat, st, &usable)) return rc;
+        if (usable) {
+            k_tet_tensor<<<emg::grid_for(pat->nt, 64), 64, 0, st>>>(pat->nt, d_nodes, d_tets, cm, cs, pat->tensor->rec);
+            launch_tensor_staged(pat, st, efm, oE, oB);
+            EMG_LAUNCH_CHECK();
+            EMG_HIP(hipEventRecord(pat->tensor->done, st));
+            return 0;
+        }
     }
+    k_assemble<<<emg::grid_for(pat->nnz_ent, ABLK), ABLK, 0, st>>>(*pat, d_nodes, d_tets, cm, cs, efm, oE, oB);
     EMG_LAUNCH_CHECK();
     return 0;
 }

@@ -61,8 +61,9 @@ int emg_pattern_assembly_tuning(const emg_pattern *pat, int *h_wg_per_cu, float 
 /* Flags for emg_assemble_*. */
 #define EMG_EXACT_FACE_MASS 1 /* use the exact face-face mass integral instead of
                                  the reference's coefficient (fem/mth/tet.py:1036) */
-#define EMG_FORCE_TWO_PHASE 2 /* isotropic assembly through per-tet element blocks in
-                                 HBM instead of the fused LDS kernel (same results) */
+#define EMG_FORCE_TWO_PHASE 2 /* without the fused LDS kernels: isotropic assembly through per-tet
+                                 element blocks in HBM (emg_assemble_iso), tensor assembly entry
+                                 by entry (emg_assemble_tensor); same results up to rounding */
 #define EMG_REFERENCE_GEOMETRY 4 /* isotropic fused path only: d_tets hold each tet in the
                                  reference's vertex order, and the vertex gradients and volume
                                  come from the reference's absolute-coordinate cofactor formulas
@@ -95,7 +96,11 @@ int emg_assemble_iso_batched(const emg_pattern *pat, int nbatch, int64_t nv, con
 
 /* Same with full 3x3 complex tensors per tet: d_mm (nt,3,3) c128 multiplies
  * the mass term (eps_r), d_ms (nt,3,3) c128 the curl term (the reference
- * passes matinv(mu_r), fem/physics/edm/optimized_assembly.py:103-107).       */
+ * passes matinv(mu_r), fem/physics/edm/optimized_assembly.py:103-107).  The
+ * pattern's per-tet records are written and read on `stream`, behind the call
+ * before on whatever stream that was, so calls on several streams may follow each
+ * other without waits of the caller's.  A call under stream capture, or without memory
+ * for the records, does without them (slower, same values up to rounding).      */
 int emg_assemble_tensor(const emg_pattern *pat, const double *d_nodes, const int32_t *d_tets,
                         const double *d_mm, const double *d_ms, int flags,
                         double *d_E, double *d_B, void *stream);

@@ -1,0 +1,50 @@
+"""What the library's host code allocates, launches and waits for, recorded on the CPU (tests/hip_recorder.c)."""
+import pytest
+
+from tests.host_calls import run
+
+PATTERN = """
+def pattern(nt):
+    h = P()
+    te = np.zeros((nt, 10), np.int32)
+    assert L.emg_pattern_build(at(te), nt, 20, P(7), ctypes.byref(h)) == 0
+    rec.rec_clear()
+    return h
+a = np.zeros(64)
+def tensor(h, stream):
+    rc = L.emg_assemble_tensor(h, at(a), at(a), at(a), at(a), 0, at(a), at(a), P(stream))
+    out([rc] + log())
+"""
+
+
+def _kernels(lines):
+    return [x.split()[1] for x in lines if x.startswith("launch")]
+
+
+def test_tensor_assemblies_on_two_streams_follow_each_other(tmp_path):
+    """The records of a pattern are one buffer: a call on another stream begins behind the last reader of the
+    call before."""
+    first, second, third = run(PATTERN + "h = pattern(4)\ntensor(h, 8)\ntensor(h, 9)\ntensor(h, 8)\n", tmp_path)
+    two = ["k_tet_tensor", "k_assemble_tensor_staged"]
+    for lines in (first, second, third):
+        assert lines[0] == 0 and _kernels(lines[1:]) == two
+    event = first[-1].split()[2]
+    assert first[-1] == f"record event {event} stream 8"
+    for lines, stream in ((second, 9), (third, 8)):
+        assert lines[1] == f"stream {stream} waits for event {event}"
+        assert lines[-1] == f"record event {event} stream {stream}"
+
+
+@pytest.mark.parametrize("nt", [4, 60000])
+def test_tensor_assembly_under_capture_uses_no_memory_of_the_pattern(tmp_path, nt):
+    """A captured call replays on any stream, so it neither allocates nor uses the pattern's records."""
+    (lines,) = run(PATTERN + f"h = pattern({nt})\nrec.rec_capturing(1)\ntensor(h, 8)\n", tmp_path)
+    assert lines[0] == 0 and len(lines) == 2 and _kernels(lines[1:]) == ["k_assemble"]
+
+
+def test_tensor_assembly_without_memory_for_the_records(tmp_path):
+    """A mesh whose records do not fit is assembled as before there were any; with memory, from them."""
+    none, some = run(PATTERN + "h = pattern(60000)\nrec.rec_budget(rec.rec_used())\ntensor(h, 8)\n"
+                     "rec.rec_budget(2 ** 62)\ntensor(h, 8)\n", tmp_path)
+    assert none[0] == 0 and _kernels(none[1:]) == ["k_assemble"]
+    assert some[0] == 0 and _kernels(some[1:]) == ["k_tet_tensor", "k_assemble_tensor_staged"]
