@@ -3072,9 +3072,10 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
         const int limit = max_refine > 0 ? max_refine : (1 << 30);
         int stall = 0;
         kept_host kh(s->cap);
-        rc = upload_kept(s, kh, st);
-        if (rc) return rc;
         while (rel > tol && ref < limit && total < maxiter) {
+            // here, not behind a cycle: nothing of a solve is in flight when it returns
+            rc = upload_kept(s, kh, st);
+            if (rc) return rc;
             const double rs = 1.0 / (rel * bn);
             k_pack_vec<float><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->r, rs, reinterpret_cast<float *>(s->w));
             // A cycle stops once complex64 GMRES has reduced its residual by CYCLE_CUT (or
@@ -3109,8 +3110,6 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
             // cycles of the same space make up in a few steps (posts box at 2.2 GHz: 244 steps to 1e-9,
             // 500 when it forgot there).
             if (it == 0 || s->cap - kh.used() < CYCLE_ROOM || (int)kh.cycles.size() == KEEP_MAX || stall >= 2) kh.cycles.clear();
-            rc = upload_kept(s, kh, st);
-            if (rc) return rc;
         }
         info->iterations = total;
         info->refinements = ref;

@@ -48,3 +48,29 @@ def test_tensor_assembly_without_memory_for_the_records(tmp_path):
                      "rec.rec_budget(2 ** 62)\ntensor(h, 8)\n", tmp_path)
     assert none[0] == 0 and _kernels(none[1:]) == ["k_assemble"]
     assert some[0] == 0 and _kernels(some[1:]) == ["k_tet_tensor", "k_assemble_tensor_staged"]
+
+
+SOLVER = """
+def solver(precision, n=20, restart=10):
+    s = P()
+    rp = np.zeros(n + 1, np.int32)
+    rp[1:] = np.arange(1, n + 1) * 2                     # entity e's rows list entity e: 2 x 2 blocks
+    c = np.stack([np.arange(n) % (n // 2), np.arange(n) % (n // 2) + n // 2], axis=1).astype(np.int32).ravel()
+    rc = L.emg_solver_create(n, 2 * n, at(rp), at(c), restart, precision, ctypes.byref(s))
+    return rc, s
+v, x = np.zeros(4000), np.zeros(4000)
+info = _lib.SolveInfo()
+"""
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_a_solve_leaves_nothing_in_flight(tmp_path, precision):
+    """emg_solver_solve synchronises its stream: no launch or copy follows its last wait, so that the caller's
+    next call may come on another stream."""
+    (lines,) = run(SOLVER + f"""
+rc, s = solver({precision})
+assert rc == 0 and L.emg_solver_set_matrix(s, at(v), None, P(9)) == 0
+rec.rec_clear()
+out([L.emg_solver_solve(s, at(v), at(x), 1e-8, 100, 0, ctypes.byref(info), P(9))] + log())
+""", tmp_path)
+    assert lines[0] == 0 and lines[-1] == "wait stream 9"
