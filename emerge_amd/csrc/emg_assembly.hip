@@ -52,7 +52,7 @@ extern "C" const char *emg_last_error(void) { return emg::g_err.c_str(); }
 // Per-tet records of the tensor path and who may write them next: a call's two launches begin after `done`
 // of the call before, whatever streams the two are on.
 struct tensor_work {
-    std::mutex mu;
+    std::mutex mu;               // of this, and of emg_pattern::spare
     double *rec = nullptr;       // nt * TREC
     hipEvent_t done = nullptr;   // recorded behind the launch that reads the records
 };
@@ -82,6 +82,11 @@ struct emg_pattern {
     int rec_batch_cap = 0;
     uint8_t *recipes = nullptr;      // 2 * 100 * RECIPE_BYTES: symmetric Gram indices, then full ones (tensors)
     tensor_work *tensor = nullptr;
+    // The build's largest sort buffer, nt * TREC doubles, until the first assembly takes it for its records,
+    // isotropic or with tensors (take_records): freeing it and allocating those costs more than either
+    // (at 7,920 / 24,480 / 49,680 tets: build 1.17 -> 0.85, 1.94 -> 1.26, 3.3 -> 2.1 ms, first tensor pass 91 -> 64,
+    // 512 -> 143, 586 -> 282 us; at 82,944 746 -> 443).
+    double *spare = nullptr;
     int wg_per_cu = 0;               // fused launch: workgroups per CU, 0 until tuned (first fused assembly)
     float wg_ms[5] = {};             // measured ms per assembly for ASM_WG[i]
 };
@@ -100,9 +105,6 @@ static constexpr int CHUNK_NMAX = 2048;  // incidences per chunk handled by the 
 static constexpr int RECIPE_BYTES = 48;
 // Doubles of a tet's record, isotropic (384 bytes, three whole 128-byte lines) and with tensors (896, seven).
 static constexpr int REC = 48, TREC = 112;
-// Up to this many tets (64 MB) the pattern build's sort buffers stay as the records' workspaces, where freeing
-// them and allocating those on the first assembly took 0.25 ms; larger meshes allocate what they use.
-static constexpr int64_t KEEP_REC_TETS = 50000;
 // A chunk's values leave in the order of the CSR rows, 2 * CHUNK values of each row mode: of every row's
 // part in the chunk the mode-0 columns, then the mode-1 columns.  A word of chunk_ent: the place of the
 // entry's mode-0 column among them (10 bits), the entries of its row in the chunk (10 bits: its mode-1
@@ -234,11 +236,14 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
         }                                                                         \
     } while (0)
     TRY(hipMalloc(&keys, n_inc * sizeof(uint64_t)));
-    const bool keep = nt <= KEEP_REC_TETS;
-    TRY(hipMalloc(&keys_s, keep ? nt * TREC * sizeof(double) : n_inc * sizeof(uint64_t)));
+    static_assert(TREC * sizeof(double) >= 100 * sizeof(uint64_t) && TREC >= REC, "the sorted keys fit the records");
+    bool keep = true;
+    if (hipMalloc(&keys_s, nt * TREC * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        keep = false;
+        TRY(hipMalloc(&keys_s, n_inc * sizeof(uint64_t)));
+    }
     TRY(hipMalloc(&vals, n_inc * sizeof(uint32_t)));
-    static_assert(TREC * sizeof(double) >= 100 * sizeof(uint64_t) && REC * sizeof(double) <= 100 * sizeof(uint32_t),
-                  "the sorted keys fit the tensor records, the isotropic records the counts");
     TRY(hipMalloc(&pat->inc, n_inc * sizeof(uint32_t)));
     k_make_keys<<<emg::grid_for(nt, 256), 256, 0, st>>>(d_tet_ent, nt, bits, keys, vals);
     TRY(hipGetLastError());
@@ -322,13 +327,9 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
     }
     TRY(hipStreamSynchronize(st));
     hfree(uniq);
-    if (keep && pat->fused_ok) {
-        pat->tet_rec = reinterpret_cast<double *>(counts);
-        pat->tensor->rec = reinterpret_cast<double *>(keys_s);
-    } else {
-        hfree(counts);
-        hfree(keys_s);
-    }
+    hfree(counts);
+    if (keep && pat->fused_ok) pat->spare = reinterpret_cast<double *>(keys_s);
+    else hfree(keys_s);
     hfree(tmp);
     hfree(d_nruns);
 #undef TRY
@@ -369,6 +370,7 @@ extern "C" void emg_pattern_destroy(emg_pattern *pat) {
     hfree(pat->tet_rec);
     hfree(pat->tet_rec_batch);
     hfree(pat->recipes);
+    hfree(pat->spare);
     hfree(pat->tensor->rec);
     if (pat->tensor->done != nullptr) (void)hipEventDestroy(pat->tensor->done);
     delete pat->tensor;
@@ -1626,12 +1628,31 @@ static void launch_tensor_staged(const emg_pattern *pat, hipStream_t st, int efm
     else k_assemble_tensor_staged<CHUNK_TMAX><<<grid, CHUNK, 0, st>>>(*pat, rec, efm, oE, oB);
 }
 
+// The pattern's spare buffer, which becomes the caller's, or else a new one of nt * doubles doubles.
+static hipError_t take_records(emg_pattern *pat, int doubles, double **rec) {
+    if (pat->spare != nullptr) {
+        *rec = pat->spare;
+        pat->spare = nullptr;
+        return hipSuccess;
+    }
+    // an allocation must not end a capture that runs on another stream
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipMalloc((void **)rec, (size_t)pat->nt * doubles * sizeof(double));
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *rec = nullptr;
+    }
+    return e;
+}
+
 // Whether a call on st may use the pattern's records, with st waiting for their last reader.  Not where
 // st is being captured, since a graph replays later, on any stream, with nothing to order it after other calls;
 // nor where there is no memory for the records.  Those calls take k_assemble, which needs none.  The event
 // and the wait take 2.6 us of 253 at 49,680 tets (a stream's handle may come back as another stream's, so
 // equal handles do not show that the order is there already).
-static int tensor_records(const emg_pattern *pat, hipStream_t st, bool *usable) {
+static int tensor_records(emg_pattern *pat, hipStream_t st, bool *usable) {
     tensor_work *w = pat->tensor;
     *usable = false;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -1640,16 +1661,8 @@ static int tensor_records(const emg_pattern *pat, hipStream_t st, bool *usable) 
         return 0;
     }
     if (w->rec == nullptr) {
-        // an allocation must not end a capture that runs on another stream
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        EMG_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-        const hipError_t e = hipMalloc((void **)&w->rec, (size_t)pat->nt * TREC * sizeof(double));
-        EMG_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            w->rec = nullptr;
-            return 0;
-        }
+        const hipError_t e = take_records(pat, TREC, &w->rec);
+        if (e == hipErrorOutOfMemory) return 0;
         EMG_HIP(e);
     }
     if (w->done == nullptr) EMG_HIP(hipEventCreateWithFlags(&w->done, hipEventDisableTiming));
@@ -1729,7 +1742,10 @@ extern "C" int emg_assemble_iso(const emg_pattern *pat, const double *d_nodes, c
         const int efm = (flags & EMG_EXACT_FACE_MASS) ? 1 : 0;
         const cplx *ce = reinterpret_cast<const cplx *>(d_eps), *cn = reinterpret_cast<const cplx *>(d_nu);
         cplx *oE = reinterpret_cast<cplx *>(d_E), *oB = reinterpret_cast<cplx *>(d_B);
-        if (!mp->tet_rec) EMG_HIP(hipMalloc(&mp->tet_rec, (size_t)pat->nt * REC * sizeof(double)));
+        if (!mp->tet_rec) {
+            std::lock_guard<std::mutex> lock(pat->tensor->mu);
+            EMG_HIP(take_records(mp, REC, &mp->tet_rec));
+        }
         auto run = [&](int wg) {
             if (flags & EMG_REFERENCE_GEOMETRY)
                 k_tet_gram<true><<<emg::grid_for(pat->nt, 64), 64, 0, st>>>(pat->nt, d_nodes, d_tets, ce, cn,
@@ -1817,7 +1833,7 @@ extern "C" int emg_assemble_tensor(const emg_pattern *pat, const double *d_nodes
     if (pat->fused_ok && !(flags & EMG_FORCE_TWO_PHASE)) {
         std::lock_guard<std::mutex> lock(pat->tensor->mu);
         bool usable = false;
-        if (int rc = tensor_records(pat, st, &usable)) return rc;
+        if (int rc = tensor_records(const_cast<emg_pattern *>(pat), st, &usable)) return rc;
         if (usable) {
             k_tet_tensor<<<emg::grid_for(pat->nt, 64), 64, 0, st>>>(pat->nt, d_nodes, d_tets, cm, cs, pat->tensor->rec);
             launch_tensor_staged(pat, st, efm, oE, oB);

@@ -35,6 +35,20 @@ def test_tensor_assemblies_on_two_streams_follow_each_other(tmp_path):
         assert lines[-1] == f"record event {event} stream {stream}"
 
 
+ISO = "assert L.emg_assemble_iso(h, at(a), at(a), at(a), at(a), 0, at(a), at(a), P(8)) == 0\nrec.rec_clear()\n"
+
+
+@pytest.mark.parametrize("nt", [4, 60000])
+def test_the_first_assembly_takes_over_the_build_s_buffer(tmp_path, nt):
+    """The sort buffer that a build leaves serves as the records of whichever assembly comes first, at every size
+    of mesh: that one allocates nothing, the other allocates its own, and a pattern that sees one kind of
+    media holds one buffer."""
+    tensor_first, tensor_after_iso, again = run(PATTERN + f"h = pattern({nt})\ntensor(h, 8)\n"
+                                                f"h = pattern({nt})\n{ISO}tensor(h, 8)\ntensor(h, 8)\n", tmp_path)
+    assert not any("malloc" in x for x in tensor_first[1:] + again[1:])
+    assert [x for x in tensor_after_iso[1:] if "malloc" in x] == [f"malloc {nt * 896} -> 0"]
+
+
 @pytest.mark.parametrize("nt", [4, 60000])
 def test_tensor_assembly_under_capture_uses_no_memory_of_the_pattern(tmp_path, nt):
     """A captured call replays on any stream, so it neither allocates nor uses the pattern's records."""
@@ -44,7 +58,7 @@ def test_tensor_assembly_under_capture_uses_no_memory_of_the_pattern(tmp_path, n
 
 def test_tensor_assembly_without_memory_for_the_records(tmp_path):
     """A mesh whose records do not fit is assembled as before there were any; with memory, from them."""
-    none, some = run(PATTERN + "h = pattern(60000)\nrec.rec_budget(rec.rec_used())\ntensor(h, 8)\n"
+    none, some = run(PATTERN + "h = pattern(60000)\n" + ISO + "rec.rec_budget(rec.rec_used())\ntensor(h, 8)\n"
                      "rec.rec_budget(2 ** 62)\ntensor(h, 8)\n", tmp_path)
     assert none[0] == 0 and _kernels(none[1:]) == ["k_assemble"]
     assert some[0] == 0 and _kernels(some[1:]) == ["k_tet_tensor", "k_assemble_tensor_staged"]
