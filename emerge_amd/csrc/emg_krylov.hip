@@ -2877,6 +2877,9 @@ struct kept_host {
 // the posts box at 40 x 20 x 8 hexes.
 static constexpr double CYCLE_CUT = 1e-1;
 static constexpr int CYCLE_ROOM = 12;       // basis vectors worth starting another kept cycle for
+// Where the caller limits the refinements, each is to reach as far as it can be worth: to 1e-2, with room for a whole
+// restart length.
+static constexpr double LIMITED_CUT = 1e-2;
 
 // What the device knows of the kept cycles: their spans, and where the next cycle begins.  (The
 // staging is not written again before the stream has been waited for.)
@@ -3069,7 +3072,8 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
         int rc = true_resid(&rel);
         if (rc) return rc;
         int total = 0, ref = 0;
-        const int limit = max_refine > 0 ? max_refine : (1 << 30);
+        const bool limited = max_refine > 0;
+        const int limit = limited ? max_refine : (1 << 30), room = limited ? s->restart : CYCLE_ROOM;
         int stall = 0;
         kept_host kh(s->cap);
         while (rel > tol && ref < limit && total < maxiter) {
@@ -3080,7 +3084,7 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
             k_pack_vec<float><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->r, rs, reinterpret_cast<float *>(s->w));
             // A cycle stops once complex64 GMRES has reduced its residual by CYCLE_CUT (or
             // reached what tol needs), so that complex64 never has to resolve more than that.
-            const double inner_tol = std::max(0.5 * tol / rel, CYCLE_CUT);
+            const double inner_tol = std::max(0.5 * tol / rel, limited ? LIMITED_CUT : CYCLE_CUT);
             int it = 0;
             double est = 0;
             rc = gmres_cycle<float>(s, 1.0, inner_tol, maxiter - total, kh, &it, &est, st);
@@ -3109,7 +3113,7 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
             // such cycle does not: rounding of a large correction can undo its gain, which the next
             // cycles of the same space make up in a few steps (posts box at 2.2 GHz: 244 steps to 1e-9,
             // 500 when it forgot there).
-            if (it == 0 || s->cap - kh.used() < CYCLE_ROOM || (int)kh.cycles.size() == KEEP_MAX || stall >= 2) kh.cycles.clear();
+            if (it == 0 || s->cap - kh.used() < room || (int)kh.cycles.size() == KEEP_MAX || stall >= 2) kh.cycles.clear();
         }
         info->iterations = total;
         info->refinements = ref;

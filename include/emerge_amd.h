@@ -185,7 +185,9 @@ int emg_solver_spmv_tuning(emg_solver *s, int *h_lanes, float *h_ms);
  * h_ms[3]: milliseconds per launch for 4, 8, 16.  EMG_GT_LANES overrides the search.
  * No reference counterpart (its solvers are direct).                                     */
 int emg_solver_smoother_tuning(emg_solver *s, int *h_lanes, float *h_ms);
-/* d_x: initial guess in, solution out (n complex128). Synchronises `stream`. */
+/* d_x: initial guess in, solution out (n complex128). Synchronises `stream`, with nothing in flight when it
+ * returns.  max_refine: most FP64 refinements (precision 32; 0: no limit).  Each reduces the residual 10-fold, or
+ * 100-fold where they are limited, unless `restart` steps do not reach that.     */
 int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, double tol, int maxiter, int max_refine,
                      emg_solve_info *info, void *stream);
 void emg_solver_destroy(emg_solver *s);
