@@ -2358,19 +2358,24 @@ extern "C" int emg_solver_spmv_tuning(emg_solver *s, int *h_lanes, float *h_ms) 
     return 0;
 }
 
+// The planes and row flags of the caller's values and mask as they are now.
+static void pack_matrix(emg_solver *s, hipStream_t st) {
+    const unsigned gp = (unsigned)((s->n_ent * SUB + 255) / 256);
+    if (s->precision == 32)
+        k_pack_matrix<float><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, s->vals, s->mask,
+                                                 static_cast<float *>(s->kre), static_cast<float *>(s->kim), s->row_flag);
+    else
+        k_pack_matrix<double><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, s->vals, s->mask,
+                                                  static_cast<double *>(s->kre), static_cast<double *>(s->kim), s->row_flag);
+}
+
 extern "C" int emg_solver_set_matrix(emg_solver *s, const double *d_vals, const uint8_t *d_mask, void *stream) {
     EMG_CHECK(s && d_vals, "emg_solver_set_matrix: null argument");
     hipStream_t st = (hipStream_t)stream;
     s->vals = d_vals;
     s->mask = d_mask;
     k_bj_setup<<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, s->rowptr, s->cols, d_vals, d_mask, s->inv64, s->inv32);
-    const unsigned gp = (unsigned)((s->n_ent * SUB + 255) / 256);
-    if (s->precision == 32)
-        k_pack_matrix<float><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, d_vals, d_mask,
-                                                 static_cast<float *>(s->kre), static_cast<float *>(s->kim), s->row_flag);
-    else
-        k_pack_matrix<double><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, d_vals, d_mask,
-                                                  static_cast<double *>(s->kre), static_cast<double *>(s->kim), s->row_flag);
+    pack_matrix(s, st);
     if (s->np2 > 0) {
         EMG_HIP(hipMemsetAsync(s->dS, 0, s->np2 * 16, st));
         k_gdiag<<<emg::grid_for(s->n * GD, RB), RB, 0, st>>>(s->n, s->rowptr, s->cols, d_vals, d_mask, s->g_rowptr,
@@ -2456,6 +2461,7 @@ extern "C" int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0
     constexpr int PROBE_H = POLY_MAX + 2;   // POLY_MAX + 1 norms
     static_assert(PROBE_H % 2 == 0 && PROBE_H + 4 * POLY_MAX * (POLY_MAX + 1) <= 4 * 2 * 512, "the probe's results fit s->h");
     double *norms = s->h, *coef = s->h + PROBE_H;
+    if (s->precision == 64) pack_matrix(s, st);   // the caller's values as they are now, as in a solve
     const int ldc = 2 * (d + 1);
     EMG_HIP(hipMemcpyAsync(V, d_v0, n * 16, hipMemcpyDeviceToDevice, st));
     k_norm2<double><<<nb, RB, 0, st>>>(n, V, s->partial);
@@ -3056,6 +3062,9 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
     double rel;
     if (s->precision == 64) {
         int it;
+        // K and the residual are the caller's values as they are now, the preconditioner the last
+        // emg_solver_set_matrix's (1 - 2 products' time)
+        pack_matrix(s, st);
         k_pack_vec<double><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, d_b, 1.0, s->r);
         k_pack_vec<double><<<emg::grid_for(s->n_ent, RB), RB, 0, st>>>(s->n_ent, d_x, 1.0, s->d);
         int rc = gmres_full(s, s->r, s->d, tol, maxiter, &it, st);
@@ -3170,9 +3179,9 @@ extern "C" int emg_spmv_blocked(int64_t n, int64_t nnz, const int32_t *d_rowptr,
     return 0;
 }
 
-// The product the solver's Arnoldi steps run: y = mask.(K (mask.x)) with the matrix of the last
-// emg_solver_set_matrix, complex128 (precision 64) or the complex64 copy (precision 32, x and y
-// complex64), PEC columns folded into that copy.
+// y = mask.(K (mask.x)) with the matrix of the last emg_solver_set_matrix, complex128 (precision 64) or the
+// complex64 copy (precision 32, x and y complex64), PEC columns folded into that copy; x and y in the caller's
+// layout (k_spmv_pk's STD form, STD_LANES lanes per entity).
 extern "C" int emg_solver_apply(emg_solver *s, int precision, const void *d_x, void *d_y, void *stream) {
     EMG_CHECK(s != nullptr && d_x && d_y, "emg_solver_apply: null argument");
     EMG_CHECK(s->vals != nullptr, "emg_solver_apply: no matrix set");

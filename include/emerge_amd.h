@@ -130,7 +130,10 @@ typedef struct {
 int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr, const int32_t *d_cols, int restart,
                       int precision, emg_solver **out);
 /* K values (nnz complex128, caller-owned, must outlive the solves) and the
- * free-DOF mask (n uint8, 1 = solve, 0 = PEC; NULL = all free). */
+ * free-DOF mask (n uint8, 1 = solve, 0 = PEC; NULL = all free).  The solver
+ * keeps copies in its own layout: the preconditioner, the complex64 steps of
+ * precision 32 and emg_solver_apply are of the values at this call.  A solve's
+ * residual, and the steps of precision 64, take the values as they are then. */
 int emg_solver_set_matrix(emg_solver *s, const double *d_vals, const uint8_t *d_mask, void *stream);
 /* Gradient correction of the smoother (no counterpart in the reference, whose
  * direct solvers need none): G (n x np2, CSR, at most 8 entries per row) maps
@@ -164,10 +167,11 @@ int emg_solver_set_poly(emg_solver *s, int degree, const double *h_coef);
  * the (d + 1) x d Hessenberg matrix column-major as complex128.  Uses the
  * solver's Krylov storage: not during a solve.  Synchronises `stream`.       */
 int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0, double *h_out, void *stream);
-/* y = mask.(K (mask.x)) as the solver's Arnoldi steps form it, with the matrix of
- * the last emg_solver_set_matrix: precision 64 complex128, precision 32 the
- * solver's complex64 copy (x, y complex64).  No counterpart in the reference
- * (scipy's CSR product inside its solvers); exported to time the product. */
+/* y = mask.(K (mask.x)) with the matrix of the last emg_solver_set_matrix from the
+ * solver's packed copy: precision 64 complex128 (of a precision-32 solver the caller's
+ * CSR values), precision 32 complex64 (x, y complex64); vectors in the caller's layout,
+ * where the Arnoldi steps hold the two modes of an entity side by side.  No counterpart
+ * in the reference (scipy's CSR product inside its solvers).                     */
 int emg_solver_apply(emg_solver *s, int precision, const void *d_x, void *d_y, void *stream);
 
 /* The solver's autotuned SpMV shape: on its first emg_solver_set_matrix the solver times
