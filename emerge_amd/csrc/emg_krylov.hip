@@ -1782,7 +1782,7 @@ struct emg_solver {
     double *inv64 = nullptr;
     float *inv32 = nullptr;
     double *V = nullptr;            // cap + 1 basis vectors, element type per precision
-    double *w = nullptr, *z = nullptr, *r = nullptr, *d = nullptr;
+    double *w = nullptr, *z = nullptr, *r = nullptr, *d = nullptr;   // d: precision 64 only
     double *partial = nullptr, *h = nullptr, *nrm = nullptr;
     int nblk = 0;
     // Arnoldi steps run from captured HIP graphs (chunks of CHUNK_IT steps)
@@ -1819,7 +1819,7 @@ struct emg_solver {
     // M p(K M) with 1 - z p(z) = prod_i (1 - z c_i), c_i = 1/theta_i on the device
     int poly_deg = 1;
     double *poly_c = nullptr;                               // POLY_MAX complex coefficients
-    double *pp = nullptr, *pt = nullptr, *py = nullptr, *pu = nullptr;   // work vectors (n complex each)
+    double *pp = nullptr, *py = nullptr, *pu = nullptr;   // work vectors (n complex each)
     // blocked-SpMV lanes per entity, [0] complex128, [1] complex64: 0 until tuned on
     // the first matrix (tune_spmv), with the measured milliseconds per variant
     int lanes[2] = {0, 0};
@@ -1856,15 +1856,27 @@ static void drop_fused(emg_solver *s) {
     s->fused = false;
 }
 
+template <typename... T>
+static void drop(T *&...p) {   // frees device buffers and forgets them
+    ((void)hipFree(p), ...);
+    ((p = nullptr), ...);
+}
+static void drop_gradient(emg_solver *s) {
+    drop(s->g_pcol, s->g_pval, s->gt_prp, s->gt_pcol, s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32);
+    drop_fused(s);
+}
+static void drop_local(emg_solver *s) { drop(s->loc_ptr, s->loc_col, s->loc_idx); }
+static void drop_buffers(emg_solver *s) {   // what emg_solver_create allocates
+    drop(s->acol, s->kre, s->kim, s->row_flag, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial, s->h, s->nrm, s->arn,
+         s->pn, s->gram, s->flag, s->poly_c, s->pp, s->py, s->pu);
+    drop_local(s);
+}
+
 static void free_solver(emg_solver *s) {
     if (!s) return;
     drop_graphs(s);
-    drop_fused(s);
-    void *ps[] = {s->acol, s->kre, s->kim, s->row_flag, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial,
-                  s->h, s->nrm, s->arn, s->pn, s->gram, s->flag, s->g_pcol, s->gt_prp, s->gt_pcol, s->g_pval,
-                  s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32, s->poly_c, s->pp, s->pt, s->py, s->pu, s->loc_ptr,
-                  s->loc_col, s->loc_idx};
-    for (void *p : ps) (void)hipFree(p);
+    drop_gradient(s);
+    drop_buffers(s);
     if (s->host) (void)hipHostFree(s->host);
     if (s->cap_stream) (void)hipStreamDestroy(s->cap_stream);
     delete s;
@@ -2058,6 +2070,19 @@ __global__ void __launch_bounds__(256) k_check_entity_pattern(int64_t ne, int64_
     }
 }
 
+// Device memory; NO_MEMORY where there is none, for callers that can do with less (the C entries return -2).
+static constexpr int NO_MEMORY = -4;
+template <typename T>
+static int device_alloc(T **p, size_t bytes) {
+    const hipError_t e = hipMalloc((void **)p, bytes);
+    if (e == hipSuccess) return 0;
+    *p = nullptr;
+    emg::set_error(std::string("emg_solver: hipMalloc: ") + hipGetErrorString(e));
+    if (e != hipErrorOutOfMemory) return -2;
+    (void)hipGetLastError();
+    return NO_MEMORY;
+}
+
 // off[i] = sum of cnt[0 .. i) for i <= n, through the host (once per solver or gradient)
 static int prefix_on_host(const int32_t *d_cnt, int64_t n, int32_t **d_off, int64_t *total, hipStream_t st) {
     std::vector<int32_t> c(n), o(n + 1, 0);
@@ -2069,7 +2094,7 @@ static int prefix_on_host(const int32_t *d_cnt, int64_t n, int32_t **d_off, int6
         EMG_CHECK(t < ((int64_t)1 << 31), "emg_solver: too many entries");
         o[i + 1] = (int32_t)t;
     }
-    EMG_HIP(hipMalloc((void **)d_off, (n + 1) * sizeof(int32_t)));
+    if (int rc = device_alloc(d_off, (n + 1) * sizeof(int32_t))) return rc;
     EMG_HIP(hipMemcpyAsync(*d_off, o.data(), (n + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
     EMG_HIP(hipStreamSynchronize(st));
     *total = t;
@@ -2082,40 +2107,78 @@ static int prefix_on_host(const int32_t *d_cnt, int64_t n, int32_t **d_off, int6
 // step at 60,000 DOFs 134 -> 140 us, at 250,000 257 -> 255; above it see k_spmv_pk.  EMG_LOCAL_COLUMNS overrides (0: never,
 // else wherever the rows fit).
 static constexpr int64_t LOC_MIN_N = 400000;
+static int fill_local(emg_solver *s, int32_t *cnt, int64_t nb) {
+    int *d_over = reinterpret_cast<int *>(s->flag), over = 0;
+    int64_t total = 0;
+    EMG_HIP(hipMemset(d_over, 0, sizeof(int)));
+    k_loc_columns<<<(unsigned)nb, 512>>>(s->n_ent, s->rowptr, s->acol, nullptr, cnt, nullptr, nullptr, d_over);
+    EMG_LAUNCH_CHECK();
+    EMG_HIP(hipMemcpy(&over, d_over, sizeof(int), hipMemcpyDeviceToHost));
+    if (over) return 0;
+    if (int rc = prefix_on_host(cnt, nb, &s->loc_ptr, &total, nullptr)) return rc;
+    if (int rc = device_alloc(&s->loc_col, std::max<int64_t>(total, 1) * sizeof(int32_t))) return rc;
+    if (int rc = device_alloc(&s->loc_idx, s->nnz / 4 * sizeof(uint16_t))) return rc;
+    k_loc_columns<<<(unsigned)nb, 512>>>(s->n_ent, s->rowptr, s->acol, s->loc_ptr, nullptr, s->loc_col, s->loc_idx, d_over);
+    EMG_LAUNCH_CHECK();
+    EMG_HIP(hipStreamSynchronize(nullptr));
+    return 0;
+}
 // The tables of the LOC form, or none where a workgroup's rows exceed it or the memory does not suffice.
 static int local_columns(emg_solver *s) {
     const char *env = getenv("EMG_LOCAL_COLUMNS");
     if (env != nullptr ? atoi(env) == 0 : s->n < LOC_MIN_N) return 0;
     const int64_t nb = (s->n_ent + LOC_ROWS - 1) / LOC_ROWS;
     int32_t *cnt = nullptr;
-    int *d_over = reinterpret_cast<int *>(s->flag), over = 0;
-    int64_t total = 0;
-    EMG_HIP(hipMalloc((void **)&cnt, nb * sizeof(int32_t)));
-    hipError_t e = hipMemset(d_over, 0, sizeof(int));
-    if (e == hipSuccess) {
-        k_loc_columns<<<(unsigned)nb, 512>>>(s->n_ent, s->rowptr, s->acol, nullptr, cnt, nullptr, nullptr, d_over);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpy(&over, d_over, sizeof(int), hipMemcpyDeviceToHost);
-    const int rc = e != hipSuccess || over ? 0 : prefix_on_host(cnt, nb, &s->loc_ptr, &total, nullptr);
+    int rc = device_alloc(&cnt, nb * sizeof(int32_t));
+    if (rc == 0) rc = fill_local(s, cnt, nb);
     (void)hipFree(cnt);
-    EMG_HIP(e);
-    if (over || rc) return rc;
-    e = hipMalloc((void **)&s->loc_col, std::max<int64_t>(total, 1) * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&s->loc_idx, s->nnz / 4 * sizeof(uint16_t));
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        void *ps[] = {s->loc_ptr, s->loc_col, s->loc_idx};
-        for (void *p : ps) (void)hipFree(p);
-        s->loc_ptr = s->loc_col = nullptr;
-        s->loc_idx = nullptr;
-        return 0;
+    if (rc != 0) drop_local(s);
+    return rc == NO_MEMORY ? 0 : rc;
+}
+
+// The solver's device buffers for a basis of s->cap + 1 vectors.
+static int allocate(emg_solver *s) {
+    const int64_t n = s->n, nnz = s->nnz;
+    const bool c64 = s->precision == 32;
+    const size_t es = c64 ? 8 : 16;   // bytes per complex element of the basis
+    const int ntile = (s->cap + 1 + DT - 1) / DT;
+    int rc = 0;
+    auto A = [&](auto **p, size_t bytes) { if (rc == 0) rc = device_alloc(p, bytes); };
+    A(&s->V, (size_t)(s->cap + 1) * n * es);
+    A(&s->w, n * 16); A(&s->z, n * 16); A(&s->r, n * 16);
+    if (!c64) A(&s->d, n * 16);
+    A(&s->partial, ((size_t)2 * ntile * 1024 * DT * 2 + 1024) * sizeof(double));
+    A(&s->gram, (size_t)(s->cap + 1) * (s->cap + 1) * 16);
+    A(&s->h, 4 * 2 * 512 * sizeof(double));   // dots | corrected | the part subtracted | y
+    A(&s->nrm, 4 * sizeof(double));
+    A(&s->inv64, s->n_ent * 4 * 16);
+    A(&s->arn, arn_off(s->cap).total * sizeof(double));
+    A(&s->pn, 1024 * sizeof(double));
+    A(&s->flag, 8 * sizeof(double));
+    if (c64) A(&s->inv32, s->n_ent * 4 * 8);
+    A(&s->acol, (size_t)nnz / 4 * sizeof(int32_t));
+    A(&s->kre, (size_t)nnz * es / 2);
+    A(&s->kim, (size_t)nnz * es / 2);
+    A(&s->row_flag, s->n_ent);
+    A(&s->poly_c, 2 * POLY_MAX * sizeof(double));
+    A(&s->pp, n * 16); A(&s->py, n * 16); A(&s->pu, n * 16);
+    if (rc == 0) s->kept = reinterpret_cast<kept_dev *>(s->arn + arn_off(s->cap).kept);
+    return rc;
+}
+
+// Gives back what a solver of a full card can do without: the tables of the LOC form and the longer half of a
+// complex64 basis.  False where there is nothing of the kind.  Not during a solve.
+static bool give_back(emg_solver *s) {
+    const bool any = s->loc_ptr != nullptr || s->cap > s->restart;
+    drop_graphs(s);
+    drop_local(s);
+    if (s->cap > s->restart) {
+        s->cap = s->restart;
+        s->kept = reinterpret_cast<kept_dev *>(s->arn + arn_off(s->cap).kept);
+        drop(s->V);
+        if (device_alloc(&s->V, (size_t)(s->cap + 1) * s->n * 8) != 0) return false;
     }
-    EMG_HIP(e);
-    k_loc_columns<<<(unsigned)nb, 512>>>(s->n_ent, s->rowptr, s->acol, s->loc_ptr, nullptr, s->loc_col, s->loc_idx, d_over);
-    EMG_LAUNCH_CHECK();
-    EMG_HIP(hipStreamSynchronize(nullptr));
-    return 0;
+    return any;
 }
 
 extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr, const int32_t *d_cols, int restart,
@@ -2127,50 +2190,32 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
     auto s = new emg_solver();
     s->n = n; s->nnz = nnz; s->n_ent = n / 2; s->restart = restart; s->precision = precision;
     s->rowptr = d_rowptr; s->cols = d_cols;
-    const size_t es = precision == 64 ? 16 : 8;   // bytes per complex element of the basis
     s->nblk = (int)std::min<int64_t>((n / 2 * maxpy_split(n) + RB - 1) / RB, 1024);
-    hipError_t e = hipSuccess;
-    auto A = [&](void **p, size_t bytes) { if (e == hipSuccess) e = hipMalloc(p, bytes); };
-    // complex64 refinement cycles keep up to two restart lengths of basis vectors (gmres_cycle), the
-    // bytes of the complex128 basis of one; where that does not fit, one
-    s->cap = precision == 32 ? std::min(2 * restart, 500) : restart;
-    A((void **)&s->V, (size_t)(s->cap + 1) * n * es);
-    if (e == hipErrorOutOfMemory && s->cap > restart) {
-        (void)hipGetLastError();
-        e = hipSuccess;
-        s->cap = restart;
-        A((void **)&s->V, (size_t)(s->cap + 1) * n * es);
-    }
-    const int ntile = (s->cap + 1 + DT - 1) / DT;
-    A((void **)&s->w, n * 16); A((void **)&s->z, n * 16); A((void **)&s->r, n * 16); A((void **)&s->d, n * 16);
-    A((void **)&s->partial, ((size_t)2 * ntile * 1024 * DT * 2 + 1024) * sizeof(double));
-    A((void **)&s->gram, (size_t)(s->cap + 1) * (s->cap + 1) * 16);
-    A((void **)&s->h, 4 * 2 * 512 * sizeof(double));   // dots | corrected | the part subtracted | y
-    A((void **)&s->nrm, 4 * sizeof(double));
-    A((void **)&s->inv64, s->n_ent * 4 * 16);
-    A((void **)&s->arn, arn_off(s->cap).total * sizeof(double));
-    A((void **)&s->pn, 1024 * sizeof(double));
-    A((void **)&s->flag, 8 * sizeof(double));
-    if (e == hipSuccess) e = hipHostMalloc((void **)&s->host, host_off(s->cap).total * sizeof(double), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->cap_stream, hipStreamNonBlocking);
-    if (precision == 32) A((void **)&s->inv32, s->n_ent * 4 * 8);
-    A((void **)&s->acol, (size_t)(nnz > 0 ? nnz : 4) / 4 * sizeof(int32_t));
-    A(&s->kre, (size_t)nnz * es / 2);
-    A(&s->kim, (size_t)nnz * es / 2);
-    A((void **)&s->row_flag, s->n_ent);
-    if (e == hipSuccess) s->kept = reinterpret_cast<kept_dev *>(s->arn + arn_off(s->cap).kept);
-    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&s->host_dev, s->host, 0);
-    A((void **)&s->poly_c, 2 * POLY_MAX * sizeof(double));
-    A((void **)&s->pp, n * 16); A((void **)&s->pt, n * 16); A((void **)&s->py, n * 16); A((void **)&s->pu, n * 16);
-    if (e != hipSuccess) {
-        emg::set_error(std::string("emg_solver_create: ") + hipGetErrorString(e));
+    // the blocked SpMV and the 2x2 block smoother need an entity pattern: check it once
+    auto refuse = [&](const char *what, hipError_t e) {
+        emg::set_error(std::string("emg_solver_create: ") + what + hipGetErrorString(e));
         free_solver(s);
         return -2;
-    }
-    // the blocked SpMV and the 2x2 block smoother need an entity pattern: check it once
-    int bad = 0;
-    if (nnz <= 0 || nnz >= ((int64_t)1 << 31)) bad = 1;
+    };
+    int bad = nnz <= 0 || nnz >= ((int64_t)1 << 31);
     if (!bad) {
+        // complex64 refinement cycles keep up to two restart lengths of basis vectors (gmres_cycle), the
+        // bytes of the complex128 basis of one; where the card does not hold everything then, one
+        s->cap = precision == 32 ? std::min(2 * restart, 500) : restart;
+        int rc = allocate(s);
+        if (rc == NO_MEMORY && s->cap > restart) {
+            drop_buffers(s);
+            s->cap = restart;
+            rc = allocate(s);
+        }
+        if (rc != 0) {
+            free_solver(s);
+            return -2;
+        }
+        hipError_t e = hipHostMalloc((void **)&s->host, host_off(s->cap).total * sizeof(double), hipHostMallocDefault);
+        if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&s->host_dev, s->host, 0);
+        if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->cap_stream, hipStreamNonBlocking);
+        if (e != hipSuccess) return refuse("", e);
         int *d_bad = reinterpret_cast<int *>(s->flag);
         e = hipMemset(d_bad, 0, sizeof(int));
         if (e == hipSuccess) {
@@ -2178,11 +2223,7 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipMemcpy(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) {
-            emg::set_error(std::string("emg_solver_create: pattern check: ") + hipGetErrorString(e));
-            free_solver(s);
-            return -2;
-        }
+        if (e != hipSuccess) return refuse("pattern check: ", e);
     }
     if (bad) {
         emg::set_error("emg_solver_create: the CSR is not on an entity pattern (emg_pattern_csr layout: rows e and "
@@ -2192,13 +2233,9 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
         return -1;
     }
     k_pack_cols<<<(unsigned)((s->n_ent * SUB + 255) / 256), 256>>>(s->n_ent, d_rowptr, d_cols, s->acol);
-    e = hipGetLastError();
+    hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-    if (e != hipSuccess) {
-        emg::set_error(std::string("emg_solver_create: packing the pattern: ") + hipGetErrorString(e));
-        free_solver(s);
-        return -2;
-    }
+    if (e != hipSuccess) return refuse("packing the pattern: ", e);
     if (int rc = local_columns(s)) {
         free_solver(s);
         return rc;
@@ -2448,6 +2485,7 @@ extern "C" int emg_solver_set_poly(emg_solver *s, int degree, const double *h_co
 extern "C" int emg_solver_arnoldi_probe(emg_solver *s, int d, const double *d_v0, double *h_out, void *stream) {
     EMG_CHECK(s && d_v0 && h_out, "emg_solver_arnoldi_probe: null argument");
     EMG_CHECK(s->vals != nullptr, "emg_solver_arnoldi_probe: emg_solver_set_matrix was not called");
+    EMG_CHECK(s->V != nullptr, "emg_solver_arnoldi_probe: no memory for the basis");
     const int64_t n = s->n;
     const size_t es = s->precision == 64 ? 16 : 8;
     EMG_CHECK(d >= 1 && d <= POLY_MAX && (size_t)(d + 1) * 16 <= (size_t)(s->restart + 1) * es,
@@ -2515,14 +2553,14 @@ static int pack_gradient(emg_solver *s, int64_t np2, const int32_t *grp, const i
         if (c < ns) before_max = std::max(before_max, wd[c]);
     }
     const int64_t slots = std::max<int64_t>(s->g_sh.first(ns), 1);
-    EMG_HIP(hipMalloc((void **)&s->g_pcol, slots * sizeof(int32_t)));
-    EMG_HIP(hipMalloc(&s->g_pval, slots * 2 * sizeof(R)));
+    if (int rc = device_alloc(&s->g_pcol, slots * sizeof(int32_t))) return rc;
+    if (int rc = device_alloc(&s->g_pval, slots * 2 * sizeof(R))) return rc;
     k_g_fill<R><<<(unsigned)ns, 64, 0, st>>>(ne, grp, gcol, gv, s->g_sh, s->g_pcol, static_cast<R *>(s->g_pval));
     k_gt_count<<<emg::grid_for(np2, RB), RB, 0, st>>>(np2, ne, tp, tcol, cnt);
     EMG_LAUNCH_CHECK();
     if (int rc = prefix_on_host(cnt, np2, &s->gt_prp, &total, st)) return rc;
-    EMG_HIP(hipMalloc((void **)&s->gt_pcol, std::max<int64_t>(total, 1) * sizeof(int32_t)));
-    EMG_HIP(hipMalloc(&s->gt_pval, std::max<int64_t>(total, 1) * 2 * sizeof(R)));
+    if (int rc = device_alloc(&s->gt_pcol, std::max<int64_t>(total, 1) * sizeof(int32_t))) return rc;
+    if (int rc = device_alloc(&s->gt_pval, std::max<int64_t>(total, 1) * 2 * sizeof(R))) return rc;
     k_gt_fill<R><<<emg::grid_for(np2, RB), RB, 0, st>>>(np2, ne, tp, tcol, tv, s->gt_prp, s->gt_pcol,
                                                         static_cast<R *>(s->gt_pval));
     EMG_LAUNCH_CHECK();
@@ -2540,12 +2578,14 @@ static int fuse_rows(int64_t rows, const GEN &gen, int32_t *cnt, int *d_over, in
     int over = 0;
     EMG_HIP(hipMemcpyAsync(&over, d_over, sizeof(int), hipMemcpyDeviceToHost, st));
     int64_t total = 0;
-    if (int rc = prefix_on_host(cnt, rows, ptr, &total, st)) return rc;
-    if (over || total == 0) { *fits = false; return 0; }   // the steps read slot 0 in place of none
-    hipError_t e = hipMalloc((void **)col, total * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(val, total * bytes);
-    if (e == hipErrorOutOfMemory) { (void)hipGetLastError(); *fits = false; return 0; }
-    EMG_HIP(e);
+    EMG_HIP(hipStreamSynchronize(st));
+    if (over) { *fits = false; return 0; }
+    int rc = prefix_on_host(cnt, rows, ptr, &total, st);
+    if (rc == 0 && total > 0) rc = device_alloc(col, total * sizeof(int32_t));
+    if (rc == 0 && total > 0) rc = device_alloc(val, total * bytes);
+    // too many entries, no memory, or none (the steps read slot 0 in place of a missing one)
+    if (rc == -1 || rc == NO_MEMORY || (rc == 0 && total == 0)) { *fits = false; return 0; }
+    if (rc != 0) return rc;
     k_distinct<<<(unsigned)rows, 256, 0, st>>>(gen, nullptr, *ptr, *col, d_over);
     EMG_LAUNCH_CHECK();
     return 0;
@@ -2563,9 +2603,9 @@ static int fuse_pattern(emg_solver *s, int64_t np2, const int32_t *grp, const in
         rc = fuse_rows(np2, gen_of_nodes{s->n_ent, trp, tcol, s->kg_ptr, s->kg_col, 0}, cnt, d_over, &s->hg_ptr, &s->hg_col, &s->hg_val,
                        8, &fits, st);
     if (rc == 0 && fits) {
-        hipError_t e = hipMalloc((void **)&s->fuse_s, (size_t)np2 * 32);
-        if (e == hipSuccess) e = hipMalloc((void **)&s->fuse_t, (size_t)np2 * 16);
-        if (e != hipSuccess) { (void)hipGetLastError(); fits = false; }
+        rc = device_alloc(&s->fuse_s, (size_t)np2 * 32);
+        if (rc == 0) rc = device_alloc(&s->fuse_t, (size_t)np2 * 16);
+        if (rc == NO_MEMORY) { rc = 0; fits = false; }
     }
     if (rc == 0 && fits) s->fused = true;
     if (rc != 0 || !fits) {
@@ -2608,23 +2648,18 @@ extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t
     // captured step graphs hold the old gradient buffers: drop them before the buffers go
     EMG_HIP(hipStreamSynchronize(st));
     drop_graphs(s);
-    void *old[] = {s->g_pcol, s->g_pval, s->gt_prp, s->gt_pcol, s->gt_pval, s->dS, s->dsinv64, s->tg, s->dsinv32};
-    for (void *p : old) (void)hipFree(p);
-    drop_fused(s);
-    s->g_pcol = s->gt_prp = s->gt_pcol = nullptr;
-    s->g_pval = s->gt_pval = nullptr;
-    s->dS = s->dsinv64 = s->tg = nullptr;
-    s->dsinv32 = nullptr;
-    s->np2 = 0;
-    EMG_HIP(hipMalloc((void **)&s->dS, (size_t)np2 * 16));
-    EMG_HIP(hipMalloc((void **)&s->dsinv64, (size_t)np2 * 16));
-    EMG_HIP(hipMalloc((void **)&s->dsinv32, (size_t)np2 * 8));
-    EMG_HIP(hipMalloc((void **)&s->tg, (size_t)np2 * 16));
-    {
-        int32_t *cnt = nullptr;
+    auto make = [&]() {
+        drop_gradient(s);
+        s->np2 = 0;
         const bool fuse = fuse_wanted(s);
-        EMG_HIP(hipMalloc((void **)&cnt, std::max<int64_t>(np2, fuse ? s->n_ent : s->n_ent / 64 + 1) * sizeof(int32_t)));
-        int rc = s->precision == 32 ? pack_gradient<float>(s, np2, d_g_rowptr, d_g_cols, d_g_vals, d_gt_rowptr, d_gt_cols,
+        int32_t *cnt = nullptr;
+        int rc = device_alloc(&s->dS, (size_t)np2 * 16);
+        if (rc == 0) rc = device_alloc(&s->dsinv64, (size_t)np2 * 16);
+        if (rc == 0) rc = device_alloc(&s->dsinv32, (size_t)np2 * 8);
+        if (rc == 0) rc = device_alloc(&s->tg, (size_t)np2 * 16);
+        if (rc == 0) rc = device_alloc(&cnt, std::max<int64_t>(np2, fuse ? s->n_ent : s->n_ent / 64 + 1) * sizeof(int32_t));
+        if (rc == 0)
+            rc = s->precision == 32 ? pack_gradient<float>(s, np2, d_g_rowptr, d_g_cols, d_g_vals, d_gt_rowptr, d_gt_cols,
                                                            d_gt_vals, cnt, st)
                                     : pack_gradient<double>(s, np2, d_g_rowptr, d_g_cols, d_g_vals, d_gt_rowptr, d_gt_cols,
                                                             d_gt_vals, cnt, st);
@@ -2633,7 +2668,11 @@ extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t
         (void)hipFree(cnt);
         if (rc) return rc;
         EMG_HIP(e);
-    }
+        return 0;
+    };
+    int rc = make();
+    if (rc == NO_MEMORY && give_back(s)) rc = make();
+    if (rc != 0) return rc == NO_MEMORY ? -2 : rc;
     s->g_rowptr = d_g_rowptr; s->g_cols = d_g_cols; s->g_vals = d_g_vals;
     s->gt_rowptr = d_gt_rowptr; s->gt_cols = d_gt_cols; s->gt_vals = d_gt_vals;
     s->np2 = np2;
@@ -3046,6 +3085,7 @@ extern "C" int emg_solver_solve(emg_solver *s, const double *d_b, double *d_x, d
                                 emg_solve_info *info, void *stream) {
     EMG_CHECK(s && d_b && d_x && info, "emg_solver_solve: null argument");
     EMG_CHECK(s->vals != nullptr, "emg_solver_solve: emg_solver_set_matrix was not called");
+    EMG_CHECK(s->V != nullptr, "emg_solver_solve: no memory for the basis");
     hipStream_t st = (hipStream_t)stream;
     memset(info, 0, sizeof(*info));
     double bn = -1.0;   // ||b||, formed with the first residual

@@ -88,3 +88,46 @@ rec.rec_clear()
 out([L.emg_solver_solve(s, at(v), at(x), 1e-8, 100, 0, ctypes.byref(info), P(9))] + log())
 """, tmp_path)
     assert lines[0] == 0 and lines[-1] == "wait stream 9"
+
+
+@pytest.mark.parametrize("local", ["0", "1"])
+def test_a_complex64_solver_is_made_wherever_one_restart_length_fits(tmp_path, local):
+    """The second restart length of the basis and the tables of the products that gather locally are taken where the
+    card has room, whichever buffer the memory ends at; what is needed without them is found by halving."""
+    tries, least, most = run(SOLVER + """
+def fits(budget):
+    rec.rec_budget(budget)
+    rc, s = solver(32, n=2000, restart=50)
+    used = rec.rec_used()
+    if rc == 0:
+        L.emg_solver_destroy(s)
+    assert rec.rec_used() == 0
+    return rc == 0, used
+most = fits(2 ** 62)[1]
+lo, hi = 0, most
+while hi - lo > 1:
+    mid = (lo + hi) // 2
+    lo, hi = (lo, mid) if fits(mid)[0] else (mid, hi)
+out([fits(b)[0] for b in np.linspace(hi, most, 400).astype(int).tolist()])
+out([hi])
+out([most])
+""", tmp_path, env={"EMG_LOCAL_COLUMNS": local})
+    assert all(tries)
+    assert most[0] - least[0] >= 50 * 2000 * 8          # a restart length of vectors
+
+
+def test_a_gradient_that_does_not_fit_gets_the_basis_second_half(tmp_path):
+    """emg_solver_set_gradient on a full card: the longer half of a complex64 basis makes room."""
+    (rc,) = run(SOLVER + """
+n, np2 = 2000, 300
+rc, s = solver(32, n=n, restart=50)
+gp, tp = np.zeros(n + 1, np.int32), np.zeros(np2 + 1, np.int32)
+gp[n] = tp[np2] = 900
+c = np.zeros(900, np.int32)
+g = np.zeros(900)
+rec.rec_budget(rec.rec_used())
+out([rc, L.emg_solver_set_gradient(s, np2, at(gp), at(c), at(g), at(tp), at(c), at(g), P(9)),
+     L.emg_solver_set_matrix(s, at(v.repeat(20)), None, P(9)),
+     L.emg_solver_solve(s, at(v), at(x), 1e-8, 100, 0, ctypes.byref(info), P(9))])
+""", tmp_path, env={"EMG_FUSED_STEPS": "0"})
+    assert rc == [0, 0, 0, 0]
