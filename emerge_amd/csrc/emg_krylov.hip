@@ -888,6 +888,12 @@ __device__ __forceinline__ unsigned xcd_run(unsigned b, unsigned n) {
     return i / XCD_RUN * (8 * XCD_RUN) + (b % 8) * XCD_RUN + i % XCD_RUN;
 }
 
+// The flags of rows whose values stay in the caller's CSR.
+__global__ void __launch_bounds__(256) k_row_flags(int64_t ne, const uint8_t *__restrict__ mask, uint8_t *__restrict__ flag) {
+    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (e < ne) flag[e] = (uint8_t)((mask == nullptr || mask[e] ? ROW0 : 0) | (mask == nullptr || mask[ne + e] ? ROW1 : 0) | ROW_CPLX);
+}
+
 // What follows a product v = K x in the same launch:
 //   SP_Y: y = v;   SP_RESID: y = b - v;
 //   SP_POLY: p = q - c_i v, y = (i == 0 ? c_0 q : y) + c_{i+1} p (apply_prec_poly; q scaled by *qs)
@@ -915,15 +921,18 @@ struct sp_args {
 // rows: 96, 66, 85; 113, 65, 86; 93, 65, 74; 2, 3 or 6 blocks in flight per lane: 95, 69, 73; 96, 68, 73; 93, 63, 89.)
 static constexpr int LOC_ROWS = 64, LOC_L = 4, LOC_MAX = 1024, LOC_CAND = 8192;
 static constexpr int LOC_LANES = LOC_ROWS * LOC_L;
+// CSR: the caller's columns and complex128 values in place of acol and kre (kim unused), for solvers without a packed
+// copy; `half` as in k_spmv_blk.
 struct loc_tab {
     const int32_t *ptr, *col;
     const uint16_t *idx;
 };
-template <typename R, int L, int EP, bool STD, bool LOC>
+template <typename R, int L, int EP, bool STD, bool LOC, bool CSR = false>
 __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, const int32_t *__restrict__ rowptr,
                                                  const int32_t *__restrict__ acol, const R *__restrict__ kre,
                                                  const R *__restrict__ kim, const uint8_t *__restrict__ flag,
-                                                 const R *__restrict__ x, sp_args<R> a, loc_tab loc) {
+                                                 const R *__restrict__ x, sp_args<R> a, loc_tab loc, int64_t half) {
+    static_assert(!CSR || (sizeof(R) == 8 && !STD && !LOC), "the caller's CSR serves complex128 steps");
     constexpr int U = L <= 4 ? 4 : L == 8 ? 3 : L == 16 ? 2 : 1;
     __shared__ __align__(16) R xs[LOC ? 4 * LOC_MAX : 4];
     const int64_t blk = xcd_run(blockIdx.x, gridDim.x);
@@ -950,6 +959,15 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
     if (e >= ne) return;
     const uint8_t fl = flag[e];
     const int32_t p0 = rowptr[e] >> 1, p1 = rowptr[e + 1] >> 1;
+    // real or imaginary parts of block q
+    auto block = [&](const R *plane, int32_t q, int im) {
+        if constexpr (CSR) {
+            const int64_t i = 2 * ((int64_t)p0 + q) + im, d = 2 * (p1 - p0);
+            return cx2<R>{kre[i], kre[i + d], kre[i + 2 * half], kre[i + 2 * half + d]};
+        } else {
+            return ld2(plane, q);
+        }
+    };
     cx2<R> own{}, qv{}, yv{};
     // the epilogue's operands, asked for before the row
     if (lane == 0) {
@@ -974,12 +992,17 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int32_t q = p + u * L < p1 ? p + u * L : p;   // past the row's end: its own entry again, not used
-                c[u] = LOC ? loc.idx[q] : acol[q];
-                k[u] = ld2(kre, q);
+                c[u] = LOC ? loc.idx[q] : acol[CSR ? p0 + q : q];
+                k[u] = block(kre, q, 0);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                if constexpr (LOC) {
+                if constexpr (CSR) {
+                    const uint8_t cf = flag[c[u]];   // the caller's values hold the PEC columns too
+                    xv[u] = ld2(x, c[u]);
+                    if (!(cf & ROW0)) xv[u].ar = xv[u].ai = 0;
+                    if (!(cf & ROW1)) xv[u].br = xv[u].bi = 0;
+                } else if constexpr (LOC) {
                     xv[u] = ld2(xs, c[u]);
                 } else if constexpr (STD) {
                     cx<R> u0 = ld(x, c[u]), u1 = ld(x, ne + c[u]);
@@ -1002,7 +1025,7 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
                               k[u].br * xv[u].ar + k[u].bi * xv[u].br, k[u].br * xv[u].ai + k[u].bi * xv[u].bi};
             if (fl & ROW_CPLX) {
 #pragma unroll
-                for (int u = 0; u < U; u++) k[u] = ld2(kim, p + u * L < p1 ? p + u * L : p);
+                for (int u = 0; u < U; u++) k[u] = block(kim, p + u * L < p1 ? p + u * L : p, 1);
 #pragma unroll
                 for (int u = 0; u < U; u++) {
                     v[u].ar -= k[u].ar * xv[u].ai + k[u].ai * xv[u].bi;
@@ -1062,17 +1085,23 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
 
 template <typename R, int EP, bool STD>
 static void launch_spmv_pk(hipStream_t st, int L, int64_t ne, const int32_t *rowptr, const int32_t *acol, const R *kre,
-                           const R *kim, const uint8_t *flag, const R *x, const sp_args<R> &a, const loc_tab &loc) {
+                           const R *kim, const uint8_t *flag, const R *x, const sp_args<R> &a, const loc_tab &loc,
+                           int64_t half = 0) {
+    if constexpr (sizeof(R) == 8 && !STD)
+        if (half > 0) {
+            k_spmv_pk<R, 16, EP, STD, false, true><<<(unsigned)((ne * 16 + 255) / 256), 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc, half);
+            return;
+        }
     if (loc.ptr != nullptr) {
-        k_spmv_pk<R, LOC_L, EP, STD, true><<<(unsigned)((ne + LOC_ROWS - 1) / LOC_ROWS), LOC_LANES, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
+        k_spmv_pk<R, LOC_L, EP, STD, true><<<(unsigned)((ne + LOC_ROWS - 1) / LOC_ROWS), LOC_LANES, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc, 0);
         return;
     }
     if (L != 4 && L != 8 && L != 32) L = 16;
     const unsigned grid = (unsigned)((ne * L + 255) / 256);
-    if (L == 4) k_spmv_pk<R, 4, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
-    else if (L == 8) k_spmv_pk<R, 8, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
-    else if (L == 32) k_spmv_pk<R, 32, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
-    else k_spmv_pk<R, 16, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc);
+    if (L == 4) k_spmv_pk<R, 4, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc, 0);
+    else if (L == 8) k_spmv_pk<R, 8, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc, 0);
+    else if (L == 32) k_spmv_pk<R, 32, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc, 0);
+    else k_spmv_pk<R, 16, EP, STD, false><<<grid, 256, 0, st>>>(ne, rowptr, acol, kre, kim, flag, x, a, loc, 0);
 }
 
 // The distinct columns of every LOC_ROWS rows, ascending, and every block's 16-bit place among them: counts first
@@ -1773,7 +1802,8 @@ struct emg_solver {
     const int32_t *rowptr = nullptr, *cols = nullptr;
     const double *vals = nullptr;   // complex128 K (caller-owned)
     const uint8_t *mask = nullptr;  // caller-owned, may be null
-    // K in the packed layout, in the precision of the solver's steps (k_pack_matrix)
+    // K in the packed layout, in the precision of the solver's steps (k_pack_matrix); at precision 64 acol and the
+    // planes are NULL where the card has no room for them, and the steps read the caller's CSR
     int32_t *acol = nullptr;        // nnz / 4 column entities
     void *kre = nullptr, *kim = nullptr;   // real and imaginary planes, nnz values each
     uint8_t *row_flag = nullptr;    // n_ent
@@ -1911,6 +1941,11 @@ static void apply_prec(emg_solver *s, const R *x, const double *xs, R *y, hipStr
 // A product with the packed matrix; L lanes per entity.
 template <typename R, int EP, bool STD>
 static void spmv_pk(emg_solver *s, int L, const R *x, const sp_args<R> &a, hipStream_t st) {
+    if constexpr (sizeof(R) == 8 && !STD)
+        if (s->kre == nullptr) {
+            launch_spmv_pk<R, EP, STD>(st, L, s->n_ent, s->rowptr, s->cols, s->vals, nullptr, s->row_flag, x, a, loc_tab{}, s->nnz / 2);
+            return;
+        }
     launch_spmv_pk<R, EP, STD>(st, L, s->n_ent, s->rowptr, s->acol, static_cast<const R *>(s->kre),
                                static_cast<const R *>(s->kim), s->row_flag, x, a, loc_tab{s->loc_ptr, s->loc_col, s->loc_idx});
 }
@@ -1923,7 +1958,7 @@ static constexpr int STD_LANES = 8;
 // y = K x, or b - K x, in complex128 and the caller's layout: the packed planes where they are
 // complex128 (precision 64), else the caller's CSR values.
 static void spmv_std(emg_solver *s, const double *x, const double *b, double *y, hipStream_t st) {
-    if (s->precision == 64) {
+    if (s->precision == 64 && s->kre != nullptr) {
         sp_args<double> a{b, y, nullptr, nullptr, 0, nullptr};
         if (b != nullptr) spmv_pk<double, SP_RESID, true>(s, STD_LANES, x, a, st);
         else spmv_pk<double, SP_Y, true>(s, STD_LANES, x, a, st);
@@ -2126,7 +2161,7 @@ static int fill_local(emg_solver *s, int32_t *cnt, int64_t nb) {
 // The tables of the LOC form, or none where a workgroup's rows exceed it or the memory does not suffice.
 static int local_columns(emg_solver *s) {
     const char *env = getenv("EMG_LOCAL_COLUMNS");
-    if (env != nullptr ? atoi(env) == 0 : s->n < LOC_MIN_N) return 0;
+    if (s->acol == nullptr || (env != nullptr ? atoi(env) == 0 : s->n < LOC_MIN_N)) return 0;
     const int64_t nb = (s->n_ent + LOC_ROWS - 1) / LOC_ROWS;
     int32_t *cnt = nullptr;
     int rc = device_alloc(&cnt, nb * sizeof(int32_t));
@@ -2136,8 +2171,8 @@ static int local_columns(emg_solver *s) {
     return rc == NO_MEMORY ? 0 : rc;
 }
 
-// The solver's device buffers for a basis of s->cap + 1 vectors.
-static int allocate(emg_solver *s) {
+// The solver's device buffers for a basis of s->cap + 1 vectors, with or without (precision 64) a packed copy of K.
+static int allocate(emg_solver *s, bool packed) {
     const int64_t n = s->n, nnz = s->nnz;
     const bool c64 = s->precision == 32;
     const size_t es = c64 ? 8 : 16;   // bytes per complex element of the basis
@@ -2156,9 +2191,11 @@ static int allocate(emg_solver *s) {
     A(&s->pn, 1024 * sizeof(double));
     A(&s->flag, 8 * sizeof(double));
     if (c64) A(&s->inv32, s->n_ent * 4 * 8);
-    A(&s->acol, (size_t)nnz / 4 * sizeof(int32_t));
-    A(&s->kre, (size_t)nnz * es / 2);
-    A(&s->kim, (size_t)nnz * es / 2);
+    if (packed) {
+        A(&s->acol, (size_t)nnz / 4 * sizeof(int32_t));
+        A(&s->kre, (size_t)nnz * es / 2);
+        A(&s->kim, (size_t)nnz * es / 2);
+    }
     A(&s->row_flag, s->n_ent);
     A(&s->poly_c, 2 * POLY_MAX * sizeof(double));
     A(&s->pp, n * 16); A(&s->py, n * 16); A(&s->pu, n * 16);
@@ -2166,12 +2203,26 @@ static int allocate(emg_solver *s) {
     return rc;
 }
 
-// Gives back what a solver of a full card can do without: the tables of the LOC form and the longer half of a
-// complex64 basis.  False where there is nothing of the kind.  Not during a solve.
+// The planes and row flags of the caller's values and mask as they are now.
+static void pack_matrix(emg_solver *s, hipStream_t st) {
+    const unsigned gp = (unsigned)((s->n_ent * SUB + 255) / 256);
+    if (s->kre == nullptr)
+        k_row_flags<<<emg::grid_for(s->n_ent, 256), 256, 0, st>>>(s->n_ent, s->mask, s->row_flag);
+    else if (s->precision == 32)
+        k_pack_matrix<float><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, s->vals, s->mask,
+                                                 static_cast<float *>(s->kre), static_cast<float *>(s->kim), s->row_flag);
+    else
+        k_pack_matrix<double><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, s->vals, s->mask,
+                                                  static_cast<double *>(s->kre), static_cast<double *>(s->kim), s->row_flag);
+}
+
+// Gives back what a solver of a full card can do without: the tables of the LOC form, and the longer half of a
+// complex64 basis or the packed complex128 copy of K.  False where there is nothing of the kind.  Not during a solve.
 static bool give_back(emg_solver *s) {
-    const bool any = s->loc_ptr != nullptr || s->cap > s->restart;
+    const bool copy = s->precision == 64 && s->kre != nullptr, any = s->loc_ptr != nullptr || s->cap > s->restart || copy;
     drop_graphs(s);
     drop_local(s);
+    if (copy) drop(s->acol, s->kre, s->kim);   // solves and probes set the row flags anew
     if (s->cap > s->restart) {
         s->cap = s->restart;
         s->kept = reinterpret_cast<kept_dev *>(s->arn + arn_off(s->cap).kept);
@@ -2200,13 +2251,15 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
     int bad = nnz <= 0 || nnz >= ((int64_t)1 << 31);
     if (!bad) {
         // complex64 refinement cycles keep up to two restart lengths of basis vectors (gmres_cycle), the
-        // bytes of the complex128 basis of one; where the card does not hold everything then, one
+        // bytes of the complex128 basis of one; where the card does not hold everything then, one.  Complex128 steps
+        // do without the packed copy of K there (883,652 DOFs: 267 -> 392 us per step, 895 -> 1,642 at degree 6).
         s->cap = precision == 32 ? std::min(2 * restart, 500) : restart;
-        int rc = allocate(s);
-        if (rc == NO_MEMORY && s->cap > restart) {
+        const char *env = getenv("EMG_PACKED_MATRIX");
+        int rc = precision == 64 && env != nullptr && atoi(env) == 0 ? NO_MEMORY : allocate(s, true);
+        if (rc == NO_MEMORY) {
             drop_buffers(s);
             s->cap = restart;
-            rc = allocate(s);
+            rc = allocate(s, precision == 32);
         }
         if (rc != 0) {
             free_solver(s);
@@ -2232,7 +2285,8 @@ extern "C" int emg_solver_create(int64_t n, int64_t nnz, const int32_t *d_rowptr
         free_solver(s);
         return -1;
     }
-    k_pack_cols<<<(unsigned)((s->n_ent * SUB + 255) / 256), 256>>>(s->n_ent, d_rowptr, d_cols, s->acol);
+    if (s->acol != nullptr)
+        k_pack_cols<<<(unsigned)((s->n_ent * SUB + 255) / 256), 256>>>(s->n_ent, d_rowptr, d_cols, s->acol);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return refuse("packing the pattern: ", e);
@@ -2335,7 +2389,9 @@ static int tune_steps(emg_solver *s, hipStream_t st) {
     auto product = [&](int L, hipStream_t rs) {
         spmv_pk<R, SP_Y, false>(s, L, pu, sp_args<R>{nullptr, pp, nullptr, nullptr, 0, nullptr}, rs);
     };
-    if (getenv("EMG_SPMV_BLK_LANES") != nullptr) {
+    if (s->kre == nullptr) {
+        s->lanes[slot] = 16;   // the only one of the CSR form
+    } else if (getenv("EMG_SPMV_BLK_LANES") != nullptr) {
         s->lanes[slot] = spmv_blk_lanes();
     } else {
         auto smooth = [&](hipStream_t rs) { apply_prec<R>(s, z, nullptr, pu, rs); };
@@ -2393,17 +2449,6 @@ extern "C" int emg_solver_spmv_tuning(emg_solver *s, int *h_lanes, float *h_ms) 
         for (int i = 0; i < 4; i++) h_ms[4 * p + i] = s->tune_ms[p][i];
     }
     return 0;
-}
-
-// The planes and row flags of the caller's values and mask as they are now.
-static void pack_matrix(emg_solver *s, hipStream_t st) {
-    const unsigned gp = (unsigned)((s->n_ent * SUB + 255) / 256);
-    if (s->precision == 32)
-        k_pack_matrix<float><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, s->vals, s->mask,
-                                                 static_cast<float *>(s->kre), static_cast<float *>(s->kim), s->row_flag);
-    else
-        k_pack_matrix<double><<<gp, 256, 0, st>>>(s->n_ent, s->nnz / 2, s->rowptr, s->acol, s->vals, s->mask,
-                                                  static_cast<double *>(s->kre), static_cast<double *>(s->kim), s->row_flag);
 }
 
 extern "C" int emg_solver_set_matrix(emg_solver *s, const double *d_vals, const uint8_t *d_mask, void *stream) {

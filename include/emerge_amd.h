@@ -117,7 +117,10 @@ int emg_assemble_tensor(const emg_pattern *pat, const double *d_nodes, const int
  * (0: never, else wherever the rows fit): products that gather x for 64 rows
  * at a time from 400,000 DOFs (EMG_LOCAL_COLUMNS, emg_solver_create), and
  * complex64 steps with one launch per smoother application and product up to
- * 50,000 (EMG_FUSED_STEPS, emg_solver_set_gradient).                        */
+ * 50,000 (EMG_FUSED_STEPS, emg_solver_set_gradient).  Chosen by the memory that is
+ * left: a complex64 basis of two restart lengths or one, and at precision 64 steps
+ * on a packed copy of K (16 bytes per entry) or on the caller's values
+ * (EMG_PACKED_MATRIX=0: these).                                              */
 typedef struct emg_solver emg_solver;
 typedef struct {
     int iterations;   /* Krylov iterations over all restarts / refinements */

@@ -90,14 +90,15 @@ out([L.emg_solver_solve(s, at(v), at(x), 1e-8, 100, 0, ctypes.byref(info), P(9))
     assert lines[0] == 0 and lines[-1] == "wait stream 9"
 
 
-@pytest.mark.parametrize("local", ["0", "1"])
-def test_a_complex64_solver_is_made_wherever_one_restart_length_fits(tmp_path, local):
-    """The second restart length of the basis and the tables of the products that gather locally are taken where the
-    card has room, whichever buffer the memory ends at; what is needed without them is found by halving."""
+@pytest.mark.parametrize("precision,local", [(32, "0"), (32, "1"), (64, "0"), (64, "1")])
+def test_a_solver_is_made_wherever_its_least_buffers_fit(tmp_path, precision, local):
+    """What serves speed (a second restart length of the complex64 basis, the packed copy of a complex128 K, the
+    tables of the products that gather locally) is taken where the card has room, whichever buffer the memory
+    ends at; what is needed without it is found by halving."""
     tries, least, most = run(SOLVER + """
 def fits(budget):
     rec.rec_budget(budget)
-    rc, s = solver(32, n=2000, restart=50)
+    rc, s = solver(PRECISION, n=2000, restart=50)
     used = rec.rec_used()
     if rc == 0:
         L.emg_solver_destroy(s)
@@ -111,16 +112,19 @@ while hi - lo > 1:
 out([fits(b)[0] for b in np.linspace(hi, most, 400).astype(int).tolist()])
 out([hi])
 out([most])
-""", tmp_path, env={"EMG_LOCAL_COLUMNS": local})
+""".replace("PRECISION", str(precision)), tmp_path, env={"EMG_LOCAL_COLUMNS": local})
     assert all(tries)
-    assert most[0] - least[0] >= 50 * 2000 * 8          # a restart length of vectors
+    # a restart length of vectors; 16 bytes per entry of the 2,000 rows of two
+    assert most[0] - least[0] >= (50 * 2000 * 8 if precision == 32 else 2000 * 2 * 16)
 
 
-def test_a_gradient_that_does_not_fit_gets_the_basis_second_half(tmp_path):
-    """emg_solver_set_gradient on a full card: the longer half of a complex64 basis makes room."""
+@pytest.mark.parametrize("precision", [32, 64])
+def test_a_gradient_that_does_not_fit_gets_room(tmp_path, precision):
+    """emg_solver_set_gradient on a full card: the longer half of a complex64 basis, or the packed copy of a
+    complex128 K, makes room."""
     (rc,) = run(SOLVER + """
 n, np2 = 2000, 300
-rc, s = solver(32, n=n, restart=50)
+rc, s = solver(PRECISION, n=n, restart=50)
 gp, tp = np.zeros(n + 1, np.int32), np.zeros(np2 + 1, np.int32)
 gp[n] = tp[np2] = 900
 c = np.zeros(900, np.int32)
@@ -129,5 +133,5 @@ rec.rec_budget(rec.rec_used())
 out([rc, L.emg_solver_set_gradient(s, np2, at(gp), at(c), at(g), at(tp), at(c), at(g), P(9)),
      L.emg_solver_set_matrix(s, at(v.repeat(20)), None, P(9)),
      L.emg_solver_solve(s, at(v), at(x), 1e-8, 100, 0, ctypes.byref(info), P(9))])
-""", tmp_path, env={"EMG_FUSED_STEPS": "0"})
+""".replace("PRECISION", str(precision)), tmp_path, env={"EMG_FUSED_STEPS": "0"})
     assert rc == [0, 0, 0, 0]
