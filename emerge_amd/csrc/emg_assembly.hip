@@ -76,7 +76,7 @@ struct emg_pattern {
     int chunk_tmax = 0;              // most tets of a chunk (sizes the fused kernel's LDS)
     uint16_t *inc_local = nullptr;   // n_inc: (local tet << 8) | (s << 4) | s'
     uint32_t *chunk_ent = nullptr;   // nchunk * CHUNK: the chunk's entries by kind and descending incidence count (ENT_*)
-    uint8_t *chunk_cnt = nullptr;    // nchunk * CHUNK: their incidences, 0 past the last entry; behind chunk_ent
+    uint16_t *chunk_cnt = nullptr;   // nchunk * CHUNK: their incidences, 0 past the last entry; behind chunk_ent
     double *tet_rec = nullptr;       // nt * REC: per-tet Gram records (fused-path workspace)
     double *tet_rec_batch = nullptr; // rec_batch_cap * nt * REC: the records of a batch of meshes
     int rec_batch_cap = 0;
@@ -111,7 +111,6 @@ static constexpr int REC = 48, TREC = 112;
 // column is that much further), its first incidence counted from the chunk's first even one (12 bits).
 static constexpr int ENT_ROW = 10, ENT_START = 20;
 static_assert(CHUNK <= 512 && CHUNK_NMAX < 1 << (32 - ENT_START), "a chunk's entries fit their words");
-static_assert(CHUNK_TMAX < 256, "an entry's incidences, each of another tet, fit chunk_cnt");
 // chunk_desc: first 32-bit word of incidence codes and their number, distinct tets, then where the values
 // go: value u of chunk c belongs at 2 c CHUNK + u + (u < N1 ? D0 : u < 2 N1 ? D1 : u >= U4 ? D4 : 0) of its
 // row mode's half (the chunk's first and last row may lie partly in its neighbours).
@@ -120,7 +119,7 @@ enum { DESC_W0, DESC_NW, DESC_NT, DESC_N1, DESC_U4, DESC_D0, DESC_D1, DESC_D4, D
 static void build_recipes(uint8_t *out, bool full);
 __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int32_t *__restrict__ chunk_tets,
                                                       int32_t *__restrict__ chunk_desc, uint16_t *__restrict__ inc_local,
-                                                      uint32_t *__restrict__ chunk_ent, uint8_t *__restrict__ chunk_cnt,
+                                                      uint32_t *__restrict__ chunk_ent, uint16_t *__restrict__ chunk_cnt,
                                                       int *__restrict__ overflow);
 
 // ------------------------------------------------------------------ symbolic
@@ -303,8 +302,8 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
         pat->chunk_desc = pat->chunk_tets + pat->nchunk * CHUNK_TMAX;
         // two spare codes: the fused kernel reads the codes as 32-bit words
         TRY(hipMalloc(&pat->inc_local, (size_t)(n_inc + 2) * sizeof(uint16_t)));
-        TRY(hipMalloc(&pat->chunk_ent, (size_t)pat->nchunk * pat->chunk * (sizeof(uint32_t) + 1)));
-        pat->chunk_cnt = reinterpret_cast<uint8_t *>(pat->chunk_ent + pat->nchunk * pat->chunk);
+        TRY(hipMalloc(&pat->chunk_ent, (size_t)pat->nchunk * pat->chunk * (sizeof(uint32_t) + sizeof(uint16_t))));
+        pat->chunk_cnt = reinterpret_cast<uint16_t *>(pat->chunk_ent + pat->nchunk * pat->chunk);
         TRY(hipMalloc(&pat->recipes, 2 * 100 * RECIPE_BYTES));
         TRY(hipMalloc(&d_over, sizeof(int)));
         TRY(hipMemsetAsync(d_over, 0, sizeof(int), st));
@@ -822,7 +821,7 @@ __device__ __forceinline__ int pair_kind(uint32_t v) { return ((v >> 4) & 15u) >
 // Distinct tets of every chunk, and chunk-local incidence codes.
 __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int32_t *__restrict__ chunk_tets,
                                                       int32_t *__restrict__ chunk_desc, uint16_t *__restrict__ inc_local,
-                                                      uint32_t *__restrict__ chunk_ent, uint8_t *__restrict__ chunk_cnt,
+                                                      uint32_t *__restrict__ chunk_ent, uint16_t *__restrict__ chunk_cnt,
                                                       int *__restrict__ overflow) {
     __shared__ uint32_t key[CHUNK_NMAX];
     __shared__ uint32_t uq[CHUNK_NMAX];
@@ -885,7 +884,7 @@ __global__ void __launch_bounds__(CHUNK) k_chunk_tets(const emg_pattern pat, int
         const int place = (int)(2 * (a - k0) + (k0 + tid - a));
         if (rank < ch) {
             chunk_ent[k0 + rank] = (uint32_t)place | (uint32_t)(b - a) << ENT_ROW | (uint32_t)(pat.pair_ptr[k0 + tid] - (q0 & ~1)) << ENT_START;
-            chunk_cnt[k0 + rank] = (uint8_t)(my_cnt < 255 ? my_cnt : 255);
+            chunk_cnt[k0 + rank] = (uint16_t)my_cnt;
         }
         int32_t *d = chunk_desc + c * DESC;
         const int64_t row_a = pat.ent_ptr[lo], row_n = pat.ent_ptr[lo + 1] - row_a;
@@ -1208,7 +1207,7 @@ __device__ __forceinline__ int out_shift(int u, int n1, int u4, int d0, int d1, 
 //  * runs of 32 chunks per XCD: workgroups that step through the whole grid drift apart, and the stores
 //    in flight spread over too much memory (store-only, 512 resident workgroups: 1.75 ms, 1.45 in runs);
 //  * the next loads issued before the stores, so that waiting for them does not wait for the stores;
-//  * an entry's place, row and incidences in five bytes, where the search for its row took nine steps in LDS;
+//  * an entry's place, row and incidences in six bytes, where the search for its row took nine steps in LDS;
 //  * formulas by kind: with edge pairs, edge-face pairs and face pairs in wavefronts of their own the
 //    incidence loop takes 118, 140 and 182 vector instructions where the common one took 190.
 // 128 registers, so 4 waves per SIMD, two workgroups per CU.  Slower: one chunk per workgroup with 4, 5 or

@@ -74,3 +74,45 @@ def test_batches_share_the_workgroups(cuda, batch):
     for i in (0, 1, batch // 2, batch - 1):
         pat.assemble_iso_device(eps[i].contiguous(), nu[i].contiguous(), 0, Es, Bs)
         assert torch.equal(E[i], Es) and torch.equal(B[i], Bs)
+
+
+@pytest.mark.parametrize("tets", [7, 8, 12])
+def test_entities_in_several_slots_of_a_tet(cuda, tets):
+    """All edges of every tet one entity and all faces another, as where a single cell lies between periodic faces:
+    the entry of the edges has 36 incidences per tet, 252, 288 and 432, and each is in it.  Against the blocks
+    of the same tets with entities of their own, summed; at most 36 * 12 * 13 * 4 terms of them per entry."""
+    import ctypes
+    import torch
+    rng = np.random.default_rng(tets)
+    nodes = torch.from_numpy(rng.uniform(0, 1, (4 * tets, 3)) + 2 * np.arange(tets).repeat(4)[:, None]).to(cuda)
+    verts = torch.arange(4 * tets, dtype=torch.int32, device=cuda).reshape(tets, 4)
+    eps, nu = (torch.from_numpy(rng.uniform(1, 4, tets) * (1 - 0.1j)).to(cuda) for _ in range(2))
+    mm, ms = (torch.eye(3, device=cuda) * v[:, None, None] for v in (eps, nu))
+    L = _lib.load()
+
+    def dense(ent, n_ent, call):
+        h, sizes = ctypes.c_void_p(), [ctypes.c_int64() for _ in range(4)]
+        _lib.check(L.emg_pattern_build(_lib.ptr(ent), tets, n_ent, _lib.stream_ptr(), ctypes.byref(h)), "emg_pattern_build")
+        _lib.check(L.emg_pattern_info(h, *(ctypes.byref(v) for v in sizes)), "emg_pattern_info")
+        n, nnz = sizes[0].value, sizes[1].value
+        rp, ci = (torch.empty(k, dtype=torch.int32, device=cuda) for k in (n + 1, nnz))
+        _lib.check(L.emg_pattern_csr(h, _lib.ptr(rp), _lib.ptr(ci), _lib.stream_ptr()), "emg_pattern_csr")
+        E, B = (torch.empty(nnz, dtype=torch.complex128, device=cuda) for _ in range(2))
+        args = (eps, nu) if call is L.emg_assemble_iso else (mm.contiguous(), ms.contiguous())
+        _lib.check(call(h, _lib.ptr(nodes), _lib.ptr(verts), _lib.ptr(args[0]), _lib.ptr(args[1]), 0, _lib.ptr(E), _lib.ptr(B),
+                        _lib.stream_ptr()), "assemble")
+        out = [torch.sparse_csr_tensor(rp.long(), ci.long(), v, (n, n)).to_dense().cpu().numpy() for v in (E, B)]
+        L.emg_pattern_destroy(h)
+        return out
+
+    own = torch.cat([torch.arange(6 * tets).reshape(tets, 6), 6 * tets + torch.arange(4 * tets).reshape(tets, 4)], dim=1).to(cuda, torch.int32)
+    shared = torch.tensor([[0] * 6 + [1] * 4] * tets, dtype=torch.int32, device=cuda)
+    fold = np.zeros((2 * 10 * tets, 4))
+    for m in range(2):
+        fold[m * 10 * tets: m * 10 * tets + 6 * tets, 2 * m] = 1
+        fold[m * 10 * tets + 6 * tets: (m + 1) * 10 * tets, 2 * m + 1] = 1
+    for call in (L.emg_assemble_iso, L.emg_assemble_tensor):
+        print("several slots", tets, call.__name__, flush=True)
+        for got, blocks in zip(dense(shared, 2, call), dense(own.contiguous(), 10 * tets, call)):
+            tol = 36 * 12 * 13 * 4 * 2.0 ** -53 * (fold.T @ np.abs(blocks) @ fold).max()
+            assert np.abs(got - fold.T @ blocks @ fold).max() <= tol
