@@ -2376,7 +2376,8 @@ static int tune_lanes(emg_solver *s, int n, const int *cand, LEAD &&lead, RUN &&
 }
 
 // Lanes per entity of the solver's products: complex128 (slot 0: the packed matrix for precision 64,
-// the caller's CSR for precision 32) and complex64 (slot 1); EMG_SPMV_BLK_LANES overrides.
+// the caller's CSR for precision 32) and complex64 (slot 1); EMG_SPMV_BLK_LANES overrides.  Fused solvers run
+// the products and the G^T product of their choice once the gradient is taken off (emg_solver_set_gradient, np2 = 0).
 static const int TUNE_LANES[4] = {4, 8, 16, 32};
 // Lanes per row of the smoother's G^T product; EMG_GT_LANES (4, 8 or 16) overrides.
 static const int GT_LANES[3] = {4, 8, 16};
@@ -2389,8 +2390,8 @@ static int tune_steps(emg_solver *s, hipStream_t st) {
     auto product = [&](int L, hipStream_t rs) {
         spmv_pk<R, SP_Y, false>(s, L, pu, sp_args<R>{nullptr, pp, nullptr, nullptr, 0, nullptr}, rs);
     };
-    if (s->kre == nullptr) {
-        s->lanes[slot] = 16;   // the only one of the CSR form
+    if (s->kre == nullptr || s->loc_ptr != nullptr) {   // these forms have one shape
+        s->lanes[slot] = s->kre == nullptr ? 16 : LOC_L;
     } else if (getenv("EMG_SPMV_BLK_LANES") != nullptr) {
         s->lanes[slot] = spmv_blk_lanes();
     } else {

@@ -282,7 +282,8 @@ class GPUSolver:
     def spmv_tuning(self) -> dict:
         """The autotuned SpMV shape of this solver (chosen on its first matrix): lanes per
         entity for complex128 and complex64 steps and the measured ms per launch of each
-        candidate (4, 8, 16, 32 lanes); lanes 0 before the first set_matrix."""
+        candidate (4, 8, 16, 32 lanes); lanes 0 before the first set_matrix.  Products that gather
+        x for 64 rows at a time have 4 lanes without a search (ms 0)."""
         lanes = (ctypes.c_int * 2)()
         ms = (ctypes.c_float * 8)()
         _lib.check(self.L.emg_solver_spmv_tuning(self.h, lanes, ms), "emg_solver_spmv_tuning")

@@ -182,7 +182,10 @@ int emg_solver_apply(emg_solver *s, int precision, const void *d_x, void *d_y, v
  * after what precedes it in a step; in complex128 and, for precision 32, complex64) and keeps the
  * fastest.  h_lanes[2]: the chosen lanes (complex128, complex64); h_ms[8]: the measured
  * milliseconds per launch (4 per precision, in the order 4, 8, 16, 32).  EMG_SPMV_BLK_LANES
- * overrides the search.  No reference counterpart (PARDISO has no shape to tune).         */
+ * overrides the search.  Products that gather x for 64 rows at a time have 4 lanes, and those
+ * on the caller's values 16, without a search (milliseconds 0); steps with one launch per
+ * smoother application and product use neither these lanes nor those of
+ * emg_solver_smoother_tuning.  No reference counterpart (PARDISO has no shape to tune).   */
 int emg_solver_spmv_tuning(emg_solver *s, int *h_lanes, float *h_ms);
 
 /* The solver's autotuned smoother shape: with the gradient correction set, the first

@@ -135,3 +135,20 @@ out([rc, L.emg_solver_set_gradient(s, np2, at(gp), at(c), at(g), at(tp), at(c), 
      L.emg_solver_solve(s, at(v), at(x), 1e-8, 100, 0, ctypes.byref(info), P(9))])
 """.replace("PRECISION", str(precision)), tmp_path, env={"EMG_FUSED_STEPS": "0"})
     assert rc == [0, 0, 0, 0]
+
+
+@pytest.mark.parametrize("precision,local,lanes,searches", [(64, "0", None, 5), (64, "1", [4, 4], 0), (32, "1", [None, 4], 5)])
+def test_products_of_one_shape_are_not_tuned(tmp_path, precision, local, lanes, searches):
+    """A search captures and times a graph per candidate and one of what precedes them: five for the products of four
+    shapes, none for those that gather x for 64 rows (precision 32 still searches for its CSR product)."""
+    lines, got = run(SOLVER + f"""
+rc, s = solver({precision}, n=2000)
+assert rc == 0
+rec.rec_clear()
+out([L.emg_solver_set_matrix(s, at(v.repeat(20)), None, P(9))] + log())
+n, ms = (ctypes.c_int * 2)(), (ctypes.c_float * 8)()
+assert L.emg_solver_spmv_tuning(s, n, ms) == 0
+out(list(n))
+""", tmp_path, env={"EMG_LOCAL_COLUMNS": local})
+    assert lines[0] == 0 and sum(x.startswith("capture") for x in lines[1:]) == searches
+    assert lanes is None or all(want in (None, have) for want, have in zip(lanes, got))
