@@ -38,3 +38,28 @@ def test_staged_equals_direct(cuda, dims, flags, kind):
     for a, b in zip(*out):
         assert torch.all(torch.isfinite(torch.view_as_real(a)))
         assert float((a - b).abs().max()) <= 64 * 13 * 4 * 16 * 2.0 ** -53 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("tets", [64, 65, 96, 97, 120])
+@pytest.mark.parametrize("flags", [0, EXACT_FACE_MASS])
+def test_staged_equals_direct_where_chunks_hold_many_tets(cuda, tets, flags):
+    """The layouts of 64, 96 and 128 records, at their edges: a fan of tets round one edge, whose row makes a chunk
+    of all of them.  Bound as in test_staged_equals_direct, with up to 120 tets per entry."""
+    import torch
+    from tests.test_assembly_chunks_gpu import _fan
+    mesh = _fan(tets)
+    pat = GPUPattern(mesh)
+    rng = np.random.default_rng(tets)
+    m = rng.standard_normal((2, mesh.n_tets, 3, 3)) + 1j * rng.standard_normal((2, mesh.n_tets, 3, 3))
+    mm, ms = (torch.from_numpy(np.ascontiguousarray(a)).to(cuda) for a in m)
+    L = _lib.load()
+    print(f"tensor fan {tets} flags={flags}", flush=True)
+    out = []
+    for f in (flags, flags | FORCE_TWO_PHASE):
+        E = torch.full((pat.nnz,), complex(np.nan, np.nan), dtype=torch.complex128, device=cuda)
+        B = torch.full_like(E, complex(np.nan, np.nan))
+        _lib.check(L.emg_assemble_tensor(pat.handle, _lib.ptr(pat.nodes), _lib.ptr(pat.tets), _lib.ptr(mm), _lib.ptr(ms),
+                                         f, _lib.ptr(E), _lib.ptr(B), _lib.stream_ptr()), "emg_assemble_tensor")
+        out.append((E, B))
+    for a, b in zip(*out):
+        assert float((a - b).abs().max()) <= 120 * 13 * 4 * 16 * 2.0 ** -53 * float(b.abs().max())
