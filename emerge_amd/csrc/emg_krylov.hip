@@ -364,7 +364,7 @@ __global__ void k_mdot_finish(int nv, int nblk, const double *__restrict__ parti
             h[2 * i + 1] = c * im;
         } else {
             const int l = nv - 1;
-            const double f = i == l ? 0.0 : c * sc[l];   // vectors are normalised: the diagonal deviates by rounding only
+            const double f = i == l ? 0.0 : c * sc[l];   // every scale is its vector's own norm's: the diagonal does not deviate
             E[2 * ((int64_t)i * ld + l)] = f * r;
             E[2 * ((int64_t)i * ld + l) + 1] = f * im;
             E[2 * ((int64_t)l * ld + i)] = f * r;
@@ -1813,7 +1813,7 @@ struct emg_solver {
     float *inv32 = nullptr;
     double *V = nullptr;            // cap + 1 basis vectors, element type per precision
     double *w = nullptr, *z = nullptr, *r = nullptr, *d = nullptr;   // d: precision 64 only
-    double *partial = nullptr, *h = nullptr, *nrm = nullptr;
+    double *partial = nullptr, *h = nullptr;
     int nblk = 0;
     // Arnoldi steps run from captured HIP graphs (chunks of CHUNK_IT steps)
     // with the Hessenberg column, Givens rotations and residual estimate
@@ -1897,7 +1897,7 @@ static void drop_gradient(emg_solver *s) {
 }
 static void drop_local(emg_solver *s) { drop(s->loc_ptr, s->loc_col, s->loc_idx); }
 static void drop_buffers(emg_solver *s) {   // what emg_solver_create allocates
-    drop(s->acol, s->kre, s->kim, s->row_flag, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial, s->h, s->nrm, s->arn,
+    drop(s->acol, s->kre, s->kim, s->row_flag, s->inv64, s->inv32, s->V, s->w, s->z, s->r, s->d, s->partial, s->h, s->arn,
          s->pn, s->gram, s->flag, s->poly_c, s->pp, s->py, s->pu);
     drop_local(s);
 }
@@ -2185,7 +2185,6 @@ static int allocate(emg_solver *s, bool packed) {
     A(&s->partial, ((size_t)2 * ntile * 1024 * DT * 2 + 1024) * sizeof(double));
     A(&s->gram, (size_t)(s->cap + 1) * (s->cap + 1) * 16);
     A(&s->h, 4 * 2 * 512 * sizeof(double));   // dots | corrected | the part subtracted | y
-    A(&s->nrm, 4 * sizeof(double));
     A(&s->inv64, s->n_ent * 4 * 16);
     A(&s->arn, arn_off(s->cap).total * sizeof(double));
     A(&s->pn, 1024 * sizeof(double));
@@ -2726,12 +2725,26 @@ extern "C" int emg_solver_set_gradient(emg_solver *s, int64_t np2, const int32_t
 }
 
 // ---------------------------------------------------------------- device Arnoldi bookkeeping
-// A cycle whose first basis vector is t0: g[t0] = beta = *nrm, V_t0 is stored normalised.
-__global__ void k_arn_init(int t0, const double *__restrict__ nrm, double *__restrict__ arn, arn_off o) {
+// A cycle whose first basis vector is V_t0 = w: g[t0] = ||w|| from its nb partial sums, and the scale 1 / ||w||.
+// Like every basis vector it is kept as it is with that scale beside it: normalised in complex64 its norm would be
+// off by the rounding, which the Gram matrix' diagonal (0 deviation) does not hold, and where the next vector
+// is all but cancelled (K M near the identity) that much of w stays in it: the bases of later cycles
+// were no longer orthogonal and one of them ran to the end of the restart without a gain.
+template <typename R>
+__global__ void __launch_bounds__(RB) k_arn_start(int64_t n, int t0, int nb, const double *__restrict__ pn,
+                                                  const R *__restrict__ w, R *__restrict__ vt, double *__restrict__ arn,
+                                                  arn_off o) {
+    for (int64_t e = blockIdx.x * (int64_t)RB + threadIdx.x; e < n; e += (int64_t)gridDim.x * RB) st(vt, e, ld(w, e));
+    if (blockIdx.x != 0) return;
+    __shared__ double sh[RB / 64];
+    double a = 0.0;
+    for (int i = threadIdx.x; i < nb; i += RB) a += pn[i];
+    a = block_sum(a, sh);
     if (threadIdx.x == 0) {
-        arn[o.g + 2 * t0] = nrm[0];
+        const double beta = sqrt(a);
+        arn[o.g + 2 * t0] = beta;
         arn[o.g + 2 * t0 + 1] = 0.0;
-        arn[o.sc + t0] = 1.0;
+        arn[o.sc + t0] = beta > 0.0 ? 1.0 / beta : 0.0;
     }
 }
 
@@ -2855,6 +2868,7 @@ __global__ void __launch_bounds__(RB) k_arn_report(int t, int m, const double *_
         hst[ho.g + i] = arn[o.fin + i];
     }
     if (threadIdx.x == 2) hst[ho.sc + t + 1] = arn[o.sc + t + 1];
+    if (threadIdx.x == 4) hst[ho.sc + t] = arn[o.sc + t];   // a cycle's first vector has a scale of its own
     if (threadIdx.x == 3) hst[ho.res + t] = arn[o.res + t];
 }
 
@@ -3018,8 +3032,7 @@ static int gmres_cycle(emg_solver *s, double unit, double tol, int maxiter, kept
     } else {
         k_norm2<R><<<nb, RB, 0, st>>>(n, w, s->pn);
     }
-    k_scale_by_norm<R><<<nb, RB, 0, st>>>(n, s->pn, nb, w, vt, s->nrm);
-    k_arn_init<<<1, 64, 0, st>>>(t0, s->nrm, s->arn, o);
+    k_arn_start<R><<<nb, RB, 0, st>>>(n, t0, nb, s->pn, w, vt, s->arn, o);
     EMG_LAUNCH_CHECK();
     const int len = chunk_it(n), most = std::min({m - t0, s->restart, maxiter});
     int k = 0;
@@ -3052,8 +3065,7 @@ static int gmres_cycle(emg_solver *s, double unit, double tol, int maxiter, kept
         for (int i = 0; i <= t; i++) kh.r(i, t) = from_host(ho.H + 2 * (int64_t)t * (m + 1), i);
         for (const auto &c : kh.cycles) kh.rotate(c, &kh.r(0, t));
     }
-    kh.sc[t0] = 1.0;
-    for (int t = t0 + 1; t <= t0 + k; t++) kh.sc[t] = s->host[ho.sc + t];
+    for (int t = t0; t <= t0 + k; t++) kh.sc[t] = s->host[ho.sc + t];
     for (const auto &c : kh.cycles) kh.rotate(c, g.data());
     kh.cycles.push_back({t0, k});
     for (int c = (int)kh.cycles.size() - 1; c >= 0; c--) {

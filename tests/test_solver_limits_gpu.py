@@ -25,14 +25,15 @@ def _matrix(rng, columns, ne):
 
 
 class _Solver:
-    def __init__(self, cuda, A, precision):
+    def __init__(self, cuda, A, precision, restart=10):
         import torch
         from emerge_amd import _lib
         self.L, self.lib, self.h = _lib.load(), _lib, ctypes.c_void_p()
         self.t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
         self.keep = [self.t(A.indptr.astype(np.int32)), self.t(A.indices.astype(np.int32)), self.t(A.data)]
         rp, ci, self.vals = self.keep
-        _lib.check(self.L.emg_solver_create(A.shape[0], A.nnz, _lib.ptr(rp), _lib.ptr(ci), 10, precision, ctypes.byref(self.h)),
+        _lib.check(self.L.emg_solver_create(A.shape[0], A.nnz, _lib.ptr(rp), _lib.ptr(ci), restart, precision,
+                                            ctypes.byref(self.h)),
                    "emg_solver_create")
 
     def matrix(self):
@@ -112,3 +113,26 @@ def test_fused_steps_at_their_limits(cuda, ne, np2, deg, monkeypatch):
     err, tol = np.linalg.norm(x.cpu().numpy() - want) / size, 16 * np.linalg.norm(rough - want) / size + 64 * 2.0 ** -24
     print("error", err, "of", tol, flush=True)
     assert err <= tol
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("shared", [0, 1, 3])
+@pytest.mark.parametrize("ne", [500, 70001])
+@pytest.mark.parametrize("restart", [10, 150])
+def test_a_krylov_space_that_ends_early(cuda, ne, shared, precision, restart):
+    """K M is the identity but for the 2 `shared` columns that every row lists, so the Krylov space holds at most 2 shared + 2
+    vectors: the next one cancels to rounding.  A space is looked at every 4 (2) steps, and complex64 may begin it
+    anew up to 4 times on the way to 1e-13: both precisions reach it in these steps."""
+    import torch
+    rng = np.random.default_rng(ne + shared)
+    A = _matrix(rng, [np.unique(np.append(np.arange(shared), e)) for e in range(ne)], ne)
+    s = _Solver(cuda, A, precision, restart)
+    s.matrix()
+    b = rng.standard_normal(2 * ne) + 1j * rng.standard_normal(2 * ne)
+    bd = s.t(b)
+    x, info = torch.zeros_like(bd), s.lib.SolveInfo()
+    print("early", ne, shared, precision, restart, flush=True)
+    s.lib.check(s.L.emg_solver_solve(s.h, s.lib.ptr(bd), s.lib.ptr(x), 1e-13, 200, 0, ctypes.byref(info), s.lib.stream_ptr()), "solve")
+    print("steps", info.iterations, "residual", info.residual, flush=True)
+    assert info.converged and info.iterations <= (2 * shared + 2 + 4) * (4 if precision == 32 else 1)
+    assert np.linalg.norm(b - A @ x.cpu().numpy()) <= 2e-13 * np.linalg.norm(b)
