@@ -26,6 +26,7 @@
 #include <cstring>
 #include <limits>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/emerge_amd.h"
@@ -984,7 +985,10 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
         if constexpr (EP == SP_POLY)
             if (a.i > 0) yv = get(a.y);
     }
-    R s0r = 0, s0i = 0, s1r = 0, s1i = 0;
+    // fewer than 16 lanes make longer chains: complex64 sums in FP64 there.  Errors against 64 bits: with 16 lanes 7.3e-8 on
+    // air and 7.4e-8 with losses, with 4 or 8 and sums in FP32 7.2e-8 and 7.7e-8, so 5.9e-8 and 6.5e-8, in the same time.
+    using S = std::conditional_t<(L < 16), double, R>;
+    S s0r = 0, s0i = 0, s1r = 0, s1i = 0;
     if (fl & (ROW0 | ROW1)) {
         for (int32_t p = p0 + lane; p < p1; p += L * U) {
             int32_t c[U];
@@ -1034,7 +1038,7 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
                     v[u].bi += k[u].br * xv[u].ar + k[u].bi * xv[u].br;
                 }
             }
-            // pairwise, then to the row's sums: the shorter chains keep few lanes per row as accurate as many
+            // pairwise, then to the row's sums
 #pragma unroll
             for (int u = 0; u < U; u++)
                 if (p + u * L >= p1) v[u] = cx2<R>{0, 0, 0, 0};
@@ -1058,7 +1062,7 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
     s1r = lane_sum<L>(s1r);
     s1i = lane_sum<L>(s1i);
     if (lane != 0) return;
-    cx2<R> v{(fl & ROW0) ? s0r : own.ar, (fl & ROW0) ? s0i : own.ai, (fl & ROW1) ? s1r : own.br, (fl & ROW1) ? s1i : own.bi};
+    cx2<R> v{(fl & ROW0) ? (R)s0r : own.ar, (fl & ROW0) ? (R)s0i : own.ai, (fl & ROW1) ? (R)s1r : own.br, (fl & ROW1) ? (R)s1i : own.bi};
     if constexpr (EP == SP_RESID) v = cx2<R>{qv.ar - v.ar, qv.ai - v.ai, qv.br - v.br, qv.bi - v.bi};
     if constexpr (EP == SP_POLY) {
         const double *cc = a.c + 2 * a.i;
