@@ -316,7 +316,11 @@ extern "C" int emg_pattern_build(const int32_t *d_tet_ent, int64_t nt, int64_t n
         TRY(hipGetLastError());
         int over = 0;
         TRY(hipMemcpyAsync(&over, d_over, sizeof(int), hipMemcpyDeviceToHost, st));
-        std::vector<int32_t> desc((size_t)pat->nchunk * DESC);
+        std::vector<int32_t> desc;
+        if (int hrc = emg::host_zeros(desc, (size_t)pat->nchunk * DESC)) {
+            hfree(d_over);
+            return fail(hrc);
+        }
         TRY(hipMemcpyAsync(desc.data(), pat->chunk_desc, desc.size() * sizeof(int32_t), hipMemcpyDeviceToHost, st));
         TRY(hipStreamSynchronize(st));
         hfree(d_over);

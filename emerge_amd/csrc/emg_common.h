@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <exception>
 #include <string>
 
 namespace emg {
@@ -47,6 +48,18 @@ __host__ __device__ inline cplx operator*(cplx a, cplx b) { return cplx(a.re * b
 __host__ __device__ inline cplx operator*(double s, cplx a) { return cplx(s * a.re, s * a.im); }
 __host__ __device__ inline cplx operator*(cplx a, double s) { return cplx(s * a.re, s * a.im); }
 __host__ __device__ inline cplx &operator+=(cplx &a, cplx b) { a.re += b.re; a.im += b.im; return a; }
+
+// n zeros of host memory, or the error of a C entry in place of an exception through it.
+template <typename V>
+int host_zeros(V &v, size_t n) {
+    try {
+        v.assign(n, typename V::value_type());
+    } catch (const std::exception &e) {
+        set_error(std::string("host memory: ") + e.what());
+        return -2;
+    }
+    return 0;
+}
 
 inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 

@@ -2124,7 +2124,9 @@ static int device_alloc(T **p, size_t bytes) {
 
 // off[i] = sum of cnt[0 .. i) for i <= n, through the host (once per solver or gradient)
 static int prefix_on_host(const int32_t *d_cnt, int64_t n, int32_t **d_off, int64_t *total, hipStream_t st) {
-    std::vector<int32_t> c(n), o(n + 1, 0);
+    std::vector<int32_t> c, o;
+    if (int rc = emg::host_zeros(c, n)) return rc;
+    if (int rc = emg::host_zeros(o, n + 1)) return rc;
     EMG_HIP(hipMemcpyAsync(c.data(), d_cnt, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
     EMG_HIP(hipStreamSynchronize(st));
     int64_t t = 0;
@@ -2590,7 +2592,9 @@ static int pack_gradient(emg_solver *s, int64_t np2, const int32_t *grp, const i
     k_g_width<<<(unsigned)ns, 64, 0, st>>>(ne, grp, gcol, cnt);
     EMG_LAUNCH_CHECK();
     // the cut between two runs of slices, each as wide as its widest, that leaves the fewest slots
-    std::vector<int32_t> wd(ns), after_max(ns + 1, 0);
+    std::vector<int32_t> wd, after_max;
+    if (int rc = emg::host_zeros(wd, ns)) return rc;
+    if (int rc = emg::host_zeros(after_max, ns + 1)) return rc;
     EMG_HIP(hipMemcpyAsync(wd.data(), cnt, ns * sizeof(int32_t), hipMemcpyDeviceToHost, st));
     EMG_HIP(hipStreamSynchronize(st));
     for (int64_t i = ns - 1; i >= 0; i--) after_max[i] = std::max(after_max[i + 1], wd[i]);

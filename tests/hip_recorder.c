@@ -1,7 +1,10 @@
 /* The HIP runtime calls of libemerge_amd.so, recorded on the CPU: device memory is host memory within a budget,
  * kernels do nothing, and every call that orders work is written to a log.  Loaded with global symbols
  * before the library (tests/host_calls.py), so that its host code runs here: what it allocates, what it does
- * when memory runs out, and in which order it launches, copies and waits. */
+ * when memory runs out, and in which order it launches, copies and waits.  Host memory of C++ containers has a
+ * limit too (build with -fexceptions). */
+#define _GNU_SOURCE
+#include <dlfcn.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -103,6 +106,17 @@ int hipMemset(void *p, int v, size_t n) { memset(p, v, n); say("memset"); return
 int hipMemsetAsync(void *p, int v, size_t n, void *st) { memset(p, v, n); say("memset stream %zu", (size_t)st); return SUCCESS; }
 int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)k; memcpy(d, s, n); say("memcpy"); return SUCCESS; }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st) { (void)k; memcpy(d, s, n); say("copy %zu stream %zu", n, (size_t)st); return SUCCESS; }
+
+/* ---- operator new: blocks above a limit are refused as the C++ library refuses them */
+static size_t g_host_block = (size_t)-1;
+void rec_host_block(size_t bytes) { g_host_block = bytes; }
+void *_Znwm(size_t n) {
+    void *p = n > g_host_block ? NULL : malloc(n ? n : 1);
+    if (!p) ((void (*)(void))dlsym(RTLD_DEFAULT, "_ZSt17__throw_bad_allocv"))();
+    return p;
+}
+void _ZdlPv(void *p) { free(p); }
+void _ZdlPvm(void *p, size_t n) { (void)n; free(p); }
 
 /* ---- order: streams, events, graphs */
 int hipStreamCreateWithFlags(void **st, unsigned f) { (void)f; *st = (void *)(size_t)1000; return SUCCESS; }

@@ -15,7 +15,8 @@ import numpy as np
 rec = ctypes.CDLL({stub!r}, mode=ctypes.RTLD_GLOBAL)
 rec.rec_log.restype = ctypes.c_char_p
 rec.rec_used.restype = ctypes.c_size_t
-rec.rec_budget.argtypes = [ctypes.c_size_t]
+rec.rec_budget.argtypes = rec.rec_host_block.argtypes = [ctypes.c_size_t]
+ctypes.CDLL("libstdc++.so.6", mode=ctypes.RTLD_GLOBAL)
 sys.path.insert(0, {root!r})
 from emerge_amd import _lib
 L = _lib.load()
@@ -31,7 +32,7 @@ def log():
 
 def run(snippet, tmp_path, env=None):
     stub = os.path.join(tmp_path, "libhip_recorder.so")
-    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", stub, os.path.join(HERE, "hip_recorder.c")], check=True)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-fexceptions", "-o", stub, os.path.join(HERE, "hip_recorder.c"), "-ldl"], check=True)
     code = PROLOGUE.format(stub=stub, root=ROOT) + snippet
     got = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env={**os.environ, **(env or {})}, capture_output=True,
                          text=True, timeout=120)

@@ -152,3 +152,20 @@ out(list(n))
 """, tmp_path, env={"EMG_LOCAL_COLUMNS": local})
     assert lines[0] == 0 and sum(x.startswith("capture") for x in lines[1:]) == searches
     assert lanes is None or all(want in (None, have) for want, have in zip(lanes, got))
+
+
+def test_host_memory_that_runs_out_is_an_error_not_an_exception(tmp_path):
+    """A table that emg_solver_set_gradient makes on the host and cannot have ends the call with an error."""
+    (rcs,) = run(SOLVER + """
+n, np2 = 2000, 300000
+rc, s = solver(32, n=n, restart=50)
+gp, tp = np.zeros(n + 1, np.int32), np.zeros(np2 + 1, np.int32)
+gp[n] = tp[np2] = 900
+c, g = np.zeros(900, np.int32), np.zeros(900)
+rcs = [rc]
+for block in (100000, 2 ** 62):
+    rec.rec_host_block(block)
+    rcs.append(L.emg_solver_set_gradient(s, np2, at(gp), at(c), at(g), at(tp), at(c), at(g), P(9)))
+out(rcs)
+""", tmp_path, env={"EMG_FUSED_STEPS": "0"})
+    assert rcs == [0, -2, 0]
