@@ -917,8 +917,9 @@ struct sp_args {
 // LOC: a workgroup first gathers x for the distinct columns of its LOC_ROWS rows into LDS (loc_tab: the columns, and
 // in acol's place 16-bit places among them).  The gathers of the other form take a line of the L2 each, 21 of them
 // per row and no two lanes of a row the same; 64 rows share theirs 3.3 times, and an index is 2 bytes.  Products of
-// the posts box: complex64 on air at 1,947,698 DOFs 114 -> 90 us (4.7 TB/s), with losses at 831,972 70 -> 63 (5.3),
-// complex128 on air at 883,652 91 -> 71 (5.1).  (8 lanes per row, which is 512 of them: 92, 61, 79; 32, 96 or 128
+// the posts box, rates by the bytes of the format: complex64 on air at 1,947,698 DOFs 114 -> 90 us (4.7 TB/s; by the HBM
+// counters 6.1, most columns' x being fetched by several XCDs), with losses at 831,972 70 -> 63 (5.3), complex128 on air at
+// 883,652 91 -> 71 (5.1).  (8 lanes per row, which is 512 of them: 92, 61, 79; 32, 96 or 128
 // rows: 96, 66, 85; 113, 65, 86; 93, 65, 74; 2, 3 or 6 blocks in flight per lane: 95, 69, 73; 96, 68, 73; 93, 63, 89.)
 static constexpr int LOC_ROWS = 64, LOC_L = 4, LOC_MAX = 1024, LOC_CAND = 8192;
 static constexpr int LOC_LANES = LOC_ROWS * LOC_L;
@@ -1375,8 +1376,8 @@ __global__ void __launch_bounds__(RB) k_bj_grad_pk(int64_t ne, const R *__restri
 // so with the matrices KG = K G, H = G^T K and HG = G^T K G at hand the polynomial's recurrence on q carries
 // G^T q along and needs one launch per product where smoother and product take three (G^T, then L and G, then
 // K).  KG's rows are the entities', with the P2 nodes of their columns' rows of G; H's and HG's are the nodes',
-// with the columns of the entities in their rows of G^T and the nodes of those' KG rows.  They are formed in
-// complex128 and kept in complex64 beside K.
+// with the columns of the entities in their rows of G^T and the nodes of those' KG rows.  KG and H are formed in
+// complex128 and kept in complex64 beside K; HG is summed in FP64 from KG as it is kept.
 
 // The distinct values that GEN(row, put) puts, ascending: their number to cnt, or with out the values
 // themselves at out[ptr[row]].  A row with more than CAND candidates or UNIQ values sets *over.
@@ -2668,11 +2669,13 @@ static int fuse_pattern(emg_solver *s, int64_t np2, const int32_t *grp, const in
     return rc;
 }
 
-// Where the fused steps are used.  KG, H and HG hold about as many bytes as K, so they pay while a launch
-// costs more than its bytes: posts box with 3,072 / 4,800 / 8,640 / 14,112 tets (20,000 / 34,000 / 60,000 / 96,000
-// DOFs), air: 124 -> 90, 123 -> 99, 134 -> 125, 158 -> 169 us per step at degree 6; lossy: 124 -> 90, 130 -> 100,
-// 140 -> 133, 178 -> 179; 38,400 tets: 258 -> 360.  Complex64 only: complex128 steps are mostly above it.
-// EMG_FUSED_STEPS overrides (0: never, else wherever the rows fit).
+// Where the fused steps are used.  KG, H and HG hold about as many bytes as K, so steps are faster while a launch
+// costs more than its bytes: posts box at 20,000 / 34,000 / 58,424 / 71,896 / 94,092 DOFs, air, degree 6: 124 -> 90, 123 -> 99,
+// 133 -> 122, 140 -> 140, 153 -> 165 us; lossy 124 -> 90, 130 -> 100, 142 -> 130, 152 -> 146, 168 -> 173.  The line lies
+// below where they cross, because the patterns are set up once (create and first matrix) and the values formed for every
+// matrix: a frequency point (matrix and one solve) takes 10.3 -> 9.4 ms at 49,414 DOFs on air for 3.0 ms of set-up,
+// and 10.7 -> 10.4 at 58,424 for 4.9, which 17 points would earn; 12.4 -> 13.0 at 71,896.
+// Complex64 only: complex128 steps are mostly above it.  EMG_FUSED_STEPS overrides (0: never, else wherever the rows fit).
 static constexpr int64_t FUSE_MAX_N = 50000;
 static bool fuse_wanted(const emg_solver *s) {
     if (s->precision != 32) return false;

@@ -79,7 +79,10 @@ int emg_pattern_assembly_tuning(const emg_pattern *pat, int *h_wg_per_cu, float 
  * Isotropic materials: one complex scalar per tet.
  *   d_nodes (nv,3) f64; d_tets (nt,4) int32 canonical (sorted);
  *   d_eps (nt) c128 (eps_r); d_nu (nt) c128 (1/mu_r);
- *   d_E, d_B (nnz) c128 outputs.                                             */
+ *   d_E, d_B (nnz) c128 outputs.
+ * The pattern's records are written and read on `stream`: assemblies of one pattern on
+ * several streams must be ordered by the caller, here and in emg_assemble_iso_batched
+ * (emg_assemble_tensor orders its own).                                          */
 int emg_assemble_iso(const emg_pattern *pat, const double *d_nodes, const int32_t *d_tets,
                      const double *d_eps, const double *d_nu, int flags,
                      double *d_E, double *d_B, void *stream);
