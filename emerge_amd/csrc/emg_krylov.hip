@@ -917,9 +917,8 @@ struct sp_args {
 // LOC: a workgroup first gathers x for the distinct columns of its LOC_ROWS rows into LDS (loc_tab: the columns, and
 // in acol's place 16-bit places among them).  The gathers of the other form take a line of the L2 each, 21 of them
 // per row and no two lanes of a row the same; 64 rows share theirs 3.3 times, and an index is 2 bytes.  Products of
-// the posts box, rates by the bytes of the format: complex64 on air at 1,947,698 DOFs 114 -> 90 us (4.7 TB/s; by the HBM
-// counters 6.1, most columns' x being fetched by several XCDs), with losses at 831,972 70 -> 63 (5.3), complex128 on air at
-// 883,652 91 -> 71 (5.1).  (8 lanes per row, which is 512 of them: 92, 61, 79; 32, 96 or 128
+// the posts box, rates by the bytes of the format: complex64 on air at 1,947,698 DOFs 114 -> 90 us (4.7 TB/s; the HBM
+// counters show 0.53 GB, 6.1), with losses at 831,972 70 -> 63 (5.3), complex128 on air at 883,652 91 -> 71 (5.1).  (8 lanes per row, which is 512 of them: 92, 61, 79; 32, 96 or 128
 // rows: 96, 66, 85; 113, 65, 86; 93, 65, 74; 2, 3 or 6 blocks in flight per lane: 95, 69, 73; 96, 68, 73; 93, 63, 89.)
 static constexpr int LOC_ROWS = 64, LOC_L = 4, LOC_MAX = 1024, LOC_CAND = 8192;
 static constexpr int LOC_LANES = LOC_ROWS * LOC_L;
