@@ -987,7 +987,9 @@ __global__ void __launch_bounds__(LOC ? LOC_LANES : 256) k_spmv_pk(int64_t ne, c
     }
     // fewer than 16 lanes make longer chains: complex64 sums in FP64 there.  Errors against 64 bits: with 16 lanes 7.3e-8 on
     // air and 7.4e-8 with losses, with 4 or 8 and sums in FP32 7.2e-8 and 7.7e-8, so 5.9e-8 and 6.5e-8, in the same time.
-    using S = std::conditional_t<(L < 16), double, R>;
+    // The Krylov steps, whose lanes are tuned, keep sums in FP32 (250,000 DOFs: 260 us a step, 266 with FP64): what they
+    // round goes into the FP64 residual that the refinement forms anew.
+    using S = std::conditional_t<(L < 16) && STD, double, R>;
     S s0r = 0, s0i = 0, s1r = 0, s1i = 0;
     if (fl & (ROW0 | ROW1)) {
         for (int32_t p = p0 + lane; p < p1; p += L * U) {
