@@ -27,9 +27,9 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per numeric assembly (k_tet_gram + k_assemble_staged) on the
 # 1,005,000-tet workload, from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE
 # runs of this benchmark (--sweep none --no-eigen --copy-calibration): FETCH (48,300 +
-# 1,064,000) KiB x 2 + WRITE (376,900 + 8,758,000) KiB x 1, the factors a 2 GiB
+# 1,106,000) KiB x 2 + WRITE (376,900 + 8,759,000) KiB x 1, the factors a 2 GiB
 # device-to-device copy in the same runs gives.
-ASSEMBLY_TRAFFIC_BYTES = ((48_300 + 1_064_000) * 2 + 376_900 + 8_758_000) * 1024
+ASSEMBLY_TRAFFIC_BYTES = ((48_300 + 1_106_000) * 2 + 376_900 + 8_759_000) * 1024
 # HBM bytes per launch of the sweep's complex64 product (k_spmv_pk) on the
 # posts box, from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs of this benchmark
 # (--spmv-kernel-only --copy-calibration): FETCH 252,900 KiB x 2 + WRITE 15,220 KiB x 1,

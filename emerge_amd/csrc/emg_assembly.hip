@@ -1203,7 +1203,7 @@ __device__ __forceinline__ int out_shift(int u, int n1, int u4, int d0, int d1, 
 //  * lane r accumulates entry chunk_ent[r] (entries by kind and descending incidence
 //    count, so the lanes of a wavefront run the same formulas a similar number of times);
 //  * the 2x2 blocks go through LDS into the order of the CSR rows and leave as whole lines.
-// What bounds it is the CSR writes, and the reads among them: at 1,005,000 tets (9.0 GB written, 2.2 read by the
+// What bounds it is the CSR writes, and the reads among them: at 1,005,000 tets (9.0 GB written, 2.3 read by the
 // counters: 4.8 TB/s, where a copy reaches 4.89) 2.31 ms, 2.22 without the incidence loop, 1.45 without the
 // stores.  (Nine tenths writes could go faster than a copy: the card fills at 6.82 TB/s and reads at 6.01, 1.7 ms for these
 // bytes, and a store-only kernel takes 1.45.)  What counts for them (2.89 ms before):
